@@ -67,7 +67,6 @@ static int ck_fields(int D, int *f)
 struct AdjArgs {
     const int *list;
     const int *cnt;
-    const int *cnt2;
     int cap;
     double *w;       // work arrays
     int64_t n;       // their stride
@@ -120,8 +119,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, i
     constexpr bool FP64 = sizeof(T) == 8;
     const int i = xcd_block() * BLOCK + threadIdx.x;
     if(i >= n) return;
-    const int cnt = a.cnt[i];
-    const int total = cnt + a.cnt2[i];
+    const int total = a.cnt[i];
     double xi[D];
     T vi[D], afi[D];
 #pragma unroll
@@ -138,7 +136,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, i
 
     Acc<T> xb[D], vb[D], hb, rhob, Ab, Bb, cb;
     for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, list_slot(kk, cnt, a.cap), a.cap)];
+        const int j = a.list[list_at(i, kk, a.cap)];
         double xj[D], dd[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
@@ -238,8 +236,7 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
 {
     const int i = xcd_block() * BLOCK + threadIdx.x;
     if(i >= n) return;
-    const int cnt = a.cnt[i];
-    const int total = cnt + a.cnt2[i];
+    const int total = a.cnt[i];
     double xi[D];
     T vi[D];
 #pragma unroll
@@ -251,7 +248,7 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
     const T ht = (T)h;
     Acc<T> rho_a, rhop_a, rhopp_a, Dv_a, Dvh_a, Rv_a[3], Rvh_a[3];
     for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, list_slot(kk, cnt, a.cap), a.cap)];
+        const int j = a.list[list_at(i, kk, a.cap)];
         double xj[D], dd[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
@@ -387,8 +384,7 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, int
 {
     const int i = xcd_block() * BLOCK + threadIdx.x;
     if(i >= n) return;
-    const int cnt = a.cnt[i];
-    const int total = cnt + a.cnt2[i];
+    const int total = a.cnt[i];
     double xi[D];
     T vi[D];
 #pragma unroll
@@ -401,7 +397,7 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, int
     const T srv_i[3] = {(T)W(a, W_SRV, i), (T)W(a, W_SRV + 1, i), (T)W(a, W_SRV + 2, i)};
     Acc<T> xb[D], vb[D];
     for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, list_slot(kk, cnt, a.cap), a.cap)];
+        const int j = a.list[list_at(i, kk, a.cap)];
         double xj[D], dd[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
@@ -485,7 +481,6 @@ int adjoint_step(Ctx &c, bool kick)
     AdjArgs a{};
     a.list = c.list;
     a.cnt = c.list_cnt;
-    a.cnt2 = c.list_cnt2;
     a.cap = c.cap;
     a.w = c.ro.work;
     a.n = c.ro.n;

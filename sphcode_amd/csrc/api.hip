@@ -40,7 +40,8 @@ __global__ void fill_int_kernel(int *p, int64_t n, int v)
 
 void reset_work(Ctx &c, int slot)
 {
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(BLOCK), 0, c.stream, c.work + NUM_XCD * slot, (int64_t)NUM_XCD, 0);
+    hipLaunchKernelGGL(fill_int_kernel, dim3(NUM_XCD * WORK_STRIDE / BLOCK), dim3(BLOCK), 0, c.stream, c.work + NUM_XCD * WORK_STRIDE * slot,
+                       (int64_t)NUM_XCD * WORK_STRIDE, 0);
 }
 
 __global__ void iota_kernel(int *p, int64_t n)
@@ -82,17 +83,17 @@ static void free_buffers(Ctx &c)
         fr(c.s.g[f]);
         c.alt.g[f] = nullptr;
     }
-    fr(c.list_rf);
     fr(c.s.id); fr(c.alt.id); fr(c.s.nb); fr(c.alt.nb);
     fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff);
-    fr(c.scan_tmp); fr(c.t.geo); fr(c.t.mom); fr(c.t.ks); fr(c.t.rng); fr(c.t.num_nodes);
+    fr(c.scan_tmp); fr(c.t.geo); fr(c.t.mom); fr(c.t.rng); fr(c.t.num_nodes);
     fr(c.lvl_nodes); fr(c.msum); fr(c.groups); fr(c.lvl);
     c.num_groups = nullptr;  // inside lvl
     fr(c.gnode); fr(c.gpart); fr(c.gacc); fr(c.leafhit); fr(c.leafcnt); fr(c.posrec); fr(c.pair_rec); fr(c.grad_rec);
     if(c.lvl_host) (void)hipHostFree(c.lvl_host);
     c.lvl_host = nullptr;
-    fr(c.list); fr(c.list_r); fr(c.list_cnt); fr(c.list_cnt2);
-    fr(c.tile_cand); fr(c.tile_mf); fr(c.tile_ma); fr(c.tile_nc); fr(c.ws_j); fr(c.ws_p);
+    fr(c.list); fr(c.list_cnt);
+    fr(c.srec); fr(c.boxes); fr(c.leaf_rad);
+    fr(c.tile_cand); fr(c.tile_ma); fr(c.tile_nc); fr(c.ws_j);
     c.tile_wcap = 0;
     c.tile_groups_cap = 0;
     c.ws_waves = 0;
@@ -129,12 +130,12 @@ static int alloc_buffers(Ctx &c, int64_t n)
     // adjoint (allocated then, ensure_lists)
     const size_t lsz = (size_t)np * (size_t)c.cap;
     SPHGPU_HIP(hipMalloc(&c.list_cnt, np * sizeof(int)));
-    SPHGPU_HIP(hipMalloc(&c.list_cnt2, np * sizeof(int)));
     // block partials: per 256 particles, or per block of four search groups
     // (up to one group per particle)
     const int64_t npart = std::max<int64_t>(grid_for(np), 1024) * 8 + np / 4 + 64;
     SPHGPU_HIP(hipMalloc(&c.partial, npart * sizeof(double)));
     int rc = tree_alloc(c);
+    if(!rc) rc = search_alloc_particles(c);
     if(rc) return rc;
     if(c.record) {
         SPHGPU_HIP(hipMalloc(&c.rec_gather, lsz * sizeof(int)));
@@ -219,9 +220,9 @@ static int launch_gravity_leaves(Ctx &c)
 // finds both the gather candidates and the symmetric pairs the force stage
 // needs (search_combined); the first call keeps the reference's initial
 // smoothing and separate searches.  With `walk` the gravity walk is started
-// on the second stream just before the search (after the search radii, the
-// cells' largest radius and the search's task counters are set, so that no
-// small kernel of the main stream waits for CUs behind the walk).
+// on the second stream just before the search (after the search radii, boxes
+// and task counters are set, so that no small kernel of the main stream
+// waits for CUs behind the walk).
 // Kernel-span marks of sphgpu_integrate's timers (ev[8 + k]).
 static void kmark(Ctx &c, int k)
 {
@@ -241,25 +242,13 @@ static int stage_pre(Ctx &c, bool walk = false)
         if((rc = search_gather(c, false))) return rc;
         kmark(c, 1);
     } else {
-        // the radii h_guess * ratio and the largest radius per cell (set by
-        // sphgpu_integrate's tree build)
-        if(!c.radius_ready && ((rc = search_guess(c)) || (rc = tree_set_kernel(c)))) return rc;
+        // the radii h_guess * ratio, and the search's records and boxes (set
+        // by sphgpu_integrate's tree build)
+        if(!c.radius_ready && (rc = search_guess(c))) return rc;
         c.radius_ready = false;
         reset_work(c, 0);  // the search's task counters
-        // The gravity walk (second stream) runs beside the search.  The
-        // search then takes two blocks of four waves per CU, leaving the
-        // other wave slots to the walk: the search waits on dependent loads
-        // and gains little from more waves, while the walk is bound by
-        // instruction issue (measured per mixed Evrard step of 2^20
-        // particles: 7.04 ms, against 7.16 ms with three blocks per CU and
-        // 7.35 ms with four).  Without gravity the best share depends on
-        // the dimension: the 2D KHI search (393,160 particles) takes
-        // 0.56 ms with two blocks per CU against 0.82 ms with eight (fewer
-        // waves keep their staging and tiles in L2), while the 3D Sedov
-        // step (2^24 particles) takes 65.8 ms with eight against 68.4 ms
-        // with four and 87.4 ms with two (its tree walks need the waves to
-        // hide their dependent loads).
-        const int bpc = (walk || c.D < 3) ? 2 : 8;
+        // the gravity walk (second stream) runs beside the search
+        const int bpc = search_blocks(c, walk);
         if(walk && (rc = launch_gravity_walk(c))) return rc;
         walk = false;
         kmark(c, 0);
@@ -267,10 +256,10 @@ static int stage_pre(Ctx &c, bool walk = false)
         kmark(c, 1);
     }
     if(c.record) {
-        if((rc = search_expand(c, c.rec_gather, c.rec_gather_cnt, nullptr, true))) return rc;
+        if((rc = search_expand(c, c.rec_gather, c.rec_gather_cnt, true))) return rc;
         c.have_gather = true;
     }
-    if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, c.list_cnt2, false))))
+    if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, false))))
         return rc;
     if(walk && (rc = launch_gravity_walk(c))) return rc;
     kmark(c, 2);
@@ -296,8 +285,7 @@ static int stage_pre(Ctx &c, bool walk = false)
         c.lists_symmetric = tr == c.trunc_seen && c.counters_host[C_OVERFLOW] == 0;
         c.trunc_seen = tr;
     }
-    if(c.lists_symmetric) return SPHGPU_OK;
-    return tree_set_kernel(c);  // BHTree::set_kernel (src/pre_interaction.cpp:166-168)
+    return SPHGPU_OK;
 }
 
 static int stage_force(Ctx &c)
@@ -305,7 +293,7 @@ static int stage_force(Ctx &c)
     int rc;
     if(!c.lists_symmetric) {
         if((rc = search_symmetric(c))) return rc;
-        if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, c.list_cnt2, false))))
+        if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, false))))
             return rc;
     }
     c.lists_symmetric = false;
@@ -320,13 +308,13 @@ static int stage_force(Ctx &c)
         const bool ok = tr == c.trunc_seen && c.counters_spec[C_OVERFLOW] == 0;
         c.trunc_seen = tr;
         if(!ok) {
-            // some h outgrew its search radius: the cells' largest h, a
-            // symmetric search, and the force pass again (it assigns acc and
+            // some h outgrew its search radius: a symmetric search with the
+            // leaves' largest h, and the force pass again (it assigns acc and
             // du/dt in full; the gravity pair pass started by the first one
             // is not started again)
             int (*hook)(Ctx &) = c.after_pack;
             c.after_pack = nullptr;
-            if((rc = tree_set_kernel(c)) || (rc = search_symmetric(c)) || (rc = force_compute(c))) {
+            if((rc = search_symmetric(c)) || (rc = force_compute(c))) {
                 c.after_pack = hook;
                 return rc;
             }
@@ -432,7 +420,7 @@ int sphgpu_create(const sphgpu_params *params, void **out)
        (e = hipHostMalloc(&c->counters_spec, NCOUNTERS * sizeof(int64_t), hipHostMallocDefault)) != hipSuccess ||
        // scalars and counters in one allocation (device and pinned host)
        (e = hipMalloc(&c->scal, SCAL_SPAN + NCOUNTER_ENTRIES * sizeof(int64_t))) != hipSuccess ||
-       (e = hipMalloc(&c->work, WORK_SLOTS * NUM_XCD * sizeof(int))) != hipSuccess ||
+       (e = hipMalloc(&c->work, WORK_SLOTS * NUM_XCD * WORK_STRIDE * sizeof(int))) != hipSuccess ||
        (e = hipHostMalloc(&c->scal_host, SCAL_SPAN + NCOUNTER_ENTRIES * sizeof(int64_t), hipHostMallocDefault)) != hipSuccess) {
         delete c;
         return hip_fail(e, "sphgpu_create");
@@ -546,7 +534,6 @@ int sphgpu_upload(void *ptr, const sphgpu_particles *h)
     }
     // list slots beyond n stay empty
     hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(c.cap_n)), dim3(BLOCK), 0, c.stream, c.list_cnt, c.cap_n, 0);
-    hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(c.cap_n)), dim3(BLOCK), 0, c.stream, c.list_cnt2, c.cap_n, 0);
     SPHGPU_HIP(hipGetLastError());
     SPHGPU_HIP(hipStreamSynchronize(c.stream));
     c.uploaded = true;

@@ -35,6 +35,19 @@ template <class T> __device__ __forceinline__ void stream_st(T *p, T v) { __buil
 // instructions take straight from the scalar registers.
 __device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
+// v with lane k's value replaced by the wave-uniform x (k wave-uniform).
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ int amdgcn_writelane(int x, int k, int v) __asm("llvm.amdgcn.writelane.i32");
+#endif
+__device__ __forceinline__ int write_lane(int x, int k, int v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return amdgcn_writelane(x, k, v);
+#else
+    return v;
+#endif
+}
+
 // 64 x 64 bit-matrix transpose across the wave: lane l returns the word
 // whose bit k is bit l of lane k's word.  Six butterfly stages: at block
 // size s, lanes l and l ^ s swap the s-bit blocks that lie across the
@@ -95,10 +108,15 @@ __device__ __forceinline__ int xcd_block() { return uniform(xcd_block((int)block
 
 // Persistent waves: tasks [0, ntask) are split into NUM_XCD contiguous
 // shares, and the waves of each XCD take the tasks of its share one at a
-// time from that XCD's counter (hardware deals block b to XCD b mod 8).
-// A wave whose share is used up moves on to the next XCD's share, so no
-// XCD idles while another still has tasks; after visiting all NUM_XCD
-// shares it gets -1.  Call with all lanes active.
+// time from that XCD's counter (hardware deals block b to XCD b mod 8).  A wave whose share is used up moves on to the next XCD's share, so no
+// XCD idles while another still has tasks; after visiting all NUM_XCD shares
+// it gets -1.  The counters lie WORK_STRIDE ints apart: updates of one cache
+// line by waves of all XCDs run one after the other at about 12 ns each,
+// and with the eight counters on one line those updates alone bounded the
+// search (2D, 393,160 particles: 327 us with 2,048 waves, 687 us with
+// 6,144).  For the same reason a share that a plain read shows to be used up
+// is passed without an update.  Call with all lanes active.
+constexpr int WORK_STRIDE = 64;
 struct TaskShare {
     int *work;
     int ntask;
@@ -117,8 +135,11 @@ struct TaskShare {
     __device__ __forceinline__ int next()
     {
         while(true) {
-            int t = 0;
-            if(wave_lane() == 0) t = atomicAdd(work + x, 1);
+            int *const c = work + x * WORK_STRIDE;
+            int t = hi - lo;
+            if(visited == 0 || lo + __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < hi) {
+                if(wave_lane() == 0) t = atomicAdd(c, 1);
+            }
             t = lo + __builtin_amdgcn_readfirstlane(t);
             if(t < hi) return t;
             if(++visited == NUM_XCD) return -1;
@@ -275,6 +296,17 @@ template <int D> __device__ __forceinline__ void min_image(const BoxDev &b, doub
         if(a1 <= a2 && a1 <= a3) r = d1;
         d[k] = r;
     }
+}
+
+// Axis k of the image of x that is nearest to c: x, x - L or x + L.
+__device__ __forceinline__ double near_image(const BoxDev &b, int k, double c, double x)
+{
+    const double d = c - x;
+    const double a1 = fabs(d), a2 = fabs(d + b.len[k]), a3 = fabs(d - b.len[k]);
+    double r = x + b.len[k];
+    if(a2 <= a3 && a2 <= a1) r = x - b.len[k];
+    if(a1 <= a2 && a1 <= a3) r = x;
+    return r;
 }
 
 // r_ij = x_i - x_j with minimum image, and its squared norm summed left to

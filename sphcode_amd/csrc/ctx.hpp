@@ -59,7 +59,6 @@ template <class T> struct Acc {
 struct TreeDev {
     double4 *geo;    // centre (x,y,z), edge
     double4 *mom;    // centre of mass (x,y,z), mass
-    double *ks;      // largest h in the subtree (BHNode::kernel_size)
     int4 *rng;       // first particle, end particle, skip (pre-order successor
                      // after the subtree), level | leaf << 8
     int *num_nodes;  // device scalar
@@ -95,6 +94,17 @@ template <> struct __align__(16) GravPart<double> {
     double x[3];
     double m, einv, pad;
 };
+
+// Neighbour search: bounding box of CHUNK key-consecutive particles (or of
+// 64 boxes of the level below), rounded outwards to FP32, with the largest
+// candidate radius in it.
+constexpr int CHUNK = 32;
+struct __align__(32) ChunkBox {
+    float lo[3], hi[3], r, pad;
+};
+static_assert(sizeof(ChunkBox) == 32, "ChunkBox is one 32-byte record");
+// flag in Ctx::tile_nc: the group's pairs take their own minimum images
+constexpr int GNC_WRAP = 1 << 30;
 
 // Neighbour records of the force pass, packed once per pass so that a pair
 // reads one FP64 (x, y, z, h) record for the cut and one record of the pair
@@ -159,10 +169,6 @@ __device__ __host__ __forceinline__ unsigned list_off(int k)
     return ((unsigned)k / LIST_C) * (WAVE * LIST_C) + (unsigned)k % LIST_C;
 }
 
-// Slot of entry kk of a list with `front` entries at the start and the rest
-// at the end (see Ctx::list).
-__device__ __forceinline__ int list_slot(int kk, int front, int cap) { return kk < front ? kk : cap - 1 - (kk - front); }
-
 // Device-side counters (int64), reduced per wave before the atomic.
 enum Counter : int {
     C_GATHER_PAIRS = 0, C_FORCE_PAIRS, C_GRAV_PP, C_GRAV_PN, C_NEWTON_FAIL, C_NEWTON_ITERS,
@@ -219,7 +225,7 @@ struct Ctx {
     hipEvent_t ev_flags = nullptr;
     bool speculate = false;      // sphgpu_integrate: assume symmetric lists, check after
     bool reorder_light = false;  // sphgpu_integrate's tree build: skip fields the step rewrites
-    bool radius_ready = false;   // that build set the search radii and the cells' largest radius
+    bool radius_ready = false;   // that build set the search radii, records and boxes
     bool stats_on = false;       // count the statistics (sphgpu_enable_stats)
     bool flags_pending = false;  // a copy behind ev_flags awaits its check
     int64_t *counters_spec = nullptr;  // pinned host copy for that check
@@ -269,39 +275,37 @@ struct Ctx {
     int *num_groups = nullptr;   // device scalar (an entry of lvl)
     int64_t group_cap = 0;
 
+    // neighbour search: position and squared candidate radius per particle,
+    // the boxes of its three levels (one after the other), and the symmetric
+    // search's candidate radii (the largest h of each particle's leaf)
+    double4 *srec = nullptr;
+    ChunkBox *boxes = nullptr;
+    double *leaf_rad = nullptr;
+
     // candidate tiles of the last neighbour search, per search group g
-    // (groups[g], at most 64 particles): tile_nc[g] candidates, stored in
-    // the group's slab of tile_wcap slots starting at g * tile_wcap.  With
-    // T = ceil(nc / 64) tiles, staging-order candidate c (the order of the
-    // reference's one-leaf-at-a-time walk) is lane k = c / T of tile
-    // t = c % T: tile t's 64 candidate indices sit at slab + 64 t (-1 past
-    // the end), and lane l of the group has the bit k of tile_mf[slab + 64 t
-    // + l] set when candidate (t, k) is in its front set (the gather
-    // candidates, r < R_l) and of tile_ma[...] when it is any of its hits
-    // (front or other symmetric candidates).  Consecutive candidates land in different
-    // tiles, so each tile samples the whole neighbourhood of the group and
-    // the group's lanes hold similar numbers of hits in every tile.
+    // (groups[g], at most 64 particles): tile_nc[g] candidates (with the flag
+    // GNC_WRAP), stored in the group's slab of tile_wcap slots starting at
+    // g * tile_wcap.  With T = ceil(nc / 64) tiles, staging-order candidate c
+    // (key order) is lane k = c / T of tile t = c % T: tile t's 64 candidate
+    // indices sit at slab + 64 t (-1 past the end), and lane l of the group
+    // has the bit k of tile_ma[slab + 64 t + l] set when candidate (t, k) is
+    // one of its hits.  Consecutive candidates land in different tiles, so
+    // each tile samples the whole neighbourhood of the group and the group's
+    // lanes hold similar numbers of hits in every tile.
     int *tile_cand = nullptr;
-    uint64_t *tile_mf = nullptr, *tile_ma = nullptr;
+    uint64_t *tile_ma = nullptr;
     int *tile_nc = nullptr;
     int tile_wcap = 0;             // slots per group (multiple of 64)
     int64_t tile_groups_cap = 0;   // groups the slabs are allocated for
-    int *ws_j = nullptr;           // search waves' staging of kept candidates:
-    double4 *ws_p = nullptr;       // index, and position with radius squared
+    int *ws_j = nullptr;           // search waves' staging of kept candidates
     int64_t ws_waves = 0;          // search waves the staging is allocated for
     int ngroups = 0;               // groups of the last tree (host copy)
 
     // neighbour lists (addressing: list_at), expanded from the tiles when
-    // the adjoint or the set record needs them (need_lists).  The first
-    // list_cnt[i] entries (k = 0, 1, ...) are the gather candidates
-    // (r < h_guess * ratio) with |r_ij| in list_r / list_rf; the combined
-    // search appends the remaining symmetric candidates from the other end
-    // (k = cap-1, cap-2, ..., list_cnt2[i] of them).
+    // the adjoint or the set record needs them (need_lists): particle i's
+    // hits are its first list_cnt[i] entries
     int *list = nullptr;
-    double *list_r = nullptr;  // |r_ij| of gather candidates (FP64 mode)
-    float *list_rf = nullptr;  // |r_ij| of gather candidates (mixed mode)
     int *list_cnt = nullptr;
-    int *list_cnt2 = nullptr;
     bool need_lists = false;       // expand every search's tiles into list
     bool lists_symmetric = false;  // the tiles hold every force pair
     int64_t trunc_seen = 0;        // truncation counter at the last check
@@ -374,14 +378,16 @@ BoxDev make_box(const Ctx &c);
 // tree.hip
 int tree_alloc(Ctx &c);
 int tree_build(Ctx &c);          // BHTree::make
-int tree_set_kernel(Ctx &c);     // BHTree::set_kernel
 // search.hip: candidate lists from the tree walk
 int search_gather(Ctx &c, bool initial);  // h from the density guess
 int search_symmetric(Ctx &c);
-int search_guess(Ctx &c);        // sml = h_guess * ratio
-int search_combined(Ctx &c, bool work_ready = false, int blocks_per_cu = 8);  // gather and symmetric candidates in one walk
+int search_guess(Ctx &c);        // sml = h_guess * ratio, search records and boxes
+int search_boxes(Ctx &c, const double *rad);  // search records and boxes with candidate radii rad
+int search_alloc_particles(Ctx &c);
+int search_combined(Ctx &c, bool work_ready, int blocks_per_cu);  // gather and symmetric candidates in one search
+int search_blocks(const Ctx &c, bool beside_walk);
 int search_alloc(Ctx &c);        // tile slabs for c.ngroups groups (after a tree build)
-int search_expand(Ctx &c, int *list, int *cnt, int *cnt2, bool front_only);  // tiles -> list_at lists
+int search_expand(Ctx &c, int *list, int *cnt, bool gather_only);  // tiles -> list_at lists
 // pre.hip
 int pre_initial(Ctx &c);         // initial_smoothing density
 int pre_compute(Ctx &c);         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients
@@ -398,7 +404,7 @@ int gravity_compute(Ctx &c);
 int gravity_walk(Ctx &c, hipStream_t st);
 int gravity_leaves(Ctx &c, hipStream_t st);
 int gravity_combine(Ctx &c, hipStream_t st);
-// Zero the NUM_XCD task counters at c.work + NUM_XCD * slot before a
+// Zero the NUM_XCD task counters (WORK_STRIDE ints apart) of a slot before a
 // persistent launch (slot 0: the neighbour search).
 void reset_work(Ctx &c, int slot);
 constexpr int WORK_SLOTS = 1;

@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         int used = 0;
         const ForceRec<T> *frec = (const ForceRec<T> *)a.frec;
         const size_t gbase = (size_t)grp * a.wcap;
-        const int nc = a.gnc[grp];
+        const int nc = a.gnc[grp] & ~GNC_WRAP;
         const int ntile = (nc + WAVE - 1) / WAVE;
         auto stage = [&](int tt) -> uint64_t {
             const size_t o = gbase + (size_t)tt * WAVE;

@@ -1,7 +1,8 @@
 // PreInteraction on the device, one wave per search group of at most 64
 // particles, one lane per particle, over the group's candidate tiles: each
 // tile's 64 neighbour records are staged once in LDS and every lane takes
-// the members of its gather candidate set (front hit mask) among them:
+// the members of its gather candidate set (the hits with r < R_i) among
+// them:
 //   SSPH  src/pre_interaction.cpp:39-169 (Newton :227-283)
 //   DISPH src/disph/d_pre_interaction.cpp:21-162 (Newton :174-230)
 //   GSPH  src/gsph/g_pre_interaction.cpp:27-144
@@ -32,7 +33,7 @@ struct PreArgs {
     const int2 *groups;
     int ngroups;
     const int *cand;      // candidate tiles (Ctx::tile_cand)
-    const uint64_t *mf;   // front (gather candidate) masks
+    const uint64_t *ma;   // hit masks
     const int *gnc;
     int wcap;
     double gamma;
@@ -134,7 +135,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
     const Kern ker(h);
     Acc<T> rho;
     const size_t gbase = (size_t)grp * a.wcap;
-    const int ntile = (a.gnc[grp] + WAVE - 1) / WAVE;
+    const int ntile = ((a.gnc[grp] & ~GNC_WRAP) + WAVE - 1) / WAVE;
     auto stage = [&](int tt) -> uint64_t {
         const size_t o = gbase + (size_t)tt * WAVE;
         const int jl = stream_ld(a.cand + o + lane);
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
             for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = s.f[F_X + k][jl];
             l_r[w][lane].m = fld<T>(s, F_MASS, jl);
         }
-        return valid ? stream_ld(a.mf + o + lane) : 0ull;
+        return valid ? stream_ld(a.ma + o + lane) : 0ull;
     };
     auto pair = [&](int kc) {
         double xj[D], d[D];
@@ -178,7 +179,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     const bool valid = have && i < gr.y;
     const int ii = valid ? i : gr.x;
     const size_t gbase = (size_t)(have ? grp : 0) * a.wcap;
-    const int ntile = have ? (a.gnc[grp] + WAVE - 1) / WAVE : 0;
+    const int ntile = have ? ((a.gnc[grp] & ~GNC_WRAP) + WAVE - 1) / WAVE : 0;
     const PreRec<T> *prec = (const PreRec<T> *)a.prec;
     double hvs = 1.7976931348623157e308;
     int64_t iters = 0, fails = 0, trunc = 0, pairs = 0;
@@ -188,6 +189,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
         const double mi = s.f[F_MASS][ii];
         const double Hs = s.f[F_SML][ii];  // search radius h_guess * ratio
+        const double Hs2 = Hs * Hs;
         double h = Hs;
         if(a.iterative) {
             // PreInteraction::newton_raphson, every lane on its own iterate;
@@ -207,7 +209,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     const size_t o = gbase + (size_t)tt * WAVE;
                     const int jl = stream_ld(a.cand + o + lane);
                     if(jl >= 0) l_pm[lane] = a.pm[jl];
-                    return done ? 0ull : stream_ld(a.mf + o + lane);
+                    return done ? 0ull : stream_ld(a.ma + o + lane);
                 };
                 auto npair = [&](int kc) {
                     const double4 pj = l_pm[kc];
@@ -215,8 +217,9 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     xj[0] = pj.x;
                     if constexpr(D > 1) xj[1] = pj.y;
                     if constexpr(D > 2) xj[2] = pj.z;
-                    const T r = gather_r<T>(sep2<D>(box, xi, xj, d));
-                    if(r < ht) {
+                    const double r2 = sep2<D>(box, xi, xj, d);
+                    const T r = gather_r<T>(r2);
+                    if(r < ht && r2 < Hs2) {
                         const T q = ker.q_of(r);
                         if constexpr(NUMBER) {
                             rho.add(ker.w(q));
@@ -268,15 +271,16 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) l_r[w][lane] = prec[jl];
             l_j[w][lane] = jl;
-            return valid ? stream_ld(a.mf + o + lane) : 0ull;
+            return valid ? stream_ld(a.ma + o + lane) : 0ull;
         };
         auto fpair = [&](int kc) {
             const PreRec<T> pj = l_r[w][kc];
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = pj.x[l];
-            const T r = gather_r<T>(sep2<D>(box, xi, xj, d));
-            if(!(r < ht)) return;
+            const double r2 = sep2<D>(box, xi, xj, d);
+            const T r = gather_r<T>(r2);
+            if(!(r < ht && r2 < Hs2)) return;
             const int j = l_j[w][kc];
             ++count;
             const T mj = pj.m;
@@ -342,7 +346,8 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = l_r[w][kc].x[l];
-            return gather_r<T>(sep2<D>(box, xi, xj, d)) < ht;
+            const double r2 = sep2<D>(box, xi, xj, d);
+            return gather_r<T>(r2) < ht && r2 < Hs2;
         };
         // refined in 3D except for GSPH (measured slower on the 3D Sedov
         // case), see tiles.hpp
@@ -452,7 +457,7 @@ static PreArgs make_args(Ctx &c)
     a.groups = c.groups;
     a.ngroups = c.ngroups;
     a.cand = c.tile_cand;
-    a.mf = c.tile_mf;
+    a.ma = c.tile_ma;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

@@ -1,77 +1,82 @@
 // Neighbour search (BHTree::neighbor_search, src/bhtree.cpp:114-126,
-// 234-270) for 64 Morton-consecutive particles per wave, in three phases:
+// 234-270) for the particles of one search group (at most 64
+// key-consecutive particles) per wave, in three phases:
 //
-//  1. Group walk.  The wave walks the pre-order tree once, 64 consecutive
-//     nodes at a time (one per lane, visited ones found by a prefix maximum
-//     of subtree ends), keeping every leaf whose cube can hold a
-//     candidate of any of its particles: per axis, the minimum-image
-//     distance between the group's box centre and the cell centre must not
-//     exceed group half-extent + edge/2 + H, with H the group's largest
-//     search radius (symmetric search: max(that, cell's largest h)).  This
-//     is implied by the reference's per-particle test, so no candidate of
-//     any lane is lost.  Leaves are collected into LDS.
-//  2. Candidate staging.  The collected leaves' particles (contiguous
-//     ranges in key order) are read 64 at a time with coalesced loads; those
-//     within the group's largest radius of the group box are kept, in
-//     staging order, in the wave's staging buffer.
+//  1. Boxes.  The key-sorted particles are cut into chunks of 32; every
+//     chunk has a bounding box with the largest candidate radius in it, 64
+//     chunks make a box of the second level and 64 of those one of the
+//     third.  The wave tests 64 boxes at a time, one per lane, against the
+//     group's own box, from the third level down, and keeps the chunks
+//     whose box lies within reach: (distance of the two boxes)^2 <= H^2,
+//     H the larger of the group's largest search radius and (symmetric
+//     search) the box's largest radius.  Every pair that the reference's
+//     test accepts is closer than that, so no candidate of any lane is lost.
+//  2. Candidate staging.  The kept chunks' particles are read two chunks at
+//     a time with coalesced loads; those within reach of the group box by
+//     their own radius are kept, in key order, in the wave's staging buffer.
 //  3. Candidate tiles.  With nc kept candidates and T = ceil(nc / 64)
 //     tiles, tile t takes candidates t, t + T, t + 2T, ... (lane k of the
-//     tile holds candidate t + kT).  Every lane applies the reference's
-//     leaf test to each of the tile's candidates: |x_i - x_j|^2 < H_i^2
-//     with H_i = h_guess * kernel_ratio (gather, src/pre_interaction.cpp:
-//     61-70) or max(h_i, leaf's largest h) (symmetric, src/bhtree.cpp:237,
-//     256), into a 64-bit hit mask, written with the tile's candidate
-//     indices to the group's slab (layout: Ctx::tile_cand).
+//     tile holds candidate t + kT).  The reference's leaf test
+//     |x_i - x_j|^2 < H_i^2 with H_i = h_guess * kernel_ratio (gather,
+//     src/pre_interaction.cpp:61-70) or max(h_i, leaf's largest h)
+//     (symmetric, src/bhtree.cpp:237, 256) is applied by every lane to its
+//     candidate for one particle i of the group after the other.  The
+//     compare's result is then particle i's 64-bit hit mask of the tile; it
+//     is moved to lane i and written with the tile's candidate indices to
+//     the group's slab (layout: Ctx::tile_cand).
+//
+// What bounds it: vector issue in phase 3 (8 FP64 operations, 1-2 compares
+// and 2 lane writes per particle and tile; vector ALUs 84 % busy on 2^21
+// particles in 3D), and the latency of the dependent box and candidate loads
+// in the first two.  Particle i's record is read with one scalar load for
+// two tiles, so a test costs no LDS read and no instruction that builds
+// bits, and the loop runs over the group's particles (47 on average in 3D)
+// with every lane busy, not over 64 candidates with a lane per particle.
+// The boxes replace a walk of the octree: their cost does not depend on
+// leafParticleNumber, where a tree with one particle per leaf has about 1.4
+// nodes per candidate to visit.  Combined search, before and after: 2D KHI,
+// 393,160 particles, 515 -> 128 us; 3D periodic, 2^21 particles, leaf 1,
+// 3,480 -> 800 us; Evrard, 2^20 particles, leaf 32, alone 1,440 -> 780 us
+// (vector instructions 4.0e8 -> 2.5e8).
 //
 // The sets are the reference's; the reference then sorts each list by
 // distance (src/bhtree.cpp:120-124) and stops at the first r >= h, whereas
 // the pair passes here test r < h on the unsorted set -- the same set.
 //
-// The combined search (split mode) walks with sml = the gather radius and
-// the cells' largest gather radius, keeps pairs with r < max(sml_i, sml_j),
-// and marks those with r^2 < sml_i^2 (the gather candidates) in the front
-// mask and the rest in the back mask, so that one walk serves both the
-// pre-interaction and the force stage.
+// The combined search takes H_ij = max(R_i, R_j) with the gather radii R,
+// so that one search serves both the pre-interaction (which keeps the pairs
+// with r < R_i) and the force stage.
 #include "ctx.hpp"
 
 #include <type_traits>
 
 namespace sphgpu {
 
+// What a hit is: r < R_i (gather), r < max(R_i, R_j) (combined), or
+// r < max(h_i, largest h of j's leaf) (symmetric).
+enum SearchMode : int { M_GATHER, M_COMBINED, M_SYMMETRIC };
+
 struct SearchArgs {
+    int n;
+    const double4 *srec;  // position and squared candidate radius per particle
+    const double *own;    // M_SYMMETRIC: h per particle (otherwise srec's radius)
+    const ChunkBox *lev[3];
+    int cnt[3];           // boxes per level
+    const int2 *groups;
+    const int *num_groups;
     int *cand;           // group slabs of candidate tiles (Ctx::tile_cand)
-    uint64_t *mf, *ma;   // front / all hit masks per (tile, lane)
-    int *gnc;            // candidates per group
+    uint64_t *ma;        // hit masks per (tile, lane)
+    int *gnc;            // candidates per group, with GNC_WRAP
     int wcap;            // slots per group slab and per staging buffer
     int *ws_j;           // staging buffers, one per persistent wave
-    double4 *ws_p;       // the staged candidate's position and (IJ) radius squared
-    int split;           // symmetric search that also marks the gather set:
-                         // r < sml_i in the front mask, the rest in the back
     int cap;             // per-particle capacity (the reference's list size)
-    int guess;           // 1: set sml = h_guess * ratio first
-    double ratio;
-    double nngb;
     int64_t *counters;
     int stats;            // add to the statistics counters (errors are always counted)
     int *work;           // per-XCD task counters, zeroed before the launch
 };
 
 constexpr int SW = BLOCK / WAVE;  // waves per block
-constexpr int LEAFCAP = 128;      // leaves collected per flush
-
-// Wave-wide exclusive prefix sum.
-__device__ __forceinline__ int wave_exclusive_scan(int v, int &total)
-{
-    const int lane = wave_lane();
-    int x = v;
-#pragma unroll
-    for(int off = 1; off < WAVE; off <<= 1) {
-        const int y = __shfl_up(x, off, WAVE);
-        if(lane >= off) x += y;
-    }
-    total = __shfl(x, WAVE - 1, WAVE);
-    return x - v;
-}
+constexpr int CHUNKCAP = 256;     // kept chunks collected per flush
 
 // Minimum-image separation of one axis (include/periodic.hpp:34-59).
 __device__ __forceinline__ double min_image1(const BoxDev &b, int k, double d)
@@ -85,324 +90,266 @@ __device__ __forceinline__ double min_image1(const BoxDev &b, int k, double d)
     return r;
 }
 
+// Does box b come within reach of the group's box (centre gc, half extents
+// ge, largest radius squared hmax2)?
 template <int D, bool IJ>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_SEARCH))) search_kernel(State s, TreeDev t, BoxDev box, const int2 *groups, const int *num_groups,
-                                                      SearchArgs a)
+__device__ __forceinline__ bool box_near(const BoxDev &box, const ChunkBox &b, const double gc[D], const double ge[D], double hmax2)
 {
-    __shared__ int l_begin[SW][LEAFCAP];
-    __shared__ int l_pre[SW][LEAFCAP + 1];
-    __shared__ double l_ks[SW][LEAFCAP];
-    // the tile's candidates: position and (IJ) radius squared
-    __shared__ double4 c_p[SW][WAVE];
+    double d2 = 0.0;
+#pragma unroll
+    for(int k = 0; k < D; ++k) {
+        const double c = 0.5 * ((double)b.lo[k] + (double)b.hi[k]), e = 0.5 * ((double)b.hi[k] - (double)b.lo[k]);
+        const double ex = fabs(min_image1(box, k, gc[k] - c)) - (ge[k] + e);
+        d2 += ex > 0.0 ? ex * ex : 0.0;
+    }
+    double H2 = hmax2;
+    if constexpr(IJ) {
+        const double r2 = (double)b.r * (double)b.r;
+        H2 = r2 > H2 ? r2 : H2;
+    }
+    return d2 <= H2 * (1.0 + 1e-6);
+}
+
+// A particle's search record through the scalar cache (i wave-uniform; the
+// records are not written by this kernel).
+__device__ __forceinline__ double4 srec_at(const double4 *p, int i) { return load_ro(p + i); }
+
+template <int D, int MODE>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_SEARCH))) search_kernel(BoxDev box, SearchArgs a)
+{
+    constexpr bool IJ = MODE != M_GATHER;
+    __shared__ int l_chunk[SW][CHUNKCAP];
 
     const int w = uniform(threadIdx.x / WAVE);
     const int lane = wave_lane();
-    const int ngroups = uniform(*num_groups);
+    const int ngroups = uniform(*a.num_groups);
+    // this wave's staging buffer
+    const size_t wbase = (size_t)(blockIdx.x * SW + w) * (size_t)a.wcap;
     // persistent waves: groups are taken one at a time from this XCD's
     // contiguous share of the Morton curve
     TaskShare share(a.work, ngroups);
     for(int grp = share.next(); grp >= 0; grp = share.next()) {
-    const int2 gr = make_int2(uniform(groups[grp].x), uniform(groups[grp].y));
-    const int i = gr.x + lane;
-    const bool valid = i < gr.y;
-
-    double xi[D], h = 0.0;
-#pragma unroll
-    for(int k = 0; k < D; ++k) xi[k] = valid ? s.f[F_X + k][i] : 0.0;
-    if(valid) {
-        if(a.guess) {
-            // p_i.sml = (N_ngb m / (rho A))^(1/D) * ratio (src/pre_interaction.cpp:61-64)
-            const double m = s.f[F_MASS][i];
-            const double rho = s.f[F_DENS][i];
-            h = sml_guess<D>(m, rho, a.nngb, a.ratio);
-            s.f[F_SML][i] = h;
-        } else {
-            h = s.f[F_SML][i];
-        }
-    }
-    const double h2_own = h * h;
-    const int64_t h2_bits = __double_as_longlong(h2_own);
-    // this wave's staging buffer, and the group's slab of tiles
-    const size_t wbase = (size_t)(blockIdx.x * SW + w) * (size_t)a.wcap;
+    const int2 gr = make_int2(uniform(a.groups[grp].x), uniform(a.groups[grp].y));
+    const int cnt = gr.y - gr.x;
+    const bool valid = lane < cnt;
     const size_t gbase = (size_t)grp * (size_t)a.wcap;
 
-    // group box: centre, half extent, largest radius (wave-uniform)
-    double gc[D], ge[D];
+    // group box: centre, half extent, largest radius squared (wave-uniform)
+    double gc[D], ge[D], hmax2;
+    {
+        const int i = gr.x + (valid ? lane : 0);
+        const double4 me = a.srec[i];
+        const double x[3] = {me.x, me.y, me.z};
 #pragma unroll
-    for(int k = 0; k < D; ++k) {
-        const double lo = wave_minv(valid ? xi[k] : 1.7976931348623157e308);
-        const double hi = wave_maxv(valid ? xi[k] : -1.7976931348623157e308);
-        gc[k] = uniform_d(0.5 * (lo + hi));
-        ge[k] = uniform_d(0.5 * (hi - lo) * (1.0 + 1e-12) + 1e-300);
-    }
-    const double hmax = uniform_d(wave_maxv(valid ? h : 0.0));
-
-    int count = 0, count2 = 0;  // hits (front / back)
-    int nkept = 0;               // staged candidates (may pass wcap: overflow)
-
-    const int total = uniform(*t.num_nodes);
-    int node = 0;
-    int64_t visited = 0, tested = 0;
-    while(node < total) {
-        // ---- phase 1: collect leaves, 64 consecutive pre-order nodes per
-        // window.  A node is visited iff every ancestor of it is opened
-        // (overlapping and internal).  Within a window the window's first
-        // node is visited, and a later node v is visited iff no earlier
-        // node of the window that is not opened has its subtree span
-        // [u, skip(u)) over v: v >= the exclusive prefix maximum of skip
-        // over the window's not-opened nodes.  The next window starts at
-        // the larger of the window's end and that maximum at the last lane.
-        // Leaves are kept in pre-order, as the one-node-at-a-time walk
-        // would keep them.
-        int nleaf = 0;
-        while(node < total && nleaf <= LEAFCAP - WAVE) {
-            node = uniform(node);
-            const int v = node + lane;
-            const bool in = v < total;
-            int closed_skip = 0;
-            bool leafhit = false;
-            int4 r = make_int4(0, 0, 0, 0);
-            double ks = 0.0;
-            if(in) {
-                const double4 g = t.geo[v];
-                r = t.rng[v];
-                double H = hmax;
-                if constexpr(IJ) {
-                    ks = t.ks[v];
-                    H = ks > H ? ks : H;
-                }
-                const double reach = g.w * 0.5 + H;
-                const double gcen[3] = {g.x, g.y, g.z};
-                bool overlap = true;
-#pragma unroll
-                for(int k = 0; k < D; ++k) {
-                    const double dd = min_image1(box, k, gc[k] - gcen[k]);
-                    overlap = overlap && fabs(dd) <= (ge[k] + reach) * (1.0 + 1e-12);
-                }
-                const bool leaf = (r.w & 256) != 0;
-                const int skip = r.z > v ? r.z : v + 1;
-                closed_skip = overlap && !leaf ? 0 : skip;
-                leafhit = overlap && leaf;
-            }
-            const int incl = wave_incl_max_nonneg(closed_skip);
-            const int excl = wave_shr1(incl);
-            const bool vis = in && v >= excl;
-            visited += __popcll(ballot(vis));
-            const bool hit = vis && leafhit;
-            const uint64_t hits = ballot(hit);
-            if(hit) {
-                const int at = nleaf + __popcll(hits & ((1ull << lane) - 1ull));
-                l_begin[w][at] = r.x;
-                l_pre[w][at] = r.y - r.x;
-                l_ks[w][at] = ks;
-            }
-            nleaf += uniform(__popcll(hits));
-            const int far = __builtin_amdgcn_readlane(incl, WAVE - 1);
-            node = node + WAVE > far ? node + WAVE : far;
+        for(int k = 0; k < D; ++k) {
+            const double lo = wave_minv(x[k]);
+            const double hi = wave_maxv(x[k]);
+            gc[k] = uniform_d(0.5 * (lo + hi));
+            ge[k] = uniform_d(0.5 * (hi - lo) * (1.0 + 1e-12) + 1e-300);
         }
-        wave_lds_sync();
-        // prefix of leaf sizes (each lane owns two slots)
-        int c0 = 0, c1 = 0;
-        if(2 * lane < nleaf) c0 = l_pre[w][2 * lane];
-        if(2 * lane + 1 < nleaf) c1 = l_pre[w][2 * lane + 1];
-        int ncand = 0;
-        const int ex = wave_exclusive_scan(c0 + c1, ncand);
-        ncand = uniform(ncand);
-        wave_lds_sync();
-        if(2 * lane < nleaf) l_pre[w][2 * lane] = ex;
-        if(2 * lane + 1 < nleaf) l_pre[w][2 * lane + 1] = ex + c0;
-        if(lane == 0) l_pre[w][nleaf] = ncand;
-        wave_lds_sync();
+        double h2 = me.w;
+        if constexpr(MODE == M_SYMMETRIC) h2 = a.own[i] * a.own[i];
+        hmax2 = uniform_d(wave_maxv(h2));
+    }
 
-        // ---- phase 2: stage the collected leaves' particles, 64 at a time.
-        // The next tile's candidates are located and their positions loaded
-        // before the current tile is tested, so the loads overlap the work.
-        int lc = 0;  // last leaf starting at or before the located tile
-        auto locate = [&](int tb, int &lo_, int &j_, double xj_[D], double &lim_, bool &has_) {
-            // each lane's candidate f = tb + lane; its leaf is the last leaf
-            // starting at or before f, found among the few leaves that start
-            // inside the tile
-            const int f = tb + lane;
-            int lo = lc, nx = lc;
-            for(int L = lc + 1; L < nleaf; ++L) {
-                const int st = uniform(l_pre[w][L]);
-                if(st > tb + WAVE) break;
-                nx = L;
-                lo = f >= st ? L : lo;
-            }
-            lc = nx;
-            has_ = f < ncand;
-            lo_ = lo;
-            j_ = has_ ? l_begin[w][lo] + (f - l_pre[w][lo]) : 0;
-            if(has_) {
-#pragma unroll
-                for(int k = 0; k < D; ++k) xj_[k] = s.f[F_X + k][j_];
-                // split mode: r < max(sml_i, sml_j) (each radius bounds that
-                // particle's final h unless truncated); otherwise the
-                // reference's r < max(h_i, leaf's largest h).  As squares:
-                // max(a, b)^2 == max(a^2, b^2) for a, b >= 0.
-                if constexpr(IJ) lim_ = a.split ? s.f[F_SML][j_] : l_ks[w][lo];
-            }
+    int nkept = 0;               // staged candidates (may pass wcap: overflow)
+    double reach2 = hmax2;       // largest squared radius among the kept candidates (per lane)
+    int64_t visited = 0, tested = 0;
+
+    // ---- phase 2: stage the particles of the collected chunks, two chunks
+    // at a time; the next two are loaded before the current ones are tested
+    int nchunk = 0;
+    auto flush = [&]() {
+        wave_lds_sync();
+        auto fetch = [&](int p, int &j, double4 &q) {
+            const int s = p + (lane >> 5);
+            j = s < nchunk ? l_chunk[w][s] * CHUNK + (lane & (CHUNK - 1)) : a.n;
+            if(j < a.n) q = a.srec[j];
         };
-        int c_lo = 0, c_jj = 0;
-        double c_xj[D], c_lm = 0.0;
-        bool c_has = false;
-        if(ncand > 0) locate(0, c_lo, c_jj, c_xj, c_lm, c_has);
-        for(int tb = 0; tb < ncand; tb += WAVE) {
-            int n_lo = 0, n_jj = 0;
-            double n_xj[D], n_lm = 0.0;
-            bool n_has = false;
-            if(tb + WAVE < ncand) locate(tb + WAVE, n_lo, n_jj, n_xj, n_lm, n_has);
-            // keep a candidate only if it lies within the group's largest
-            // radius of the group box (the box contains every x_i, so each
-            // lane's own test implies this)
+        int c_j = a.n;
+        double4 c_q = make_double4(0.0, 0.0, 0.0, 0.0);
+        fetch(0, c_j, c_q);
+        for(int p = 0; p < nchunk; p += 2) {
+            int n_j = a.n;
+            double4 n_q = make_double4(0.0, 0.0, 0.0, 0.0);
+            if(p + 2 < nchunk) fetch(p + 2, n_j, n_q);
             bool keep = false;
-            if(c_has) {
+            if(c_j < a.n) {
+                // keep a candidate only if it lies within reach of the group
+                // box (the box contains every x_i, so each lane's own test
+                // implies this)
+                const double x[3] = {c_q.x, c_q.y, c_q.z};
                 double d2b = 0.0;
 #pragma unroll
                 for(int k = 0; k < D; ++k) {
-                    const double ex = fabs(min_image1(box, k, c_xj[k] - gc[k])) - ge[k];
+                    const double ex = fabs(min_image1(box, k, x[k] - gc[k])) - ge[k];
                     d2b += ex > 0.0 ? ex * ex : 0.0;
                 }
-                double Hc = hmax;
-                if constexpr(IJ) {
-                    const double ksj = l_ks[w][c_lo];
-                    Hc = ksj > Hc ? ksj : Hc;
-                }
-                keep = d2b <= Hc * Hc * (1.0 + 1e-9);
+                double H2 = hmax2;
+                if constexpr(IJ) H2 = c_q.w > H2 ? c_q.w : H2;
+                keep = d2b <= H2 * (1.0 + 1e-9);
+                if constexpr(IJ) reach2 = keep && H2 > reach2 ? H2 : reach2;
             }
             const uint64_t kept = ballot(keep);
             if(keep) {
                 const int at = nkept + __popcll(kept & ((1ull << lane) - 1ull));
-                if(at < a.wcap) {
-                    a.ws_j[wbase + at] = c_jj;
-                    // the position and radius are staged only where phase 3
-                    // cannot read them back from the particle (the leaf's
-                    // largest h of an unsplit symmetric search)
-                    if(IJ && !a.split) a.ws_p[wbase + at] = make_double4(c_xj[0], D > 1 ? c_xj[1] : 0.0, D > 2 ? c_xj[2] : 0.0, c_lm * c_lm);
-                }
+                if(at < a.wcap) a.ws_j[wbase + at] = c_j;
             }
             const int m = uniform(__popcll(kept));
             nkept += m;
             tested += m;
-            c_lo = n_lo;
-            c_jj = n_jj;
-#pragma unroll
-            for(int k = 0; k < D; ++k) c_xj[k] = n_xj[k];
-            c_lm = n_lm;
-            c_has = n_has;
+            c_j = n_j;
+            c_q = n_q;
         }
-        wave_lds_sync();  // leaf tables are rewritten by the next batch
+        nchunk = 0;
+        wave_lds_sync();
+    };
+
+    // ---- phase 1: boxes near the group's box, 64 per window
+    auto window = [&](int level, int base) -> uint64_t {
+        const int v = base + lane;
+        bool hit = false;
+        if(v < a.cnt[level]) hit = box_near<D, IJ>(box, a.lev[level][v], gc, ge, hmax2);
+        visited += min(WAVE, a.cnt[level] - base);
+        return ballot(hit);
+    };
+    for(int b3 = 0; b3 < a.cnt[2]; b3 += WAVE) {
+        // a level with one box is not tested
+        uint64_t m3 = a.cnt[2] > 1 ? window(2, b3) : 1ull;
+        while(m3) {
+            const int k3 = (int)__builtin_ctzll(m3);
+            m3 &= m3 - 1ull;
+            const int b2 = (b3 + k3) * WAVE;
+            uint64_t m2 = a.cnt[1] > 1 ? window(1, b2) : 1ull;
+            while(m2) {
+                const int k2 = (int)__builtin_ctzll(m2);
+                m2 &= m2 - 1ull;
+                const int b1 = (b2 + k2) * WAVE;
+                const uint64_t m1 = window(0, b1);
+                if((m1 >> lane) & 1) l_chunk[w][nchunk + __popcll(m1 & ((1ull << lane) - 1ull))] = b1 + lane;
+                nchunk += uniform(__popcll(m1));
+                if(nchunk > CHUNKCAP - WAVE) flush();
+            }
+        }
     }
+    if(nchunk) flush();
 
     // ---- phase 3: strided tiles of the kept candidates, the next tile's
     // records loaded while the current one is tested
     const int nc = nkept < a.wcap ? nkept : a.wcap;
     const int T = (nc + WAVE - 1) / WAVE;
+    // Periodic box: every lane's minimum image of a candidate that can be a
+    // hit is the one nearest to the group's centre, if the group and its
+    // reach span less than half the box; the candidate is then moved there
+    // once.  Otherwise (the flag GNC_WRAP, also read by the pair passes)
+    // every pair takes its own minimum image.
+    bool wrap = false;
+    if(box.on) {
+        const double H = sqrt(uniform_d(wave_maxv(reach2)));
+#pragma unroll
+        for(int k = 0; k < D; ++k) wrap = wrap || !(2.0 * ge[k] + H < 0.499 * box.len[k]);
+    }
     // the staging writes of all lanes before their reads by other lanes
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    int p_j = -1;
-    double4 p_p = make_double4(0.0, 0.0, 0.0, 0.0);
-    // a kept candidate's position and radius squared: staged, or read back
-    // from the particle arrays (mostly still in L2 from phase 2)
-    const bool staged_p = IJ && !a.split;
-    auto fetch_p = [&](int j) -> double4 {
-        double4 q;
-        q.x = s.f[F_X][j];
-        q.y = D > 1 ? s.f[F_X + 1][j] : 0.0;
-        q.z = D > 2 ? s.f[F_X + 2][j] : 0.0;
-        if constexpr(IJ) {
-            const double l = s.f[F_SML][j];
-            q.w = l * l;
-        } else {
-            q.w = 0.0;
+    auto fetch_c = [&](int c, int &j, double4 &q) {
+        j = -1;
+        // past the tile's end: at no finite distance
+        q = make_double4(1e200, 1e200, 1e200, 0.0);
+        if(c < nc) {
+            j = a.ws_j[wbase + c];
+            q = a.srec[j];
         }
-        return q;
     };
-    if(T > 0 && lane * T < nc) {
-        p_j = a.ws_j[wbase + lane * T];
-        p_p = staged_p ? a.ws_p[wbase + lane * T] : fetch_p(p_j);
-    }
-    for(int tt = 0; tt < T; ++tt) {
-        const int m = (nc - tt + T - 1) / T;  // candidates of this tile (a prefix of its lanes)
-        const int j = p_j;
-        if(j >= 0) c_p[w][lane] = p_p;
-        stream_st(a.cand + gbase + (size_t)tt * WAVE + lane, j);
-        // next tile's records
-        const int cn = tt + 1 + lane * T;
-        p_j = -1;
-        if(tt + 1 < T && cn < nc) {
-            p_j = a.ws_j[wbase + cn];
-            p_p = staged_p ? a.ws_p[wbase + cn] : fetch_p(p_j);
+    int count = 0;  // hits of particle `lane`
+    // V consecutive tiles from tt on, the candidates' records in p_j and p_q
+    int p_j[2] = {-1, -1};
+    double4 p_q[2];
+    auto tiles = [&](int tt, auto pairwise, auto width) {
+        constexpr bool PER = decltype(pairwise)::value;
+        constexpr int V = decltype(width)::value;
+        constexpr int U = PER ? 1 : 4;  // particles per pass
+        int j[V];
+        double x[V][3], cw[V];
+#pragma unroll
+        for(int v = 0; v < V; ++v) {
+            j[v] = p_j[v];
+            x[v][0] = p_q[v].x;
+            x[v][1] = p_q[v].y;
+            x[v][2] = p_q[v].z;
+            cw[v] = p_q[v].w;
+            stream_st(a.cand + gbase + (size_t)(tt + v) * WAVE + lane, j[v]);
+            if(!PER && box.on && j[v] >= 0) {
+#pragma unroll
+                for(int k = 0; k < D; ++k) x[v][k] = near_image(box, k, gc[k], x[v][k]);
+            }
         }
-        wave_lds_sync();
-        // every lane tests every candidate of the tile (uniform loop,
-        // broadcast LDS reads) into a hit mask, and a mask of the hits
-        // inside its own radius (the gather entries of a split search;
-        // every hit otherwise).  Two candidates per pass, their records
-        // read together (one with periodic boundaries); the slots past the
-        // tile's m candidates hold stale records, whose bits are cleared.
-        // (Four per pass spilled registers at this kernel's budget and was
-        // no faster.)
-        uint64_t mine = 0, mfront = 0;
-        if(valid) {
-            auto sweep = [&](auto periodic) {
+        // the next tiles' records, while these are tested
+        if(tt + V < T) fetch_c(tt + V + lane * T, p_j[0], p_q[0]);
+        if(V > 1 && tt + V + 1 < T) fetch_c(tt + V + 1 + lane * T, p_j[1], p_q[1]);
+        // particle after particle: the lanes' compares are its hit mask
+        int lo[V] = {}, hi[V] = {};
+        for(int i0 = 0; i0 < cnt; i0 += U) {
 #pragma clang fp contract(off)
-                constexpr bool PER = decltype(periodic)::value;
-                constexpr int U = PER ? 1 : 2;
-                uint64_t hm = 0, fm = 0;
-                for(int cc = 0; cc < m; cc += U) {
-                    double4 q[U];
+            // records past the group's last particle (srec has a spare
+            // tile of them) fill lanes that are masked off below
+            double4 q[U];
+            double o2[U];
 #pragma unroll
-                    for(int u = 0; u < U; ++u) q[u] = c_p[w][cc + u];
-                    uint32_t hn = 0, fn = 0;
+            for(int u = 0; u < U; ++u) {
+                q[u] = srec_at(a.srec, gr.x + i0 + u);
+                o2[u] = q[u].w;
+            }
+            if constexpr(MODE == M_SYMMETRIC) {
 #pragma unroll
-                    for(int u = 0; u < U; ++u) {
-                        double d[D];
-                        d[0] = xi[0] - q[u].x;
-                        if constexpr(D > 1) d[1] = xi[1] - q[u].y;
-                        if constexpr(D > 2) d[2] = xi[2] - q[u].z;
-                        if constexpr(PER) min_image<D>(box, d);
-                        double r2 = d[0] * d[0];
-#pragma unroll
-                        for(int k = 1; k < D; ++k) r2 = r2 + d[k] * d[k];
-                        // r2 < max(h_i^2, kl^2) as two tests; all three are
-                        // non-negative, so their bit patterns order as integers
-                        const int64_t rb = __double_as_longlong(r2);
-                        const bool f = rb < h2_bits;
-                        bool hh = f;
-                        if constexpr(IJ) hh = f | (rb < __double_as_longlong(q[u].w));
-                        hn |= (uint32_t)hh << u;
-                        fn |= (uint32_t)f << u;
-                    }
-                    hm |= (uint64_t)hn << cc;
-                    fm |= (uint64_t)fn << cc;
+                for(int u = 0; u < U; ++u) {
+                    const double h = a.own[gr.x + min(i0 + u, cnt - 1)];
+                    o2[u] = h * h;
                 }
-                const uint64_t live = m >= WAVE ? ~0ull : (1ull << m) - 1ull;
-                mine = hm & live;
-                mfront = a.split ? fm & live : mine;
-            };
-            if(box.on) sweep(std::true_type{});
-            else sweep(std::false_type{});
+            }
+#pragma unroll
+            for(int u = 0; u < U; ++u) {
+#pragma unroll
+                for(int v = 0; v < V; ++v) {
+                    double d[D];
+                    d[0] = q[u].x - x[v][0];
+                    if constexpr(D > 1) d[1] = q[u].y - x[v][1];
+                    if constexpr(D > 2) d[2] = q[u].z - x[v][2];
+                    if constexpr(PER) min_image<D>(box, d);
+                    double r2 = d[0] * d[0];
+#pragma unroll
+                    for(int k = 1; k < D; ++k) r2 = r2 + d[k] * d[k];
+                    uint64_t m = ballot(r2 < o2[u]);
+                    if constexpr(IJ) m |= ballot(r2 < cw[v]);
+                    lo[v] = write_lane((int)(uint32_t)m, i0 + u, lo[v]);
+                    hi[v] = write_lane((int)(uint32_t)(m >> 32), i0 + u, hi[v]);
+                }
+            }
         }
-        const size_t mo = gbase + (size_t)tt * WAVE + lane;
-        stream_st(a.mf + mo, mfront);
-        stream_st(a.ma + mo, mine);
-        count += __popcll(mfront);
-        count2 += __popcll(mine & ~mfront);
-        wave_lds_sync();
+#pragma unroll
+        for(int v = 0; v < V; ++v) {
+            uint64_t mine = valid ? ((uint64_t)(uint32_t)hi[v] << 32) | (uint32_t)lo[v] : 0ull;
+            if constexpr(PER) mine &= ballot(j[v] >= 0);  // a wrapped distance is always finite
+            stream_st(a.ma + gbase + (size_t)(tt + v) * WAVE + lane, mine);
+            count += __popcll(mine);
+        }
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if(T > 0) fetch_c(lane * T, p_j[0], p_q[0]);
+    int tt = 0;
+    if(wrap) {
+        for(; tt < T; ++tt) tiles(tt, std::true_type{}, One{});
+    } else {
+        if(T > 1) fetch_c(1 + lane * T, p_j[1], p_q[1]);
+        for(; tt + 1 < T; tt += 2) tiles(tt, std::false_type{}, Two{});
+        if(tt < T) tiles(tt, std::false_type{}, One{});
     }
-    if(lane == 0) a.gnc[grp] = nc;
+    if(lane == 0) a.gnc[grp] = nc | (wrap ? GNC_WRAP : 0);
 
-    int over = 0, len = 0;
-    if(valid) {
-        // past the reference's list capacity (its unchecked write,
-        // src/bhtree.cpp:257-258) the search reports an overflow
-        over = count + count2 > a.cap ? 1 : 0;
-        len = count + count2;
-    }
-    over = wave_sum(over);
-    len = wave_maxv(len);
+    // past the reference's list capacity (its unchecked write,
+    // src/bhtree.cpp:257-258) the search reports an overflow
+    const int over = wave_sum(count > a.cap ? 1 : 0);
+    const int len = wave_maxv(count);
     if(lane == 0) {
         if(a.stats) {
             stat_add(a.counters, grp, C_SEARCH_NODES, visited);
@@ -415,7 +362,123 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     }  // groups
 }
 
-template <int D, bool IJ> static void launch_search(Ctx &c, const SearchArgs &a, bool work_ready, int blocks_per_cu)
+// ------------------------------------------------------------------- boxes
+// Search records (position, squared candidate radius) and the boxes of the
+// first two levels: a workgroup takes the 2,048 particles of one
+// second-level box.  rad may be null (gather search: its boxes need none;
+// the records' radius is then `own2`'s, the group's own radii).
+constexpr int BOX_THREADS = 1024;
+constexpr int SUPER = CHUNK * WAVE;  // particles per second-level box
+
+__device__ __forceinline__ void box_join(ChunkBox &a, const ChunkBox &b)
+{
+#pragma unroll
+    for(int k = 0; k < 3; ++k) {
+        a.lo[k] = b.lo[k] < a.lo[k] ? b.lo[k] : a.lo[k];
+        a.hi[k] = b.hi[k] > a.hi[k] ? b.hi[k] : a.hi[k];
+    }
+    a.r = b.r > a.r ? b.r : a.r;
+}
+
+__device__ __forceinline__ ChunkBox box_none()
+{
+    ChunkBox b;
+#pragma unroll
+    for(int k = 0; k < 3; ++k) {
+        b.lo[k] = 3.4028234e38f;
+        b.hi[k] = -3.4028234e38f;
+    }
+    b.r = 0.0f;
+    b.pad = 0.0f;
+    return b;
+}
+
+// box of W consecutive lanes' boxes, in every one of them
+template <int W> __device__ __forceinline__ ChunkBox box_lanes(ChunkBox b)
+{
+#pragma unroll
+    for(int off = W / 2; off > 0; off >>= 1) {
+        ChunkBox o;
+#pragma unroll
+        for(int k = 0; k < 3; ++k) {
+            o.lo[k] = __shfl_xor(b.lo[k], off, WAVE);
+            o.hi[k] = __shfl_xor(b.hi[k], off, WAVE);
+        }
+        o.r = __shfl_xor(b.r, off, WAVE);
+        box_join(b, o);
+    }
+    return b;
+}
+
+template <int D>
+__global__ void __launch_bounds__(BOX_THREADS) chunk_boxes_kernel(State s, const double *rad, int n, double4 *srec, ChunkBox *l1, ChunkBox *l2)
+{
+    __shared__ ChunkBox sh[WAVE];
+    for(int r = 0; r < SUPER / BOX_THREADS; ++r) {
+        const int slot = r * BOX_THREADS + threadIdx.x;
+        const int64_t i = (int64_t)blockIdx.x * SUPER + slot;
+        ChunkBox b = box_none();
+        if(i < n) {
+            double4 q;
+            q.x = s.f[F_X][i];
+            q.y = D > 1 ? s.f[F_X + 1][i] : 0.0;
+            q.z = D > 2 ? s.f[F_X + 2][i] : 0.0;
+            const double h = rad[i];
+            q.w = h * h;
+            srec[i] = q;
+            const double x[3] = {q.x, q.y, q.z};
+#pragma unroll
+            for(int k = 0; k < 3; ++k) {
+                // FP32, rounded outwards (a NaN coordinate stays out of the box)
+                const float f = (float)x[k], e = fabsf(f) * 1.2e-7f + 1e-37f;
+                if(f == f) {
+                    b.lo[k] = f - e;
+                    b.hi[k] = f + e;
+                }
+            }
+            const float f = (float)h;
+            b.r = f == f ? f + f * 1.2e-7f + 1e-37f : 0.0f;
+        }
+        b = box_lanes<CHUNK>(b);
+        if((slot & (CHUNK - 1)) == 0) sh[slot / CHUNK] = b;
+    }
+    __syncthreads();
+    if(threadIdx.x < WAVE) {
+        const ChunkBox b = sh[threadIdx.x];
+        const int64_t at = (int64_t)blockIdx.x * WAVE + threadIdx.x;
+        if(at * CHUNK < n) l1[at] = b;
+        const ChunkBox t = box_lanes<WAVE>(b);
+        if(threadIdx.x == 0) l2[blockIdx.x] = t;
+    }
+}
+
+// third level: one box per 64 of the second
+__global__ void __launch_bounds__(BLOCK) upper_boxes_kernel(const ChunkBox *l2, int n2, ChunkBox *l3)
+{
+    const int b = (int)(blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE);
+    const int v = b * WAVE + wave_lane();
+    if(b * WAVE >= n2) return;
+    const ChunkBox t = box_lanes<WAVE>(v < n2 ? l2[v] : box_none());
+    if(wave_lane() == 0) l3[b] = t;
+}
+
+// Records and boxes of the current particles with candidate radii `rad`.
+int search_boxes(Ctx &c, const double *rad)
+{
+    const int n = (int)c.n, n2 = grid_for(n, SUPER), n3 = grid_for(n2, WAVE);
+    ChunkBox *l1 = c.boxes, *l2 = l1 + grid_for(c.cap_n, CHUNK), *l3 = l2 + grid_for(c.cap_n, SUPER);
+    switch(c.D) {
+    case 1: hipLaunchKernelGGL(chunk_boxes_kernel<1>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
+    case 2: hipLaunchKernelGGL(chunk_boxes_kernel<2>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
+    default: hipLaunchKernelGGL(chunk_boxes_kernel<3>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
+    }
+    // with one third-level box the search starts at the second
+    if(n3 > 1) hipLaunchKernelGGL(upper_boxes_kernel, dim3(grid_for(n3, SW)), dim3(BLOCK), 0, c.stream, l2, n2, l3);
+    SPHGPU_HIP(hipGetLastError());
+    return SPHGPU_OK;
+}
+
+template <int D, int MODE> static void launch_search(Ctx &c, const SearchArgs &a, bool work_ready, int blocks_per_cu)
 {
     const BoxDev box = make_box(c);
     // blocks_per_cu blocks of 4 waves per CU (8 fill every CU), a multiple
@@ -424,22 +487,22 @@ template <int D, bool IJ> static void launch_search(Ctx &c, const SearchArgs &a,
     if(!work_ready) reset_work(c, 0);
     SearchArgs aw = a;
     aw.work = c.work;
-    hipLaunchKernelGGL((search_kernel<D, IJ>), dim3(blocks), dim3(BLOCK), 0, c.stream, c.s, c.t, box, c.groups, c.num_groups, aw);
+    hipLaunchKernelGGL((search_kernel<D, MODE>), dim3(blocks), dim3(BLOCK), 0, c.stream, box, aw);
 }
 
-template <bool IJ> static int search_dispatch(Ctx &c, const SearchArgs &a, bool work_ready = false, int blocks_per_cu = 8)
+template <int MODE> static int search_dispatch(Ctx &c, const SearchArgs &a, bool work_ready, int blocks_per_cu)
 {
     switch(c.D) {
-    case 1: launch_search<1, IJ>(c, a, work_ready, blocks_per_cu); break;
-    case 2: launch_search<2, IJ>(c, a, work_ready, blocks_per_cu); break;
-    default: launch_search<3, IJ>(c, a, work_ready, blocks_per_cu); break;
+    case 1: launch_search<1, MODE>(c, a, work_ready, blocks_per_cu); break;
+    case 2: launch_search<2, MODE>(c, a, work_ready, blocks_per_cu); break;
+    default: launch_search<3, MODE>(c, a, work_ready, blocks_per_cu); break;
     }
     SPHGPU_HIP(hipGetLastError());
     return SPHGPU_OK;
 }
 
-// sml = h_guess * ratio (src/pre_interaction.cpp:61-64), the gather
-// search radius, before the combined search
+// sml = h_guess * ratio (src/pre_interaction.cpp:61-64), the gather search
+// radius
 template <int D> __global__ void __launch_bounds__(BLOCK) guess_kernel(State s, int n, double nngb, double ratio)
 {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
@@ -447,9 +510,8 @@ template <int D> __global__ void __launch_bounds__(BLOCK) guess_kernel(State s, 
     s.f[F_SML][i] = sml_guess<D>(s.f[F_MASS][i], s.f[F_DENS][i], nngb, ratio);
 }
 
-int search_guess(Ctx &c)
+static int guess(Ctx &c, double ratio)
 {
-    const double ratio = c.p.iterative_sml ? 1.2 : 1.0;
     const double nngb = (double)c.p.neighbor_number;
     switch(c.D) {
     case 1: hipLaunchKernelGGL(guess_kernel<1>, dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, nngb, ratio); break;
@@ -457,62 +519,107 @@ int search_guess(Ctx &c)
     default: hipLaunchKernelGGL(guess_kernel<3>, dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, nngb, ratio); break;
     }
     SPHGPU_HIP(hipGetLastError());
-    return SPHGPU_OK;
+    return search_boxes(c, c.s.f[F_SML]);
 }
+
+int search_guess(Ctx &c) { return guess(c, c.p.iterative_sml ? 1.2 : 1.0); }
+
+// The largest h of every particle's leaf (BHTree::set_kernel's value for it,
+// src/bhtree.cpp:206-232): the symmetric search's candidate radius.
+__global__ void __launch_bounds__(BLOCK) leaf_radius_kernel(TreeDev t, const double *sml, int64_t cap, double *out)
+{
+    const int total = *t.num_nodes;
+    for(int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x; v < total && v < cap; v += (int64_t)gridDim.x * BLOCK) {
+        const int4 r = t.rng[v];
+        if(!(r.w & 256)) continue;
+        double h = 0.0;
+        for(int i = r.x; i < r.y; ++i) h = sml[i] > h ? sml[i] : h;
+        for(int i = r.x; i < r.y; ++i) out[i] = h;
+    }
+}
+
+// Blocks of four persistent waves per CU.  More waves hide the dependent
+// loads of the first two phases; fewer leave the scalar cache (which holds
+// the groups' records) and L2 to each.  Beside the gravity walk, which is
+// bound by instruction issue, the step is shortest with two (mixed Evrard
+// step, 2^20 particles: 5.13 ms, against 5.15, 5.19 and 5.29 with three,
+// four and six).  Alone: 2D KHI, 393,160 particles: 128 us with four (137
+// with two, 143 with six); 3D, 2^21 particles: 800 us with six (1,122 with
+// two, 865 with four, 824 with eight).
+int search_blocks(const Ctx &c, bool beside_walk) { return beside_walk ? 2 : c.D < 3 ? 4 : 6; }
 
 static SearchArgs base_args(Ctx &c)
 {
     SearchArgs a{};
+    a.n = (int)c.n;
+    a.srec = c.srec;
+    a.own = c.s.f[F_SML];
+    a.lev[0] = c.boxes;
+    a.lev[1] = c.boxes + grid_for(c.cap_n, CHUNK);
+    a.lev[2] = a.lev[1] + grid_for(c.cap_n, SUPER);
+    a.cnt[0] = grid_for(c.n, CHUNK);
+    a.cnt[1] = grid_for(c.n, SUPER);
+    a.cnt[2] = grid_for(a.cnt[1], WAVE);
+    a.groups = c.groups;
+    a.num_groups = c.num_groups;
     a.cand = c.tile_cand;
-    a.mf = c.tile_mf;
     a.ma = c.tile_ma;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.ws_j = c.ws_j;
-    a.ws_p = c.ws_p;
     a.cap = c.cap;
     a.counters = c.counters;
     a.stats = c.stats_on ? 1 : 0;
     return a;
 }
 
-// One walk for both sets: with sml = h_guess * ratio and the cells' largest
-// sml from tree_set_kernel, the test r < max(sml_i, sml_j) finds every
-// gather candidate (r < sml_i, in the front masks) and every pair with
-// r < max(h_i, h_j) for the final h, as long as no final h exceeds its
-// search radius (the caller checks the truncation counter).  With
+// One search for both sets: with the records' radii h_guess * ratio, the
+// test r < max(R_i, R_j) finds every gather candidate (r < R_i) and every
+// pair with r < max(h_i, h_j) for the final h, as long as no final h exceeds
+// its search radius (the caller checks the truncation counter).  With
 // `work_ready` the caller has already cleared the task counters
-// (reset_work(c, 0)); `blocks_per_cu` sets how many of the CUs' wave slots
-// the search's persistent waves take (8: all of them).
+// (reset_work(c, 0)); `blocks_per_cu` sets how many blocks of four
+// persistent waves each CU gets.
 int search_combined(Ctx &c, bool work_ready, int blocks_per_cu)
 {
-    SearchArgs a = base_args(c);
-    a.split = 1;
-    a.guess = 0;
-    return search_dispatch<true>(c, a, work_ready, blocks_per_cu);
+    return search_dispatch<M_COMBINED>(c, base_args(c), work_ready, blocks_per_cu);
 }
 
 int search_gather(Ctx &c, bool initial)
 {
-    SearchArgs a = base_args(c);
-    a.guess = 1;
-    a.ratio = initial ? 1.0 : (c.p.iterative_sml ? 1.2 : 1.0);  // src/pre_interaction.cpp:31-35
-    a.nngb = (double)c.p.neighbor_number;
-    return search_dispatch<false>(c, a, false, c.D < 3 ? 2 : 8);  // blocks per CU: see stage_pre
+    int rc = guess(c, initial ? 1.0 : (c.p.iterative_sml ? 1.2 : 1.0));  // src/pre_interaction.cpp:31-35
+    if(rc) return rc;
+    return search_dispatch<M_GATHER>(c, base_args(c), false, search_blocks(c, false));
 }
 
 int search_symmetric(Ctx &c)
 {
-    SearchArgs a = base_args(c);
-    a.guess = 0;
-    return search_dispatch<true>(c, a, false, c.D < 3 ? 2 : 8);
+    hipLaunchKernelGGL(leaf_radius_kernel, dim3(std::min<int64_t>(grid_for(c.node_cap), 2048)), dim3(BLOCK), 0, c.stream, c.t,
+                       c.s.f[F_SML], c.node_cap, c.leaf_rad);
+    SPHGPU_HIP(hipGetLastError());
+    int rc = search_boxes(c, c.leaf_rad);
+    if(rc) return rc;
+    return search_dispatch<M_SYMMETRIC>(c, base_args(c), false, search_blocks(c, false));
+}
+
+// Search records and boxes of up to n particles, and the symmetric search's
+// radii.  The records have a spare tile behind the last particle (the search
+// reads a group's records four at a time).
+int search_alloc_particles(Ctx &c)
+{
+    const int64_t n = c.cap_n;
+    SPHGPU_HIP(hipMalloc(&c.srec, (n + WAVE) * sizeof(double4)));
+    const int64_t nb = grid_for(n, CHUNK) + grid_for(n, SUPER) + grid_for(grid_for(n, SUPER), WAVE);
+    SPHGPU_HIP(hipMalloc(&c.boxes, nb * sizeof(ChunkBox)));
+    SPHGPU_HIP(hipMalloc(&c.leaf_rad, n * sizeof(double)));
+    return SPHGPU_OK;
 }
 
 // Slabs of candidate tiles for the c.ngroups groups of the last tree, and
 // the staging buffers of the search's persistent waves.  A slab holds
 // tile_wcap candidates: the larger of eight times the per-particle capacity
-// and 48 times neighborNumber.  A group of 64 particles keeps about 19
-// times neighborNumber in 3D (1,220 at 64 neighbours in the Evrard
+// and 48 times neighborNumber.  A group of 64 particles keeps about 11
+// times neighborNumber in 3D (690 at 64 neighbours in the Evrard
 // benchmark).
 int search_alloc(Ctx &c)
 {
@@ -521,26 +628,21 @@ int search_alloc(Ctx &c)
     const int64_t waves = (int64_t)8 * c.num_cu * SW + SW;
     if(wcap != c.tile_wcap || waves > c.ws_waves) {
         if(c.ws_j) (void)hipFree(c.ws_j);
-        if(c.ws_p) (void)hipFree(c.ws_p);
         c.ws_j = nullptr;
-        c.ws_p = nullptr;
         SPHGPU_HIP(hipMalloc(&c.ws_j, (size_t)waves * wcap * sizeof(int)));
-        SPHGPU_HIP(hipMalloc(&c.ws_p, (size_t)waves * wcap * sizeof(double4)));
         c.ws_waves = waves;
     }
     if(wcap != c.tile_wcap || c.ngroups > c.tile_groups_cap) {
         // grow with headroom: the group count changes a little every step
         const int64_t groups = std::max<int64_t>((int64_t)c.ngroups + c.ngroups / 4 + 64, c.tile_groups_cap);
         if(c.tile_cand) (void)hipFree(c.tile_cand);
-        if(c.tile_mf) (void)hipFree(c.tile_mf);
         if(c.tile_ma) (void)hipFree(c.tile_ma);
         if(c.tile_nc) (void)hipFree(c.tile_nc);
         c.tile_cand = nullptr;
-        c.tile_mf = c.tile_ma = nullptr;
+        c.tile_ma = nullptr;
         c.tile_nc = nullptr;
         const size_t slots = (size_t)groups * wcap;
         SPHGPU_HIP(hipMalloc(&c.tile_cand, slots * sizeof(int)));
-        SPHGPU_HIP(hipMalloc(&c.tile_mf, slots * sizeof(uint64_t)));
         SPHGPU_HIP(hipMalloc(&c.tile_ma, slots * sizeof(uint64_t)));
         SPHGPU_HIP(hipMalloc(&c.tile_nc, groups * sizeof(int)));
         c.tile_groups_cap = groups;
@@ -550,14 +652,13 @@ int search_alloc(Ctx &c)
 }
 
 // Lists in list_at layout from the tiles of the last search: lane l of a
-// group appends its front hits from slot 0 on and its back hits from slot
-// cap - 1 down, both in staging order (candidate c = t + kT is bit k of
-// tile t), which is the order the reference's one-leaf-at-a-time walk
-// finds them in.  cnt / cnt2 receive the counts (cnt2 may be null with
-// front_only).  Entries past cap are dropped (the search reports them).
-__global__ void __launch_bounds__(BLOCK) expand_kernel(const int2 *groups, int ngroups, const int *gnc, const int *cand,
-                                                       const uint64_t *mf, const uint64_t *ma, int wcap, int cap,
-                                                       int front_only, int *list, int *cnt, int *cnt2)
+// group appends its hits in staging order (candidate c = t + kT is bit k of
+// tile t).  gather_only keeps the gather candidates r < R_i (sml before the
+// pre-interaction).  Entries past cap are dropped (the search reports them).
+template <int D>
+__global__ void __launch_bounds__(BLOCK) expand_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
+                                                       const int *cand, const uint64_t *ma, int wcap, int cap,
+                                                       int gather_only, int *list, int *cnt)
 {
     const int grp = xcd_block() * (BLOCK / WAVE) + (int)(threadIdx.x / WAVE);
     if(grp >= ngroups) return;
@@ -566,31 +667,45 @@ __global__ void __launch_bounds__(BLOCK) expand_kernel(const int2 *groups, int n
     const int i = gr.x + lane;
     if(i >= gr.y) return;
     const size_t gbase = (size_t)grp * wcap;
-    const int nc = gnc[grp];
+    const int nc = gnc[grp] & ~GNC_WRAP;
     const int T = (nc + WAVE - 1) / WAVE;
     const size_t lb = list_base(i, cap);
-    int wf = 0, wb = 0;  // entries written (at most cap in total)
+    double xi[D];
+#pragma unroll
+    for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][i];
+    const double h2 = s.f[F_SML][i] * s.f[F_SML][i];
+    int wf = 0;  // entries written (at most cap)
     for(int k = 0; k < WAVE; ++k) {
         for(int t = 0; t < T; ++t) {
             if(t + k * T >= nc) break;
             const size_t o = gbase + (size_t)t * WAVE;
-            const uint64_t bit = 1ull << k;
-            const bool room = wf + wb < cap;
-            if(mf[o + lane] & bit) {
-                if(room) list[lb + list_off(wf++)] = cand[o + k];
-            } else if(!front_only && (ma[o + lane] & bit)) {
-                if(room) list[lb + list_off(cap - 1 - wb++)] = cand[o + k];
+            if(!((ma[o + lane] >> k) & 1ull)) continue;
+            const int j = cand[o + k];
+            if(gather_only) {
+                double xj[D], d[D];
+#pragma unroll
+                for(int q = 0; q < D; ++q) xj[q] = s.f[F_X + q][j];
+                if(!(sep2<D>(box, xi, xj, d) < h2)) continue;
             }
+            if(wf < cap) list[lb + list_off(wf++)] = j;
         }
     }
     cnt[i] = wf;
-    if(cnt2) cnt2[i] = wb;
 }
 
-int search_expand(Ctx &c, int *list, int *cnt, int *cnt2, bool front_only)
+template <int D> static void launch_expand(Ctx &c, int *list, int *cnt, bool gather_only)
 {
-    hipLaunchKernelGGL(expand_kernel, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.groups, c.ngroups, c.tile_nc,
-                       c.tile_cand, c.tile_mf, c.tile_ma, c.tile_wcap, c.cap, front_only ? 1 : 0, list, cnt, cnt2);
+    hipLaunchKernelGGL(expand_kernel<D>, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
+                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, gather_only ? 1 : 0, list, cnt);
+}
+
+int search_expand(Ctx &c, int *list, int *cnt, bool gather_only)
+{
+    switch(c.D) {
+    case 1: launch_expand<1>(c, list, cnt, gather_only); break;
+    case 2: launch_expand<2>(c, list, cnt, gather_only); break;
+    default: launch_expand<3>(c, list, cnt, gather_only); break;
+    }
     SPHGPU_HIP(hipGetLastError());
     return SPHGPU_OK;
 }

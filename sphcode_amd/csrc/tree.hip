@@ -1,5 +1,4 @@
-// Octree build on the device (replaces BHTree::make, src/bhtree.cpp:55-107,
-// and BHTree::set_kernel, src/bhtree.cpp:109-112, 206-232).
+// Octree build on the device (replaces BHTree::make, src/bhtree.cpp:55-107).
 //
 // The reference builds a pointer octree top-down, serially: the root cube
 // is the bounding box (centre, largest extent) or the periodic box
@@ -19,9 +18,8 @@
 // b begins a level-L cell whose parent holds more than leafParticleNumber
 // particles.  Each particle emits the nodes that start at it, so an
 // exclusive scan of those counts is the pre-order numbering.  Mass moments
-// and the largest h per subtree are reduced bottom-up, one tree level per
-// launch (the upper levels, which hold few nodes, in one single-workgroup
-// launch).  The root keeps zero mass and centre of mass,
+// are reduced bottom-up, one tree level per launch (the upper levels, which
+// hold few nodes, in one single-workgroup launch).  The root keeps zero mass and centre of mass,
 // as the reference never accumulates them (include/bhtree.hpp:46-53).
 #include <cstring>
 
@@ -381,13 +379,10 @@ __global__ void __launch_bounds__(BLOCK) level_scatter_kernel(TreeDev t, int *lv
 // particles, an internal node its children (one level deeper, done by the
 // previous launch), in child order.  The root's moments stay zero, as the
 // reference never accumulates them (include/bhtree.hpp:46-53).
-// With KS, also the node's largest smoothing length (kernel_size_node's
-// result) in the same pass.
-template <int D, bool KS> __device__ __forceinline__ void moments_node(const State &s, const TreeDev &t, int p, int total, double4 *msum)
+template <int D> __device__ __forceinline__ void moments_node(const State &s, const TreeDev &t, int p, int total, double4 *msum)
 {
     const int4 r = t.rng[p];
     double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
-    double h = 0.0;
     if(r.w & 256) {
         double mx[3] = {0.0, 0.0, 0.0};
         for(int i = r.x; i < r.y; ++i) {
@@ -395,10 +390,6 @@ template <int D, bool KS> __device__ __forceinline__ void moments_node(const Sta
             acc.w += mi;
 #pragma unroll
             for(int q = 0; q < D; ++q) mx[q] += s.f[F_X + q][i] * mi;
-            if constexpr(KS) {
-                const double hi = s.f[F_SML][i];
-                h = hi > h ? hi : h;
-            }
         }
         acc.x = mx[0];
         acc.y = mx[1];
@@ -408,24 +399,19 @@ template <int D, bool KS> __device__ __forceinline__ void moments_node(const Sta
         for(int c = p + 1; c < r.z && c < total && guard < 8; c = t.rng[c].z, ++guard) {
             const double4 v = msum[c];
             acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-            if constexpr(KS) {
-                const double hc = t.ks[c];
-                h = hc > h ? hc : h;
-            }
         }
     }
-    if constexpr(KS) t.ks[p] = h;
     msum[p] = acc;
     if(p == 0) t.mom[0] = make_double4(0.0, 0.0, 0.0, 0.0);
     else t.mom[p] = make_double4(acc.x / acc.w, acc.y / acc.w, acc.z / acc.w, acc.w);
 }
 
-template <int D, bool KS>
+template <int D>
 __global__ void __launch_bounds__(BLOCK) moments_level_kernel(State s, TreeDev t, const int *nodes, int count, double4 *msum)
 {
     const int k = blockIdx.x * BLOCK + threadIdx.x;
     if(k >= count) return;
-    moments_node<D, KS>(s, t, nodes[k], *t.num_nodes, msum);
+    moments_node<D>(s, t, nodes[k], *t.num_nodes, msum);
 }
 
 // The upper levels, which hold few nodes, in one launch of one workgroup:
@@ -441,12 +427,12 @@ struct TopLevels {
     int offset[16];
 };
 
-template <int D, bool KS>
+template <int D>
 __global__ void __launch_bounds__(TOP_THREADS) moments_top_kernel(State s, TreeDev t, const int *nodes, TopLevels tl, double4 *msum)
 {
     const int total = *t.num_nodes;
     for(int L = tl.nlev - 1; L >= 0; --L) {
-        for(int k = threadIdx.x; k < tl.count[L]; k += TOP_THREADS) moments_node<D, KS>(s, t, nodes[tl.offset[L] + k], total, msum);
+        for(int k = threadIdx.x; k < tl.count[L]; k += TOP_THREADS) moments_node<D>(s, t, nodes[tl.offset[L] + k], total, msum);
         __syncthreads();
     }
 }
@@ -518,43 +504,6 @@ __global__ void __launch_bounds__(BLOCK) level_count_groups_kernel(TreeDev t, in
     }
 }
 
-// Largest smoothing length per subtree (BHNode::set_kernel,
-// src/bhtree.cpp:206-232), one level per launch as the moments.
-__device__ __forceinline__ void kernel_size_node(const State &s, const TreeDev &t, int p, int total)
-{
-    const int4 r = t.rng[p];
-    double h = 0.0;
-    if(r.w & 256) {
-        for(int i = r.x; i < r.y; ++i) {
-            const double hi = s.f[F_SML][i];
-            h = hi > h ? hi : h;
-        }
-    } else {
-        int guard = 0;
-        for(int c = p + 1; c < r.z && c < total && guard < 8; c = t.rng[c].z, ++guard) {
-            const double v = t.ks[c];
-            h = v > h ? v : h;
-        }
-    }
-    t.ks[p] = h;
-}
-
-__global__ void __launch_bounds__(BLOCK) kernel_size_level_kernel(State s, TreeDev t, const int *nodes, int count)
-{
-    const int k = blockIdx.x * BLOCK + threadIdx.x;
-    if(k >= count) return;
-    kernel_size_node(s, t, nodes[k], *t.num_nodes);
-}
-
-__global__ void __launch_bounds__(TOP_THREADS) kernel_size_top_kernel(State s, TreeDev t, const int *nodes, TopLevels tl)
-{
-    const int total = *t.num_nodes;
-    for(int L = tl.nlev - 1; L >= 0; --L) {
-        for(int k = threadIdx.x; k < tl.count[L]; k += TOP_THREADS) kernel_size_node(s, t, nodes[tl.offset[L] + k], total);
-        __syncthreads();
-    }
-}
-
 // ------------------------------------------------------------------ host
 int tree_alloc(Ctx &c)
 {
@@ -569,7 +518,6 @@ int tree_alloc(Ctx &c)
     SPHGPU_HIP(hipMalloc(&c.noff, n * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.t.geo, c.node_cap * sizeof(double4)));
     SPHGPU_HIP(hipMalloc(&c.t.mom, c.node_cap * sizeof(double4)));
-    SPHGPU_HIP(hipMalloc(&c.t.ks, c.node_cap * sizeof(double)));
     SPHGPU_HIP(hipMalloc(&c.t.rng, c.node_cap * sizeof(int4)));
     SPHGPU_HIP(hipMalloc(&c.t.num_nodes, sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.lvl_nodes, c.node_cap * sizeof(int)));
@@ -663,8 +611,8 @@ template <int D> static int tree_build_d(Ctx &c)
     }
     r.isrc[0] = c.s.id; r.idst[0] = c.alt.id;
     r.isrc[1] = c.reorder_light ? nullptr : c.s.nb; r.idst[1] = c.alt.nb;
-    // sphgpu_integrate's combined search needs the radii h_guess * ratio and
-    // the cells' largest radius: set here, by the reorder and the moments
+    // sphgpu_integrate's combined search needs the radii h_guess * ratio, set
+    // here by the reorder, and its records and boxes
     const bool radius = c.reorder_light;
     if(radius) {
         r.sml = c.alt.f[F_SML];
@@ -678,6 +626,10 @@ template <int D> static int tree_build_d(Ctx &c)
     for(int f = 0; f < NF; ++f) std::swap(c.s.f[f], c.alt.f[f]);
     std::swap(c.s.id, c.alt.id);
     std::swap(c.s.nb, c.alt.nb);
+    if(radius) {
+        int rc = search_boxes(c, c.s.f[F_SML]);
+        if(rc) return rc;
+    }
 
     const TreeShape ts{n, G, D, c.p.tree_leaf_particle_num, c.p.tree_max_level};
     hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn);
@@ -704,19 +656,10 @@ template <int D> static int tree_build_d(Ctx &c)
     for(int L = NLEVEL - 1; L >= tl.first + tl.nlev; --L) {
         const int cnt = c.lvl_host[L];
         if(cnt <= 0) continue;
-        if(radius)
-            hipLaunchKernelGGL((moments_level_kernel<D, true>), dim3(grid_for(cnt)), dim3(BLOCK), 0, c.stream, c.s, c.t,
-                               c.lvl_nodes + c.lvl_host[NLEVEL + L], cnt, c.msum);
-        else
-            hipLaunchKernelGGL((moments_level_kernel<D, false>), dim3(grid_for(cnt)), dim3(BLOCK), 0, c.stream, c.s, c.t,
-                               c.lvl_nodes + c.lvl_host[NLEVEL + L], cnt, c.msum);
+        hipLaunchKernelGGL(moments_level_kernel<D>, dim3(grid_for(cnt)), dim3(BLOCK), 0, c.stream, c.s, c.t,
+                           c.lvl_nodes + c.lvl_host[NLEVEL + L], cnt, c.msum);
     }
-    if(tl.nlev > 0) {
-        if(radius)
-            hipLaunchKernelGGL((moments_top_kernel<D, true>), dim3(1), dim3(TOP_THREADS), 0, c.stream, c.s, c.t, c.lvl_nodes, tl, c.msum);
-        else
-            hipLaunchKernelGGL((moments_top_kernel<D, false>), dim3(1), dim3(TOP_THREADS), 0, c.stream, c.s, c.t, c.lvl_nodes, tl, c.msum);
-    }
+    if(tl.nlev > 0) hipLaunchKernelGGL(moments_top_kernel<D>, dim3(1), dim3(TOP_THREADS), 0, c.stream, c.s, c.t, c.lvl_nodes, tl, c.msum);
     SPHGPU_HIP(hipGetLastError());
     c.radius_ready = radius;
     return search_alloc(c);
@@ -729,22 +672,6 @@ int tree_build(Ctx &c)
     case 2: return tree_build_d<2>(c);
     default: return tree_build_d<3>(c);
     }
-}
-
-int tree_set_kernel(Ctx &c)
-{
-    // level lists and counts from the last tree build
-    const TopLevels tl = top_levels(c);
-    for(int L = NLEVEL - 1; L >= tl.first + tl.nlev; --L) {
-        const int cnt = c.lvl_host[L];
-        if(cnt <= 0) continue;
-        hipLaunchKernelGGL(kernel_size_level_kernel, dim3(grid_for(cnt)), dim3(BLOCK), 0, c.stream, c.s, c.t,
-                           c.lvl_nodes + c.lvl_host[NLEVEL + L], cnt);
-    }
-    if(tl.nlev > 0)
-        hipLaunchKernelGGL(kernel_size_top_kernel, dim3(1), dim3(TOP_THREADS), 0, c.stream, c.s, c.t, c.lvl_nodes, tl);
-    SPHGPU_HIP(hipGetLastError());
-    return SPHGPU_OK;
 }
 
 }  // namespace sphgpu
