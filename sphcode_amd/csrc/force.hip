@@ -169,14 +169,20 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         int used = 0;
         const ForceRec<T> *frec = (const ForceRec<T> *)a.frec;
         const size_t gbase = (size_t)grp * a.wcap;
-        const int nc = a.gnc[grp] & ~GNC_WRAP;
+        const int gnc = uniform(a.gnc[grp]);
+        const int nc = gnc & ~GNC_WRAP;
+        const GroupImage<D> img(box, gnc, xi);
         const int ntile = (nc + WAVE - 1) / WAVE;
         auto stage = [&](int tt) -> uint64_t {
             const size_t o = gbase + (size_t)tt * WAVE;
             // lane k loads candidate k's records
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) {
-                l_p[w][lane] = a.posrec[jl];
+                double4 q = a.posrec[jl];
+                q.x = img.at(0, q.x);
+                if constexpr(D > 1) q.y = img.at(1, q.y);
+                if constexpr(D > 2) q.z = img.at(2, q.z);
+                l_p[w][lane] = q;
                 l_f[w][lane] = frec[jl];
                 if constexpr(GS)
                     if(a.second_order) l_g[GS ? w : 0][lane] = ((const GradRec<T> *)a.grec)[jl];
@@ -191,7 +197,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             xj[0] = pj4.x;
             if constexpr(D > 1) xj[1] = pj4.y;
             if constexpr(D > 2) xj[2] = pj4.z;
-            const double r2 = sep2<D>(box, xi, xj, d);
+            const double r2 = sep2<D>(img.pairs, xi, xj, d);
             const double hj_d = pj4.w;
             const double hmax = hi_d < hj_d ? hj_d : hi_d;
             T r;
@@ -338,7 +344,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             xj[0] = pj4.x;
             if constexpr(D > 1) xj[1] = pj4.y;
             if constexpr(D > 2) xj[2] = pj4.z;
-            const double r2 = sep2<D>(box, xi, xj, d);
+            const double r2 = sep2<D>(img.pairs, xi, xj, d);
             const double hmax = hi_d < pj4.w ? pj4.w : hi_d;
             if constexpr(FP64) {
                 const double r = sqrt(r2);

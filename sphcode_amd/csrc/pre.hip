@@ -131,17 +131,19 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
     double xi[D];
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
+    const int gnc = uniform(a.gnc[grp]);
+    const GroupImage<D> img(box, gnc, xi);
     const T h = (T)s.f[F_SML][ii];
     const Kern ker(h);
     Acc<T> rho;
     const size_t gbase = (size_t)grp * a.wcap;
-    const int ntile = ((a.gnc[grp] & ~GNC_WRAP) + WAVE - 1) / WAVE;
+    const int ntile = ((gnc & ~GNC_WRAP) + WAVE - 1) / WAVE;
     auto stage = [&](int tt) -> uint64_t {
         const size_t o = gbase + (size_t)tt * WAVE;
         const int jl = stream_ld(a.cand + o + lane);
         if(jl >= 0) {
 #pragma unroll
-            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = s.f[F_X + k][jl];
+            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl]);
             l_r[w][lane].m = fld<T>(s, F_MASS, jl);
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
@@ -150,7 +152,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         double xj[D], d[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = l_r[w][kc].x[k];
-        const T r = gather_r<T>(sep2<D>(box, xi, xj, d));
+        const T r = gather_r<T>(sep2<D>(img.pairs, xi, xj, d));
         if(r < h) rho.add(l_r[w][kc].m * ker.w(ker.q_of(r)));
     };
     tile_sweep(ntile, stage, pair);
@@ -179,7 +181,8 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     const bool valid = have && i < gr.y;
     const int ii = valid ? i : gr.x;
     const size_t gbase = (size_t)(have ? grp : 0) * a.wcap;
-    const int ntile = have ? ((a.gnc[grp] & ~GNC_WRAP) + WAVE - 1) / WAVE : 0;
+    const int gnc = have ? uniform(a.gnc[grp]) : 0;
+    const int ntile = ((gnc & ~GNC_WRAP) + WAVE - 1) / WAVE;
     const PreRec<T> *prec = (const PreRec<T> *)a.prec;
     double hvs = 1.7976931348623157e308;
     int64_t iters = 0, fails = 0, trunc = 0, pairs = 0;
@@ -187,6 +190,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         double xi[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
+        const GroupImage<D> img(box, gnc, xi);
         const double mi = s.f[F_MASS][ii];
         const double Hs = s.f[F_SML][ii];  // search radius h_guess * ratio
         const double Hs2 = Hs * Hs;
@@ -208,7 +212,13 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 auto nstage = [&](int tt) -> uint64_t {
                     const size_t o = gbase + (size_t)tt * WAVE;
                     const int jl = stream_ld(a.cand + o + lane);
-                    if(jl >= 0) l_pm[lane] = a.pm[jl];
+                    if(jl >= 0) {
+                        double4 q = a.pm[jl];
+                        q.x = img.at(0, q.x);
+                        if constexpr(D > 1) q.y = img.at(1, q.y);
+                        if constexpr(D > 2) q.z = img.at(2, q.z);
+                        l_pm[lane] = q;
+                    }
                     return done ? 0ull : stream_ld(a.ma + o + lane);
                 };
                 auto npair = [&](int kc) {
@@ -217,7 +227,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     xj[0] = pj.x;
                     if constexpr(D > 1) xj[1] = pj.y;
                     if constexpr(D > 2) xj[2] = pj.z;
-                    const double r2 = sep2<D>(box, xi, xj, d);
+                    const double r2 = sep2<D>(img.pairs, xi, xj, d);
                     const T r = gather_r<T>(r2);
                     if(r < ht && r2 < Hs2) {
                         const T q = ker.q_of(r);
@@ -269,7 +279,12 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         auto fstage = [&](int tt) -> uint64_t {
             const size_t o = gbase + (size_t)tt * WAVE;
             const int jl = stream_ld(a.cand + o + lane);
-            if(jl >= 0) l_r[w][lane] = prec[jl];
+            if(jl >= 0) {
+                PreRec<T> q = prec[jl];
+#pragma unroll
+                for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k]);
+                l_r[w][lane] = q;
+            }
             l_j[w][lane] = jl;
             return valid ? stream_ld(a.ma + o + lane) : 0ull;
         };
@@ -278,7 +293,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = pj.x[l];
-            const double r2 = sep2<D>(box, xi, xj, d);
+            const double r2 = sep2<D>(img.pairs, xi, xj, d);
             const T r = gather_r<T>(r2);
             if(!(r < ht && r2 < Hs2)) return;
             const int j = l_j[w][kc];
@@ -346,7 +361,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = l_r[w][kc].x[l];
-            const double r2 = sep2<D>(box, xi, xj, d);
+            const double r2 = sep2<D>(img.pairs, xi, xj, d);
             return gather_r<T>(r2) < ht && r2 < Hs2;
         };
         // refined in 3D except for GSPH (measured slower on the 3D Sedov

@@ -25,6 +25,29 @@
 
 namespace sphgpu {
 
+// Periodic images of a group's candidates.  Unless the group's entry in
+// Ctx::tile_nc carries GNC_WRAP, every pair's minimum image of a candidate
+// is the image nearest to any one particle of the group (the search checked
+// that the group and its reach span less than half the box), so a candidate
+// is moved there once, when it is staged, and the pairs subtract plain
+// coordinates: `pairs` is the box that sep2 gets, switched off then.  The
+// three minimum images of a pair cost some 30 FP64 operations and compares.
+template <int D> struct GroupImage {
+    const BoxDev &box;
+    BoxDev pairs;
+    bool move;
+    double x0[D];
+    __device__ __forceinline__ GroupImage(const BoxDev &b, int gnc, const double xi[D]) : box(b), pairs(b)
+    {
+        pairs.on = b.on && (gnc & GNC_WRAP);
+        move = b.on && !(gnc & GNC_WRAP);
+#pragma unroll
+        for(int k = 0; k < D; ++k) x0[k] = uniform_d(xi[k]);
+    }
+    // axis k of a staged candidate's position
+    __device__ __forceinline__ double at(int k, double x) const { return move ? near_image(box, k, x0[k], x) : x; }
+};
+
 struct NoRefine {
     __device__ __forceinline__ uint64_t operator()(uint64_t m) const { return m; }
 };
