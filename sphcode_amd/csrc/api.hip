@@ -61,6 +61,24 @@ __global__ void fill_i64_kernel(int64_t *p, int n)
     for(int k = threadIdx.x; k < n; k += blockDim.x) p[k] = 0;
 }
 
+// A wave takes one group through its tiles in a serial chain of some 100 to
+// 500 us, so with few groups most SIMDs idle while a few waves finish; the
+// four waves of a block then share each group's tiles (and the search's
+// chunks) and add up their sums.  With many groups the sums' LDS exchange
+// and the boxes that each wave of the search tests again cost more than the
+// shorter chains give.  Measured on 256 CUs, one wave against four:
+//   search  435 groups (3D) 150 -> 52 us, 634 110 -> 45; 2,300 110 -> 121,
+//           5,600 123 -> 179
+//   pre     200 groups (2D) 126 -> 46 us, 435 (3D) 245 -> 83, 2,300 186 ->
+//           153, 2,800 392 -> 282, 5,600 190 -> 184; 8,400 (2D) 283 -> 309
+//   force   200 groups (2D) 61 -> 26 us, 435 (3D) 113 -> 41, 2,300 117 ->
+//           107, 5,600 137 -> 120; 8,400 (2D) 195 -> 197
+int group_waves(const Ctx &c, GroupPass pass)
+{
+    const int most = (pass == GROUP_SEARCH ? 6 : 24) * c.num_cu;
+    return c.ngroups <= most ? BLOCK / WAVE : 1;
+}
+
 static bool field_used(const Ctx &c, int f)
 {
     const int D = c.D;

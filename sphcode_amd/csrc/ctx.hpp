@@ -411,6 +411,10 @@ constexpr int WORK_SLOTS = 1;
 // one wave per search group: grid of ceil(ngroups / 4) blocks of 4 waves,
 // block b serving groups 4 xcd_block() .. + 3
 inline int group_grid(const Ctx &c) { return std::max(1, (c.ngroups + BLOCK / WAVE - 1) / (BLOCK / WAVE)); }
+// Waves that take a search group together in the search and the pair
+// passes (1, or the four of a block).
+enum GroupPass : int { GROUP_SEARCH, GROUP_PAIRS };
+int group_waves(const Ctx &c, GroupPass pass);
 // step.hip
 int step_init_fields(Ctx &c);
 int step_timestep(Ctx &c);       // dt into scal[S_DT]

@@ -116,7 +116,9 @@ template <int D, class T> __device__ __forceinline__ T dotd(const T a[D], const 
     return s;
 }
 
-template <int D, int K, int TYPE, class T>
+// NW waves take a group together (group_waves): 1, or the block's four,
+// which then share its tiles.
+template <int D, int K, int TYPE, class T, int NW>
 __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n, ForceArgs a)
 {
     using Kern = typename KernelOf<D, K, T>::type;
@@ -127,9 +129,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
     __shared__ ForceRec<T> l_f[SW][WAVE];
     __shared__ GradRec<T> l_g[GS ? SW : 1][GS ? WAVE : 1];
     __shared__ int l_j[SW][WAVE];
+    __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
-    const int grp = xcd_block() * SW + w;
+    const int part = w % NW;
+    const int grp = xcd_block() * (SW / NW) + w / NW;
     if(grp >= a.ngroups) return;
     const int2 gr = a.groups[grp];
     const int i = gr.x + lane;
@@ -356,16 +360,19 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         // refined in 3D only, see tiles.hpp
         if constexpr(D == 3) {
             auto refine = [&](uint64_t m) { return refine_bits(m, keep); };
-            tile_sweep(ntile, stage, refine, pair);
+            tile_sweep<NW>(part, ntile, stage, refine, pair);
         } else {
-            tile_sweep(ntile, stage, pair);
+            tile_sweep<NW>(part, ntile, stage, pair);
         }
-        if(valid) {
+        if constexpr(D == 3) parts_sum<NW, 4>(red, part, {&acc[0].s, &acc[1].s, &acc[2].s, &dene.s});
+        else if constexpr(D == 2) parts_sum<NW, 3>(red, part, {&acc[0].s, &acc[1].s, &dene.s});
+        else parts_sum<NW, 2>(red, part, {&acc[0].s, &dene.s});
+        pairs = used;
+        if(valid && part == 0) {
 #pragma unroll
             for(int k = 0; k < D; ++k) s.f[F_A + k][i] = acc[k].val();
             s.f[F_DENE][i] = dene.val();
             if(a.rec_cnt) a.rec_cnt[i] = used < a.cap ? used : a.cap;
-            pairs = used;
         }
     }
     if(a.stats) {
@@ -380,7 +387,11 @@ template <int D, int K, int TYPE, class T> static void launch_force(Ctx &c, cons
     hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
                        c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec);
     if(c.after_pack) c.after_pack_rc = c.after_pack(c);
-    hipLaunchKernelGGL((force_kernel<D, K, TYPE, T>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
+    // (recorded sets are numbered by one wave per group)
+    if(group_waves(c, GROUP_PAIRS) > 1 && !a.rec)
+        hipLaunchKernelGGL((force_kernel<D, K, TYPE, T, BLOCK / WAVE>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
+    else
+        hipLaunchKernelGGL((force_kernel<D, K, TYPE, T, 1>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
 }
 
 template <int D, int K, class T> static void launch_force_t(Ctx &c, const ForceArgs &a, const BoxDev &box)

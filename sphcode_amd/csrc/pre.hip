@@ -115,14 +115,16 @@ template <class T> struct PosMass {
     T m;
 };
 
-template <int D, int K, class T>
+template <int D, int K, class T, int NW>
 __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box, PreArgs a)
 {
     using Kern = typename KernelOf<D, K, T>::type;
     __shared__ PosMass<T> l_r[PSW][WAVE];
+    __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
-    const int grp = xcd_block() * PSW + w;
+    const int part = w % NW;
+    const int grp = xcd_block() * (PSW / NW) + w / NW;
     if(grp >= a.ngroups) return;
     const int2 gr = a.groups[grp];
     const int i = gr.x + lane;
@@ -155,18 +157,23 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         const T r = gather_r<T>(sep2<D>(img.pairs, xi, xj, d));
         if(r < h) rho.add(l_r[w][kc].m * ker.w(ker.q_of(r)));
     };
-    tile_sweep(ntile, stage, pair);
-    if(valid) s.f[F_DENS][i] = rho.val();
+    tile_sweep<NW>(part, ntile, stage, pair);
+    parts_sum<NW, 1>(red, part, {&rho.s});
+    if(valid && part == 0) s.f[F_DENS][i] = rho.val();
 }
 
-template <int D, int K, int TYPE, class T>
+// NW waves take a group together (group_waves): 1, or the block's four,
+// which then share its tiles.
+template <int D, int K, int TYPE, class T, int NW>
 __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, PreArgs a)
 {
     using Kern = typename KernelOf<D, K, T>::type;
     constexpr bool NUMBER = TYPE == SPHGPU_DISPH;
     __shared__ PreRec<T> l_r[PSW][WAVE];
     __shared__ int l_j[PSW][WAVE];
+    __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
+    const int part = w % NW;
     // the Newton sweeps stage 32-byte position and mass records in the same
     // LDS as the final sweep's records (64 of them per wave)
     double4 *const l_pm = reinterpret_cast<double4 *>(&l_r[w][0]);
@@ -174,7 +181,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                   "position and mass records fit the final sweep's slot");
     const int lane = wave_lane();
     // waves past the last group take part in the block's reduction only
-    const int grp = xcd_block() * PSW + w;
+    const int grp = xcd_block() * (PSW / NW) + w / NW;
     const bool have = grp < a.ngroups;
     const int2 gr = have ? a.groups[grp] : make_int2(0, 0);
     const int i = gr.x + lane;
@@ -241,9 +248,10 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                         }
                     }
                 };
-                tile_sweep(ntile, nstage, npair);
+                tile_sweep<NW>(part, ntile, nstage, npair);
+                parts_sum<NW, 2>(red, part, {&rho.s, &drho.s});
                 if(!done) {
-                    ++iters;
+                    iters += part == 0;
                     const double f = rho.val() * pow_dim<D>(hn) - b;
                     const double df = drho.val() * pow_dim<D>(hn) + D * rho.val() * pow_dim1<D>(hn);
                     hn -= f / df;
@@ -255,9 +263,9 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     h = hn;
                 } else {
                     h = Hs / a.ratio;
-                    ++fails;
+                    fails += part == 0;
                 }
-                if(h > Hs) ++trunc;
+                if(h > Hs) trunc += part == 0;
             }
         }
 
@@ -368,11 +376,39 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         // case), see tiles.hpp
         if constexpr(D == 3 && TYPE != SPHGPU_GSPH) {
             auto frefine = [&](uint64_t m) { return refine_bits(m, fkeep); };
-            tile_sweep(ntile, fstage, frefine, fpair);
+            tile_sweep<NW>(part, ntile, fstage, frefine, fpair);
         } else {
-            tile_sweep(ntile, fstage, fpair);
+            tile_sweep<NW>(part, ntile, fstage, fpair);
         }
-        if(valid) {
+        if constexpr(NW > 1) {
+            // whole sums in every part, of which the first writes the results
+            double cnt_d = (double)count;
+            parts_sum<NW, 2>(red, part, {&rho.s, &cnt_d});
+            count = (int)cnt_d;
+            if constexpr(TYPE == SPHGPU_DISPH) parts_sum<NW, 4>(red, part, {&nd.s, &dnd.s, &pb.s, &dpb.s});
+            if constexpr(TYPE == SPHGPU_SSPH) parts_sum<NW, 1>(red, part, {&drho.s});
+            if constexpr(TYPE == SPHGPU_GSPH) {
+                if(a.second_order) {
+#pragma unroll
+                    for(int l = 0; l < D; ++l) {
+                        parts_sum<NW, 2>(red, part, {&gd[l].s, &gu[l].s});
+#pragma unroll
+                        for(int c = 0; c < D; ++c) parts_sum<NW, 1>(red, part, {&gv[c][l].s});
+                    }
+                }
+            } else if(need_dv) {
+                parts_sum<NW, 4>(red, part, {&divv.s, &rot.c[0].s, &rot.c[1].s, &rot.c[2].s});
+            }
+            __syncthreads();
+            red.v[0][part][lane] = (double)vsig_max;
+            __syncthreads();
+#pragma unroll
+            for(int p = 0; p < NW; ++p) {
+                const T o = (T)red.v[0][p][lane];
+                vsig_max = o > vsig_max ? o : vsig_max;
+            }
+        }
+        if(valid && part == 0) {
             pairs = count;
             const double gm1 = a.gamma - 1.0;
             const double rho_d = rho.val();
@@ -502,7 +538,10 @@ constexpr int kNumPreInputs = 8;
 
 template <int D, int K, class T> static void launch_initial(Ctx &c, const PreArgs &a)
 {
-    hipLaunchKernelGGL((pre_initial_kernel<D, K, T>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), a);
+    if(group_waves(c, GROUP_PAIRS) > 1)
+        hipLaunchKernelGGL((pre_initial_kernel<D, K, T, PSW>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, make_box(c), a);
+    else
+        hipLaunchKernelGGL((pre_initial_kernel<D, K, T, 1>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), a);
 }
 
 template <class T> static void initial_t(Ctx &c, const PreArgs &a)
@@ -530,7 +569,10 @@ template <int D, int K, int TYPE, class T> static void launch_pre(Ctx &c, const 
 {
     hipLaunchKernelGGL((pack_pre_kernel<D, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n,
                        (PreRec<T> *)c.pair_rec, c.posrec);
-    hipLaunchKernelGGL((pre_kernel<D, K, TYPE, T>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
+    if(group_waves(c, GROUP_PAIRS) > 1)
+        hipLaunchKernelGGL((pre_kernel<D, K, TYPE, T, PSW>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
+    else
+        hipLaunchKernelGGL((pre_kernel<D, K, TYPE, T, 1>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
 }
 
 template <int D, int K, class T> static void launch_pre_t(Ctx &c, const PreArgs &a, const BoxDev &box)
@@ -563,7 +605,7 @@ int pre_compute(Ctx &c)
     else pre_t<double>(c, a, box);
     SPHGPU_HIP(hipGetLastError());
     c.gpart_fresh = a.gpart != nullptr;
-    return reduce_min_partials(c, group_grid(c), S_HVS);
+    return reduce_min_partials(c, group_waves(c, GROUP_PAIRS) > 1 ? c.ngroups : group_grid(c), S_HVS);
 }
 
 }  // namespace sphgpu

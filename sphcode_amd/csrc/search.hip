@@ -114,21 +114,35 @@ __device__ __forceinline__ bool box_near(const BoxDev &box, const ChunkBox &b, c
 // records are not written by this kernel).
 __device__ __forceinline__ double4 srec_at(const double4 *p, int i) { return load_ro(p + i); }
 
-template <int D, int MODE>
+// NW waves take a group together: 1, or the block's four.  Each of the four
+// tests all the boxes, stages every fourth pair of chunks in a buffer of its
+// own and tests every fourth pair of tiles.
+template <int D, int MODE, int NW>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_SEARCH))) search_kernel(BoxDev box, SearchArgs a)
 {
     constexpr bool IJ = MODE != M_GATHER;
+    static_assert(NW == 1 || NW == SW, "one wave or the whole block per group");
     __shared__ int l_chunk[SW][CHUNKCAP];
+    __shared__ int l_kept[NW > 1 ? SW : 1], l_hits[NW > 1 ? SW : 1][NW > 1 ? WAVE : 1];
+    __shared__ double l_reach[NW > 1 ? SW : 1];
 
     const int w = uniform(threadIdx.x / WAVE);
+    const int part = NW > 1 ? w : 0;  // this wave's part of the group
     const int lane = wave_lane();
     const int ngroups = uniform(*a.num_groups);
     // this wave's staging buffer
     const size_t wbase = (size_t)(blockIdx.x * SW + w) * (size_t)a.wcap;
     // persistent waves: groups are taken one at a time from this XCD's
-    // contiguous share of the Morton curve
+    // contiguous share of the Morton curve (a whole block: in turn)
     TaskShare share(a.work, ngroups);
-    for(int grp = share.next(); grp >= 0; grp = share.next()) {
+    int turn = NW > 1 ? xcd_block() : 0;
+    auto next = [&]() -> int {
+        if constexpr(NW == 1) return share.next();
+        const int t = turn < ngroups ? turn : -1;
+        turn += (int)gridDim.x;
+        return t;
+    };
+    for(int grp = next(); grp >= 0; grp = next()) {
     const int2 gr = make_int2(uniform(a.groups[grp].x), uniform(a.groups[grp].y));
     const int cnt = gr.y - gr.x;
     const bool valid = lane < cnt;
@@ -168,11 +182,11 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
         };
         int c_j = a.n;
         double4 c_q = make_double4(0.0, 0.0, 0.0, 0.0);
-        fetch(0, c_j, c_q);
-        for(int p = 0; p < nchunk; p += 2) {
+        fetch(2 * part, c_j, c_q);
+        for(int p = 2 * part; p < nchunk; p += 2 * NW) {
             int n_j = a.n;
             double4 n_q = make_double4(0.0, 0.0, 0.0, 0.0);
-            if(p + 2 < nchunk) fetch(p + 2, n_j, n_q);
+            if(p + 2 * NW < nchunk) fetch(p + 2 * NW, n_j, n_q);
             bool keep = false;
             if(c_j < a.n) {
                 // keep a candidate only if it lies within reach of the group
@@ -236,6 +250,25 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 
     // ---- phase 3: strided tiles of the kept candidates, the next tile's
     // records loaded while the current one is tested
+    // the staging writes of all lanes before their reads by other lanes
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    double reach = box.on ? wave_maxv(reach2) : 0.0;
+    int before[NW];  // candidates staged by the parts before each
+    before[0] = 0;
+    if constexpr(NW > 1) {
+        if(lane == 0) {
+            l_kept[w] = nkept;
+            l_reach[w] = reach;
+        }
+        __syncthreads();
+        nkept = 0;
+#pragma unroll
+        for(int k = 0; k < NW; ++k) {
+            before[k] = nkept;
+            nkept += uniform(l_kept[k]);
+            reach = l_reach[k] > reach ? l_reach[k] : reach;
+        }
+    }
     const int nc = nkept < a.wcap ? nkept : a.wcap;
     const int T = (nc + WAVE - 1) / WAVE;
     // Periodic box: every lane's minimum image of a candidate that can be a
@@ -245,18 +278,27 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     // every pair takes its own minimum image.
     bool wrap = false;
     if(box.on) {
-        const double H = sqrt(uniform_d(wave_maxv(reach2)));
+        const double H = sqrt(uniform_d(reach));
 #pragma unroll
         for(int k = 0; k < D; ++k) wrap = wrap || !(2.0 * ge[k] + H < 0.499 * box.len[k]);
     }
-    // the staging writes of all lanes before their reads by other lanes
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     auto fetch_c = [&](int c, int &j, double4 &q) {
         j = -1;
         // past the tile's end: at no finite distance
         q = make_double4(1e200, 1e200, 1e200, 0.0);
         if(c < nc) {
-            j = a.ws_j[wbase + c];
+            if constexpr(NW == 1) {
+                j = a.ws_j[wbase + c];
+            } else {
+                int k = 0, b = 0;
+#pragma unroll
+                for(int u = 1; u < NW; ++u)
+                    if(c >= before[u]) {
+                        k = u;
+                        b = before[u];
+                    }
+                j = a.ws_j[(size_t)(blockIdx.x * SW + k) * (size_t)a.wcap + (c - b)];
+            }
             q = a.srec[j];
         }
     };
@@ -284,8 +326,9 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
             }
         }
         // the next tiles' records, while these are tested
-        if(tt + V < T) fetch_c(tt + V + lane * T, p_j[0], p_q[0]);
-        if(V > 1 && tt + V + 1 < T) fetch_c(tt + V + 1 + lane * T, p_j[1], p_q[1]);
+        constexpr int S = V * NW;
+        if(tt + S < T) fetch_c(tt + S + lane * T, p_j[0], p_q[0]);
+        if(V > 1 && tt + S + 1 < T) fetch_c(tt + S + 1 + lane * T, p_j[1], p_q[1]);
         // particle after particle: the lanes' compares are its hit mask
         int lo[V] = {}, hi[V] = {};
         for(int i0 = 0; i0 < cnt; i0 += U) {
@@ -335,15 +378,27 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     };
     using One = std::integral_constant<int, 1>;
     using Two = std::integral_constant<int, 2>;
-    if(T > 0) fetch_c(lane * T, p_j[0], p_q[0]);
-    int tt = 0;
     if(wrap) {
-        for(; tt < T; ++tt) tiles(tt, std::true_type{}, One{});
+        int tt = part;
+        if(tt < T) fetch_c(tt + lane * T, p_j[0], p_q[0]);
+        for(; tt < T; tt += NW) tiles(tt, std::true_type{}, One{});
     } else {
-        if(T > 1) fetch_c(1 + lane * T, p_j[1], p_q[1]);
-        for(; tt + 1 < T; tt += 2) tiles(tt, std::false_type{}, Two{});
+        int tt = 2 * part;
+        if(tt < T) fetch_c(tt + lane * T, p_j[0], p_q[0]);
+        if(tt + 1 < T) fetch_c(tt + 1 + lane * T, p_j[1], p_q[1]);
+        for(; tt + 1 < T; tt += 2 * NW) tiles(tt, std::false_type{}, Two{});
         if(tt < T) tiles(tt, std::false_type{}, One{});
     }
+    if constexpr(NW > 1) {
+        l_hits[w][lane] = count;
+        __syncthreads();
+        count = 0;
+#pragma unroll
+        for(int k = 0; k < NW; ++k) count += l_hits[k][lane];
+        // (the next group's first barrier comes after these reads)
+        tested = part == 0 ? nkept : 0;
+    }
+    if(part != 0) continue;
     if(lane == 0) a.gnc[grp] = nc | (wrap ? GNC_WRAP : 0);
 
     // past the reference's list capacity (its unchecked write,
@@ -480,6 +535,11 @@ int search_boxes(Ctx &c, const double *rad)
 
 template <int D, int MODE> static void launch_search(Ctx &c, const SearchArgs &a, bool work_ready, int blocks_per_cu)
 {
+    if(group_waves(c, GROUP_SEARCH) > 1) {
+        const int blocks = std::min(c.ngroups, 8 * c.num_cu);
+        hipLaunchKernelGGL((search_kernel<D, MODE, SW>), dim3(blocks), dim3(BLOCK), 0, c.stream, make_box(c), a);
+        return;
+    }
     const BoxDev box = make_box(c);
     // blocks_per_cu blocks of 4 waves per CU (8 fill every CU), a multiple
     // of the XCD count; blocks beyond what the CUs hold find no task and leave
@@ -487,7 +547,7 @@ template <int D, int MODE> static void launch_search(Ctx &c, const SearchArgs &a
     if(!work_ready) reset_work(c, 0);
     SearchArgs aw = a;
     aw.work = c.work;
-    hipLaunchKernelGGL((search_kernel<D, MODE>), dim3(blocks), dim3(BLOCK), 0, c.stream, box, aw);
+    hipLaunchKernelGGL((search_kernel<D, MODE, 1>), dim3(blocks), dim3(BLOCK), 0, c.stream, box, aw);
 }
 
 template <int MODE> static int search_dispatch(Ctx &c, const SearchArgs &a, bool work_ready, int blocks_per_cu)

@@ -8,7 +8,8 @@
 // first anyway), each lane testing its own bits once the tile is visible
 // to the whole wave; pair(k) handles candidate k of the tile for this lane.
 // Each lane then walks the set bits of its mask, as a divergent loop, and
-// the wave moves to the next tile when every lane is done.
+// the wave moves to the next tile when every lane is done.  With NW waves
+// per group, wave `part` takes every NW-th tile.
 //
 // Refining pays where the search radius holds many more candidates than
 // the pair's cut-off keeps: in 3D a candidate within 1.2 h_guess passes
@@ -52,10 +53,10 @@ struct NoRefine {
     __device__ __forceinline__ uint64_t operator()(uint64_t m) const { return m; }
 };
 
-template <class Stage, class Refine, class Pair>
-__device__ __forceinline__ void tile_sweep(int ntile, Stage &&stage, Refine &&refine, Pair &&pair)
+template <int NW, class Stage, class Refine, class Pair>
+__device__ __forceinline__ void tile_sweep(int part, int ntile, Stage &&stage, Refine &&refine, Pair &&pair)
 {
-    for(int t = 0; t < ntile; ++t) {
+    for(int t = part; t < ntile; t += NW) {
         uint64_t m = stage(t);
         wave_lds_sync();
         m = refine(m);
@@ -68,10 +69,37 @@ __device__ __forceinline__ void tile_sweep(int ntile, Stage &&stage, Refine &&re
     }
 }
 
-template <class Stage, class Pair>
-__device__ __forceinline__ void tile_sweep(int ntile, Stage &&stage, Pair &&pair)
+template <int NW, class Stage, class Pair>
+__device__ __forceinline__ void tile_sweep(int part, int ntile, Stage &&stage, Pair &&pair)
 {
-    tile_sweep(ntile, stage, NoRefine{}, pair);
+    tile_sweep<NW>(part, ntile, stage, NoRefine{}, pair);
+}
+
+// Sums of the parts' values, lane by lane and part after part (a fixed
+// order), in every part: N values at a time through `red`, which all the
+// block's waves share.  Nothing to do with one wave per group.
+template <int NW> struct PartsLds {
+    double v[NW > 1 ? 4 : 1][NW][NW > 1 ? WAVE : 1];
+};
+
+template <int NW, int N>
+__device__ __forceinline__ void parts_sum(PartsLds<NW> &red, int part, double *const (&v)[N])
+{
+    static_assert(N <= 4, "four values at a time");
+    if constexpr(NW > 1) {
+        const int lane = wave_lane();
+        __syncthreads();  // the previous values have been read
+#pragma unroll
+        for(int k = 0; k < N; ++k) red.v[k][part][lane] = *v[k];
+        __syncthreads();
+#pragma unroll
+        for(int k = 0; k < N; ++k) {
+            double s = red.v[k][0][lane];
+#pragma unroll
+            for(int p = 1; p < NW; ++p) s += red.v[k][p][lane];
+            *v[k] = s;
+        }
+    }
 }
 
 // The bits of m whose candidate passes keep(k), tested by this lane.
