@@ -401,6 +401,7 @@ int force_compute(Ctx &c);
 // assigned acc).  gravity_compute runs all three on c.stream;
 // sphgpu_integrate overlaps the first two with the hydrodynamic stages.
 int gravity_compute(Ctx &c);
+int gravity_parts(int64_t n, int num_cu);  // waves per 64-particle group
 int gravity_walk(Ctx &c, hipStream_t st);
 int gravity_leaves(Ctx &c, hipStream_t st);
 int gravity_combine(Ctx &c, hipStream_t st);

@@ -126,6 +126,21 @@ template <int D, class T, bool RECORD = false> struct GravityVisitor {
         return om;
     }
 
+    // The lanes of `act` that open the node, by the same test.
+    __device__ __forceinline__ uint64_t opens(const GravNode &g, uint64_t act) const
+    {
+#pragma clang fp contract(off)
+        double d[D];
+        d[0] = xi[0] - g.cx;
+        if constexpr(D > 1) d[1] = xi[1] - g.cy;
+        if constexpr(D > 2) d[2] = xi[2] - g.cz;
+        min_image<D>(box, d);
+        double d2 = d[0] * d[0];
+#pragma unroll
+        for(int k = 1; k < D; ++k) d2 = d2 + d[k] * d[k];
+        return act & ballot(g.edge2 > theta2 * d2);
+    }
+
     __device__ __forceinline__ void leaf(int b, int e, uint64_t open)
     {
         if constexpr(RECORD) {
@@ -182,12 +197,48 @@ template <int D, class T, bool RECORD = false> struct GravityVisitor {
     }
 };
 
-// Split pass, part 1: the walk with monopoles only (no h needed), which
-// records the opened leaves per wave for part 2.
-template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(GravityOcc<T>::value))) gravity_walk_kernel(State s, TreeDev t, BoxDev box, int n, GravArgs a)
+// K waves share a 64-particle group: 1 (a block then holds four groups) or
+// more (a block holds one group's K waves).
+template <int K> struct GravShape {
+    static constexpr int waves = K > 1 ? K : BLOCK / WAVE;  // per block
+    static constexpr int threads = waves * WAVE;
+    static constexpr int groups = waves / K;
+};
+
+// Sums over a group's waves, lane by lane and part after part, in part 0.
+template <int D, int K, class V> __device__ __forceinline__ void join_parts(V &v, int part)
 {
-    const int i = xcd_block() * BLOCK + threadIdx.x;
-    const int task = uniform(i / WAVE);
+    if constexpr(K > 1) {
+        __shared__ double red[K][D + 1][WAVE];
+        const int lane = wave_lane();
+        if(part > 0) {
+#pragma unroll
+            for(int k = 0; k < D; ++k) red[part][k][lane] = v.acc[k].s;
+            red[part][D][lane] = v.phi.s;
+        }
+        __syncthreads();
+        if(part == 0)
+            for(int p = 1; p < K; ++p) {
+#pragma unroll
+                for(int k = 0; k < D; ++k) v.acc[k].s += red[p][k][lane];
+                v.phi.s += red[p][D][lane];
+            }
+    }
+}
+
+// Split pass, part 1: the walk with monopoles only (no h needed), which
+// records the opened leaves per wave for part 2.  With K waves, each walks
+// an equal share of the nodes.
+template <int D, class T, bool STATS, int K>
+__global__ void __launch_bounds__(GravShape<K>::threads) __attribute__((amdgpu_waves_per_eu(GravityOcc<T>::value)))
+gravity_walk_kernel(State s, TreeDev t, BoxDev box, int n, GravArgs a)
+{
+    constexpr int NW = GravShape<K>::waves;
+    const int w = uniform(threadIdx.x / WAVE);
+    const int part = w % K;
+    const int group = uniform(xcd_block() * GravShape<K>::groups + w / K);
+    const int i = group * WAVE + wave_lane();
+    const int task = group * K + part;
     const bool valid = i < n;
     GravityVisitor<D, T, true> v(box, nullptr);
     v.G = a.G;
@@ -196,20 +247,32 @@ template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) _
     v.rec = a.leafhit + (int64_t)task * LEAFHIT_CAP;
 #pragma unroll
     for(int k = 0; k < D; ++k) v.xi[k] = valid ? s.f[F_X + k][i] : 0.0;
-    __shared__ int stk_node[BLOCK / WAVE][WALK_STACK];
-    __shared__ uint64_t stk_mask[BLOCK / WAVE][WALK_STACK];
-    const int w = uniform(threadIdx.x / WAVE);
-    const WalkCount wc = tree_walk<STATS>(a.gnode, uniform(*t.num_nodes), valid, v, stk_node[w], stk_mask[w]);
-    if(valid) {
+    __shared__ int stk_node[NW][WALK_STACK];
+    __shared__ uint64_t stk_mask[NW][WALK_STACK];
+    const int total = uniform(*t.num_nodes);
+    const int first = K > 1 ? (int)((int64_t)total * part / K) : 0;
+    const int last = K > 1 ? (int)((int64_t)total * (part + 1) / K) : total;
+    const WalkCount wc = tree_walk<STATS>(a.gnode, first, last, valid, v, stk_node[w], stk_mask[w]);
+    join_parts<D, K>(v, part);
+    if(valid && part == 0) {
         s.f[F_PHI][i] = v.phi.val();
 #pragma unroll
         for(int k = 0; k < D; ++k) a.gacc[k * a.stride + i] = v.acc[k].val();
     }
+    // the leaves that the group opened
+    int nrec = v.nrec;
+    if constexpr(K > 1) {
+        __shared__ int l_rec[K];
+        if(wave_lane() == 0) l_rec[part] = v.nrec;
+        __syncthreads();
+        nrec = 0;
+        for(int p = 0; p < K; ++p) nrec += l_rec[p];
+    }
     if(wave_lane() == 0) {
         a.leafcnt[task] = v.nrec;
-        if(v.nrec > LEAFHIT_CAP) atomicAdd((unsigned long long *)&a.counters[C_GRAV_REWALK], 1ull);
+        if(part == 0 && nrec > LEAFHIT_CAP) atomicAdd((unsigned long long *)&a.counters[C_GRAV_REWALK], 1ull);
         if constexpr(STATS) {
-            stat_max(a.counters, task, C_GRAV_MAXREC, (unsigned)v.nrec);
+            if(part == 0) stat_max(a.counters, task, C_GRAV_MAXREC, (unsigned)nrec);
             stat_add(a.counters, task, C_GRAV_PP, (unsigned)wc.pairs);
             stat_add(a.counters, task, C_GRAV_PN, (unsigned)wc.accepted);
             stat_add(a.counters, task, C_GRAV_OPEN, (unsigned)wc.opened);
@@ -219,30 +282,44 @@ template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) _
 }
 
 // Split pass, part 2: the particle pairs of the recorded leaves (softened
-// with h_i and h_j), added to part 1's sums.  A wave whose record overflowed
-// walks the tree again in full and overwrites part 1's sums.
-template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(GravityOcc<T>::value))) gravity_leaf_kernel(State s, TreeDev t, BoxDev box, int n, GravArgs a)
+// with h_i and h_j), added to part 1's sums.  With K waves, each takes every
+// K-th of the group's records.  A group whose record overflowed is walked
+// again in full by its first wave, which overwrites part 1's sums.
+template <int D, class T, bool STATS, int K>
+__global__ void __launch_bounds__(GravShape<K>::threads) __attribute__((amdgpu_waves_per_eu(GravityOcc<T>::value)))
+gravity_leaf_kernel(State s, TreeDev t, BoxDev box, int n, GravArgs a)
 {
-    const int i = xcd_block() * BLOCK + threadIdx.x;
-    const int task = uniform(i / WAVE);
+    constexpr int NWV = GravShape<K>::waves;
+    const int w = uniform(threadIdx.x / WAVE);
+    const int part = w % K;
+    const int group = uniform(xcd_block() * GravShape<K>::groups + w / K);
+    const int lane = wave_lane();
+    const int i = group * WAVE + lane;
+    const int task = group * K + part;
     const bool valid = i < n;
-    const int nrec = uniform(a.leafcnt[task]);
+    // records of the group's waves, one list after the other
+    int before[K], nrec = 0;
+#pragma unroll
+    for(int p = 0; p < K; ++p) {
+        before[p] = nrec;
+        nrec += uniform(a.leafcnt[group * K + p]);
+    }
     double xi[D];
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = valid ? s.f[F_X + k][i] : 0.0;
     const T einv_i = valid ? (T)(2.0 * s.f[F_HINV][i]) : T(0);
     if(nrec > LEAFHIT_CAP) {
+        if(part != 0) return;
         GravityVisitor<D, T> v(box, (const GravPart<T> *)a.gpart);
         v.G = a.G;
         v.theta2 = a.theta2;
         v.einv_i = einv_i;
 #pragma unroll
         for(int k = 0; k < D; ++k) v.xi[k] = xi[k];
-        __shared__ int stk_node[BLOCK / WAVE][WALK_STACK];
-        __shared__ uint64_t stk_mask[BLOCK / WAVE][WALK_STACK];
-        const int w = uniform(threadIdx.x / WAVE);
-        const WalkCount wc = tree_walk<STATS>(a.gnode, uniform(*t.num_nodes), valid, v, stk_node[w], stk_mask[w]);
-        if(STATS && wave_lane() == 0) stat_add(a.counters, task, C_GRAV_SLOTS, (int64_t)WAVE * (unsigned)wc.slots);
+        __shared__ int stk_node[GravShape<K>::groups][WALK_STACK];
+        __shared__ uint64_t stk_mask[GravShape<K>::groups][WALK_STACK];
+        const WalkCount wc = tree_walk<STATS>(a.gnode, 0, uniform(*t.num_nodes), valid, v, stk_node[w / K], stk_mask[w / K]);
+        if(STATS && lane == 0) stat_add(a.counters, task, C_GRAV_SLOTS, (int64_t)WAVE * (unsigned)wc.slots);
         if(valid) {
             s.f[F_PHI][i] = v.phi.val();
 #pragma unroll
@@ -261,18 +338,17 @@ template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) _
     // every lane steps through the (leaf, particle) sequence of its set
     // bits at its own pace, so no lane waits on leaves that it did not
     // open.  A lane adds its pairs in the same order as a sweep over all
-    // records would (records in walk order, particles in tree order).  The
-    // records are taken LEAFHIT_CHUNK at a time, in order.
-    const LeafHit *rec = a.leafhit + (int64_t)task * LEAFHIT_CAP;
-    const int lane = wave_lane();
-    const int w = uniform(threadIdx.x / WAVE);
-    __shared__ int2 srec[BLOCK / WAVE][LEAFHIT_CHUNK];
+    // of the wave's records would (records in walk order, particles in tree
+    // order).  The records are taken LEAFHIT_CHUNK at a time, in order.
+    const LeafHit *rec = a.leafhit + (int64_t)group * K * LEAFHIT_CAP;
+    const int mycount = nrec > part ? (nrec - part + K - 1) / K : 0;
+    __shared__ int2 srec[NWV][LEAFHIT_CHUNK];
     constexpr int NW = LEAFHIT_CHUNK / WAVE;
     static_assert(NW == 4, "four record words per lane");
     const GravPart<T> *gp = (const GravPart<T> *)a.gpart;
     int iters = 0;
-    for(int base = 0; base < nrec; base += LEAFHIT_CHUNK) {
-        const int cnt = min(nrec - base, LEAFHIT_CHUNK);
+    for(int base = 0; base < mycount; base += LEAFHIT_CHUNK) {
+        const int cnt = min(mycount - base, LEAFHIT_CHUNK);
         const int nwords = (cnt + WAVE - 1) / WAVE;
         uint64_t mine[NW];
 #pragma unroll
@@ -282,7 +358,14 @@ template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) _
                 const int k = c * WAVE + lane;
                 uint64_t m = 0;
                 if(k < cnt) {
-                    const LeafHit h = rec[base + k];
+                    int r = (base + k) * K + part, p = 0, b = 0;
+#pragma unroll
+                    for(int u = 1; u < K; ++u)
+                        if(r >= before[u]) {
+                            p = u;
+                            b = before[u];
+                        }
+                    const LeafHit h = rec[(int64_t)p * LEAFHIT_CAP + (r - b)];
                     m = h.mask;
                     srec[w][k] = make_int2(h.b, h.e);
                 }
@@ -324,11 +407,29 @@ template <int D, class T, bool STATS> __global__ void __launch_bounds__(BLOCK) _
         wave_lds_sync();  // srec is refilled by the next round
     }
     if(STATS && lane == 0) stat_add(a.counters, task, C_GRAV_SLOTS, (int64_t)(2 * WAVE) * (unsigned)iters);
-    if(valid) {
+    join_parts<D, K>(v, part);
+    if(valid && part == 0) {
         s.f[F_PHI][i] += v.phi.val();
 #pragma unroll
         for(int k = 0; k < D; ++k) a.gacc[k * a.stride + i] += v.acc[k].val();
     }
+}
+
+// Waves that share a 64-particle group's walk and pair pass.  A group's walk
+// is a serial chain of some 1,500 node visits, so one wave per group needs
+// many groups to fill the chip; with more waves per group, each goes down to
+// its first node again and the scalar cache holds fewer of the nodes that
+// the block's waves read.  Whole step at leafParticleNumber 32, FP64 / mixed
+// (ms), with one, four and eight waves on 256 CUs:
+//    20,011        - / 0.89     - / 0.53     - / 0.49
+//    65,536     1.35 / 1.16  1.05 / 0.84  1.03 / 0.82
+//   131,072     1.92 / -     1.69 / -     1.76 / -
+//   200,000     1.94 / 1.59  1.93 / 1.48  2.16 / 1.63
+//   400,000     3.74 / 2.70  3.79 / 2.71  4.23 / 3.18
+int gravity_parts(int64_t n, int num_cu)
+{
+    const int64_t groups = grid_for(n, WAVE);
+    return groups <= 4 * num_cu ? 8 : groups <= 12 * num_cu ? 4 : 1;
 }
 
 static GravArgs grav_args(Ctx &c)
@@ -346,23 +447,40 @@ static GravArgs grav_args(Ctx &c)
     return a;
 }
 
+template <int D, class T, bool STATS, int K> static void launch_walk(Ctx &c, const GravArgs &a, const BoxDev &box, hipStream_t st)
+{
+    hipLaunchKernelGGL((gravity_walk_kernel<D, T, STATS, K>), dim3(grid_for(grid_for(c.n, WAVE), GravShape<K>::groups)),
+                       dim3(GravShape<K>::threads), 0, st, c.s, c.t, box, (int)c.n, a);
+}
+
+template <int D, class T, bool STATS, int K> static void launch_leaves(Ctx &c, const GravArgs &a, const BoxDev &box, hipStream_t st)
+{
+    hipLaunchKernelGGL((gravity_leaf_kernel<D, T, STATS, K>), dim3(grid_for(grid_for(c.n, WAVE), GravShape<K>::groups)),
+                       dim3(GravShape<K>::threads), 0, st, c.s, c.t, box, (int)c.n, a);
+}
+
+#define SPHGPU_GRAV_PARTS(LAUNCH, D)                                        \
+    switch(gravity_parts(c.n, c.num_cu)) {                                    \
+    case 1: LAUNCH<D, T, STATS, 1>(c, a, box, st); break;                     \
+    case 4: LAUNCH<D, T, STATS, 4>(c, a, box, st); break;                     \
+    default: LAUNCH<D, T, STATS, 8>(c, a, box, st); break;                    \
+    }
+
 template <class T, bool STATS> static void walk_d(Ctx &c, const GravArgs &a, const BoxDev &box, hipStream_t st)
 {
-    const int n = (int)c.n;
     switch(c.D) {
-    case 1: hipLaunchKernelGGL((gravity_walk_kernel<1, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
-    case 2: hipLaunchKernelGGL((gravity_walk_kernel<2, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
-    default: hipLaunchKernelGGL((gravity_walk_kernel<3, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
+    case 1: SPHGPU_GRAV_PARTS(launch_walk, 1); break;
+    case 2: SPHGPU_GRAV_PARTS(launch_walk, 2); break;
+    default: SPHGPU_GRAV_PARTS(launch_walk, 3); break;
     }
 }
 
 template <class T, bool STATS> static void leaves_d(Ctx &c, const GravArgs &a, const BoxDev &box, hipStream_t st)
 {
-    const int n = (int)c.n;
     switch(c.D) {
-    case 1: hipLaunchKernelGGL((gravity_leaf_kernel<1, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
-    case 2: hipLaunchKernelGGL((gravity_leaf_kernel<2, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
-    default: hipLaunchKernelGGL((gravity_leaf_kernel<3, T, STATS>), dim3(grid_for(n)), dim3(BLOCK), 0, st, c.s, c.t, box, n, a); break;
+    case 1: SPHGPU_GRAV_PARTS(launch_leaves, 1); break;
+    case 2: SPHGPU_GRAV_PARTS(launch_leaves, 2); break;
+    default: SPHGPU_GRAV_PARTS(launch_leaves, 3); break;
     }
 }
 

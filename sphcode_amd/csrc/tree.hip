@@ -527,8 +527,9 @@ int tree_alloc(Ctx &c)
         // one spare record: a scalar load may fetch a whole record past the last
         SPHGPU_HIP(hipMalloc(&c.gpart, (n + 1) * sizeof(GravPart<double>)));
         SPHGPU_HIP(hipMalloc(&c.gacc, (size_t)c.D * n * sizeof(double)));
-        // one record slot per wave of a grid_for(n)-block launch
-        const size_t waves = (size_t)grid_for(n) * (BLOCK / WAVE);
+        // one record list per wave: a wave per 64 particles in blocks of
+        // four, or several
+        const size_t waves = (size_t)grid_for(n) * (BLOCK / WAVE) * gravity_parts(n, c.num_cu);
         SPHGPU_HIP(hipMalloc(&c.leafhit, waves * LEAFHIT_CAP * sizeof(LeafHit)));
         SPHGPU_HIP(hipMalloc(&c.leafcnt, waves * sizeof(int)));
     }

@@ -50,8 +50,14 @@ struct WalkCount {
     int opened = 0, accepted = 0, pairs = 0;
 };
 
+//
+// A walk may cover only the nodes [first, total) of the pre-order (several
+// waves then share a group's walk): it first goes down from the root to
+// `first` along that node's ancestors, where the lanes take the same opening
+// decisions (v.opens, which sums nothing); the lanes that do not open an
+// ancestor are parked at its skip index as ever.
 template <bool STATS, class V>
-__device__ __forceinline__ WalkCount tree_walk(const GravNode *gn, int total, bool valid, V &v, int *stk_node,
+__device__ __forceinline__ WalkCount tree_walk(const GravNode *gn, int first, int total, bool valid, V &v, int *stk_node,
                                                uint64_t *stk_mask)
 {
     WalkCount wc;
@@ -79,20 +85,59 @@ __device__ __forceinline__ WalkCount tree_walk(const GravNode *gn, int total, bo
     // lane keeps one.
     // The loop tests for the end at the bottom only, so the visitor's sums
     // stay in the same registers from one visit to the next.
-    if(active == 0 || total <= 0) return wc;
+    if(active == 0 || total <= first) return wc;
     const char *gnb = reinterpret_cast<const char *>(gn);
+    // the whole 64-byte record in one scalar load (the compiler would
+    // otherwise split it by the fields used into five); the empty asm
+    // statement only keeps all sixteen words live
+    auto load = [&](int k) -> GravNode {
+        GravNode g;
+        typedef uint32_t u16v __attribute__((ext_vector_type(16)));
+        const u16v raw = *(const __attribute__((address_space(4))) u16v *)(gnb + ((uint32_t)k << 6));
+        asm volatile("" ::"s"(raw));
+        __builtin_memcpy(&g, &raw, sizeof(GravNode));
+        return g;
+    };
+    // parks lanes at a skip index (the stack stays sorted: an index pushed
+    // is never above the top's)
+    auto park = [&](int skip, uint64_t fm) {
+        if(top_node == skip) {
+            top_mask |= fm;
+        } else {
+            if(top_node != WALK_DONE && sp < WALK_STACK) {
+                stk_node[sp] = top_node;
+                stk_mask[sp] = top_mask;
+                ++sp;
+            }
+            top_node = skip;
+            top_mask = fm;
+        }
+    };
+    if(first > 0) {
+        while(node < first) {
+            const GravNode g = load(node);
+            if(g.skip <= first) {
+                node = g.skip;
+                continue;
+            }
+            // an ancestor of `first`, so it has children
+            const uint64_t om = v.opens(g, active);
+            if(active & ~om) park(g.skip, active & ~om);
+            active = om;
+            if(active == 0) break;
+            node = node + 1;
+        }
+        if(active == 0) {
+            // no lane gets to `first`: on to the first parked ones
+            node = top_node;
+            active = top_mask;
+            pop();
+            if(node >= total) return wc;
+        }
+    }
     do {
         if constexpr(STATS) ++wc.visits;
-        // the whole 64-byte record in one scalar load (the compiler would
-        // otherwise split it by the fields used into five); the empty asm
-        // statement only keeps all sixteen words live
-        GravNode g;
-        {
-            typedef uint32_t u16v __attribute__((ext_vector_type(16)));
-            const u16v raw = *(const __attribute__((address_space(4))) u16v *)(gnb + ((uint32_t)node << 6));
-            asm volatile("" ::"s"(raw));
-            __builtin_memcpy(&g, &raw, sizeof(GravNode));
-        }
+        const GravNode g = load(node);
         const int skip = g.skip;
         const uint64_t om = v.node(g, active);
         if constexpr(STATS) {
@@ -111,20 +156,7 @@ __device__ __forceinline__ WalkCount tree_walk(const GravNode *gn, int total, bo
             node = skip;
         } else {
             const uint64_t fm = active & ~om;
-            if(fm) {
-                // park the lanes that accepted this node at its skip index
-                if(top_node == skip) {
-                    top_mask |= fm;
-                } else {
-                    if(top_node != WALK_DONE && sp < WALK_STACK) {
-                        stk_node[sp] = top_node;
-                        stk_mask[sp] = top_mask;
-                        ++sp;
-                    }
-                    top_node = skip;
-                    top_mask = fm;
-                }
-            }
+            if(fm) park(skip, fm);  // the lanes that accepted this node
             active = om;
             node = node + 1;
         }
