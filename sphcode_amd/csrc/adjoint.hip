@@ -14,9 +14,9 @@
 // implicit function theorem on G(h, x) = rho(h, x) h^D - m N_ngb / A_D = 0,
 // which the Newton iteration solves (src/pre_interaction.cpp:227-283).
 //
-// All pair sums of the adjoint are gathers over the symmetric force list
-// (r < max(h_i, h_j)), which contains every pair of the gather sets
-// (r < h_i) in either direction: particle k collects the derivative of every
+// All pair sums of the adjoint are gathers over the search's candidate tiles,
+// whose hits hold every force pair (r < max(h_i, h_j)) and with them every
+// pair of the gather sets (r < h_i) in either direction: particle k collects the derivative of every
 // pair term with respect to its own variables, so no atomics are needed.
 // Three passes per force evaluation:
 //   1. force pairs  -> adjoints of x, v (direct), h, rho, A = P Omega / rho^2,
@@ -26,9 +26,20 @@
 //   3. gather pairs -> adjoints of x and v through those sums
 // The pair arithmetic follows the context's precision (FP64, or FP32 with
 // FP64 accumulation); the per-particle chain rule and the IFT are FP64.
+//
+// Each pass runs as the forward pair passes do (tiles.hpp): a wave or four
+// per search group, the neighbours' records staged through LDS once per
+// group.  They are bound by vector issue.  Reading per-particle neighbour
+// lists expanded from the tiles instead, one global load per field and pair,
+// they were bound by those scattered loads and by the expansion (mixed,
+// 262,144 particles: lists 574 us and passes 426, 124 and 344 us, now 170,
+// 97 and 171 us; FP64, 29,791 particles: 243, 146, 81 and 124 us, now 55, 34
+// and 53 us).  The records' sizes are no multiple of 64 bytes: lanes reading
+// different records of a tile would meet in a few LDS banks.
 #include <vector>
 
-#include "ctx.hpp"
+#include "tiles.hpp"
+
 #include "kderiv.hpp"
 
 namespace sphgpu {
@@ -44,12 +55,8 @@ enum Work : int {
     W_AB = 12,     // adjoint of A = P Omega / rho^2
     W_BB = 13,     // adjoint of the Balsara switch
     W_CB = 14,     // adjoint of the sound speed
-    W_SRHO = 15,   // seed on sum m W
-    W_SRHOP = 16,  // seed on sum m dW/dh
-    W_SDV = 17,    // seed on sum m v_ij . grad W
-    W_SRV = 18,    // seed on sum m v_ij x grad W (3)
-    W_UB = 21,     // adjoint of u
-    NWORK = 22
+    W_UB = 15,     // adjoint of u
+    NWORK = 16
 };
 
 // checkpointed fields: what one step or Solver::initialize reads
@@ -64,10 +71,31 @@ static int ck_fields(int D, int *f)
     return k;
 }
 
+// Neighbour records: the fields of j read by passes 1 and 2 ...
+template <class T> struct __align__(16) AdjRec {
+    T hinv, rho, A, bal, c, alpha, m, duf;  // A = P Omega / rho^2
+    T v[3], af[3];
+    T pad[sizeof(T) == 4 ? 6 : 4];
+};
+static_assert(sizeof(AdjRec<float>) == 80 && sizeof(AdjRec<double>) == 144, "AdjRec size");
+// ... and by pass 3, written by pass 2
+template <class T> struct __align__(16) SeedRec {
+    T h, hinv, m, srho, srhop, sdv;
+    T v[3], srv[3];
+    T pad[sizeof(T) == 4 ? 8 : 2];
+};
+static_assert(sizeof(SeedRec<float>) == 80 && sizeof(SeedRec<double>) == 112, "SeedRec size");
+
 struct AdjArgs {
-    const int *list;
-    const int *cnt;
-    int cap;
+    const int2 *groups;
+    int ngroups;
+    const int *cand;     // candidate tiles (Ctx::tile_cand)
+    const uint64_t *ma;
+    const int *gnc;
+    int wcap;
+    double4 *pos;        // x, y, z, h
+    void *rec;           // AdjRec<T>
+    void *seed;          // SeedRec<T>
     double *w;       // work arrays
     int64_t n;       // their stride
     double *adj;     // adjoint state, caller order
@@ -89,17 +117,35 @@ template <int D> struct AdjLayout {
     static constexpr int X = 0, V = D, U = 2 * D, A = 2 * D + 1, DU = 3 * D + 1, N = 3 * D + 2;
 };
 
-// seeds of F from the adjoint of the step's output state
-template <int D> __global__ void __launch_bounds__(BLOCK) adj_seed_kernel(State s, int n, AdjArgs a)
+// Seeds of F from the adjoint of the step's output state, and the records
+// of passes 1 and 2.
+template <int D, class T> __global__ void __launch_bounds__(BLOCK) adj_seed_kernel(State s, int n, AdjArgs a)
 {
     using L = AdjLayout<D>;
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     if(i >= n) return;
     const int id = s.id[i];
     const double half = a.kick ? 0.5 * a.dt : 0.0;
+    AdjRec<T> r{};
 #pragma unroll
-    for(int k = 0; k < D; ++k) W(a, W_AF + k, i) = ADJ<D>(a, L::A + k, id) + half * ADJ<D>(a, L::V + k, id);
-    W(a, W_DUF, i) = ADJ<D>(a, L::DU, id) + half * ADJ<D>(a, L::U, id);
+    for(int k = 0; k < D; ++k) {
+        const double af = ADJ<D>(a, L::A + k, id) + half * ADJ<D>(a, L::V + k, id);
+        W(a, W_AF + k, i) = af;
+        r.af[k] = (T)af;
+        r.v[k] = fld<T>(s, F_V + k, i);
+    }
+    const double duf = ADJ<D>(a, L::DU, id) + half * ADJ<D>(a, L::U, id);
+    W(a, W_DUF, i) = duf;
+    r.duf = (T)duf;
+    r.hinv = T(1) / fld<T>(s, F_SML, i);
+    r.rho = fld<T>(s, F_DENS, i);
+    r.A = fld<T>(s, F_PRES, i) * fld<T>(s, F_GRADH, i) / (r.rho * r.rho);
+    r.bal = fld<T>(s, F_BAL, i);
+    r.c = fld<T>(s, F_SOUND, i);
+    r.alpha = fld<T>(s, F_ALPHA, i);
+    r.m = fld<T>(s, F_MASS, i);
+    ((AdjRec<T> *)a.rec)[i] = r;
+    a.pos[i] = make_double4(s.f[F_X][i], D > 1 ? s.f[F_X + 1][i] : 0.0, D > 2 ? s.f[F_X + 2][i] : 0.0, s.f[F_SML][i]);
 }
 
 // Pair arithmetic of the passes: T = double, or float in mixed precision
@@ -112,14 +158,81 @@ template <class T> __device__ __forceinline__ T pair_r(double r2)
     else return gather_r_f32(r2);
 }
 
+// One wave's view of its group: particle, tiles, and the staging of the
+// candidates' positions (and a record each) in LDS.
+constexpr int ASW = BLOCK / WAVE;
+template <int D, int NW> struct AdjGroup {
+    int w, lane, part, grp, i;
+    bool have, valid;
+    size_t gbase;
+    int gnc, ntile;
+    __device__ __forceinline__ explicit AdjGroup(const AdjArgs &a)
+    {
+        w = threadIdx.x / WAVE;
+        lane = wave_lane();
+        part = w % NW;
+        grp = xcd_block() * (ASW / NW) + w / NW;
+        have = grp < a.ngroups;
+        const int2 gr = have ? a.groups[grp] : make_int2(0, 0);
+        i = gr.x + lane;
+        valid = have && i < gr.y;
+        if(!valid) i = gr.x;
+        gbase = (size_t)(have ? grp : 0) * a.wcap;
+        gnc = have ? uniform(a.gnc[grp]) : 0;
+        ntile = ((gnc & ~GNC_WRAP) + WAVE - 1) / WAVE;
+    }
+    template <class R>
+    __device__ __forceinline__ uint64_t stage(const AdjArgs &a, const GroupImage<D> &img, int tt, double4 *l_p, R *l_r, const R *rec) const
+    {
+        const size_t o = gbase + (size_t)tt * WAVE;
+        const int jl = stream_ld(a.cand + o + lane);
+        if(jl >= 0) {
+            double4 q = a.pos[jl];
+            q.x = img.at(0, q.x);
+            if constexpr(D > 1) q.y = img.at(1, q.y);
+            if constexpr(D > 2) q.z = img.at(2, q.z);
+            l_p[lane] = q;
+            l_r[lane] = rec[jl];
+        }
+        return valid ? stream_ld(a.ma + o + lane) : 0ull;
+    }
+};
+
+template <int D> __device__ __forceinline__ double pair_sep2(const GroupImage<D> &img, const double xi[D], const double4 &q, double d[D])
+{
+    double xj[D];
+    xj[0] = q.x;
+    if constexpr(D > 1) xj[1] = q.y;
+    if constexpr(D > 2) xj[2] = q.z;
+    return sep2<D>(img.pairs, xi, xj, d);
+}
+
+// The sweep of a pass: in 3D each lane's hits are first narrowed to those
+// that `keep` accepts (see tiles.hpp).
+template <int D, int NW, class Stage, class Keep, class Pair>
+__device__ __forceinline__ void adj_sweep(const AdjGroup<D, NW> &g, Stage &&stage, Keep &&keep, Pair &&pair)
+{
+    if constexpr(D == 3) {
+        auto refine = [&](uint64_t m) { return refine_bits(m, keep); };
+        tile_sweep<NW>(g.part, g.ntile, stage, refine, pair);
+    } else {
+        tile_sweep<NW>(g.part, g.ntile, stage, [&](int k) {
+            if(keep(k)) pair(k);
+        });
+    }
+}
+
 // pass 1: force pairs (src/fluid_force.cpp:26-106)
-template <int D, int K, class T>
-__global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, int n, AdjArgs a)
+template <int D, int K, class T, int NW>
+__global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, AdjArgs a)
 {
     constexpr bool FP64 = sizeof(T) == 8;
-    const int i = xcd_block() * BLOCK + threadIdx.x;
-    if(i >= n) return;
-    const int total = a.cnt[i];
+    __shared__ double4 l_p[ASW][WAVE];
+    __shared__ AdjRec<T> l_r[ASW][WAVE];
+    __shared__ PartsLds<NW> red;
+    const AdjGroup<D, NW> g(a);
+    if(!g.have) return;  // (one wave per group only)
+    const int i = g.i, w = g.w;
     double xi[D];
     T vi[D], afi[D];
 #pragma unroll
@@ -128,58 +241,57 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, i
         vi[k] = (T)s.f[F_V + k][i];
         afi[k] = (T)W(a, W_AF + k, i);
     }
+    const GroupImage<D> img(box, g.gnc, xi);
     const double hi_d = s.f[F_SML][i];
-    const T hi = (T)hi_d, rhoi = (T)s.f[F_DENS][i], pi_ = (T)s.f[F_PRES][i], omi = (T)s.f[F_GRADH][i];
+    const T hi_inv = T(1) / (T)hi_d, rhoi = (T)s.f[F_DENS][i], pi_ = (T)s.f[F_PRES][i], omi = (T)s.f[F_GRADH][i];
     const T bi = (T)s.f[F_BAL][i], ci = (T)s.f[F_SOUND][i], ali = (T)s.f[F_ALPHA][i], mi = (T)s.f[F_MASS][i];
     const T dufi = (T)W(a, W_DUF, i);
     const T Ai = pi_ * omi / (rhoi * rhoi);
 
     Acc<T> xb[D], vb[D], hb, rhob, Ab, Bb, cb;
-    for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, kk, a.cap)];
-        double xj[D], dd[D];
-#pragma unroll
-        for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
-        const double r2 = sep2<D>(box, xi, xj, dd);
-        const double hj_d = s.f[F_SML][j];
-        const double hmax = hi_d < hj_d ? hj_d : hi_d;
-        T r;
+    auto keep = [&](int kc) -> bool {
+        const double4 q = l_p[w][kc];
+        double dd[D];
+        const double r2 = pair_sep2<D>(img, xi, q, dd);
+        const double hmax = hi_d < q.w ? q.w : hi_d;
         if constexpr(FP64) {
-            r = sqrt(r2);
-            if(r >= hmax || r == 0.0) continue;
+            const double r = sqrt(r2);
+            return !(r >= hmax || r == 0.0);
         } else {
-            if(!(r2 < hmax * hmax) || r2 == 0.0) continue;
-            r = sqrtf((float)r2);
+            return r2 < hmax * hmax && r2 != 0.0;
         }
+    };
+    auto pair = [&](int kc) {
+        const AdjRec<T> &j = l_r[w][kc];
+        double dd[D];
+        const double r2 = pair_sep2<D>(img, xi, l_p[w][kc], dd);
+        T r;
+        if constexpr(FP64) r = sqrt(r2);
+        else r = sqrtf((float)r2);
         T d[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) d[k] = (T)dd[k];
-        const T hj = fld<T>(s, F_SML, j);
-        const T rhoj = fld<T>(s, F_DENS, j), pj = fld<T>(s, F_PRES, j), omj = fld<T>(s, F_GRADH, j);
-        const T bj = fld<T>(s, F_BAL, j), cj = fld<T>(s, F_SOUND, j), alj = fld<T>(s, F_ALPHA, j);
-        const T mj = fld<T>(s, F_MASS, j);
-        const T dufj = (T)W(a, W_DUF, j);
-        const T Aj = pj * omj / (rhoj * rhoj);
-        const KernelDerivs<T> ki = kernel_derivs<D, K, T>(r, hi);
-        const KernelDerivs<T> kj = kernel_derivs<D, K, T>(r, hj);
+        const T rhoj = j.rho, bj = j.bal, cj = j.c, alj = j.alpha, mj = j.m, dufj = j.duf, Aj = j.A;
+        const KernelDerivs<T> ki = kernel_derivs_inv<D, K, T>(r, hi_inv);
+        const KernelDerivs<T> kj = kernel_derivs_inv<D, K, T>(r, j.hinv);
         const T gi = ki.f, gj = kj.f, gb = T(0.5) * (gi + gj);
         T v[D], beta[D];
         T sv = T(0), b = T(0);
 #pragma unroll
         for(int k = 0; k < D; ++k) {
-            v[k] = vi[k] - fld<T>(s, F_V + k, j);
-            beta[k] = mi * (T)W(a, W_AF + k, j) - mj * afi[k];
+            v[k] = vi[k] - j.v[k];
+            beta[k] = mi * j.af[k] - mj * afi[k];
             sv += v[k] * d[k];
             b += beta[k] * d[k];
         }
         const T psii = mj * dufi, psij = mi * dufj, psis = psii + psij;
         // Monaghan viscosity Pi = K (C - 3 w) w for w = v.r / r < 0
-        T Pi = T(0), Kv = T(0), w = T(0);
+        T Pi = T(0), Kv = T(0), wv = T(0);
         const T Cs = ci + cj, rhos = rhoi + rhoj, al2 = ali + alj;
         if(sv < T(0)) {
-            w = sv / r;
+            wv = sv / r;
             Kv = T(-0.25) * (bi + bj) * al2 / rhos;
-            Pi = Kv * (Cs - T(3) * w) * w;
+            Pi = Kv * (Cs - T(3) * wv) * wv;
         }
         const T Phi = Ai * gi + Aj * gj + Pi * gb;
         const T EPi = (b + T(0.5) * sv * psis) * gb;
@@ -188,12 +300,12 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, i
         T Es = psii * Ai * gi + psij * Aj * gj + T(0.5) * psis * Pi * gb;
         T Er = Egi * ki.fr + Egj * kj.fr;
         if(sv < T(0)) {
-            const T Piw = Kv * (Cs - T(6) * w);
+            const T Piw = Kv * (Cs - T(6) * wv);
             Es += EPi * Piw / r;
-            Er -= EPi * Piw * w / r;
+            Er -= EPi * Piw * wv / r;
             rhob.add(-(EPi * Pi / rhos));
-            cb.add(EPi * Kv * w);
-            Bb.add(EPi * (Cs - T(3) * w) * w * (T(-0.25) * al2 / rhos));
+            cb.add(EPi * Kv * wv);
+            Bb.add(EPi * (Cs - T(3) * wv) * wv * (T(-0.25) * al2 / rhos));
         }
         const T er = Er / r;
 #pragma unroll
@@ -203,7 +315,14 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, i
         }
         hb.add(Egi * ki.fh);
         Ab.add((b + sv * psii) * gi);
-    }
+    };
+    const AdjRec<T> *rec = (const AdjRec<T> *)a.rec;
+    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
+#pragma unroll
+    for(int k = 0; k < D; ++k) parts_sum<NW, 2>(red, g.part, {&xb[k].s, &vb[k].s});
+    parts_sum<NW, 4>(red, g.part, {&hb.s, &rhob.s, &Ab.s, &Bb.s});
+    parts_sum<NW, 1>(red, g.part, {&cb.s});
+    if(!g.valid || g.part != 0) return;
 #pragma unroll
     for(int k = 0; k < D; ++k) {
         W(a, W_XB + k, i) = xb[k].val();
@@ -231,12 +350,15 @@ template <int D, class T> __device__ __forceinline__ void cross_vr(const T v[D],
 
 // pass 2: gather sums of particle i and the chain rule through its
 // derived quantities (src/pre_interaction.cpp:66-169), the latter in FP64
-template <int D, int K, class T>
-__global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int n, AdjArgs a)
+template <int D, int K, class T, int NW>
+__global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, AdjArgs a)
 {
-    const int i = xcd_block() * BLOCK + threadIdx.x;
-    if(i >= n) return;
-    const int total = a.cnt[i];
+    __shared__ double4 l_p[ASW][WAVE];
+    __shared__ AdjRec<T> l_r[ASW][WAVE];
+    __shared__ PartsLds<NW> red;
+    const AdjGroup<D, NW> gp(a);
+    if(!gp.have) return;  // (one wave per group only)
+    const int i = gp.i, w = gp.w;
     double xi[D];
     T vi[D];
 #pragma unroll
@@ -244,28 +366,31 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
         xi[k] = s.f[F_X + k][i];
         vi[k] = (T)s.f[F_V + k][i];
     }
+    const GroupImage<D> img(box, gp.gnc, xi);
     const double h = s.f[F_SML][i];
-    const T ht = (T)h;
+    const T ht = (T)h, ht_inv = T(1) / ht;
     Acc<T> rho_a, rhop_a, rhopp_a, Dv_a, Dvh_a, Rv_a[3], Rvh_a[3];
-    for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, kk, a.cap)];
-        double xj[D], dd[D];
-#pragma unroll
-        for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
-        const double r2 = sep2<D>(box, xi, xj, dd);
+    auto keep = [&](int kc) -> bool {
+        double dd[D];
+        return pair_r<T>(pair_sep2<D>(img, xi, l_p[w][kc], dd)) < ht;
+    };
+    auto pair = [&](int kc) {
+        const AdjRec<T> &j = l_r[w][kc];
+        double dd[D];
+        const double r2 = pair_sep2<D>(img, xi, l_p[w][kc], dd);
         const T r = pair_r<T>(r2);
-        if(!(r < ht)) continue;
-        const T mj = fld<T>(s, F_MASS, j);
-        const KernelDerivs<T> kd = kernel_derivs<D, K, T>(r, ht);
+        const T mj = j.m;
+        const KernelDerivs<T> kd = kernel_derivs_inv<D, K, T>(r, ht_inv);
         rho_a.add(mj * kd.w);
         rhop_a.add(mj * kd.wh);
         rhopp_a.add(mj * kd.whh);
-        if(j != i && a.balsara && D > 1) {
+        // (particle i itself adds nothing to the sums over v_ij)
+        if(a.balsara && D > 1) {
             T v[D], d[D], sv = T(0);
 #pragma unroll
             for(int k = 0; k < D; ++k) {
                 d[k] = (T)dd[k];
-                v[k] = vi[k] - fld<T>(s, F_V + k, j);
+                v[k] = vi[k] - j.v[k];
                 sv += v[k] * d[k];
             }
             T cr[3];
@@ -278,7 +403,15 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
                 Rvh_a[k].add(mj * cr[k] * kd.fh);
             }
         }
+    };
+    const AdjRec<T> *rec = (const AdjRec<T> *)a.rec;
+    adj_sweep<D, NW>(gp, [&](int tt) { return gp.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
+    parts_sum<NW, 3>(red, gp.part, {&rho_a.s, &rhop_a.s, &rhopp_a.s});
+    if(a.balsara && D > 1) {
+        parts_sum<NW, 4>(red, gp.part, {&Dv_a.s, &Rv_a[0].s, &Rv_a[1].s, &Rv_a[2].s});
+        parts_sum<NW, 4>(red, gp.part, {&Dvh_a.s, &Rvh_a[0].s, &Rvh_a[1].s, &Rvh_a[2].s});
     }
+    if(!gp.valid || gp.part != 0) return;
     const double rho = rho_a.val(), rhop = rhop_a.val(), rhopp = rhopp_a.val(), Dv = Dv_a.val(), Dvh = Dvh_a.val();
     const double Rv[3] = {Rv_a[0].val(), Rv_a[1].val(), Rv_a[2].val()};
     const double Rvh[3] = {Rvh_a[0].val(), Rvh_a[1].val(), Rvh_a[2].val()};
@@ -332,11 +465,18 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
     const double hD1 = ipow<double, D - 1>(h);
     const double Gh = rhop * hD1 * h + D * rho * hD1;
     const double g = -hb / Gh;
-    W(a, W_SRHO, i) = rhob + g * hD1 * h;
-    W(a, W_SRHOP, i) = rhopb;
-    W(a, W_SDV, i) = Dvb;
+    SeedRec<T> o{};
+    o.h = fld<T>(s, F_SML, i);
+    o.hinv = T(1) / o.h;
+    o.m = fld<T>(s, F_MASS, i);
+    o.srho = (T)(rhob + g * hD1 * h);
+    o.srhop = (T)rhopb;
+    o.sdv = (T)Dvb;
 #pragma unroll
-    for(int k = 0; k < 3; ++k) W(a, W_SRV + k, i) = Rvb[k];
+    for(int k = 0; k < D; ++k) o.v[k] = fld<T>(s, F_V + k, i);
+#pragma unroll
+    for(int k = 0; k < 3; ++k) o.srv[k] = (T)Rvb[k];
+    ((SeedRec<T> *)a.seed)[i] = o;
     // c = sqrt(gamma (gamma - 1) u)
     if(ci > 0.0) ub += cb * a.gamma * gm1 / (2.0 * ci);
     W(a, W_UB, i) = ub;
@@ -345,10 +485,10 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, int
 // derivative of the seeded sum terms of one pair with respect to r_ij and
 // v_ij; the terms are even in (r_ij, v_ij), so both ends use the same form
 template <int D, int K, class T>
-__device__ __forceinline__ void sum_term(T r, const T d[D], const T v[D], T sv, T m, T h, T srho, T srhop, T sdv,
+__device__ __forceinline__ void sum_term(T r, const T d[D], const T v[D], T sv, T m, T hinv, T srho, T srhop, T sdv,
                                          const T srv[3], Acc<T> xb[D], Acc<T> vb[D])
 {
-    const KernelDerivs<T> kd = kernel_derivs<D, K, T>(r, h);
+    const KernelDerivs<T> kd = kernel_derivs_inv<D, K, T>(r, hinv);
     T gQd[D], gQv[D], Q = T(0);
     if constexpr(D == 3) {
         // Q = srv . (v x r):  dQ/dr = srv x v,  dQ/dv = r x srv
@@ -379,12 +519,15 @@ __device__ __forceinline__ void sum_term(T r, const T d[D], const T v[D], T sv, 
 
 // pass 3: adjoint of x and v through the seeded gather sums of i (pairs
 // with r < h_i) and of its neighbours j (pairs with r < h_j)
-template <int D, int K, class T>
-__global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, int n, AdjArgs a)
+template <int D, int K, class T, int NW>
+__global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, AdjArgs a)
 {
-    const int i = xcd_block() * BLOCK + threadIdx.x;
-    if(i >= n) return;
-    const int total = a.cnt[i];
+    __shared__ double4 l_p[ASW][WAVE];
+    __shared__ SeedRec<T> l_r[ASW][WAVE];
+    __shared__ PartsLds<NW> red;
+    const AdjGroup<D, NW> g(a);
+    if(!g.have) return;  // (one wave per group only)
+    const int i = g.i, w = g.w;
     double xi[D];
     T vi[D];
 #pragma unroll
@@ -392,33 +535,33 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, int
         xi[k] = s.f[F_X + k][i];
         vi[k] = (T)s.f[F_V + k][i];
     }
-    const T hi = (T)s.f[F_SML][i], mi = (T)s.f[F_MASS][i];
-    const T srho_i = (T)W(a, W_SRHO, i), srhop_i = (T)W(a, W_SRHOP, i), sdv_i = (T)W(a, W_SDV, i);
-    const T srv_i[3] = {(T)W(a, W_SRV, i), (T)W(a, W_SRV + 1, i), (T)W(a, W_SRV + 2, i)};
+    const GroupImage<D> img(box, g.gnc, xi);
+    const SeedRec<T> *rec = (const SeedRec<T> *)a.seed;
+    const SeedRec<T> me = rec[i];
     Acc<T> xb[D], vb[D];
-    for(int kk = 0; kk < total; ++kk) {
-        const int j = a.list[list_at(i, kk, a.cap)];
-        double xj[D], dd[D];
-#pragma unroll
-        for(int k = 0; k < D; ++k) xj[k] = s.f[F_X + k][j];
-        const T r = pair_r<T>(sep2<D>(box, xi, xj, dd));
-        const T hj = fld<T>(s, F_SML, j);
-        const bool in_i = r < hi, in_j = r < hj;
-        if(r == T(0) || !(in_i || in_j)) continue;
+    auto keep = [&](int kc) -> bool {
+        double dd[D];
+        const T r = pair_r<T>(pair_sep2<D>(img, xi, l_p[w][kc], dd));
+        return r != T(0) && (r < me.h || r < l_r[w][kc].h);
+    };
+    auto pair = [&](int kc) {
+        const SeedRec<T> &j = l_r[w][kc];
+        double dd[D];
+        const T r = pair_r<T>(pair_sep2<D>(img, xi, l_p[w][kc], dd));
         T v[D], d[D], sv = T(0);
 #pragma unroll
         for(int k = 0; k < D; ++k) {
             d[k] = (T)dd[k];
-            v[k] = vi[k] - fld<T>(s, F_V + k, j);
+            v[k] = vi[k] - j.v[k];
             sv += v[k] * d[k];
         }
-        if(in_i) sum_term<D, K, T>(r, d, v, sv, fld<T>(s, F_MASS, j), hi, srho_i, srhop_i, sdv_i, srv_i, xb, vb);
-        if(in_j) {
-            const T srv_j[3] = {(T)W(a, W_SRV, j), (T)W(a, W_SRV + 1, j), (T)W(a, W_SRV + 2, j)};
-            sum_term<D, K, T>(r, d, v, sv, mi, hj, (T)W(a, W_SRHO, j), (T)W(a, W_SRHOP, j), (T)W(a, W_SDV, j), srv_j,
-                              xb, vb);
-        }
-    }
+        if(r < me.h) sum_term<D, K, T>(r, d, v, sv, j.m, me.hinv, me.srho, me.srhop, me.sdv, me.srv, xb, vb);
+        if(r < j.h) sum_term<D, K, T>(r, d, v, sv, me.m, j.hinv, j.srho, j.srhop, j.sdv, j.srv, xb, vb);
+    };
+    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
+#pragma unroll
+    for(int k = 0; k < D; ++k) parts_sum<NW, 2>(red, g.part, {&xb[k].s, &vb[k].s});
+    if(!g.valid || g.part != 0) return;
 #pragma unroll
     for(int k = 0; k < D; ++k) {
         W(a, W_XB + k, i) += xb[k].val();
@@ -460,13 +603,20 @@ template <int D> __global__ void __launch_bounds__(BLOCK) adj_state_kernel(State
     }
 }
 
+template <int D, int K, class T, int NW> static void launch_pairs(Ctx &c, const AdjArgs &a, const BoxDev &box)
+{
+    const int g = NW > 1 ? c.ngroups : group_grid(c);
+    hipLaunchKernelGGL((adj_force_kernel<D, K, T, NW>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, a);
+    hipLaunchKernelGGL((adj_pre_kernel<D, K, T, NW>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, a);
+    hipLaunchKernelGGL((adj_sum_kernel<D, K, T, NW>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, a);
+}
+
 template <int D, int K, class T> static void launch_passes_t(Ctx &c, const AdjArgs &a, const BoxDev &box)
 {
     const int g = grid_for(c.n);
-    hipLaunchKernelGGL((adj_seed_kernel<D>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, a);
-    hipLaunchKernelGGL((adj_force_kernel<D, K, T>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
-    hipLaunchKernelGGL((adj_pre_kernel<D, K, T>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
-    hipLaunchKernelGGL((adj_sum_kernel<D, K, T>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
+    hipLaunchKernelGGL((adj_seed_kernel<D, T>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, a);
+    if(group_waves(c, GROUP_PAIRS) > 1) launch_pairs<D, K, T, ASW>(c, a, box);
+    else launch_pairs<D, K, T, 1>(c, a, box);
     hipLaunchKernelGGL((adj_state_kernel<D>), dim3(g), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, a);
 }
 
@@ -479,9 +629,15 @@ template <int D, int K> static void launch_passes(Ctx &c, const AdjArgs &a, cons
 int adjoint_step(Ctx &c, bool kick)
 {
     AdjArgs a{};
-    a.list = c.list;
-    a.cnt = c.list_cnt;
-    a.cap = c.cap;
+    a.groups = c.groups;
+    a.ngroups = c.ngroups;
+    a.cand = c.tile_cand;
+    a.ma = c.tile_ma;
+    a.gnc = c.tile_nc;
+    a.wcap = c.tile_wcap;
+    a.pos = c.posrec;  // free after the force pass
+    a.rec = c.ro.rec;
+    a.seed = c.ro.seed;
     a.w = c.ro.work;
     a.n = c.ro.n;
     a.adj = c.ro.adj;
@@ -507,6 +663,8 @@ void adjoint_free(Ctx &c)
     if(c.ro.ck_id) (void)hipFree(c.ro.ck_id);
     if(c.ro.adj) (void)hipFree(c.ro.adj);
     if(c.ro.work) (void)hipFree(c.ro.work);
+    if(c.ro.rec) (void)hipFree(c.ro.rec);
+    if(c.ro.seed) (void)hipFree(c.ro.seed);
     c.ro = Ctx::Rollout{};
 }
 
@@ -527,6 +685,9 @@ int adjoint_alloc(Ctx &c, int steps)
     SPHGPU_HIP(hipMalloc(&c.ro.ck_id, (size_t)slots * n * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.ro.adj, (size_t)(3 * c.D + 2) * n * sizeof(double)));
     SPHGPU_HIP(hipMalloc(&c.ro.work, (size_t)NWORK * n * sizeof(double)));
+    const bool mixed = c.p.precision == SPHGPU_MIXED;
+    SPHGPU_HIP(hipMalloc(&c.ro.rec, n * (mixed ? sizeof(AdjRec<float>) : sizeof(AdjRec<double>))));
+    SPHGPU_HIP(hipMalloc(&c.ro.seed, n * (mixed ? sizeof(SeedRec<float>) : sizeof(SeedRec<double>))));
     c.ro.n = c.n;
     c.ro.slots = slots;
     c.ro.steps = 0;

@@ -109,7 +109,6 @@ static void free_buffers(Ctx &c)
     fr(c.gnode); fr(c.gpart); fr(c.gacc); fr(c.leafhit); fr(c.leafcnt); fr(c.posrec); fr(c.pair_rec); fr(c.grad_rec);
     if(c.lvl_host) (void)hipHostFree(c.lvl_host);
     c.lvl_host = nullptr;
-    fr(c.list); fr(c.list_cnt);
     fr(c.srec); fr(c.boxes); fr(c.leaf_rad);
     fr(c.tile_cand); fr(c.tile_ma); fr(c.tile_nc); fr(c.ws_j);
     c.tile_wcap = 0;
@@ -144,10 +143,7 @@ static int alloc_buffers(Ctx &c, int64_t n)
     SPHGPU_HIP(hipMalloc(&c.alt.id, np * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.s.nb, np * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.alt.nb, np * sizeof(int)));
-    // per-particle lists are expanded from the candidate tiles only for the
-    // adjoint (allocated then, ensure_lists)
     const size_t lsz = (size_t)np * (size_t)c.cap;
-    SPHGPU_HIP(hipMalloc(&c.list_cnt, np * sizeof(int)));
     // block partials: per 256 particles, or per block of four search groups
     // (up to one group per particle)
     const int64_t npart = std::max<int64_t>(grid_for(np), 1024) * 8 + np / 4 + 64;
@@ -166,14 +162,6 @@ static int alloc_buffers(Ctx &c, int64_t n)
 
 // Reads the error counters; a list overflow or node-pool exhaustion since
 // the last check becomes an error status.
-// Neighbour lists in list_at layout (the adjoint's input), allocated on
-// first use.
-static int ensure_lists(Ctx &c)
-{
-    if(!c.list) SPHGPU_HIP(hipMalloc(&c.list, (size_t)c.cap_n * (size_t)c.cap * sizeof(int)));
-    return SPHGPU_OK;
-}
-
 // Reads the counters (and, with the scalars, the scalars as well: they
 // share one allocation, so one copy brings both) and reports the errors
 // they record.
@@ -274,11 +262,9 @@ static int stage_pre(Ctx &c, bool walk = false)
         kmark(c, 1);
     }
     if(c.record) {
-        if((rc = search_expand(c, c.rec_gather, c.rec_gather_cnt, true))) return rc;
+        if((rc = search_record(c, c.rec_gather, c.rec_gather_cnt))) return rc;
         c.have_gather = true;
     }
-    if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, false))))
-        return rc;
     if(walk && (rc = launch_gravity_walk(c))) return rc;
     kmark(c, 2);
     if((rc = pre_compute(c))) return rc;
@@ -287,7 +273,7 @@ static int stage_pre(Ctx &c, bool walk = false)
     if(combined) {
         // the combined lists hold every force pair unless some h outgrew its
         // search radius (src/pre_interaction.cpp:70 truncates the gather set)
-        if(c.speculate && !c.need_lists && !c.record) {
+        if(c.speculate && !c.record) {
             // sphgpu_integrate: the force pass starts on the combined lists
             // at once and stage_force checks the counters once it is queued
             // (a truncation, which needs a new search, is rare)
@@ -311,8 +297,6 @@ static int stage_force(Ctx &c)
     int rc;
     if(!c.lists_symmetric) {
         if((rc = search_symmetric(c))) return rc;
-        if(c.need_lists && ((rc = ensure_lists(c)) || (rc = search_expand(c, c.list, c.list_cnt, false))))
-            return rc;
     }
     c.lists_symmetric = false;
     kmark(c, 4);
@@ -550,8 +534,6 @@ int sphgpu_upload(void *ptr, const sphgpu_particles *h)
     } else {
         hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s.nb, n, 0);
     }
-    // list slots beyond n stay empty
-    hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(c.cap_n)), dim3(BLOCK), 0, c.stream, c.list_cnt, c.cap_n, 0);
     SPHGPU_HIP(hipGetLastError());
     SPHGPU_HIP(hipStreamSynchronize(c.stream));
     c.uploaded = true;
@@ -885,14 +867,6 @@ int sphgpu_rollout_adjoint(void *ptr, const double *dl_dx, const double *dl_dv, 
     if(c.ro.steps < 1 || c.ro.n != c.n) return set_error(SPHGPU_E_STATE, "rollout adjoint: no stored rollout");
     const int K = c.ro.steps;
     if((rc = adjoint_seed(c, dl_dx, dl_dv, dl_du))) return rc;
-    if((rc = ensure_lists(c))) return rc;
-    // the recomputed steps expand their candidate tiles into lists, which
-    // the adjoint passes read
-    struct ListsOn {
-        Ctx &c;
-        explicit ListsOn(Ctx &c_) : c(c_) { c.need_lists = true; }
-        ~ListsOn() { c.need_lists = false; }
-    } lists_on(c);
     for(int k = K; k >= 0; --k) {
         if((rc = rollout_recompute(c, k))) return rc;
         if((rc = adjoint_step(c, k > 0))) return rc;

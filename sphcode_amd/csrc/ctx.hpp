@@ -301,15 +301,10 @@ struct Ctx {
     int64_t ws_waves = 0;          // search waves the staging is allocated for
     int ngroups = 0;               // groups of the last tree (host copy)
 
-    // neighbour lists (addressing: list_at), expanded from the tiles when
-    // the adjoint or the set record needs them (need_lists): particle i's
-    // hits are its first list_cnt[i] entries
-    int *list = nullptr;
-    int *list_cnt = nullptr;
-    bool need_lists = false;       // expand every search's tiles into list
     bool lists_symmetric = false;  // the tiles hold every force pair
     int64_t trunc_seen = 0;        // truncation counter at the last check
-    int *rec_gather = nullptr, *rec_gather_cnt = nullptr;  // recorded sets (debug)
+    // recorded sets (debug): lists in list_at addressing
+    int *rec_gather = nullptr, *rec_gather_cnt = nullptr;
     int *rec_force = nullptr, *rec_force_cnt = nullptr;
     bool record = false;
     bool have_gather = false, have_force = false;
@@ -340,6 +335,8 @@ struct Ctx {
         int *ck_id = nullptr;   // (K + 2) slots x n
         double *adj = nullptr;  // adjoint of the state, caller order
         double *work = nullptr; // per-stage adjoint arrays, device order
+        void *rec = nullptr;    // neighbour records of the adjoint's pair passes
+        void *seed = nullptr;
         int slots = 0;          // allocated slots
     } ro;
 
@@ -387,7 +384,7 @@ int search_alloc_particles(Ctx &c);
 int search_combined(Ctx &c, bool work_ready, int blocks_per_cu);  // gather and symmetric candidates in one search
 int search_blocks(const Ctx &c, bool beside_walk);
 int search_alloc(Ctx &c);        // tile slabs for c.ngroups groups (after a tree build)
-int search_expand(Ctx &c, int *list, int *cnt, bool gather_only);  // tiles -> list_at lists
+int search_record(Ctx &c, int *list, int *cnt);  // the gather sets of the tiles as list_at lists
 // pre.hip
 int pre_initial(Ctx &c);         // initial_smoothing density
 int pre_compute(Ctx &c);         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients

@@ -77,12 +77,11 @@ template <class T, int D> KD_FN T ipow(T x)
     return y;
 }
 
-// K = 0: cubic spline, K = 1: Wendland C4
-template <int D, int K, class T> KD_FN KernelDerivs<T> kernel_derivs(T r, T h)
+// K = 0: cubic spline, K = 1: Wendland C4; hinv = 1/h
+template <int D, int K, class T> KD_FN KernelDerivs<T> kernel_derivs_inv(T r, T hinv)
 {
     constexpr T kappa = K == 0 ? T(2) : T(1);
     const T C = K == 0 ? T(KernelConst<D>::cubic) : T(KernelConst<D>::wendland);
-    const T hinv = T(1) / h;
     const T q = kappa * r * hinv;
     T phi, d1, d2, psi, dpsi;
     if constexpr(K == 0) cubic_shape<T>(q, phi, d1, d2, psi, dpsi);
@@ -100,6 +99,11 @@ template <int D, int K, class T> KD_FN KernelDerivs<T> kernel_derivs(T r, T h)
     o.fr = kappa * kappa * kappa * h3 * dpsi;
     o.fh = -kappa * kappa * h3 * (T(D + 2) * psi + q * dpsi);
     return o;
+}
+
+template <int D, int K, class T> KD_FN KernelDerivs<T> kernel_derivs(T r, T h)
+{
+    return kernel_derivs_inv<D, K, T>(r, T(1) / h);
 }
 
 }  // namespace sphgpu

@@ -711,14 +711,14 @@ int search_alloc(Ctx &c)
     return SPHGPU_OK;
 }
 
-// Lists in list_at layout from the tiles of the last search: lane l of a
-// group appends its hits in staging order (candidate c = t + kT is bit k of
-// tile t).  gather_only keeps the gather candidates r < R_i (sml before the
-// pre-interaction).  Entries past cap are dropped (the search reports them).
+// The gather sets as lists in list_at layout, from the tiles of the last
+// search (debug): lane l of a group appends its hits with r < R_i (sml before
+// the pre-interaction) in staging order (candidate c = t + kT is bit k of
+// tile t).  Entries past cap are dropped (the search reports them).
 template <int D>
-__global__ void __launch_bounds__(BLOCK) expand_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
+__global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
                                                        const int *cand, const uint64_t *ma, int wcap, int cap,
-                                                       int gather_only, int *list, int *cnt)
+                                                       int *list, int *cnt)
 {
     const int grp = xcd_block() * (BLOCK / WAVE) + (int)(threadIdx.x / WAVE);
     if(grp >= ngroups) return;
@@ -741,30 +741,28 @@ __global__ void __launch_bounds__(BLOCK) expand_kernel(State s, BoxDev box, cons
             const size_t o = gbase + (size_t)t * WAVE;
             if(!((ma[o + lane] >> k) & 1ull)) continue;
             const int j = cand[o + k];
-            if(gather_only) {
-                double xj[D], d[D];
+            double xj[D], d[D];
 #pragma unroll
-                for(int q = 0; q < D; ++q) xj[q] = s.f[F_X + q][j];
-                if(!(sep2<D>(box, xi, xj, d) < h2)) continue;
-            }
+            for(int q = 0; q < D; ++q) xj[q] = s.f[F_X + q][j];
+            if(!(sep2<D>(box, xi, xj, d) < h2)) continue;
             if(wf < cap) list[lb + list_off(wf++)] = j;
         }
     }
     cnt[i] = wf;
 }
 
-template <int D> static void launch_expand(Ctx &c, int *list, int *cnt, bool gather_only)
+template <int D> static void launch_record(Ctx &c, int *list, int *cnt)
 {
-    hipLaunchKernelGGL(expand_kernel<D>, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
-                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, gather_only ? 1 : 0, list, cnt);
+    hipLaunchKernelGGL(record_kernel<D>, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
+                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, list, cnt);
 }
 
-int search_expand(Ctx &c, int *list, int *cnt, bool gather_only)
+int search_record(Ctx &c, int *list, int *cnt)
 {
     switch(c.D) {
-    case 1: launch_expand<1>(c, list, cnt, gather_only); break;
-    case 2: launch_expand<2>(c, list, cnt, gather_only); break;
-    default: launch_expand<3>(c, list, cnt, gather_only); break;
+    case 1: launch_record<1>(c, list, cnt); break;
+    case 2: launch_record<2>(c, list, cnt); break;
+    default: launch_record<3>(c, list, cnt); break;
     }
     SPHGPU_HIP(hipGetLastError());
     return SPHGPU_OK;
