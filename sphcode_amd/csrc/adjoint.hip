@@ -694,29 +694,46 @@ int adjoint_alloc(Ctx &c, int steps)
     return SPHGPU_OK;
 }
 
-int adjoint_save(Ctx &c, int slot)
+// Copies of a slot's fields and ids in one launch (the state's arrays are
+// separate allocations; a copy call for each took 18 launches of 5 us).
+struct SlotCopy {
+    const double *src[20];
+    double *dst[20];
+    const int *isrc;
+    int *idst;
+    int nf;
+};
+
+__global__ void __launch_bounds__(BLOCK) slot_copy_kernel(SlotCopy c, int n)
+{
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if(i >= n) return;
+    for(int k = 0; k < c.nf; ++k) c.dst[k][i] = c.src[k][i];
+    c.idst[i] = c.isrc[i];
+}
+
+static int slot_copy(Ctx &c, int slot, bool save)
 {
     int f[32];
     const int nck = ck_fields(c.D, f);
     const size_t n = (size_t)c.n;
-    for(int k = 0; k < nck; ++k)
-        SPHGPU_HIP(hipMemcpyAsync(c.ro.ck + ((size_t)slot * nck + k) * n, c.s.f[f[k]], n * sizeof(double),
-                                  hipMemcpyDeviceToDevice, c.stream));
-    SPHGPU_HIP(hipMemcpyAsync(c.ro.ck_id + (size_t)slot * n, c.s.id, n * sizeof(int), hipMemcpyDeviceToDevice, c.stream));
+    SlotCopy s{};
+    s.nf = nck;
+    for(int k = 0; k < nck; ++k) {
+        double *ck = c.ro.ck + ((size_t)slot * nck + k) * n;
+        s.src[k] = save ? c.s.f[f[k]] : ck;
+        s.dst[k] = save ? ck : c.s.f[f[k]];
+    }
+    int *id = c.ro.ck_id + (size_t)slot * n;
+    s.isrc = save ? c.s.id : id;
+    s.idst = save ? id : c.s.id;
+    hipLaunchKernelGGL(slot_copy_kernel, dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, s, (int)c.n);
+    SPHGPU_HIP(hipGetLastError());
     return SPHGPU_OK;
 }
 
-int adjoint_restore(Ctx &c, int slot)
-{
-    int f[32];
-    const int nck = ck_fields(c.D, f);
-    const size_t n = (size_t)c.n;
-    for(int k = 0; k < nck; ++k)
-        SPHGPU_HIP(hipMemcpyAsync(c.s.f[f[k]], c.ro.ck + ((size_t)slot * nck + k) * n, n * sizeof(double),
-                                  hipMemcpyDeviceToDevice, c.stream));
-    SPHGPU_HIP(hipMemcpyAsync(c.s.id, c.ro.ck_id + (size_t)slot * n, n * sizeof(int), hipMemcpyDeviceToDevice, c.stream));
-    return SPHGPU_OK;
-}
+int adjoint_save(Ctx &c, int slot) { return slot_copy(c, slot, true); }
+int adjoint_restore(Ctx &c, int slot) { return slot_copy(c, slot, false); }
 
 // host seeds (caller order, n*D for vectors; NULL = 0) into the adjoint state
 int adjoint_seed(Ctx &c, const double *dx, const double *dv, const double *du)
