@@ -739,35 +739,35 @@ int adjoint_restore(Ctx &c, int slot) { return slot_copy(c, slot, false); }
 int adjoint_seed(Ctx &c, const double *dx, const double *dv, const double *du)
 {
     const int D = c.D;
-    const size_t n = (size_t)c.n;
-    std::vector<double> h((size_t)(3 * D + 2) * n, 0.0);
-    for(size_t i = 0; i < n; ++i)
-        for(int k = 0; k < D; ++k) {
-            if(dx) h[(size_t)k * n + i] = dx[i * D + k];
-            if(dv) h[(size_t)(D + k) * n + i] = dv[i * D + k];
-        }
-    if(du)
-        for(size_t i = 0; i < n; ++i) h[(size_t)2 * D * n + i] = du[i];
-    SPHGPU_HIP(hipMemcpyAsync(c.ro.adj, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
-    return SPHGPU_OK;
+    const int64_t n = c.n;
+    Xfer x;
+    auto put = [&](const double *src, int comps, int row) {
+        const int off = src ? x.add(const_cast<double *>(src), comps) : -1;
+        for(int k = 0; k < comps; ++k) x.field(c.ro.adj + (row + k) * n, off, comps, k);
+    };
+    // the rows of AdjLayout: x, v, u, a, du
+    put(dx, D, 0);
+    put(dv, D, D);
+    put(du, 1, 2 * D);
+    put(nullptr, D, 2 * D + 1);
+    put(nullptr, 1, 3 * D + 1);
+    return xfer_upload(c, x, n);
 }
 
 int adjoint_fetch(Ctx &c, double *dx, double *dv, double *du)
 {
     const int D = c.D;
-    const size_t n = (size_t)c.n;
-    std::vector<double> h((size_t)(2 * D + 1) * n);
-    SPHGPU_HIP(hipMemcpyAsync(h.data(), c.ro.adj, h.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
-    for(size_t i = 0; i < n; ++i)
-        for(int k = 0; k < D; ++k) {
-            if(dx) dx[i * D + k] = h[(size_t)k * n + i];
-            if(dv) dv[i * D + k] = h[(size_t)(D + k) * n + i];
-        }
-    if(du)
-        for(size_t i = 0; i < n; ++i) du[i] = h[(size_t)2 * D * n + i];
-    return SPHGPU_OK;
+    const int64_t n = c.n;
+    Xfer x;
+    auto get = [&](double *dst, int comps, int row) {
+        if(!dst) return;
+        const int off = x.add(dst, comps);
+        for(int k = 0; k < comps; ++k) x.field(c.ro.adj + (row + k) * n, off, comps, k);
+    };
+    get(dx, D, 0);
+    get(dv, D, D);
+    get(du, 1, 2 * D);
+    return xfer_download(c, x, n);
 }
 
 }  // namespace sphgpu

@@ -44,12 +44,6 @@ void reset_work(Ctx &c, int slot)
                        (int64_t)NUM_XCD * WORK_STRIDE, 0);
 }
 
-__global__ void iota_kernel(int *p, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if(i < n) p[i] = (int)i;
-}
-
 __global__ void fill_double_kernel(double *p, int64_t n, double v)
 {
     const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
@@ -459,6 +453,7 @@ int sphgpu_destroy(void *ptr)
     (void)hipStreamSynchronize(c->stream);
     if(c->gstream) (void)hipStreamSynchronize(c->gstream);
     adjoint_free(*c);
+    xfer_free(*c);
     free_buffers(*c);
     if(c->scal) (void)hipFree(c->scal);  // with the counters
     if(c->work) (void)hipFree(c->work);
@@ -502,40 +497,34 @@ int sphgpu_upload(void *ptr, const sphgpu_particles *h)
         if(rc) return rc;
     }
     c.n = n;
-    std::vector<double> tmp(n);
-    auto put = [&](int f, const double *src, int stride, int comp) -> int {
-        if(!c.s.f[f]) return SPHGPU_OK;
-        if(!src) {
-            hipLaunchKernelGGL(fill_double_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s.f[f], n, 0.0);
-            return SPHGPU_OK;
+    // every field is written: from the caller's array, or zero
+    Xfer x;
+    auto put = [&](int f, const double *src, int comps, auto slot) {
+        int off = -1;
+        for(int k = 0; k < comps; ++k) {
+            double *dev = c.s.f[slot(f, k)];
+            if(!dev) continue;
+            if(src && off < 0) off = x.add(const_cast<double *>(src), comps);
+            x.field(dev, off, comps, k);
         }
-        for(int64_t i = 0; i < n; ++i) tmp[i] = src[i * stride + comp];
-        SPHGPU_HIP(hipMemcpy(c.s.f[f], tmp.data(), n * sizeof(double), hipMemcpyHostToDevice));
-        return SPHGPU_OK;
     };
-    int rc = 0;
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
-    for(int k = 0; k < D && !rc; ++k) {
-        rc = rc ? rc : put(F_X + k, h->pos, D, k);
-        rc = rc ? rc : put(F_V + k, h->vel, D, k);
-        rc = rc ? rc : put(F_VP + k, h->vel_p, D, k);
-        rc = rc ? rc : put(F_A + k, h->acc, D, k);
-        rc = rc ? rc : put(F_GD + k, h->grad_density, D, k);
-        rc = rc ? rc : put(F_GP + k, h->grad_pressure, D, k);
-        for(int l = 0; l < D && !rc; ++l) rc = put(F_GV + 3 * k + l, h->grad_velocity, D * D, k * D + l);
-    }
+    auto vec = [](int f, int k) { return f + k; };
+    auto mat = [D](int f, int k) { return f + 3 * (k / D) + k % D; };
+    put(F_X, h->pos, D, vec);
+    put(F_V, h->vel, D, vec);
+    put(F_VP, h->vel_p, D, vec);
+    put(F_A, h->acc, D, vec);
+    put(F_GD, h->grad_density, D, vec);
+    put(F_GP, h->grad_pressure, D, vec);
+    put(F_GV, h->grad_velocity, D * D, mat);
     const double *sc[] = {h->mass, h->dens, h->pres, h->ene, h->ene_p, h->dene, h->sml, h->sound, h->balsara, h->alpha, h->gradh, h->phi};
-    for(int f = F_MASS; f <= F_PHI && !rc; ++f) rc = put(f, sc[f - F_MASS], 1, 0);
-    if(!rc && c.s.f[F_HINV]) rc = put(F_HINV, nullptr, 1, 0);
+    for(int f = F_MASS; f <= F_PHI; ++f) put(f, sc[f - F_MASS], 1, vec);
+    put(F_HINV, nullptr, 1, vec);
+    x.dev_ints = c.s.nb;
+    x.user_ints = const_cast<int32_t *>(h->neighbor);
+    x.dev_id = c.s.id;
+    int rc = xfer_upload(c, x, n);
     if(rc) return rc;
-    hipLaunchKernelGGL(iota_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s.id, n);
-    if(h->neighbor) {
-        SPHGPU_HIP(hipMemcpy(c.s.nb, h->neighbor, n * sizeof(int), hipMemcpyHostToDevice));
-    } else {
-        hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s.nb, n, 0);
-    }
-    SPHGPU_HIP(hipGetLastError());
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
     c.uploaded = true;
     c.first_pre = true;
     c.tree_ready = false;
@@ -550,40 +539,30 @@ int sphgpu_download(void *ptr, sphgpu_particles *h)
     if(!h || h->n != c.n) return set_error(SPHGPU_E_INVALID, "particle count mismatch");
     const int64_t n = c.n;
     const int D = c.D;
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
-    std::vector<int> id(n);
-    SPHGPU_HIP(hipMemcpy(id.data(), c.s.id, n * sizeof(int), hipMemcpyDeviceToHost));
-    std::vector<double> tmp(n);
-    auto get = [&](int f, double *dst, int stride, int comp) -> int {
-        if(!dst) return SPHGPU_OK;
-        if(!c.s.f[f]) {
-            for(int64_t i = 0; i < n; ++i) dst[(int64_t)id[i] * stride + comp] = 0.0;
-            return SPHGPU_OK;
-        }
-        SPHGPU_HIP(hipMemcpy(tmp.data(), c.s.f[f], n * sizeof(double), hipMemcpyDeviceToHost));
-        for(int64_t i = 0; i < n; ++i) dst[(int64_t)id[i] * stride + comp] = tmp[i];
-        return SPHGPU_OK;
+    Xfer x;
+    auto get = [&](int f, double *dst, int comps, auto slot) {
+        if(!dst) return;
+        const int off = x.add(dst, comps);
+        for(int k = 0; k < comps; ++k) x.field(c.s.f[slot(f, k)], off, comps, k);  // (zeros if the field has no array)
     };
-    int rc = 0;
-    for(int k = 0; k < D && !rc; ++k) {
-        rc = rc ? rc : get(F_X + k, h->pos, D, k);
-        rc = rc ? rc : get(F_V + k, h->vel, D, k);
-        rc = rc ? rc : get(F_VP + k, h->vel_p, D, k);
-        rc = rc ? rc : get(F_A + k, h->acc, D, k);
-        rc = rc ? rc : get(F_GD + k, h->grad_density, D, k);
-        rc = rc ? rc : get(F_GP + k, h->grad_pressure, D, k);
-        for(int l = 0; l < D && !rc; ++l) rc = get(F_GV + 3 * k + l, h->grad_velocity, D * D, k * D + l);
-    }
+    auto vec = [](int f, int k) { return f + k; };
+    auto mat = [D](int f, int k) { return f + 3 * (k / D) + k % D; };
+    get(F_X, h->pos, D, vec);
+    get(F_V, h->vel, D, vec);
+    get(F_VP, h->vel_p, D, vec);
+    get(F_A, h->acc, D, vec);
+    get(F_GD, h->grad_density, D, vec);
+    get(F_GP, h->grad_pressure, D, vec);
+    get(F_GV, h->grad_velocity, D * D, mat);
     double *sc[] = {h->mass, h->dens, h->pres, h->ene, h->ene_p, h->dene, h->sml, h->sound, h->balsara, h->alpha, h->gradh, h->phi};
-    for(int f = F_MASS; f <= F_PHI && !rc; ++f) rc = get(f, sc[f - F_MASS], 1, 0);
+    for(int f = F_MASS; f <= F_PHI; ++f) get(f, sc[f - F_MASS], 1, vec);
+    x.dev_ints = c.s.nb;
+    x.user_ints = h->neighbor;
+    x.dev_id = c.s.id;
+    int rc = xfer_download(c, x, n);
     if(rc) return rc;
     if(h->id)
-        for(int64_t i = 0; i < n; ++i) h->id[id[i]] = id[i];
-    if(h->neighbor) {
-        std::vector<int> nb(n);
-        SPHGPU_HIP(hipMemcpy(nb.data(), c.s.nb, n * sizeof(int), hipMemcpyDeviceToHost));
-        for(int64_t i = 0; i < n; ++i) h->neighbor[id[i]] = nb[i];
-    }
+        for(int64_t i = 0; i < n; ++i) h->id[i] = (int32_t)i;
     return SPHGPU_OK;
 }
 

@@ -207,6 +207,28 @@ __device__ __forceinline__ void stat_max(int64_t *counters, int task, int k, int
 }
 
 
+// A transfer between the caller's arrays and device fields (transfer.hip).
+struct Xfer {
+    static constexpr int MAX_FIELDS = NF, MAX_ARRAYS = 24;
+    struct Field {
+        double *dev;
+        int off;     // the array's offset in doubles per particle, -1: zeros
+        int stride;  // doubles per particle in the array
+        int comp;
+    };
+    struct Array {
+        char *user;
+        int bytes;  // per particle
+    };
+    Field f[MAX_FIELDS];
+    Array arrays[MAX_ARRAYS];
+    int nf = 0, narrays = 0, doubles = 0;
+    int *user_ints = nullptr, *dev_ints = nullptr;  // one int field
+    int *dev_id = nullptr;  // upload: receives 0, 1, ...; download: the caller index of each slot
+    int add(void *user, int comps);  // an array of comps doubles per particle; returns its offset
+    void field(double *dev, int off, int stride, int comp);
+};
+
 constexpr int TIMER_SETS = 32;
 constexpr int TIMER_EVENTS = 20;
 
@@ -319,6 +341,12 @@ struct Ctx {
     int64_t *counters_host = nullptr;  // (char *)scal_host + SCAL_SPAN
     double *scal_host = nullptr;
 
+    // staging of particle transfers: two buffers on the host (pinned) and
+    // two on the device, of xfer_half bytes each
+    void *xfer_host = nullptr, *xfer_dev = nullptr;
+    int64_t xfer_half = 0;
+    hipEvent_t ev_xfer[2] = {nullptr, nullptr};
+
     // host mirror of simulation scalars
     double time = 0.0, dt = 0.0, h_per_v_sig = 0.0;
     bool uploaded = false, first_pre = true, tree_ready = false;
@@ -372,6 +400,10 @@ inline int grid_for(int64_t n, int block = BLOCK) { return (int)((n + block - 1)
 BoxDev make_box(const Ctx &c);
 
 // ------------------------------------------------------------- launchers
+// transfer.hip
+int xfer_upload(Ctx &c, const Xfer &x, int64_t n);    // returns when the caller's arrays are free
+int xfer_download(Ctx &c, const Xfer &x, int64_t n);
+void xfer_free(Ctx &c);
 // tree.hip
 int tree_alloc(Ctx &c);
 int tree_build(Ctx &c);          // BHTree::make
