@@ -256,7 +256,7 @@ static int stage_pre(Ctx &c, bool walk = false)
         kmark(c, 1);
     }
     if(c.record) {
-        if((rc = search_record(c, c.rec_gather, c.rec_gather_cnt))) return rc;
+        if((rc = search_record(c, c.rec_gather, c.rec_gather_cnt, false))) return rc;
         c.have_gather = true;
     }
     if(walk && (rc = launch_gravity_walk(c))) return rc;
@@ -317,7 +317,10 @@ static int stage_force(Ctx &c)
             c.after_pack = hook;
         }
     }
-    if(c.record) c.have_force = true;
+    if(c.record) {
+        if((rc = search_record(c, c.rec_force, c.rec_force_cnt, true))) return rc;
+        c.have_force = true;
+    }
     return SPHGPU_OK;
 }
 

@@ -354,6 +354,22 @@ template <class T> __device__ __forceinline__ T rsqrt_t(T x)
     else return rsqrt(x);
 }
 
+// a / b and sqrt(x) of pair terms.  The FP32 forms are the hardware
+// reciprocal (times a) and square root, each about 1 ulp, without the
+// rescaling of operands or results beyond 2^126 in size (a division in
+// frexp/ldexp form takes eight instructions, about 38 cycles a wave, against
+// 12; a rescaled square root 28 against 9).
+template <class T> __device__ __forceinline__ T div_t(T a, T b)
+{
+    if constexpr(sizeof(T) == 4) return a * __builtin_amdgcn_rcpf(b);
+    else return a / b;
+}
+template <class T> __device__ __forceinline__ T sqrt_t(T x)
+{
+    if constexpr(sizeof(T) == 4) return __builtin_amdgcn_sqrtf(x);
+    else return sqrt(x);
+}
+
 template <int D, class T> struct Cubic {
     static constexpr double sigma_d = D == 1 ? 2.0 / 3.0 : D == 2 ? 10.0 / (7.0 * 3.14159265358979323846) : 1.0 / 3.14159265358979323846;
     T qscale;   // 1/H
@@ -377,8 +393,13 @@ template <int D, class T> struct Cubic {
     __device__ __forceinline__ T dw_coef(T q, T r) const
     {
         if(r == T(0)) return T(0);
+        return dw_coef_inv(q, div_t<T>(T(1), r));
+    }
+    // the same given 1/r, r != 0
+    __device__ __forceinline__ T dw_coef_inv(T q, T rinv) const
+    {
         const T a = fmax(T(2) - q, T(0)), b = fmax(T(1) - q, T(0));
-        return -gnorm / r * (T(0.75) * a * a - T(3) * b * b);
+        return -gnorm * rinv * (T(0.75) * a * a - T(3) * b * b);
     }
     __device__ __forceinline__ T dhw(T q) const
     {
@@ -416,6 +437,7 @@ template <int D, class T> struct WendlandC4 {
         const T t2 = t * t;
         return -gnorm * (t2 * t2 * t) * (T(1) + T(5) * q);
     }
+    __device__ __forceinline__ T dw_coef_inv(T q, T /*rinv*/) const { return dw_coef(q, T(0)); }
     __device__ __forceinline__ T dhw(T q) const
     {
         const T t = fmax(T(1) - q, T(0));

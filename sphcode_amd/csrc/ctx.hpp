@@ -108,20 +108,30 @@ constexpr int GNC_WRAP = 1 << 30;
 
 // Neighbour records of the force pass, packed once per pass so that a pair
 // reads one FP64 (x, y, z, h) record for the cut and one record of the pair
-// fields (FP32 mirrors in mixed mode) instead of one load per field.
+// fields (rounded to FP32 in mixed mode) instead of one load per field, and
+// divides by nothing of particle j's alone: `q` is u/P (DISPH), P/rho^2
+// (SSPH) or 1/rho^2 (GSPH), `p` is grad-h (DISPH, SSPH) or P (GSPH).  The sizes of
+// the records that lie in LDS are odd multiples of 16 bytes: lanes that read
+// different records of a tile then spread over all banks (a stride of 64
+// bytes would use a quarter of them).
 template <class T> struct __align__(16) ForceRec {
-    T hinv, m, rho, p, c, alpha, bal, u, gradh;  // the kernels need 1/h only
+    T hinv, m, rho, p, c, alpha, bal, u, q;  // the kernels need 1/h only
     T v[3];
 };
-static_assert(sizeof(ForceRec<float>) == 48 && sizeof(ForceRec<double>) == 96, "ForceRec size");
+template <> struct __align__(16) ForceRec<double> {
+    double hinv, m, rho, p, c, alpha, bal, u, q;
+    double v[3];
+    double pad[2];
+};
+static_assert(sizeof(ForceRec<float>) == 48 && sizeof(ForceRec<double>) == 112, "ForceRec size");
 
 // GSPH second order: the MUSCL gradients of a particle (density,
 // pressure, velocity component c along l at gv[3c + l]) in one record.
 template <class T> struct __align__(16) GradRec {
     T gd[3], gp[3], gv[9];
-    T pad;
+    T pad[sizeof(T) == 4 ? 5 : 3];
 };
-static_assert(sizeof(GradRec<float>) == 64 && sizeof(GradRec<double>) == 128, "GradRec size");
+static_assert(sizeof(GradRec<float>) == 80 && sizeof(GradRec<double>) == 144, "GradRec size");
 
 // Neighbour records of the pre-interaction's final sweep: FP64 position,
 // and m, u, c, v in the pair type.
@@ -416,7 +426,9 @@ int search_alloc_particles(Ctx &c);
 int search_combined(Ctx &c, bool work_ready, int blocks_per_cu);  // gather and symmetric candidates in one search
 int search_blocks(const Ctx &c, bool beside_walk);
 int search_alloc(Ctx &c);        // tile slabs for c.ngroups groups (after a tree build)
-int search_record(Ctx &c, int *list, int *cnt);  // the gather sets of the tiles as list_at lists
+// the gather sets (before the pre-interaction) or the force sets (after it)
+// of the tiles as list_at lists
+int search_record(Ctx &c, int *list, int *cnt, bool force);
 // pre.hip
 int pre_initial(Ctx &c);         // initial_smoothing density
 int pre_compute(Ctx &c);         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients

@@ -8,9 +8,16 @@
 //   GSPH  src/gsph/g_fluid_force.cpp:39-166, limiter :27-36, HLL :168-199
 // acc and dene are assigned, not accumulated, as in the reference.
 //
-// T is the pair arithmetic (double, or float in mixed mode: j fields from
-// FP32 mirrors, separations taken in FP64 then rounded, FP32 terms
-// accumulated in FP64; the pair cut is tested on the FP64 squared distance).
+// T is the pair arithmetic (double, or float in mixed mode: j fields rounded
+// to FP32, separations taken in FP64 then rounded, FP32 terms accumulated in
+// FP64; the pair cut is tested on the FP64 squared distance).
+//
+// Bound by vector issue (ALUs fully busy at 46 % of their lanes, 67 % in the
+// second-order GSPH pass).  FP32 quotients use the hardware reciprocal, the
+// quotients of j's own fields come with its record, and positions and
+// gradients lie in LDS with strides that spread over all banks: alone, Evrard
+// 2^20 DISPH 725 -> 589 us (4.6e8 -> 3.9e8 vector instructions), 2^21 GSPH
+// second order 2,361 -> 1,690 us (1.53e9 -> 0.99e9).
 #include "tiles.hpp"
 
 namespace sphgpu {
@@ -22,7 +29,6 @@ struct ForceArgs {
     const uint64_t *ma;     // hit masks per (tile, lane): every symmetric pair
     const int *gnc;
     int wcap;
-    int cap;
     double gamma;
     int use_ac;
     double alpha_ac;
@@ -31,15 +37,13 @@ struct ForceArgs {
     const double *scal;   // S_DT
     int64_t *counters;
     int stats;            // add to the statistics counters (errors are always counted)
-    int *rec;             // recorded force sets (debug), list_at layout
-    int *rec_cnt;
     const double4 *posrec;  // x, y, z, h (FP64)
     const void *frec;       // ForceRec<T>
     const void *grec;       // GradRec<T> (GSPH second order)
 };
 
-// One pass over the particles: the records the pair loop reads for j, with
-// the fields the formulation reads (FP32 mirrors in mixed mode).
+// One pass over the particles: the records the pair loop reads for j
+// (rounded to the pair type), and the quotients of j's own fields.
 template <int D, int TYPE, class T>
 __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, double4 *pr, ForceRec<T> *fr,
                                                            GradRec<T> *gr)
@@ -52,30 +56,39 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
     p.z = D > 2 ? s.f[F_X + 2][i] : 0.0;
     p.w = s.f[F_SML][i];
     pr[i] = p;
+    const double rho = s.f[F_DENS][i], pres = s.f[F_PRES][i];
     ForceRec<T> r{};
-    r.hinv = fld<T>(s, F_HINV, i);
-    r.m = fld<T>(s, F_MASS, i);
-    r.rho = fld<T>(s, F_DENS, i);
-    r.p = fld<T>(s, F_PRES, i);
-    r.c = fld<T>(s, F_SOUND, i);
+    r.hinv = (T)s.f[F_HINV][i];
+    r.m = (T)s.f[F_MASS][i];
+    r.rho = (T)rho;
+    r.c = (T)s.f[F_SOUND][i];
 #pragma unroll
-    for(int l = 0; l < D; ++l) r.v[l] = fld<T>(s, F_V + l, i);
+    for(int l = 0; l < D; ++l) r.v[l] = (T)s.f[F_V + l][i];
     if constexpr(TYPE != SPHGPU_GSPH) {
-        r.alpha = fld<T>(s, F_ALPHA, i);
-        r.bal = fld<T>(s, F_BAL, i);
-        r.gradh = fld<T>(s, F_GRADH, i);
+        r.alpha = (T)s.f[F_ALPHA][i];
+        r.bal = (T)s.f[F_BAL][i];
     }
-    if(use_u) r.u = fld<T>(s, F_ENE, i);
+    if(use_u) r.u = (T)s.f[F_ENE][i];
+    if constexpr(TYPE == SPHGPU_DISPH) {
+        r.p = (T)s.f[F_GRADH][i];
+        r.q = (T)(s.f[F_ENE][i] / pres);
+    } else if constexpr(TYPE == SPHGPU_SSPH) {
+        r.p = (T)s.f[F_GRADH][i];
+        r.q = div_t<T>((T)pres, r.rho * r.rho);
+    } else {
+        r.p = (T)pres;
+        r.q = (T)(1.0 / (rho * rho));
+    }
     fr[i] = r;
     if constexpr(TYPE == SPHGPU_GSPH) {
         if(gr) {
             GradRec<T> g{};
 #pragma unroll
             for(int l = 0; l < D; ++l) {
-                g.gd[l] = fld<T>(s, F_GD + l, i);
-                g.gp[l] = fld<T>(s, F_GP + l, i);
+                g.gd[l] = (T)s.f[F_GD + l][i];
+                g.gp[l] = (T)s.f[F_GP + l][i];
 #pragma unroll
-                for(int c = 0; c < D; ++c) g.gv[3 * c + l] = fld<T>(s, F_GV + 3 * c + l, i);
+                for(int c = 0; c < D; ++c) g.gv[3 * c + l] = (T)s.f[F_GV + 3 * c + l][i];
             }
             gr[i] = g;
         }
@@ -86,22 +99,22 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
 template <class T> __device__ __forceinline__ T van_leer(T a, T b)
 {
     const T ab = a * b;
-    return ab <= T(0) ? T(0) : T(2) * ab / (a + b);
+    return ab <= T(0) ? T(0) : div_t<T>(T(2) * ab, a + b);
 }
 
 // HLL with Roe-averaged wave speeds (src/gsph/g_fluid_force.cpp:168-199);
 // states are (velocity along e, density, pressure, sound speed).
 template <class T> __device__ __forceinline__ void hll(const T L[4], const T R[4], T &pstar, T &vstar)
 {
-    const T sl = sqrt(L[1]), sr = sqrt(R[1]);
-    const T inv = T(1) / (sl + sr);
+    const T sl = sqrt_t<T>(L[1]), sr = sqrt_t<T>(R[1]);
+    const T inv = div_t<T>(T(1), sl + sr);
     const T ut = (sl * L[0] + sr * R[0]) * inv;
     const T ct = (sl * L[3] + sr * R[3]) * inv;
     const T s_l = fmin(L[0] - L[3], ut - ct);
     const T s_r = fmax(R[0] + R[3], ut + ct);
     const T c1 = L[1] * (s_l - L[0]);
     const T c2 = R[1] * (s_r - R[0]);
-    const T c3 = T(1) / (c1 - c2);
+    const T c3 = div_t<T>(T(1), c1 - c2);
     const T c4 = L[2] - L[0] * c1;
     const T c5 = R[2] - R[0] * c2;
     vstar = (c5 - c4) * c3;
@@ -125,10 +138,9 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
     constexpr bool FP64 = sizeof(T) == 8;
     constexpr bool GS = TYPE == SPHGPU_GSPH;
     constexpr int SW = BLOCK / WAVE;
-    __shared__ double4 l_p[SW][WAVE];
+    __shared__ double2 l_xy[SW][WAVE], l_zh[SW][WAVE];
     __shared__ ForceRec<T> l_f[SW][WAVE];
     __shared__ GradRec<T> l_g[GS ? SW : 1][GS ? WAVE : 1];
-    __shared__ int l_j[SW][WAVE];
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -186,41 +198,46 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 q.x = img.at(0, q.x);
                 if constexpr(D > 1) q.y = img.at(1, q.y);
                 if constexpr(D > 2) q.z = img.at(2, q.z);
-                l_p[w][lane] = q;
+                l_xy[w][lane] = make_double2(q.x, q.y);
+                l_zh[w][lane] = make_double2(q.z, q.w);
                 l_f[w][lane] = frec[jl];
                 if constexpr(GS)
                     if(a.second_order) l_g[GS ? w : 0][lane] = ((const GradRec<T> *)a.grec)[jl];
             }
-            l_j[w][lane] = jl;
             return valid ? stream_ld(a.ma + o + lane) : 0ull;
         };
+        // separation from candidate kc, its square, and max(h_i, h_j)
+        auto sep = [&](int kc, double d[D], double &hmax) -> double {
+            const double2 xy = l_xy[w][kc], zh = l_zh[w][kc];
+            double xj[D];
+            xj[0] = xy.x;
+            if constexpr(D > 1) xj[1] = xy.y;
+            if constexpr(D > 2) xj[2] = zh.x;
+            hmax = hi_d < zh.y ? zh.y : hi_d;
+            return sep2<D>(img.pairs, xi, xj, d);
+        };
         auto pair = [&](int kc) {
-            const int j = l_j[w][kc];
-            const double4 pj4 = l_p[w][kc];
-            double xj[D], d[D];
-            xj[0] = pj4.x;
-            if constexpr(D > 1) xj[1] = pj4.y;
-            if constexpr(D > 2) xj[2] = pj4.z;
-            const double r2 = sep2<D>(img.pairs, xi, xj, d);
-            const double hj_d = pj4.w;
-            const double hmax = hi_d < hj_d ? hj_d : hi_d;
-            T r;
+            double d[D], hmax;
+            const double r2 = sep(kc, d, hmax);
+            T r, rinv;
             if constexpr(FP64) {
                 r = sqrt(r2);
                 if(r >= hmax || r == 0.0) return;  // src/fluid_force.cpp:62-64
+                rinv = 1.0 / r;
             } else {
                 if(!(r2 < hmax * hmax) || r2 == 0.0) return;
-                r = sqrtf((float)r2);
+                const float r2f = fmaxf((float)r2, 1.17549435e-38f);
+                r = __builtin_amdgcn_sqrtf(r2f);
+                rinv = __builtin_amdgcn_rcpf(r);
             }
-            if(a.rec && used < a.cap) a.rec[list_at(i, used, a.cap)] = j;
             ++used;
             T rij[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) rij[l] = (T)d[l];
             const ForceRec<T> fj = l_f[w][kc];
             const Kern kj(T(0), fj.hinv);  // the kernel object reads 1/h only
-            const T cwi = ki.dw_coef(ki.q_of(r), r);
-            const T cwj = kj.dw_coef(kj.q_of(r), r);
+            const T cwi = ki.dw_coef_inv(ki.q_of(r), rinv);
+            const T cwj = kj.dw_coef_inv(kj.q_of(r), rinv);
             T dwi[D], dwj[D], vj[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) {
@@ -230,11 +247,10 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             }
             const T mj = fj.m;
             const T rhoj = fj.rho;
-            const T pj = fj.p;
             const T cj = fj.c;
 
             if constexpr(TYPE == SPHGPU_GSPH) {
-                const T rinv = T(1) / r;
+                const T pj = fj.p;
                 T e[D];
 #pragma unroll
                 for(int l = 0; l < D; ++l) e[l] = rij[l] * rinv;
@@ -279,8 +295,8 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     const T dp = pi_ - pj;
                     R[2] = pi_ - van_leer(dp, gpi * r) * di;
                     L[2] = pj + van_leer(dp, gpj * r) * dj;
-                    R[3] = sqrt(gam * R[2] / R[1]);
-                    L[3] = sqrt(gam * L[2] / L[1]);
+                    R[3] = sqrt_t<T>(div_t<T>(gam * R[2], R[1]));
+                    L[3] = sqrt_t<T>(div_t<T>(gam * L[2], L[1]));
                     hll(L, R, pstar, vstar);
                 } else {
                     const T R[4] = {ve_i, rhoi, pi_, ci};
@@ -288,11 +304,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     hll(L, R, pstar, vstar);
                 }
                 const T fi = mj * pstar * rho2_inv_i;
-                const T fj = mj * pstar / (rhoj * rhoj);
+                const T fjj = mj * pstar * fj.q;
                 T fdv = T(0);
 #pragma unroll
                 for(int l = 0; l < D; ++l) {
-                    const T f = dwi[l] * fi + dwj[l] * fj;
+                    const T f = dwi[l] * fi + dwj[l] * fjj;
                     acc[l].add(-f);
                     fdv += f * (e[l] * vstar - vi[l]);
                 }
@@ -310,30 +326,30 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 if(vr < T(0)) {
                     const T alpha = T(0.5) * (alphai + fj.alpha);
                     const T bal = T(0.5) * (bali + fj.bal);
-                    const T w = vr / r;
-                    const T vsig = ci + cj - T(3) * w;
-                    pij = T(-0.5) * bal * alpha * vsig * w * (T(2) / (rhoi + rhoj));
+                    const T wv = vr * rinv;
+                    const T vsig = ci + cj - T(3) * wv;
+                    pij = T(-0.5) * bal * alpha * vsig * wv * div_t<T>(T(2), rhoi + rhoj);
                 }
                 T ac = T(0);
                 if(a.use_ac) {
                     const T uj = fj.u;
-                    const T vs = a.gravity ? fabs(vr / r) : sqrt(T(2) * fabs(pi_ - pj) / (rhoi + rhoj));
-                    ac = (T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij) / r;
+                    const T pj = TYPE == SPHGPU_DISPH ? div_t<T>(uj, fj.q) : fj.q * rhoj * rhoj;
+                    const T vs = a.gravity ? fabs(vr * rinv) : sqrt_t<T>(div_t<T>(T(2) * fabs(pi_ - pj), rhoi + rhoj));
+                    ac = (T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij) * rinv;
                 }
                 const T vdwi = dotd<D, T>(vij, dwi);
                 const T vdwij = dotd<D, T>(vij, dwij);
                 T ci_f, cj_f, de;
                 if constexpr(TYPE == SPHGPU_DISPH) {
-                    const T uj = fj.u;
-                    const T fij = T(1) - gradhi / (mj * uj);
-                    const T fji = T(1) - fj.gradh * mu_inv_i;
-                    const T u_p_j = uj / pj;
-                    ci_f = mj * (g2u_p_i * uj * fij + T(0.5) * pij);
-                    cj_f = mj * (g2u_i * u_p_j * fji + T(0.5) * pij);
-                    de = mj * g2u_p_i * uj * fij * vdwi;
+                    // m_j u_j f_ij = m_j u_j - grad-h_i, f_ji = 1 - grad-h_j / (m_i u_i)
+                    const T pi_i = g2u_p_i * (mj * fj.u - gradhi);
+                    const T fji = T(1) - fj.p * mu_inv_i;
+                    ci_f = pi_i + T(0.5) * mj * pij;
+                    cj_f = mj * (g2u_i * fj.q * fji + T(0.5) * pij);
+                    de = pi_i * vdwi;
                 } else {
                     ci_f = mj * (p_rho2_i * gradhi + T(0.5) * pij);
-                    cj_f = mj * (pj / (rhoj * rhoj) * fj.gradh + T(0.5) * pij);
+                    cj_f = mj * (fj.q * fj.p + T(0.5) * pij);
                     de = mj * p_rho2_i * gradhi * vdwi;
                 }
 #pragma unroll
@@ -343,13 +359,8 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         };
         // the cut-off r < max(h_i, h_j), r > 0 of the pair, tested ahead
         auto keep = [&](int kc) -> bool {
-            const double4 pj4 = l_p[w][kc];
-            double xj[D], d[D];
-            xj[0] = pj4.x;
-            if constexpr(D > 1) xj[1] = pj4.y;
-            if constexpr(D > 2) xj[2] = pj4.z;
-            const double r2 = sep2<D>(img.pairs, xi, xj, d);
-            const double hmax = hi_d < pj4.w ? pj4.w : hi_d;
+            double d[D], hmax;
+            const double r2 = sep(kc, d, hmax);
             if constexpr(FP64) {
                 const double r = sqrt(r2);
                 return !(r >= hmax || r == 0.0);
@@ -372,7 +383,6 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
 #pragma unroll
             for(int k = 0; k < D; ++k) s.f[F_A + k][i] = acc[k].val();
             s.f[F_DENE][i] = dene.val();
-            if(a.rec_cnt) a.rec_cnt[i] = used < a.cap ? used : a.cap;
         }
     }
     if(a.stats) {
@@ -387,8 +397,7 @@ template <int D, int K, int TYPE, class T> static void launch_force(Ctx &c, cons
     hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
                        c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec);
     if(c.after_pack) c.after_pack_rc = c.after_pack(c);
-    // (recorded sets are numbered by one wave per group)
-    if(group_waves(c, GROUP_PAIRS) > 1 && !a.rec)
+    if(group_waves(c, GROUP_PAIRS) > 1)
         hipLaunchKernelGGL((force_kernel<D, K, TYPE, T, BLOCK / WAVE>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
     else
         hipLaunchKernelGGL((force_kernel<D, K, TYPE, T, 1>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
@@ -422,7 +431,6 @@ int force_compute(Ctx &c)
     a.ma = c.tile_ma;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
-    a.cap = c.cap;
     a.gamma = c.p.gamma;
     a.use_ac = c.p.ac_is_valid;
     a.alpha_ac = c.p.ac_alpha;
@@ -431,8 +439,6 @@ int force_compute(Ctx &c)
     a.scal = c.scal;
     a.counters = c.counters;
     a.stats = c.stats_on ? 1 : 0;
-    a.rec = c.record ? c.rec_force : nullptr;
-    a.rec_cnt = c.record ? c.rec_force_cnt : nullptr;
     a.posrec = c.posrec;
     a.frec = c.pair_rec;
     a.grec = c.grad_rec;

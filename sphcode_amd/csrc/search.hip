@@ -711,11 +711,13 @@ int search_alloc(Ctx &c)
     return SPHGPU_OK;
 }
 
-// The gather sets as lists in list_at layout, from the tiles of the last
-// search (debug): lane l of a group appends its hits with r < R_i (sml before
-// the pre-interaction) in staging order (candidate c = t + kT is bit k of
-// tile t).  Entries past cap are dropped (the search reports them).
-template <int D>
+// The gather sets (FORCE = 0: r < R_i, sml before the pre-interaction) or the
+// force sets (r < max(h_i, h_j), r != 0, as the force pass of the precision
+// tests it: 1 FP64, 2 mixed) as lists in list_at layout, from the tiles of
+// the last search (debug): lane l of a group appends its hits in staging
+// order (candidate c = t + kT is bit k of tile t).  Entries past cap are
+// dropped (the search reports them).
+template <int D, int FORCE>
 __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
                                                        const int *cand, const uint64_t *ma, int wcap, int cap,
                                                        int *list, int *cnt)
@@ -733,7 +735,7 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     double xi[D];
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][i];
-    const double h2 = s.f[F_SML][i] * s.f[F_SML][i];
+    const double h = s.f[F_SML][i], h2 = h * h;
     int wf = 0;  // entries written (at most cap)
     for(int k = 0; k < WAVE; ++k) {
         for(int t = 0; t < T; ++t) {
@@ -744,25 +746,44 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
             double xj[D], d[D];
 #pragma unroll
             for(int q = 0; q < D; ++q) xj[q] = s.f[F_X + q][j];
-            if(!(sep2<D>(box, xi, xj, d) < h2)) continue;
+            const double r2 = sep2<D>(box, xi, xj, d);
+            if constexpr(FORCE == 0) {
+                if(!(r2 < h2)) continue;
+            } else {
+                const double hj = s.f[F_SML][j];
+                const double hmax = h < hj ? hj : h;
+                if constexpr(FORCE == 1) {
+                    const double r = sqrt(r2);
+                    if(r >= hmax || r == 0.0) continue;
+                } else if(!(r2 < hmax * hmax) || r2 == 0.0) {
+                    continue;
+                }
+            }
             if(wf < cap) list[lb + list_off(wf++)] = j;
         }
     }
     cnt[i] = wf;
 }
 
-template <int D> static void launch_record(Ctx &c, int *list, int *cnt)
+template <int D, int FORCE> static void launch_record_t(Ctx &c, int *list, int *cnt)
 {
-    hipLaunchKernelGGL(record_kernel<D>, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
+    hipLaunchKernelGGL((record_kernel<D, FORCE>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
                        c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, list, cnt);
 }
 
-int search_record(Ctx &c, int *list, int *cnt)
+template <int D> static void launch_record(Ctx &c, int *list, int *cnt, bool force)
+{
+    if(!force) launch_record_t<D, 0>(c, list, cnt);
+    else if(c.p.precision == SPHGPU_FP64) launch_record_t<D, 1>(c, list, cnt);
+    else launch_record_t<D, 2>(c, list, cnt);
+}
+
+int search_record(Ctx &c, int *list, int *cnt, bool force)
 {
     switch(c.D) {
-    case 1: launch_record<1>(c, list, cnt); break;
-    case 2: launch_record<2>(c, list, cnt); break;
-    default: launch_record<3>(c, list, cnt); break;
+    case 1: launch_record<1>(c, list, cnt, force); break;
+    case 2: launch_record<2>(c, list, cnt, force); break;
+    default: launch_record<3>(c, list, cnt, force); break;
     }
     SPHGPU_HIP(hipGetLastError());
     return SPHGPU_OK;
