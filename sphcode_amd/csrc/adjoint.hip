@@ -132,25 +132,25 @@ template <int D, class T> __global__ void __launch_bounds__(BLOCK) adj_seed_kern
         const double af = ADJ<D>(a, L::A + k, id) + half * ADJ<D>(a, L::V + k, id);
         W(a, W_AF + k, i) = af;
         r.af[k] = (T)af;
-        r.v[k] = fld<T>(s, F_V + k, i);
+        r.v[k] = (T)s.f[F_V + k][i];
     }
     const double duf = ADJ<D>(a, L::DU, id) + half * ADJ<D>(a, L::U, id);
     W(a, W_DUF, i) = duf;
     r.duf = (T)duf;
-    r.hinv = T(1) / fld<T>(s, F_SML, i);
-    r.rho = fld<T>(s, F_DENS, i);
-    r.A = fld<T>(s, F_PRES, i) * fld<T>(s, F_GRADH, i) / (r.rho * r.rho);
-    r.bal = fld<T>(s, F_BAL, i);
-    r.c = fld<T>(s, F_SOUND, i);
-    r.alpha = fld<T>(s, F_ALPHA, i);
-    r.m = fld<T>(s, F_MASS, i);
+    r.hinv = T(1) / (T)s.f[F_SML][i];
+    r.rho = (T)s.f[F_DENS][i];
+    r.A = (T)s.f[F_PRES][i] * (T)s.f[F_GRADH][i] / (r.rho * r.rho);
+    r.bal = (T)s.f[F_BAL][i];
+    r.c = (T)s.f[F_SOUND][i];
+    r.alpha = (T)s.f[F_ALPHA][i];
+    r.m = (T)s.f[F_MASS][i];
     ((AdjRec<T> *)a.rec)[i] = r;
     a.pos[i] = make_double4(s.f[F_X][i], D > 1 ? s.f[F_X + 1][i] : 0.0, D > 2 ? s.f[F_X + 2][i] : 0.0, s.f[F_SML][i]);
 }
 
 // Pair arithmetic of the passes: T = double, or float in mixed precision
-// (separations taken in FP64 and rounded, fields of j from the FP32
-// mirrors, terms accumulated in FP64 by Acc<T>); the pair-set tests are
+// (separations taken in FP64 and rounded, fields of j rounded to
+// FP32, terms accumulated in FP64 by Acc<T>); the pair-set tests are
 // those of the forward stages in the same precision.
 template <class T> __device__ __forceinline__ T pair_r(double r2)
 {
@@ -466,14 +466,14 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, Adj
     const double Gh = rhop * hD1 * h + D * rho * hD1;
     const double g = -hb / Gh;
     SeedRec<T> o{};
-    o.h = fld<T>(s, F_SML, i);
+    o.h = (T)s.f[F_SML][i];
     o.hinv = T(1) / o.h;
-    o.m = fld<T>(s, F_MASS, i);
+    o.m = (T)s.f[F_MASS][i];
     o.srho = (T)(rhob + g * hD1 * h);
     o.srhop = (T)rhopb;
     o.sdv = (T)Dvb;
 #pragma unroll
-    for(int k = 0; k < D; ++k) o.v[k] = fld<T>(s, F_V + k, i);
+    for(int k = 0; k < D; ++k) o.v[k] = (T)s.f[F_V + k][i];
 #pragma unroll
     for(int k = 0; k < 3; ++k) o.srv[k] = (T)Rvb[k];
     ((SeedRec<T> *)a.seed)[i] = o;

@@ -92,8 +92,6 @@ static void free_buffers(Ctx &c)
     for(int f = 0; f < NF; ++f) {
         fr(c.s.f[f]);
         fr(c.alt.f[f]);
-        fr(c.s.g[f]);
-        c.alt.g[f] = nullptr;
     }
     fr(c.s.id); fr(c.alt.id); fr(c.s.nb); fr(c.alt.nb);
     fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff);
@@ -124,7 +122,6 @@ static int alloc_buffers(Ctx &c, int64_t n)
         if(!field_used(c, f)) continue;
         SPHGPU_HIP(hipMalloc(&c.s.f[f], np * sizeof(double)));
         SPHGPU_HIP(hipMalloc(&c.alt.f[f], np * sizeof(double)));
-        if(mixed && f >= F_V) SPHGPU_HIP(hipMalloc(&c.s.g[f], np * sizeof(float)));
     }
     SPHGPU_HIP(hipMalloc(&c.posrec, np * sizeof(double4)));
     // one buffer for the records of either pair pass (ForceRec is the larger)

@@ -29,18 +29,9 @@ enum Field : int {
 // Kernel-argument view of the state.
 struct State {
     double *f[NF];
-    float *g[NF];  // FP32 mirrors read by the mixed-precision pair kernels
-                   // (positions excepted; allocated in mixed mode only)
     int *id;       // caller index of the particle in each sorted slot
     int *nb;       // neighbour count (SPHParticle::neighbor)
 };
-
-// FP64 master field, or its FP32 mirror, as the pair arithmetic type.
-template <class T> __device__ __forceinline__ T fld(const State &s, int f, int i)
-{
-    if constexpr(sizeof(T) == 8) return s.f[f][i];
-    else return s.g[f][i];
-}
 
 // Per-particle sums.  FP32 pair terms are compensated by accumulating them
 // in FP64: every FP32 term is exact in FP64, so the sum's error does not
@@ -86,7 +77,7 @@ struct __align__(16) LeafHit {
 constexpr int LEAFHIT_CAP = 1024;   // recorded leaves per wave before it falls back
 constexpr int LEAFHIT_CHUNK = 256;  // records the pair pass takes per round
 template <class T> struct GravPart;
-template <> struct __align__(32) GravPart<float> {  // mixed: FP32 mirrors of m and 2/h
+template <> struct __align__(32) GravPart<float> {  // mixed: m and 2/h in FP32
     double x[3];
     float m, einv;
 };
@@ -463,8 +454,6 @@ int step_timestep(Ctx &c);       // dt into scal[S_DT]
 int step_predict(Ctx &c);
 int step_correct(Ctx &c, bool add_gravity = false);  // add_gravity: acc += the gravity pass's sums first
 int step_energy(Ctx &c, double *out);
-// FP32 mirrors of the listed fields (mixed precision only; no-op in FP64)
-int mirror_fields(Ctx &c, const int *fields, int nfields);
 int reduce_min_partials(Ctx &c, int nblocks, int slot);
 // adjoint.hip: vector-Jacobian product of one force evaluation
 // (pre-interaction + fluid force at the current state and lists) and the

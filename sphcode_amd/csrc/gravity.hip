@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(BLOCK) pack_nodes_kernel(TreeDev t, GravNode *
 }
 
 // Particle records in tree order: position, mass and 2/h in the pair type
-// (FP32 mirrors in mixed mode, as the pair kernels read them).
+// (rounded as the pair kernels read them).
 template <int D, class T> __global__ void __launch_bounds__(BLOCK) pack_parts_kernel(State s, int n, GravPart<T> *out)
 {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
@@ -75,8 +75,8 @@ template <int D, class T> __global__ void __launch_bounds__(BLOCK) pack_parts_ke
     if(i < n) {
 #pragma unroll
         for(int k = 0; k < 3; ++k) p.x[k] = k < D ? s.f[F_X + k][i] : 0.0;
-        p.m = fld<T>(s, F_MASS, i);
-        p.einv = T(2) * fld<T>(s, F_HINV, i);
+        p.m = (T)s.f[F_MASS][i];
+        p.einv = T(2) * (T)s.f[F_HINV][i];
     }
     out[i] = p;  // i == n: the spare record
 }

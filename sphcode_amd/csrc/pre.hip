@@ -63,8 +63,8 @@ template <class T> __device__ __forceinline__ T gather_r(double r2)
     else return gather_r_f32(r2);
 }
 
-// Records read for j by the final sweep (FP32 mirrors in mixed mode), and
-// the 32-byte position and mass records the Newton sweeps read.
+// Records read for j by the final sweep (rounded to the pair type), and the
+// 32-byte position and mass records the Newton sweeps read.
 template <int D, class T> __global__ void __launch_bounds__(BLOCK) pack_pre_kernel(State s, int n, PreRec<T> *out, double4 *pm)
 {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
@@ -73,19 +73,12 @@ template <int D, class T> __global__ void __launch_bounds__(BLOCK) pack_pre_kern
 #pragma unroll
     for(int k = 0; k < 3; ++k) r.x[k] = k < D ? s.f[F_X + k][i] : 0.0;
     pm[i] = make_double4(r.x[0], r.x[1], r.x[2], s.f[F_MASS][i]);
-    r.m = fld<T>(s, F_MASS, i);
-    r.u = fld<T>(s, F_ENE, i);
-    r.c = fld<T>(s, F_SOUND, i);
+    r.m = (T)s.f[F_MASS][i];
+    r.u = (T)s.f[F_ENE][i];
+    r.c = (T)s.f[F_SOUND][i];
 #pragma unroll
-    for(int k = 0; k < D; ++k) r.v[k] = fld<T>(s, F_V + k, i);
+    for(int k = 0; k < D; ++k) r.v[k] = (T)s.f[F_V + k][i];
     out[i] = r;
-}
-
-// Writes an FP64 result and, in mixed mode, its FP32 mirror.
-template <class T> __device__ __forceinline__ void put(const State &s, int f, int i, double v)
-{
-    s.f[f][i] = v;
-    if constexpr(sizeof(T) == 4) s.g[f][i] = (float)v;
 }
 
 template <int D, class T> struct CurlAcc {
@@ -146,7 +139,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         if(jl >= 0) {
 #pragma unroll
             for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl]);
-            l_r[w][lane].m = fld<T>(s, F_MASS, jl);
+            l_r[w][lane].m = (T)s.f[F_MASS][jl];
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
     };
@@ -412,28 +405,28 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             pairs = count;
             const double gm1 = a.gamma - 1.0;
             const double rho_d = rho.val();
-            put<T>(s, F_SML, i, h);
-            put<T>(s, F_HINV, i, 1.0 / h);
+            s.f[F_SML][i] = h;
+            s.f[F_HINV][i] = 1.0 / h;
             if(a.gpart) {
                 // the gravity leaf pass's record of i, as pack_parts_kernel writes it
                 GravPart<T> gp{};
 #pragma unroll
                 for(int k = 0; k < 3; ++k) gp.x[k] = k < D ? xi[k] : 0.0;
                 gp.m = (T)mi;
-                gp.einv = T(2) * (T)(1.0 / h);  // 2 x the FP32 mirror of 1/h in mixed mode
+                gp.einv = T(2) * (T)(1.0 / h);
                 ((GravPart<T> *)a.gpart)[i] = gp;
             }
-            put<T>(s, F_DENS, i, rho_d);
+            s.f[F_DENS][i] = rho_d;
             double pres;
             if constexpr(TYPE == SPHGPU_DISPH) {
                 pres = gm1 * pb.val();
                 const double nv = nd.val();
-                put<T>(s, F_GRADH, i, h / (D * nv) * dpb.val() / (1.0 + h / (D * nv) * dnd.val()));
+                s.f[F_GRADH][i] = h / (D * nv) * dpb.val() / (1.0 + h / (D * nv) * dnd.val());
             } else {
                 pres = gm1 * rho_d * ui;
-                if constexpr(TYPE == SPHGPU_SSPH) put<T>(s, F_GRADH, i, 1.0 / (1.0 + h / (D * rho_d) * drho.val()));
+                if constexpr(TYPE == SPHGPU_SSPH) s.f[F_GRADH][i] = 1.0 / (1.0 + h / (D * rho_d) * drho.val());
             }
-            put<T>(s, F_PRES, i, pres);
+            s.f[F_PRES][i] = pres;
             s.nb[i] = count;
             hvs = h / (double)vsig_max;
 
@@ -442,13 +435,13 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     const double rinv = 1.0 / rho_d;
 #pragma unroll
                     for(int l = 0; l < D; ++l) {
-                        put<T>(s, F_GD + l, i, gd[l].val());
-                        put<T>(s, F_GP + l, i, (gd[l].val() * ui + gu[l].val()) * gm1);
+                        s.f[F_GD + l][i] = gd[l].val();
+                        s.f[F_GP + l][i] = (gd[l].val() * ui + gu[l].val()) * gm1;
                     }
 #pragma unroll
                     for(int c = 0; c < D; ++c)
 #pragma unroll
-                        for(int l = 0; l < D; ++l) put<T>(s, F_GV + 3 * c + l, i, gv[c][l].val() * rinv);
+                        for(int l = 0; l < D; ++l) s.f[F_GV + 3 * c + l][i] = gv[c][l].val() * rinv;
                 }
             } else {
                 const double dt = a.scal[S_DT];
@@ -464,18 +457,18 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                         dv /= rho_d;
                         rm = rot.magnitude() / rho_d;
                     }
-                    put<T>(s, F_BAL, i, fabs(dv) / (fabs(dv) + rm + 1e-4 * ci / h));
+                    s.f[F_BAL][i] = fabs(dv) / (fabs(dv) + rm + 1e-4 * ci / h);
                     if(a.tdav) {
                         const double tau_inv = a.eps_av * ci / h;
                         const double da = (-(alpha - a.amin) * tau_inv + fmax(-dv, 0.0) * (a.amax - alpha)) * dt;
-                        put<T>(s, F_ALPHA, i, alpha + da);
+                        s.f[F_ALPHA][i] = alpha + da;
                     }
                 } else if(a.tdav) {
                     if constexpr(TYPE == SPHGPU_DISPH) dv *= gm1 / pres;
                     else dv /= rho_d;
                     const double tau_inv = a.eps_av * ci / h;
                     const double si = fmax(-dv, 0.0);
-                    put<T>(s, F_ALPHA, i, (alpha + dt * tau_inv * a.amin + si * dt * a.amax) / (1.0 + dt * tau_inv + si * dt));
+                    s.f[F_ALPHA][i] = (alpha + dt * tau_inv * a.amin + si * dt * a.amax) / (1.0 + dt * tau_inv + si * dt);
                 }
             }
         }
@@ -530,12 +523,6 @@ static PreArgs make_args(Ctx &c)
     return a;
 }
 
-// Fields of j read by the pair sums, mirrored to FP32 before the stage
-// (alpha and the Balsara switch too: the force reads their mirrors, and
-// the stage rewrites them only when their switches are on).
-static const int kPreInputs[] = {F_V, F_V + 1, F_V + 2, F_MASS, F_ENE, F_SOUND, F_ALPHA, F_BAL};
-constexpr int kNumPreInputs = 8;
-
 template <int D, int K, class T> static void launch_initial(Ctx &c, const PreArgs &a)
 {
     if(group_waves(c, GROUP_PAIRS) > 1)
@@ -556,8 +543,6 @@ template <class T> static void initial_t(Ctx &c, const PreArgs &a)
 
 int pre_initial(Ctx &c)
 {
-    int rc = mirror_fields(c, kPreInputs, kNumPreInputs);
-    if(rc) return rc;
     const PreArgs a = make_args(c);
     if(c.p.precision == SPHGPU_MIXED) initial_t<float>(c, a);
     else initial_t<double>(c, a);
@@ -596,8 +581,6 @@ template <class T> static void pre_t(Ctx &c, const PreArgs &a, const BoxDev &box
 
 int pre_compute(Ctx &c)
 {
-    int rc = mirror_fields(c, kPreInputs, kNumPreInputs);
-    if(rc) return rc;
     PreArgs a = make_args(c);
     a.gpart = c.p.gravity_is_valid ? c.gpart : nullptr;
     const BoxDev box = make_box(c);

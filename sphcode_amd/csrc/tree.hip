@@ -623,7 +623,6 @@ template <int D> static int tree_build_d(Ctx &c)
         r.ratio = c.p.iterative_sml ? 1.2 : 1.0;
     }
     hipLaunchKernelGGL(reorder_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, r, c.perm, n, nf);
-    // swap master buffers; FP32 mirrors stay (they are rewritten before use)
     for(int f = 0; f < NF; ++f) std::swap(c.s.f[f], c.alt.f[f]);
     std::swap(c.s.id, c.alt.id);
     std::swap(c.s.nb, c.alt.nb);
