@@ -20,6 +20,8 @@
 // gathers in a second loop over the same set (Balsara switch and
 // time-dependent viscosity, or the GSPH MUSCL gradients).
 //
+// Bound by vector issue (ALUs fully busy at about 45 % of their lanes).
+//
 // T is the pair arithmetic: double, or float for the mixed mode, where
 // pair terms are evaluated in FP32 relative to particle i (separations
 // taken in FP64, then rounded) and accumulated in FP64 (Acc in ctx.hpp),
@@ -34,6 +36,7 @@ struct PreArgs {
     int ngroups;
     const int *cand;      // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;   // hit masks
+    uint64_t *mn;         // narrowed masks (Ctx::tile_mn)
     const int *gnc;
     int wcap;
     double gamma;
@@ -54,6 +57,14 @@ struct PreArgs {
 };
 
 constexpr int PSW = BLOCK / WAVE;  // waves (groups) per block
+
+// The Newton solve's first sweep keeps the hits within NARROW times its h.
+// The search radius holds 1.2^3 = 1.7 times as many candidates as r < h (in
+// 3D), and the solve moves h by a percent or so in a running simulation, so
+// the later sweeps, the final one among them, run over little more than the
+// pairs they sum (steps: Evrard 2^20 5.12 -> 4.92 ms, 2D KHI 0.895 -> 0.848,
+// rollout of 262,144 0.79 -> 0.755; 1.02 and 1.035 measured the same).
+constexpr double NARROW = 1.05;
 
 // |r_ij| of a gather candidate in the pair type from the FP64 r^2: the
 // correctly rounded FP64 square root, or its FP32 form (gather_r_f32)
@@ -163,15 +174,15 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     using Kern = typename KernelOf<D, K, T>::type;
     constexpr bool NUMBER = TYPE == SPHGPU_DISPH;
     __shared__ PreRec<T> l_r[PSW][WAVE];
-    __shared__ int l_j[PSW][WAVE];
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int part = w % NW;
     // the Newton sweeps stage 32-byte position and mass records in the same
     // LDS as the final sweep's records (64 of them per wave)
-    double4 *const l_pm = reinterpret_cast<double4 *>(&l_r[w][0]);
-    static_assert(sizeof(PreRec<T>) >= sizeof(double4) && (WAVE * sizeof(PreRec<T>)) % alignof(double4) == 0,
-                  "position and mass records fit the final sweep's slot");
+    // (two halves of 16 bytes, so that lanes reading different candidates
+    // spread over all banks)
+    double2 *const l_xy = reinterpret_cast<double2 *>(&l_r[w][0]), *const l_zm = l_xy + WAVE;
+    static_assert(sizeof(PreRec<T>) >= 2 * sizeof(double2), "position and mass records fit the final sweep's slot");
     const int lane = wave_lane();
     // waves past the last group take part in the block's reduction only
     const int grp = xcd_block() * (PSW / NW) + w / NW;
@@ -195,12 +206,20 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         const double Hs = s.f[F_SML][ii];  // search radius h_guess * ratio
         const double Hs2 = Hs * Hs;
         double h = Hs;
+        double lim2 = 0.0;
+        bool narrowed = false;  // the narrowed masks hold every r < h
         if(a.iterative) {
             // PreInteraction::newton_raphson, every lane on its own iterate;
             // the wave sweeps the tiles once per iteration for the lanes
             // still iterating
             const double b = NUMBER ? a.nngb / UnitVolume<D>::value : mi * a.nngb / UnitVolume<D>::value;
             double hn = Hs / a.ratio;
+            // the first sweep also narrows the hits to r < lim, a little
+            // above its h: a wave whose iterates stay below takes the later
+            // sweeps over those
+            const double lim = NARROW * hn;
+            lim2 = lim * lim;
+            auto narrow_holds = [&](double h_now) -> bool { return ballot(valid && !(h_now <= lim)) == 0; };
             bool done = !valid;
             int it = 0;
             for(; it < 10; ++it) {
@@ -209,24 +228,23 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 const T ht = (T)hn;
                 const Kern ker(ht);
                 Acc<T> rho, drho;
+                const uint64_t *masks = it == 0 || !narrow_holds(hn) ? a.ma : a.mn;
                 auto nstage = [&](int tt) -> uint64_t {
                     const size_t o = gbase + (size_t)tt * WAVE;
                     const int jl = stream_ld(a.cand + o + lane);
                     if(jl >= 0) {
-                        double4 q = a.pm[jl];
-                        q.x = img.at(0, q.x);
-                        if constexpr(D > 1) q.y = img.at(1, q.y);
-                        if constexpr(D > 2) q.z = img.at(2, q.z);
-                        l_pm[lane] = q;
+                        const double4 q = a.pm[jl];
+                        l_xy[lane] = make_double2(img.at(0, q.x), D > 1 ? img.at(1, q.y) : 0.0);
+                        l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z) : 0.0, q.w);
                     }
-                    return done ? 0ull : stream_ld(a.ma + o + lane);
+                    return done ? 0ull : stream_ld(masks + o + lane);
                 };
-                auto npair = [&](int kc) {
-                    const double4 pj = l_pm[kc];
+                auto npair = [&](int kc) -> bool {
+                    const double2 xy = l_xy[kc], zm = l_zm[kc];
                     double xj[D], d[D];
-                    xj[0] = pj.x;
-                    if constexpr(D > 1) xj[1] = pj.y;
-                    if constexpr(D > 2) xj[2] = pj.z;
+                    xj[0] = xy.x;
+                    if constexpr(D > 1) xj[1] = xy.y;
+                    if constexpr(D > 2) xj[2] = zm.x;
                     const double r2 = sep2<D>(img.pairs, xi, xj, d);
                     const T r = gather_r<T>(r2);
                     if(r < ht && r2 < Hs2) {
@@ -235,13 +253,19 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                             rho.add(ker.w(q));
                             drho.add(ker.dhw(q));
                         } else {
-                            const T mj = (T)pj.w;
+                            const T mj = (T)zm.y;
                             rho.add(mj * ker.w(q));
                             drho.add(mj * ker.dhw(q));
                         }
                     }
+                    return r2 < lim2;
                 };
-                tile_sweep<NW>(part, ntile, nstage, npair);
+                if(it == 0)
+                    tile_sweep_keep<NW>(part, ntile, nstage, npair, [&](int tt, uint64_t kept) {
+                        stream_st(a.mn + gbase + (size_t)tt * WAVE + lane, kept);
+                    });
+                else
+                    tile_sweep<NW>(part, ntile, nstage, npair);
                 parts_sum<NW, 2>(red, part, {&rho.s, &drho.s});
                 if(!done) {
                     iters += part == 0;
@@ -260,6 +284,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 }
                 if(h > Hs) trunc += part == 0;
             }
+            narrowed = narrow_holds(h);
         }
 
         // final sums over r < h
@@ -286,8 +311,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k]);
                 l_r[w][lane] = q;
             }
-            l_j[w][lane] = jl;
-            return valid ? stream_ld(a.ma + o + lane) : 0ull;
+            return valid ? stream_ld((narrowed ? a.mn : a.ma) + o + lane) : 0ull;
         };
         auto fpair = [&](int kc) {
             const PreRec<T> pj = l_r[w][kc];
@@ -297,7 +321,6 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             const double r2 = sep2<D>(img.pairs, xi, xj, d);
             const T r = gather_r<T>(r2);
             if(!(r < ht && r2 < Hs2)) return;
-            const int j = l_j[w][kc];
             ++count;
             const T mj = pj.m;
             const T q = ker.q_of(r);
@@ -322,11 +345,11 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 rij[l] = (T)d[l];
                 vij[l] = vi[l] - pj.v[l];
             }
-            if(j != i) {
+            if(r2 != 0.0) {  // not particle i itself
                 T rv = rij[0] * vij[0];
 #pragma unroll
                 for(int l = 1; l < D; ++l) rv += rij[l] * vij[l];
-                const T vs = ci_t + pj.c - T(3) * rv / r;
+                const T vs = ci_t + pj.c - div_t<T>(T(3) * rv, r);
                 vsig_max = vs > vsig_max ? vs : vsig_max;
             }
             if(need_dv) {
@@ -365,10 +388,10 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             const double r2 = sep2<D>(img.pairs, xi, xj, d);
             return gather_r<T>(r2) < ht && r2 < Hs2;
         };
-        // refined in 3D except for GSPH (measured slower on the 3D Sedov
-        // case), see tiles.hpp
+        // with all the hits, refined in 3D except for GSPH (measured slower
+        // on the 3D Sedov case), see tiles.hpp; the narrowed ones need none
         if constexpr(D == 3 && TYPE != SPHGPU_GSPH) {
-            auto frefine = [&](uint64_t m) { return refine_bits(m, fkeep); };
+            auto frefine = [&](uint64_t m) { return narrowed ? m : refine_bits(m, fkeep); };
             tile_sweep<NW>(part, ntile, fstage, frefine, fpair);
         } else {
             tile_sweep<NW>(part, ntile, fstage, fpair);
@@ -502,6 +525,7 @@ static PreArgs make_args(Ctx &c)
     a.ngroups = c.ngroups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
+    a.mn = c.tile_mn;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

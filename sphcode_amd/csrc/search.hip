@@ -697,13 +697,15 @@ int search_alloc(Ctx &c)
         const int64_t groups = std::max<int64_t>((int64_t)c.ngroups + c.ngroups / 4 + 64, c.tile_groups_cap);
         if(c.tile_cand) (void)hipFree(c.tile_cand);
         if(c.tile_ma) (void)hipFree(c.tile_ma);
+        if(c.tile_mn) (void)hipFree(c.tile_mn);
         if(c.tile_nc) (void)hipFree(c.tile_nc);
         c.tile_cand = nullptr;
-        c.tile_ma = nullptr;
+        c.tile_ma = c.tile_mn = nullptr;
         c.tile_nc = nullptr;
         const size_t slots = (size_t)groups * wcap;
         SPHGPU_HIP(hipMalloc(&c.tile_cand, slots * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.tile_ma, slots * sizeof(uint64_t)));
+        SPHGPU_HIP(hipMalloc(&c.tile_mn, slots * sizeof(uint64_t)));
         SPHGPU_HIP(hipMalloc(&c.tile_nc, groups * sizeof(int)));
         c.tile_groups_cap = groups;
     }

@@ -75,6 +75,26 @@ __device__ __forceinline__ void tile_sweep(int part, int ntile, Stage &&stage, P
     tile_sweep<NW>(part, ntile, stage, NoRefine{}, pair);
 }
 
+// A sweep that also narrows: pair(k) says whether candidate k is to be kept,
+// and keep(t, m) receives this lane's kept hits of tile t.
+template <int NW, class Stage, class Pair, class Keep>
+__device__ __forceinline__ void tile_sweep_keep(int part, int ntile, Stage &&stage, Pair &&pair, Keep &&keep)
+{
+    for(int t = part; t < ntile; t += NW) {
+        uint64_t m = stage(t);
+        wave_lds_sync();
+        uint64_t kept = 0;
+        while(m) {
+            const int k = (int)__builtin_ctzll(m);
+            const uint64_t rest = m & (m - 1ull);
+            if(pair(k)) kept |= m ^ rest;
+            m = rest;
+        }
+        keep(t, kept);
+        wave_lds_sync();
+    }
+}
+
 // Sums of the parts' values, lane by lane and part after part (a fixed
 // order), in every part: N values at a time through `red`, which all the
 // block's waves share.  Nothing to do with one wave per group.
