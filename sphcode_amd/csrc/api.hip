@@ -94,7 +94,7 @@ static void free_buffers(Ctx &c)
         fr(c.alt.f[f]);
     }
     fr(c.s.id); fr(c.alt.id); fr(c.s.nb); fr(c.alt.nb);
-    fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff);
+    fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.bucket_cnt); fr(c.bucket_off); fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff);
     fr(c.scan_tmp); fr(c.t.geo); fr(c.t.mom); fr(c.t.rng); fr(c.t.num_nodes);
     fr(c.lvl_nodes); fr(c.msum); fr(c.groups); fr(c.lvl);
     c.num_groups = nullptr;  // inside lvl

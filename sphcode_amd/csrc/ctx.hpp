@@ -272,6 +272,11 @@ struct Ctx {
     // tree build
     uint64_t *keys = nullptr, *keys_sorted = nullptr;
     int *idx = nullptr, *perm = nullptr;
+    // sort by buckets (tree.hip): particles per bucket and the buckets' starts
+    int *bucket_cnt = nullptr, *bucket_off = nullptr;
+    int bucket_bits = 0;       // leading key bits that number a bucket
+    bool bucket_clear = false; // bucket_cnt is all zero
+    int bucket_wait = 0;       // tree builds before the buckets are tried again
     void *sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     uint8_t *delta = nullptr;

@@ -96,11 +96,34 @@ template <int D> __global__ void bbox_final(const double *partial, int nblocks, 
 }
 
 // ------------------------------------------------------------------- keys
+// The keys' sort.  The particles of one cell of an upper level (a bucket: the
+// cells numbered by the leading bucket_bits of the key, at most twice as many
+// as there are particles) are counted as the keys are made, the counts
+// scanned, the particles moved to their bucket's range, and each finds its
+// place there by counting the smaller (key, index) pairs: the order of a
+// stable sort by key, whatever order the counting took.  What bounds it is
+// launch latency and one pass over keys and indices each; with some ten
+// particles to a bucket the comparisons are few (reorder included 99 us at
+// 1M particles, 24 us at 393k).  Steps against the library's merge sort (up
+// to 1M keys) and radix sort: 2D KHI at 393k 0.863 -> 0.766 ms, the blast at
+// 2M 5.31 -> 5.05, Evrard at 20k 0.470 -> 0.445 and at 1M 4.92 -> 4.82; at
+// 400 and 4,096 particles the launches are as many and the time the same.
+// A bucket of more than BUCKET_MOST particles would make the counting
+// quadratic: the build is then done again with the library's sort, which is
+// kept for the next BUCKET_WAIT builds.
+constexpr int BUCKET_MOST = 512;
+constexpr int BUCKET_WAIT = 16;
+
 // The reference's descent, one level per slot group (src/bhtree.cpp:163-204).
-template <int D> __global__ void __launch_bounds__(BLOCK) keys_kernel(State s, int n, const double *scal, int levels, uint64_t *keys, int *idx)
+// With cnt, also each particle's rank in its bucket, in idx (otherwise idx
+// receives the index).
+template <int D>
+__global__ void __launch_bounds__(BLOCK) keys_kernel(State s, int n, const double *scal, int levels, uint64_t *keys, int *idx,
+                                                     int *cnt, int shift, int *sort_flag)
 {
 #pragma clang fp contract(off)
     const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if(i == 0) *sort_flag = 0;
     if(i >= n) return;
     double c[D], x[D];
 #pragma unroll
@@ -119,7 +142,37 @@ template <int D> __global__ void __launch_bounds__(BLOCK) keys_kernel(State s, i
         key = (key << D) | slot;
     }
     keys[i] = key;
-    idx[i] = i;
+    if(!cnt) {
+        idx[i] = i;
+        return;
+    }
+    // Neighbouring lanes are mostly in one bucket (the particles are nearly
+    // in key order): the first lane of each run counts for the run, as many
+    // updates of one counter would run one after the other.
+    const int b = (int)(key >> shift);
+    const int lane = wave_lane();
+    const int before = __shfl_up(b, 1, WAVE);  // by every lane: lane 1 reads lane 0
+    const bool head = lane == 0 || before != b;
+    const uint64_t heads = ballot(head), here = ballot(true);
+    const int first = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
+    const uint64_t later = lane == 63 ? 0 : heads >> (lane + 1) << (lane + 1);
+    const int end = later ? (int)__builtin_ctzll(later) : __popcll(here);
+    int base = 0;
+    if(head) base = atomicAdd(cnt + b, end - lane);
+    idx[i] = __shfl(base, first, WAVE) + (lane - first);
+}
+
+// Keys and indices into their buckets' ranges; clears the counts.
+__global__ void __launch_bounds__(BLOCK) bucket_scatter_kernel(const uint64_t *keys, const int *rank, int n, int shift, const int *off,
+                                                               int *cnt, int nbucket, uint64_t *bkeys, int *bidx)
+{
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if(i < nbucket) cnt[i] = 0;
+    if(i >= n) return;
+    const uint64_t key = keys[i];
+    const int p = off[key >> shift] + rank[i];
+    bkeys[p] = key;
+    bidx[p] = i;
 }
 
 // --------------------------------------------------------------- reorder
@@ -133,13 +186,37 @@ struct Reorder {
     double *sml;
     const double *mass, *dens;
     double nngb, ratio;
+    // sort by buckets: the keys in their buckets' ranges, the buckets' starts
+    // and the sorted keys (off null: perm is sorted)
+    const uint64_t *bkeys;
+    const int *off;
+    int shift, nbucket;
+    uint64_t *keys;
+    int *sort_flag;
 };
 
 template <int D> __global__ void __launch_bounds__(BLOCK) reorder_kernel(Reorder r, const int *perm, int n, int nfields)
 {
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if(i >= n) return;
-    const int j = perm[i];
+    const int p = blockIdx.x * BLOCK + threadIdx.x;
+    if(p >= n) return;
+    const int j = perm[p];
+    int i = p;  // the particle's place
+    if(r.off) {
+        const uint64_t key = r.bkeys[p];
+        const int b = (int)(key >> r.shift);
+        const int lo = r.off[b], hi = b + 1 < r.nbucket ? r.off[b + 1] : n;
+        if(hi - lo <= BUCKET_MOST) {
+            i = lo;
+#pragma unroll 4
+            for(int q = lo; q < hi; ++q) {
+                const uint64_t k = r.bkeys[q];
+                i += k < key || (k == key && perm[q] < j);
+            }
+        } else {
+            *r.sort_flag = 1;
+        }
+        r.keys[i] = key;
+    }
     for(int f = 0; f < nfields; ++f) r.dst[f][i] = r.src[f][j];
     r.idst[0][i] = r.isrc[0][j];
     if(r.isrc[1]) r.idst[1][i] = r.isrc[1][j];
@@ -244,10 +321,16 @@ __device__ int nodes_at(const uint64_t *keys, int delta_b, const TreeShape &ts, 
 }
 
 // Nodes beginning at each particle, and the deltas for emit_nodes_kernel.
-__global__ void __launch_bounds__(BLOCK) count_nodes_kernel(const uint64_t *keys, TreeShape ts, uint8_t *delta, int *nn)
+// None where the sort has given up: the keys are then in no order, and the
+// host builds again.
+__global__ void __launch_bounds__(BLOCK) count_nodes_kernel(const uint64_t *keys, TreeShape ts, uint8_t *delta, int *nn, const int *sort_flag)
 {
     const int b = blockIdx.x * BLOCK + threadIdx.x;
     if(b >= ts.n) return;
+    if(*sort_flag) {
+        nn[b] = 0;
+        return;
+    }
     const int d = key_delta(keys, b, ts.G, ts.D);
     delta[b] = (uint8_t)d;
     int lvl0 = 0;
@@ -340,9 +423,9 @@ __global__ void __launch_bounds__(BLOCK) emit_nodes_kernel(const uint64_t *keys,
 __device__ __forceinline__ int node_level(const int4 &r) { return (r.w & 255) < NLEVEL ? (r.w & 255) : NLEVEL - 1; }
 
 // Layout of lvl: counts [0, NLEVEL), offsets [NLEVEL, 2 NLEVEL), the number
-// of search groups at 2 NLEVEL (so that one copy takes all three to the
-// host), fill counters from LVL_FILL on.
-constexpr int LVL_FILL = 2 * NLEVEL + 1;
+// of search groups at LVL_GROUPS, the sort's flag at LVL_SORT (so that one
+// copy takes all four to the host), fill counters from LVL_FILL on.
+constexpr int LVL_GROUPS = 2 * NLEVEL, LVL_SORT = 2 * NLEVEL + 1, LVL_FILL = 2 * NLEVEL + 2;
 
 // offsets (lvl[NLEVEL + L]) from the counts; clears the fill counters
 __global__ void level_offsets_kernel(int *lvl)
@@ -534,10 +617,19 @@ int tree_alloc(Ctx &c)
         SPHGPU_HIP(hipMalloc(&c.leafcnt, waves * sizeof(int)));
     }
     if(!c.lvl) SPHGPU_HIP(hipMalloc(&c.lvl, (LVL_FILL + NLEVEL) * sizeof(int)));
-    c.num_groups = c.lvl + 2 * NLEVEL;
-    // per-level counts and offsets, then the number of search groups
-    if(!c.lvl_host) SPHGPU_HIP(hipHostMalloc(&c.lvl_host, (2 * NLEVEL + 1) * sizeof(int), hipHostMallocDefault));
-    for(int k = 0; k < 2 * NLEVEL + 1; ++k) c.lvl_host[k] = 0;
+    c.num_groups = c.lvl + LVL_GROUPS;
+    // per-level counts and offsets, the number of search groups, the sort's flag
+    if(!c.lvl_host) SPHGPU_HIP(hipHostMalloc(&c.lvl_host, LVL_FILL * sizeof(int), hipHostMallocDefault));
+    for(int k = 0; k < LVL_FILL; ++k) c.lvl_host[k] = 0;
+    // buckets: the cells of the deepest level that has at most twice as many
+    // cells as there are particles
+    int levels = 0;
+    while(levels < c.p.tree_max_level && (levels + 1) * c.D <= 30 && ((int64_t)1 << ((levels + 1) * c.D)) <= 2 * (int64_t)n) ++levels;
+    c.bucket_bits = levels * c.D;
+    c.bucket_clear = false;
+    c.bucket_wait = 0;
+    SPHGPU_HIP(hipMalloc(&c.bucket_cnt, ((size_t)1 << c.bucket_bits) * sizeof(int)));
+    SPHGPU_HIP(hipMalloc(&c.bucket_off, ((size_t)1 << c.bucket_bits) * sizeof(int)));
     c.group_cap = c.node_cap + n / 64 + 1;
     SPHGPU_HIP(hipMalloc(&c.groups, c.group_cap * sizeof(int2)));
     size_t bytes = 0;
@@ -547,6 +639,9 @@ int tree_alloc(Ctx &c)
     SPHGPU_HIP(hipMalloc(&c.sort_tmp, bytes));
     bytes = 0;
     SPHGPU_HIP(rocprim::exclusive_scan(nullptr, bytes, c.nn, c.noff, 0, (size_t)n, rocprim::plus<int>(), c.stream));
+    size_t bucket_bytes = 0;
+    SPHGPU_HIP(rocprim::exclusive_scan(nullptr, bucket_bytes, c.bucket_cnt, c.bucket_off, 0, (size_t)1 << c.bucket_bits, rocprim::plus<int>(), c.stream));
+    bytes = std::max(bytes, bucket_bytes);
     c.scan_tmp_bytes = bytes;
     SPHGPU_HIP(hipMalloc(&c.scan_tmp, bytes));
     return SPHGPU_OK;
@@ -585,20 +680,44 @@ static bool rewritten_in_step(const Ctx &c, int f)
     return false;
 }
 
+__global__ void __launch_bounds__(BLOCK) clear_kernel(int *p, int n)
+{
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if(i < n) p[i] = 0;
+}
+
 template <int D> static int tree_build_d(Ctx &c)
 {
     const int n = (int)c.n;
     const int G = c.p.tree_max_level;
     c.radius_ready = false;
+    const bool buckets = c.bucket_wait == 0;
+    if(!buckets) --c.bucket_wait;
+    const int nbucket = 1 << c.bucket_bits, shift = G * D - c.bucket_bits;
     // root geometry
     if(!c.p.periodic_is_valid) {
         const int nb = std::min(grid_for(n), 1024);
         hipLaunchKernelGGL(bbox_partial<D>, dim3(nb), dim3(BLOCK), 0, c.stream, c.s, n, c.partial);
         hipLaunchKernelGGL(bbox_final<D>, dim3(1), dim3(WAVE), 0, c.stream, c.partial, nb, c.scal);
     }
-    hipLaunchKernelGGL(keys_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s, n, c.scal, G, c.keys, c.idx);
-    size_t bytes = c.sort_tmp_bytes;
-    SPHGPU_HIP(rocprim::radix_sort_pairs(c.sort_tmp, bytes, c.keys, c.keys_sorted, c.idx, c.perm, (unsigned)n, 0, (unsigned)(G * D), c.stream));
+    if(buckets && !c.bucket_clear)
+        hipLaunchKernelGGL(clear_kernel, dim3(grid_for(nbucket)), dim3(BLOCK), 0, c.stream, c.bucket_cnt, nbucket);
+    c.bucket_clear = false;
+    hipLaunchKernelGGL(keys_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s, n, c.scal, G, c.keys, c.idx,
+                       buckets ? c.bucket_cnt : nullptr, shift, c.lvl + LVL_SORT);
+    size_t bytes = 0;
+    if(buckets) {
+        bytes = c.scan_tmp_bytes;
+        SPHGPU_HIP(rocprim::exclusive_scan(c.scan_tmp, bytes, c.bucket_cnt, c.bucket_off, 0, (size_t)nbucket, rocprim::plus<int>(), c.stream));
+        hipLaunchKernelGGL(bucket_scatter_kernel, dim3(grid_for(std::max(n, nbucket))), dim3(BLOCK), 0, c.stream, c.keys, c.idx, n, shift, c.bucket_off,
+                           c.bucket_cnt, nbucket, c.keys_sorted, c.perm);
+        c.bucket_clear = true;
+        // the keys in bucket order are read, the sorted ones written
+        std::swap(c.keys, c.keys_sorted);
+    } else {
+        bytes = c.sort_tmp_bytes;
+        SPHGPU_HIP(rocprim::radix_sort_pairs(c.sort_tmp, bytes, c.keys, c.keys_sorted, c.idx, c.perm, (unsigned)n, 0, (unsigned)(G * D), c.stream));
+    }
     // gather the state into key order (in sphgpu_integrate, without the
     // fields that the step rewrites before anything reads them)
     Reorder r{};
@@ -622,17 +741,29 @@ template <int D> static int tree_build_d(Ctx &c)
         r.nngb = (double)c.p.neighbor_number;
         r.ratio = c.p.iterative_sml ? 1.2 : 1.0;
     }
+    if(buckets) {
+        r.bkeys = c.keys;
+        r.off = c.bucket_off;
+        r.shift = shift;
+        r.nbucket = nbucket;
+        r.keys = c.keys_sorted;
+        r.sort_flag = c.lvl + LVL_SORT;
+    }
     hipLaunchKernelGGL(reorder_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, r, c.perm, n, nf);
-    for(int f = 0; f < NF; ++f) std::swap(c.s.f[f], c.alt.f[f]);
-    std::swap(c.s.id, c.alt.id);
-    std::swap(c.s.nb, c.alt.nb);
+    const auto swap_state = [&c] {
+        for(int f = 0; f < NF; ++f) std::swap(c.s.f[f], c.alt.f[f]);
+        std::swap(c.s.id, c.alt.id);
+        std::swap(c.s.nb, c.alt.nb);
+    };
+    swap_state();
     if(radius) {
         int rc = search_boxes(c, c.s.f[F_SML]);
         if(rc) return rc;
     }
 
     const TreeShape ts{n, G, D, c.p.tree_leaf_particle_num, c.p.tree_max_level};
-    hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn);
+    hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn,
+                       c.lvl + LVL_SORT);
     bytes = c.scan_tmp_bytes;
     SPHGPU_HIP(rocprim::exclusive_scan(c.scan_tmp, bytes, c.nn, c.noff, 0, (size_t)n, rocprim::plus<int>(), c.stream));
     hipLaunchKernelGGL(emit_nodes_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, c.delta, ts, c.nn, c.noff,
@@ -648,9 +779,16 @@ template <int D> static int tree_build_d(Ctx &c)
                        c.group_cap, D < 3 ? 1 : 0);
     hipLaunchKernelGGL(level_offsets_kernel, dim3(1), dim3(WAVE), 0, c.stream, c.lvl);
     hipLaunchKernelGGL(level_scatter_kernel, dim3(ngrid), dim3(BLOCK), 0, c.stream, c.t, c.lvl, c.lvl_nodes);
-    SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, (2 * NLEVEL + 1) * sizeof(int), hipMemcpyDeviceToHost, c.stream));
+    SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_FILL * sizeof(int), hipMemcpyDeviceToHost, c.stream));
     SPHGPU_HIP(hipStreamSynchronize(c.stream));
-    c.ngroups = c.lvl_host[2 * NLEVEL];
+    if(buckets && c.lvl_host[LVL_SORT]) {
+        // a bucket was too full to be sorted: build again from the state as
+        // it was, with the library's sort
+        swap_state();
+        c.bucket_wait = BUCKET_WAIT;
+        return tree_build_d<D>(c);
+    }
+    c.ngroups = c.lvl_host[LVL_GROUPS];
     if(c.ngroups < 1 || c.ngroups > c.group_cap) return set_error(SPHGPU_E_TREE, "search groups out of range");
     const TopLevels tl = top_levels(c);
     for(int L = NLEVEL - 1; L >= tl.first + tl.nlev; --L) {
