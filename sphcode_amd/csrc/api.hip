@@ -94,9 +94,10 @@ static void free_buffers(Ctx &c)
         fr(c.alt.f[f]);
     }
     fr(c.s.id); fr(c.alt.id); fr(c.s.nb); fr(c.alt.nb);
-    fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.bucket_cnt); fr(c.bucket_off); fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff);
-    fr(c.scan_tmp); fr(c.t.geo); fr(c.t.mom); fr(c.t.rng); fr(c.t.num_nodes);
-    fr(c.lvl_nodes); fr(c.msum); fr(c.groups); fr(c.lvl);
+    fr(c.keys); fr(c.keys_sorted); fr(c.idx); fr(c.perm); fr(c.bucket_cnt); fr(c.bucket_off); fr(c.bucket_base);
+    fr(c.sort_tmp); fr(c.delta); fr(c.nn); fr(c.noff); fr(c.nbase);
+    fr(c.t.geo); fr(c.t.mom); fr(c.t.rng); fr(c.t.num_nodes);
+    fr(c.span); fr(c.span_child); fr(c.msum); fr(c.groups); fr(c.lvl);
     c.num_groups = nullptr;  // inside lvl
     fr(c.gnode); fr(c.gpart); fr(c.gacc); fr(c.leafhit); fr(c.leafcnt); fr(c.posrec); fr(c.pair_rec); fr(c.grad_rec);
     if(c.lvl_host) (void)hipHostFree(c.lvl_host);
@@ -187,10 +188,9 @@ static int stage_tree(Ctx &c)
 }
 
 // sphgpu_integrate's gravity walk on the second stream, ordered after the
-// work queued so far on the main stream.
+// main stream's work before ev_pre.
 static int launch_gravity_walk(Ctx &c)
 {
-    SPHGPU_HIP(hipEventRecord(c.ev_pre, c.stream));
     SPHGPU_HIP(hipStreamWaitEvent(c.gstream, c.ev_pre, 0));
     if(c.timers_on) (void)hipEventRecord(c.ev_g[0], c.gstream);
     int rc = gravity_walk(c, c.gstream);
@@ -217,9 +217,9 @@ static int launch_gravity_leaves(Ctx &c)
 // finds both the gather candidates and the symmetric pairs the force stage
 // needs (search_combined); the first call keeps the reference's initial
 // smoothing and separate searches.  With `walk` the gravity walk is started
-// on the second stream just before the search (after the search radii, boxes
-// and task counters are set, so that no small kernel of the main stream
-// waits for CUs behind the walk).
+// on the second stream just after the search's launch (mixed Evrard step
+// 4.87 -> 4.62 ms at 2^20 particles, 0.418 -> 0.398 at 20k, FP64 at 131k
+// 1.27 -> 1.20 against starting it just before).
 // Kernel-span marks of sphgpu_integrate's timers (ev[8 + k]).
 static void kmark(Ctx &c, int k)
 {
@@ -244,19 +244,26 @@ static int stage_pre(Ctx &c, bool walk = false)
         if(!c.radius_ready && (rc = search_guess(c))) return rc;
         c.radius_ready = false;
         reset_work(c, 0);  // the search's task counters
-        // the gravity walk (second stream) runs beside the search
+        // the gravity walk (second stream) runs beside the search, which is
+        // launched first: the walk's waves take what the search leaves free,
+        // so that the longer path (search, pre-interaction, force) is not
+        // held up
         const int bpc = search_blocks(c, walk);
-        if(walk && (rc = launch_gravity_walk(c))) return rc;
-        walk = false;
+        if(walk) SPHGPU_HIP(hipEventRecord(c.ev_pre, c.stream));
         kmark(c, 0);
         if((rc = search_combined(c, true, bpc))) return rc;
+        if(walk && (rc = launch_gravity_walk(c))) return rc;
+        walk = false;
         kmark(c, 1);
     }
     if(c.record) {
         if((rc = search_record(c, c.rec_gather, c.rec_gather_cnt, false))) return rc;
         c.have_gather = true;
     }
-    if(walk && (rc = launch_gravity_walk(c))) return rc;
+    if(walk) {
+        SPHGPU_HIP(hipEventRecord(c.ev_pre, c.stream));
+        if((rc = launch_gravity_walk(c))) return rc;
+    }
     kmark(c, 2);
     if((rc = pre_compute(c))) return rc;
     kmark(c, 3);
@@ -413,6 +420,7 @@ int sphgpu_create(const sphgpu_params *params, void **out)
        (e = hipEventCreateWithFlags(&c->ev_pre, hipEventDisableTiming | EV_SCOPE)) != hipSuccess ||
        (e = hipEventCreateWithFlags(&c->ev_grav, hipEventDisableTiming | EV_SCOPE)) != hipSuccess ||
        (e = hipEventCreateWithFlags(&c->ev_flags, hipEventDisableTiming)) != hipSuccess ||
+       (e = hipEventCreateWithFlags(&c->ev_tree, hipEventDisableTiming)) != hipSuccess ||
        (e = hipHostMalloc(&c->counters_spec, NCOUNTERS * sizeof(int64_t), hipHostMallocDefault)) != hipSuccess ||
        // scalars and counters in one allocation (device and pinned host)
        (e = hipMalloc(&c->scal, SCAL_SPAN + NCOUNTER_ENTRIES * sizeof(int64_t))) != hipSuccess ||
@@ -464,7 +472,7 @@ int sphgpu_destroy(void *ptr)
             if(c->tev[t][k]) (void)hipEventDestroy(c->tev[t][k]);
     if(c->stream) (void)hipStreamDestroy(c->stream);
     if(c->gstream) (void)hipStreamDestroy(c->gstream);
-    for(hipEvent_t e : {c->ev_pre, c->ev_grav, c->ev_flags})
+    for(hipEvent_t e : {c->ev_pre, c->ev_grav, c->ev_flags, c->ev_tree})
         if(e) (void)hipEventDestroy(e);
     delete c;
     return SPHGPU_OK;

@@ -273,20 +273,22 @@ struct Ctx {
     uint64_t *keys = nullptr, *keys_sorted = nullptr;
     int *idx = nullptr, *perm = nullptr;
     // sort by buckets (tree.hip): particles per bucket and the buckets' starts
-    int *bucket_cnt = nullptr, *bucket_off = nullptr;
+    // (in and over the scan's tiles)
+    int *bucket_cnt = nullptr, *bucket_off = nullptr, *bucket_base = nullptr;
     int bucket_bits = 0;       // leading key bits that number a bucket
     bool bucket_clear = false; // bucket_cnt is all zero
     int bucket_wait = 0;       // tree builds before the buckets are tried again
     void *sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     uint8_t *delta = nullptr;
-    int *nn = nullptr, *noff = nullptr;
-    void *scan_tmp = nullptr;
-    size_t scan_tmp_bytes = 0;
+    int *nn = nullptr, *noff = nullptr, *nbase = nullptr; // nodes per particle, their scan in and over tiles
     TreeDev t{};
-    int *lvl_nodes = nullptr;  // node ids grouped by tree level
-    int *lvl = nullptr;        // per-level node counts, offsets, fill (device)
-    int *lvl_host = nullptr;   // per-level counts and offsets (pinned host)
+    int *span = nullptr;       // cells that span slices of nodes, span_cap per level
+    int4 *span_child = nullptr; // and their children
+    int span_cap = 0;
+    int *lvl = nullptr;        // the build's counters (tree.hip's LVL_...)
+    int *lvl_host = nullptr;   // the first of them (pinned host)
+    hipEvent_t ev_tree = nullptr; // they are on the host
     double4 *msum = nullptr;   // raw mass moments (sum m x, sum m)
     GravNode *gnode = nullptr; // gravity node records (gravity on)
     double *gacc = nullptr;    // gravity's acceleration, D x cap_n (gravity on)

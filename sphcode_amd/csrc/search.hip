@@ -602,7 +602,7 @@ __global__ void __launch_bounds__(BLOCK) leaf_radius_kernel(TreeDev t, const dou
 // loads of the first two phases; fewer leave the scalar cache (which holds
 // the groups' records) and L2 to each.  Beside the gravity walk, which is
 // bound by instruction issue, the step is shortest with two (mixed Evrard
-// step, 2^20 particles: 5.13 ms, against 5.15, 5.19 and 5.29 with three,
+// step, 2^20 particles: 4.62 ms, against 4.63, 4.66 and 4.75 with three,
 // four and six).  Alone: 2D KHI, 393,160 particles: 128 us with four (137
 // with two, 143 with six); 3D, 2^21 particles: 800 us with six (1,122 with
 // two, 865 with four, 824 with eight).

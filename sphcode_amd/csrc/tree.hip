@@ -18,9 +18,10 @@
 // b begins a level-L cell whose parent holds more than leafParticleNumber
 // particles.  Each particle emits the nodes that start at it, so an
 // exclusive scan of those counts is the pre-order numbering.  Mass moments
-// are reduced bottom-up, one tree level per launch (the upper levels, which
-// hold few nodes, in one single-workgroup launch).  The root keeps zero mass and centre of mass,
-// as the reference never accumulates them (include/bhtree.hpp:46-53).
+// are reduced bottom-up, in slices of consecutive nodes by one workgroup each
+// and then, for the few cells that span slices, by a single workgroup.  The
+// root keeps zero mass and centre of mass, as the reference never
+// accumulates them (include/bhtree.hpp:46-53).
 #include <cstring>
 
 #include "ctx.hpp"
@@ -95,6 +96,73 @@ template <int D> __global__ void bbox_final(const double *partial, int nblocks, 
     scal[S_ROOT_EDGE] = edge;
 }
 
+// Levels of the tree (> deepest level: max_level + 1 <= 65).
+constexpr int NLEVEL = 72;
+
+// Layout of lvl, all cleared by the keys' kernel: the number of search
+// groups and the sort's flag (one copy takes both to the host), the scans'
+// tickets, and the number of slice-spanning cells of each level.
+constexpr int LVL_GROUPS = 0, LVL_SORT = 1, LVL_HOST = 2, LVL_TICKET = 2, LVL_SPAN = 4, LVL_SIZE = LVL_SPAN + NLEVEL;
+
+// ------------------------------------------------------------------- scan
+// Exclusive scans by tiles: a block scans its tile and publishes the tile's
+// sum; the block that publishes last replaces the sums by their own scan
+// (their total at [gridDim.x]).  An element's prefix is its place in the
+// tile plus the tile's, two loads instead of a second pass; one launch.
+constexpr int SCAN_THREADS = 1024;
+
+// Exclusive scan over a block of SCAN_THREADS.
+__device__ __forceinline__ int block_scan(int v, int *sh, int &total)
+{
+    constexpr int NWAVE = SCAN_THREADS / WAVE;
+    const int lane = wave_lane(), w = threadIdx.x / WAVE;
+    int inc = v;
+#pragma unroll
+    for(int d = 1; d < WAVE; d *= 2) {
+        const int u = __shfl_up(inc, d, WAVE);
+        if(lane >= d) inc += u;
+    }
+    __syncthreads();  // sh is free
+    if(lane == WAVE - 1) sh[w] = inc;
+    __syncthreads();
+    int before = 0;
+    total = 0;
+#pragma unroll
+    for(int k = 0; k < NWAVE; ++k) {
+        const int x = sh[k];
+        before += k < w ? x : 0;
+        total += x;
+    }
+    return before + inc - v;
+}
+
+__device__ __forceinline__ void scan_publish(int sum, int *base, int *ticket, int *sh)
+{
+    __shared__ int last;
+    const int nb = gridDim.x;
+    if(threadIdx.x == 0) {
+        // The sum alone passes between the blocks, through atomics of device
+        // scope: it is out before the ticket is taken (a release would also
+        // write back all that the block's L2 holds; with it the nodes' count
+        // took 84 us instead of 34 at 2M particles).
+        __hip_atomic_store(base + blockIdx.x, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+    }
+    __syncthreads();
+    if(!last) return;
+    int carry = 0;
+    for(int k0 = 0; k0 < nb; k0 += SCAN_THREADS) {
+        const int k = k0 + threadIdx.x;
+        const int v = k < nb ? __hip_atomic_load(base + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        int total;
+        const int ex = block_scan(v, sh, total);
+        if(k < nb) base[k] = carry + ex;
+        carry += total;
+    }
+    if(threadIdx.x == 0) base[nb] = carry;
+}
+
 // ------------------------------------------------------------------- keys
 // The keys' sort.  The particles of one cell of an upper level (a bucket: the
 // cells numbered by the leading bucket_bits of the key, at most twice as many
@@ -119,11 +187,11 @@ constexpr int BUCKET_WAIT = 16;
 // receives the index).
 template <int D>
 __global__ void __launch_bounds__(BLOCK) keys_kernel(State s, int n, const double *scal, int levels, uint64_t *keys, int *idx,
-                                                     int *cnt, int shift, int *sort_flag)
+                                                     int *cnt, int shift, int *lvl)
 {
 #pragma clang fp contract(off)
     const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if(i == 0) *sort_flag = 0;
+    if(i < LVL_SIZE) lvl[i] = 0;  // the first block has them all
     if(i >= n) return;
     double c[D], x[D];
 #pragma unroll
@@ -162,15 +230,38 @@ __global__ void __launch_bounds__(BLOCK) keys_kernel(State s, int n, const doubl
     idx[i] = __shfl(base, first, WAVE) + (lane - first);
 }
 
-// Keys and indices into their buckets' ranges; clears the counts.
-__global__ void __launch_bounds__(BLOCK) bucket_scatter_kernel(const uint64_t *keys, const int *rank, int n, int shift, const int *off,
-                                                               int *cnt, int nbucket, uint64_t *bkeys, int *bidx)
+static_assert(LVL_SIZE <= BLOCK, "one block of the keys' kernel clears lvl");
+
+// The buckets' starts; clears their counts.
+constexpr int BUCKET_TILE = 4 * SCAN_THREADS;
+struct BucketOff {
+    const int *off, *base;
+    __device__ __forceinline__ int operator()(int b) const { return off[b] + base[b / BUCKET_TILE]; }
+};
+
+__global__ void __launch_bounds__(SCAN_THREADS) bucket_scan_kernel(int4 *cnt, int nbucket, int4 *off, int *base, int *ticket)
+{
+    __shared__ int sh[SCAN_THREADS / WAVE];
+    const int i = blockIdx.x * SCAN_THREADS + threadIdx.x;
+    int4 v = make_int4(0, 0, 0, 0);
+    if(i < nbucket / 4) {
+        v = cnt[i];
+        cnt[i] = make_int4(0, 0, 0, 0);
+    }
+    int total;
+    const int ex = block_scan(v.x + v.y + v.z + v.w, sh, total);
+    if(i < nbucket / 4) off[i] = make_int4(ex, ex + v.x, ex + v.x + v.y, ex + v.x + v.y + v.z);
+    scan_publish(total, base, ticket, sh);
+}
+
+// Keys and indices into their buckets' ranges.
+__global__ void __launch_bounds__(BLOCK) bucket_scatter_kernel(const uint64_t *keys, const int *rank, int n, int shift, BucketOff off,
+                                                               uint64_t *bkeys, int *bidx)
 {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if(i < nbucket) cnt[i] = 0;
     if(i >= n) return;
     const uint64_t key = keys[i];
-    const int p = off[key >> shift] + rank[i];
+    const int p = off((int)(key >> shift)) + rank[i];
     bkeys[p] = key;
     bidx[p] = i;
 }
@@ -187,9 +278,9 @@ struct Reorder {
     const double *mass, *dens;
     double nngb, ratio;
     // sort by buckets: the keys in their buckets' ranges, the buckets' starts
-    // and the sorted keys (off null: perm is sorted)
+    // and the sorted keys (bkeys null: perm is sorted)
     const uint64_t *bkeys;
-    const int *off;
+    BucketOff off;
     int shift, nbucket;
     uint64_t *keys;
     int *sort_flag;
@@ -201,10 +292,10 @@ template <int D> __global__ void __launch_bounds__(BLOCK) reorder_kernel(Reorder
     if(p >= n) return;
     const int j = perm[p];
     int i = p;  // the particle's place
-    if(r.off) {
+    if(r.bkeys) {
         const uint64_t key = r.bkeys[p];
         const int b = (int)(key >> r.shift);
-        const int lo = r.off[b], hi = b + 1 < r.nbucket ? r.off[b + 1] : n;
+        const int lo = r.off(b), hi = b + 1 < r.nbucket ? r.off(b + 1) : n;
         if(hi - lo <= BUCKET_MOST) {
             i = lo;
 #pragma unroll 4
@@ -234,9 +325,6 @@ __device__ __forceinline__ int key_delta(const uint64_t *k, int i, int G, int D)
     const int lz = __clzll((long long)x) - (64 - G * D);
     return lz / D;
 }
-
-// Levels of the per-level node lists (> deepest level: max_level + 1 <= 65).
-constexpr int NLEVEL = 72;
 
 // Search groups: compact sets of at most 64 key-consecutive particles.
 // Every cell holding more than 64 particles packs its children that hold at
@@ -306,10 +394,10 @@ __device__ __forceinline__ bool parent_split(const uint64_t *keys, const TreeSha
 }
 
 // Number of nodes that begin at particle b (all at consecutive levels).
-__device__ int nodes_at(const uint64_t *keys, int delta_b, const TreeShape &ts, int b, int &lvl0)
+__device__ __forceinline__ int nodes_at(const uint64_t *keys, int delta_b, const TreeShape &ts, int b)
 {
     if(b > 0 && delta_b >= ts.G) return 0;  // same deepest cell as b-1
-    lvl0 = first_level(delta_b, b);
+    const int lvl0 = first_level(delta_b, b);
     if(lvl0 > 2 && !parent_split(keys, ts, b, lvl0 - 1)) return 0;
     int k = 0;
     for(int L = lvl0;; ++L) {
@@ -320,270 +408,362 @@ __device__ int nodes_at(const uint64_t *keys, int delta_b, const TreeShape &ts, 
     return k;
 }
 
-// Nodes beginning at each particle, and the deltas for emit_nodes_kernel.
-// None where the sort has given up: the keys are then in no order, and the
-// host builds again.
-__global__ void __launch_bounds__(BLOCK) count_nodes_kernel(const uint64_t *keys, TreeShape ts, uint8_t *delta, int *nn, const int *sort_flag)
+// Nodes beginning at each particle, scanned by tiles of SCAN_THREADS, and
+// the deltas for emit_nodes_kernel.  None where the sort has given up: the
+// keys are then in no order, and the host builds again.
+__global__ void __launch_bounds__(SCAN_THREADS) count_nodes_kernel(const uint64_t *keys, TreeShape ts, uint8_t *delta, int *nn, int *noff,
+                                                                int *base, int *lvl)
 {
-    const int b = blockIdx.x * BLOCK + threadIdx.x;
-    if(b >= ts.n) return;
-    if(*sort_flag) {
-        nn[b] = 0;
-        return;
+    __shared__ int sh[SCAN_THREADS / WAVE];
+    const int b = blockIdx.x * SCAN_THREADS + threadIdx.x;
+    int k = 0;
+    if(b < ts.n && !lvl[LVL_SORT]) {
+        const int d = key_delta(keys, b, ts.G, ts.D);
+        delta[b] = (uint8_t)d;
+        k = nodes_at(keys, d, ts, b);
     }
-    const int d = key_delta(keys, b, ts.G, ts.D);
-    delta[b] = (uint8_t)d;
-    int lvl0 = 0;
-    nn[b] = nodes_at(keys, d, ts, b, lvl0);
+    int total;
+    const int ex = block_scan(k, sh, total);
+    if(b < ts.n) {
+        nn[b] = k;
+        noff[b] = ex;
+    }
+    scan_publish(total, base, lvl + LVL_TICKET + 1, sh);
 }
 
 // End (exclusive) of the level-L cell that begins at b: first particle
-// whose key differs in the first L-1 slot groups.
+// whose key differs in the first L-1 slot groups.  Most cells are small, so
+// steps of 16, 64, ... look for a stretch that holds the end first.
 __device__ __forceinline__ int cell_end(const uint64_t *keys, const TreeShape &ts, int b, int L)
 {
     const int shift = (ts.G - (L - 1)) * ts.D;
-    const uint64_t pre = shift >= 64 ? 0 : keys[b] >> shift;
-    int lo = b + 1, hi = ts.n;
+    const uint64_t pre = cell_prefix(keys[b], shift);
+    int in = b, step = 16;
+    while(step < ts.n - in && cell_prefix(keys[in + step], shift) == pre) {
+        in += step;
+        step = step < 1 << 28 ? step * 4 : step;
+    }
+    int lo = in + 1, hi = step < ts.n - in ? in + step : ts.n;
     while(lo < hi) {
         const int mid = (lo + hi) >> 1;
-        const uint64_t pm = shift >= 64 ? 0 : keys[mid] >> shift;
-        if(pm > pre) hi = mid;
+        if(cell_prefix(keys[mid], shift) > pre) hi = mid;
         else lo = mid + 1;
     }
     return lo;
 }
 
-// Also clears the per-level counters (lvl) and the search groups: the
-// groups of a root holding at most GROUP particles, none otherwise.
-template <int D>
-__global__ void __launch_bounds__(BLOCK) emit_nodes_kernel(const uint64_t *keys, const uint8_t *delta, TreeShape ts, const int *nn,
-                                                        const int *noff, const double *scal, TreeDev t, int64_t node_cap,
-                                                        int64_t *counters, int *lvl, int2 *groups, int *num_groups)
+// Mass and centre of mass of a node from its sums.  The root's stay zero.
+__device__ __forceinline__ void store_mom(const TreeDev &t, int p, const double4 &acc)
 {
-#pragma clang fp contract(off)
-    const int b = blockIdx.x * BLOCK + threadIdx.x;
-    if(b < NLEVEL) lvl[b] = 0;  // the level counts (the grid has at least BLOCK > NLEVEL threads)
-    if(b >= ts.n) return;
-    const int total = 1 + noff[ts.n - 1] + nn[ts.n - 1];
-    if(b == 0) {
-        *t.num_nodes = total <= node_cap ? total : (int)node_cap;
-        if(total > node_cap) atomicAdd((unsigned long long *)&counters[C_TREE_ERR], 1ull);
-        t.geo[0] = make_double4(scal[S_ROOT_CX], D > 1 ? scal[S_ROOT_CY] : 0.0, D > 2 ? scal[S_ROOT_CZ] : 0.0, scal[S_ROOT_EDGE]);
-        t.rng[0] = make_int4(0, ts.n, total, 1);
-        int ng = 0;
-        if(ts.n <= GROUP) groups[ng++] = make_int2(0, ts.n);
-        *num_groups = ng;
-    }
-    const int cnt = nn[b];
-    if(cnt == 0) return;
-    int lvl0 = 0;
-    nodes_at(keys, (int)delta[b], ts, b, lvl0);
-    const int base = 1 + noff[b];
-    const uint64_t key = keys[b];
-    const uint64_t mask = (1ull << D) - 1ull;
-    double c[D];
-#pragma unroll
-    for(int k = 0; k < D; ++k) c[k] = scal[S_ROOT_CX + k];
-    double e = scal[S_ROOT_EDGE];
-    // replay the descent down to level lvl0 - 1
-    int g = 0;
-    for(; g < lvl0 - 2; ++g) {
-        const uint64_t slot = (key >> ((ts.G - 1 - g) * D)) & mask;
-#pragma unroll
-        for(int k = 0; k < D; ++k) c[k] = c[k] + (((slot >> k) & 1) ? 1.0 : -1.0) * e * 0.25;
-        e = e * 0.5;
-    }
-    for(int j = 0; j < cnt; ++j) {
-        const int L = lvl0 + j;
-        // descend one more level: cell of level L
-        const uint64_t slot = (key >> ((ts.G - 1 - g) * D)) & mask;
-#pragma unroll
-        for(int k = 0; k < D; ++k) c[k] = c[k] + (((slot >> k) & 1) ? 1.0 : -1.0) * e * 0.25;
-        e = e * 0.5;
-        ++g;
-        const int node = base + j;
-        const bool leaf = j == cnt - 1;
-        int end;
-        if(leaf && L <= ts.max_level) end = b + cell_count_bounded(keys, ts, b, L);
-        else end = cell_end(keys, ts, b, L);
-        const int skip = end < ts.n ? 1 + noff[end] : total;
-        if(node < node_cap) {
-            t.geo[node] = make_double4(c[0], D > 1 ? c[D > 1 ? 1 : 0] : 0.0, D > 2 ? c[D > 2 ? 2 : 0] : 0.0, e);
-            t.rng[node] = make_int4(b, end, skip, L | (leaf ? 256 : 0));
-        }
-    }
-}
-
-// ------------------------------------------------- level-by-level reductions
-// Node sums are formed bottom-up one tree level per launch: a launch
-// boundary orders the children's results before the parents read them, so
-// no cross-XCD atomics or cache maintenance are needed.  The nodes of each
-// level are listed once per tree build (level_bins / level_scatter).
-
-__device__ __forceinline__ int node_level(const int4 &r) { return (r.w & 255) < NLEVEL ? (r.w & 255) : NLEVEL - 1; }
-
-// Layout of lvl: counts [0, NLEVEL), offsets [NLEVEL, 2 NLEVEL), the number
-// of search groups at LVL_GROUPS, the sort's flag at LVL_SORT (so that one
-// copy takes all four to the host), fill counters from LVL_FILL on.
-constexpr int LVL_GROUPS = 2 * NLEVEL, LVL_SORT = 2 * NLEVEL + 1, LVL_FILL = 2 * NLEVEL + 2;
-
-// offsets (lvl[NLEVEL + L]) from the counts; clears the fill counters
-__global__ void level_offsets_kernel(int *lvl)
-{
-    if(threadIdx.x != 0) return;
-    int o = 0;
-    for(int k = 0; k < NLEVEL; ++k) {
-        lvl[NLEVEL + k] = o;
-        lvl[LVL_FILL + k] = 0;
-        o += lvl[k];
-    }
-}
-
-__global__ void __launch_bounds__(BLOCK) level_scatter_kernel(TreeDev t, int *lvl, int *nodes)
-{
-    __shared__ int bins[NLEVEL], base[NLEVEL];
-    for(int k = threadIdx.x; k < NLEVEL; k += BLOCK) bins[k] = 0;
-    __syncthreads();
-    const int p = blockIdx.x * BLOCK + threadIdx.x;
-    const int total = *t.num_nodes;
-    int L = 0, rank = 0;
-    if(p < total) {
-        L = node_level(t.rng[p]);
-        rank = atomicAdd(&bins[L], 1);
-    }
-    __syncthreads();
-    for(int k = threadIdx.x; k < NLEVEL; k += BLOCK)
-        base[k] = bins[k] ? atomicAdd(&lvl[LVL_FILL + k], bins[k]) : 0;
-    __syncthreads();
-    if(p < total) nodes[lvl[NLEVEL + L] + base[L] + rank] = p;
-}
-
-// Mass and centre of mass of the nodes of one level: a leaf sums its
-// particles, an internal node its children (one level deeper, done by the
-// previous launch), in child order.  The root's moments stay zero, as the
-// reference never accumulates them (include/bhtree.hpp:46-53).
-template <int D> __device__ __forceinline__ void moments_node(const State &s, const TreeDev &t, int p, int total, double4 *msum)
-{
-    const int4 r = t.rng[p];
-    double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
-    if(r.w & 256) {
-        double mx[3] = {0.0, 0.0, 0.0};
-        for(int i = r.x; i < r.y; ++i) {
-            const double mi = s.f[F_MASS][i];
-            acc.w += mi;
-#pragma unroll
-            for(int q = 0; q < D; ++q) mx[q] += s.f[F_X + q][i] * mi;
-        }
-        acc.x = mx[0];
-        acc.y = mx[1];
-        acc.z = mx[2];
-    } else {
-        int guard = 0;
-        for(int c = p + 1; c < r.z && c < total && guard < 8; c = t.rng[c].z, ++guard) {
-            const double4 v = msum[c];
-            acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-        }
-    }
-    msum[p] = acc;
     if(p == 0) t.mom[0] = make_double4(0.0, 0.0, 0.0, 0.0);
     else t.mom[p] = make_double4(acc.x / acc.w, acc.y / acc.w, acc.z / acc.w, acc.w);
 }
 
-template <int D>
-__global__ void __launch_bounds__(BLOCK) moments_level_kernel(State s, TreeDev t, const int *nodes, int count, double4 *msum)
+template <int D> __device__ __forceinline__ void leaf_moments(const State &s, const TreeDev &t, int p, int begin, int end, double4 *msum)
 {
-    const int k = blockIdx.x * BLOCK + threadIdx.x;
-    if(k >= count) return;
-    moments_node<D>(s, t, nodes[k], *t.num_nodes, msum);
+    double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
+    double mx[3] = {0.0, 0.0, 0.0};
+    for(int j = begin; j < end; ++j) {
+        const double mj = s.f[F_MASS][j];
+        acc.w += mj;
+#pragma unroll
+        for(int q = 0; q < D; ++q) mx[q] += s.f[F_X + q][j] * mj;
+    }
+    acc.x = mx[0];
+    acc.y = mx[1];
+    acc.z = mx[2];
+    msum[p] = acc;
+    store_mom(t, p, acc);
 }
 
-// The upper levels, which hold few nodes, in one launch of one workgroup:
-// level after level bottom-up, a barrier between levels orders the
-// children's results before their parents read them (one workgroup runs on
-// one CU, whose waves see each other's stores once past the barrier).
-constexpr int TOP_THREADS = 1024;
-constexpr int TOP_MAXNODES = 512;  // a level is one of the upper ones up to this many nodes
-struct TopLevels {
-    int first;        // levels first .. first + nlev - 1 (entry k is level first + k)
-    int nlev;
-    int count[16];
-    int offset[16];
-};
-
+// The nodes that begin at a block's particles: a node per lane (they are
+// consecutive; the particle by bisection in LDS), so that no lane walks a
+// chain of searches for a particle where many cells begin.  Also the search
+// group of a root that holds at most GROUP particles, and the leaves' moments
+// (their particles in order).  At 400 particles (11
+// levels) 13 us, without the leaves' moments and with a particle per lane 26;
+// in 2D at 393k 15 (39), in 3D at 2M 109 (126).
 template <int D>
-__global__ void __launch_bounds__(TOP_THREADS) moments_top_kernel(State s, TreeDev t, const int *nodes, TopLevels tl, double4 *msum)
+__global__ void __launch_bounds__(BLOCK) emit_nodes_kernel(const uint64_t *keys, const uint8_t *delta, TreeShape ts, const int *nn,
+                                                        const int *noff, const int *base, const double *scal, State s, TreeDev t, double4 *msum,
+                                                        int64_t node_cap, int64_t *counters, int2 *groups, int *num_groups)
 {
-    const int total = *t.num_nodes;
-    for(int L = tl.nlev - 1; L >= 0; --L) {
-        for(int k = threadIdx.x; k < tl.count[L]; k += TOP_THREADS) moments_node<D>(s, t, nodes[tl.offset[L] + k], total, msum);
-        __syncthreads();
-    }
-}
-
-
-// Per node: the per-level node counts (block histograms, one atomic per bin
-// and block), and the groups of a packing cell.
-__global__ void __launch_bounds__(BLOCK) level_count_groups_kernel(TreeDev t, int *lvl, int2 *groups, int *num_groups,
-                                                                int64_t group_cap, int runs)
-{
-    __shared__ int bins[NLEVEL];
-    for(int k = threadIdx.x; k < NLEVEL; k += BLOCK) bins[k] = 0;
-    __syncthreads();
-    const int q = blockIdx.x * BLOCK + threadIdx.x;
-    const int total = *t.num_nodes;
-    int4 rq = make_int4(0, 0, 0, 0);
-    if(q < total) {
-        rq = t.rng[q];
-        atomicAdd(&bins[node_level(rq)], 1);
-    }
-    __syncthreads();
-    for(int k = threadIdx.x; k < NLEVEL; k += BLOCK)
-        if(bins[k]) atomicAdd(&lvl[k], bins[k]);
-    if(q >= total) return;
-    if((rq.w & 256) || rq.y - rq.x <= GROUP) return;  // not a packing cell
-    const int end = rq.z > q ? rq.z : total;
-    // two passes over the children: count the groups, then write them
-    int g0 = 0;
-    for(int pass = 0; pass < 2; ++pass) {
-        int ng = 0, cb = -1, ce = -1;
-        auto emit = [&](int b, int e) {
-            if(pass == 1 && g0 + ng < group_cap) groups[g0 + ng] = make_int2(b, e);
-            ++ng;
-        };
-        // runs: a stretch [b, e) of consecutive small children is cut into
-        // ceil((e - b) / GROUP) groups of equal size, which fills the waves
-        // but does not keep whole cells together
-        auto cut = [&](int b, int e) {
-            const int k = (e - b + GROUP - 1) / GROUP;
-            for(int j = 0; j < k; ++j) emit(b + (int)((int64_t)(e - b) * j / k), b + (int)((int64_t)(e - b) * (j + 1) / k));
-        };
-        for(int c = q + 1; c < end;) {
-            const int4 rc = t.rng[c];
-            const int cnt = rc.y - rc.x;
-            const bool leaf = (rc.w & 256) != 0;
-            if(cnt > GROUP) {
-                if(cb >= 0) {
-                    if(runs) cut(cb, ce);
-                    else emit(cb, ce);
-                }
-                cb = -1;
-                if(leaf)
-                    for(int b = rc.x; b < rc.y; b += GROUP) emit(b, b + GROUP < rc.y ? b + GROUP : rc.y);
-            } else if(cnt > 0) {
-                if(!runs && cb >= 0 && rc.y - cb > GROUP) {
-                    emit(cb, ce);
-                    cb = -1;
-                }
-                if(cb < 0) cb = rc.x;
-                ce = rc.y;
+#pragma clang fp contract(off)
+    __shared__ int first[BLOCK + 1];  // first node of each particle
+    const int b0 = blockIdx.x * BLOCK, nb = min(BLOCK, ts.n - b0);
+    const int total = 1 + base[(ts.n + SCAN_THREADS - 1) / SCAN_THREADS];
+    const auto node_of = [&](int b) { return 1 + noff[b] + base[b / SCAN_THREADS]; };
+    if((int)threadIdx.x < nb) {
+        const int b = b0 + threadIdx.x;
+        const int f = node_of(b);
+        first[threadIdx.x] = f;
+        if((int)threadIdx.x == nb - 1) first[nb] = f + nn[b];
+        if(b == 0) {
+            *t.num_nodes = total <= node_cap ? total : (int)node_cap;
+            if(total > node_cap) atomicAdd((unsigned long long *)&counters[C_TREE_ERR], 1ull);
+            t.geo[0] = make_double4(scal[S_ROOT_CX], D > 1 ? scal[S_ROOT_CY] : 0.0, D > 2 ? scal[S_ROOT_CZ] : 0.0, scal[S_ROOT_EDGE]);
+            t.rng[0] = make_int4(0, ts.n, total, 1);
+            if(ts.n <= GROUP) {
+                groups[0] = make_int2(0, ts.n);
+                *num_groups = 1;
             }
-            c = rc.z > c ? rc.z : c + 1;
         }
-        if(cb >= 0) {
-            if(runs) cut(cb, ce);
-            else emit(cb, ce);
+    }
+    __syncthreads();
+    const uint64_t mask = (1ull << D) - 1ull;
+    const int end_node = min((int64_t)first[nb], node_cap);
+    for(int node = first[0] + threadIdx.x; node < end_node; node += BLOCK) {
+        int lo = 0, hi = nb - 1;  // last particle whose first node is not past this one
+        while(lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if(first[mid] <= node) lo = mid;
+            else hi = mid - 1;
         }
-        if(pass == 0) g0 = atomicAdd(num_groups, ng);
+        const int b = b0 + lo;
+        const int L = first_level((int)delta[b], b) + node - first[lo];
+        const bool leaf = node == first[lo + 1] - 1;
+        const uint64_t key = keys[b];
+        const int end = leaf && L <= ts.max_level ? b + cell_count_bounded(keys, ts, b, L) : cell_end(keys, ts, b, L);
+        const int skip = end < ts.n ? node_of(end) : total;
+        // replay the descent down to level L
+        double c[D];
+#pragma unroll
+        for(int k = 0; k < D; ++k) c[k] = scal[S_ROOT_CX + k];
+        double e = scal[S_ROOT_EDGE];
+        for(int g = 0; g < L - 1; ++g) {
+            const uint64_t slot = (key >> ((ts.G - 1 - g) * D)) & mask;
+#pragma unroll
+            for(int k = 0; k < D; ++k) c[k] = c[k] + (((slot >> k) & 1) ? 1.0 : -1.0) * e * 0.25;
+            e = e * 0.5;
+        }
+        t.geo[node] = make_double4(c[0], D > 1 ? c[D > 1 ? 1 : 0] : 0.0, D > 2 ? c[D > 2 ? 2 : 0] : 0.0, e);
+        t.rng[node] = make_int4(b, end, skip, L | (leaf ? 256 : 0));
+        if(leaf) leaf_moments<D>(s, t, node, b, end, msum);
+    }
+}
+
+// ---------------------------------------------------- moments and groups
+__device__ __forceinline__ int node_level(const int4 &r) { return (r.w & 255) < NLEVEL ? (r.w & 255) : NLEVEL - 1; }
+
+// The search groups of a packing cell (range rq, first child q + 1):
+// emit(begin, end) for each.  small(c) is the number of particles of node c
+// if it is at most GROUP, otherwise -1; next(c) the node after its subtree.
+template <class Small, class Next, class Emit>
+__device__ __forceinline__ void pack_groups(const int4 *rng, int q, const int4 &rq, int total, bool runs, Small &&small, Next &&next, Emit &&emit)
+{
+    // runs: a stretch [b, e) of consecutive small children is cut into
+    // ceil((e - b) / GROUP) groups of equal size, which fills the waves
+    // but does not keep whole cells together
+    auto cut = [&](int b, int e) {
+        const int k = runs ? (e - b + GROUP - 1) / GROUP : 1;
+        for(int j = 0; j < k; ++j) emit(b + (e - b) * j / k, b + (e - b) * (j + 1) / k);  // at most 8 GROUP particles
+    };
+    const int end = min(rq.z, total);
+    int cb = -1, ce = rq.x;  // the open stretch; the children cover the cell in order
+    for(int c = q + 1; c < end; c = next(c)) {
+        const int cnt = small(c);
+        if(cnt < 0) {
+            if(cb >= 0) cut(cb, ce);
+            cb = -1;
+            const int4 rc = rng[c];
+            if(rc.w & 256)
+                for(int b = rc.x; b < rc.y; b += GROUP) emit(b, b + GROUP < rc.y ? b + GROUP : rc.y);
+            ce = rc.y;
+        } else {
+            if(!runs && cb >= 0 && ce + cnt - cb > GROUP) {
+                cut(cb, ce);
+                cb = -1;
+            }
+            if(cb < 0) cb = ce;
+            ce += cnt;
+        }
+    }
+    if(cb >= 0) cut(cb, ce);
+}
+
+// Moments of the internal cells and search groups of SLICE consecutive
+// nodes.  A cell sums its children, in child order: the cells whose whole
+// subtree lies in the slice, level after level in LDS.  For those that reach
+// past it (one to a level at most) the children are listed for
+// spanning_kernel, and the sums that these need go to msum.  What bounds it
+// is latency (about eight dependent LDS reads per cell and level); one
+// launch takes the place of node lists by level and a launch for each
+// level: 29 us (with the moments of leaves 61) in 2D at 393k
+// particles, 39 (153) at 1M and 105 (400) at 2M in 3D.
+constexpr int SLICE = 2048;  // the larger, the fewer cells span slices; 74 KB of LDS
+constexpr int NO_CHILD = -1;  // a child c that spans slices itself is listed as -2 - c
+constexpr int SLICE_PER = SLICE / SCAN_THREADS;
+__global__ void __launch_bounds__(SCAN_THREADS) slice_kernel(TreeDev t, double4 *msum, int *span_cnt, int *span, int4 *span_child, int span_cap,
+                                                          int2 *groups, int *num_groups, int64_t group_cap, int runs)
+{
+    __shared__ double4 m[SLICE];
+    __shared__ uint16_t skip[SLICE];   // of the cells within the slice: the node after the subtree
+    __shared__ uint8_t count[SLICE];   // particles, or 255 (more than GROUP)
+    __shared__ uint8_t used[SLICE];    // internal cells: summed into the parent
+    __shared__ int deepest, ngroups, group0;
+    const int total = *t.num_nodes;
+    for(int v0 = blockIdx.x * SLICE; v0 < total; v0 += gridDim.x * SLICE) {
+        const int nloc = min(SLICE, total - v0), v1 = v0 + nloc;
+        if(threadIdx.x == 0) {
+            deepest = 0;
+            ngroups = 0;
+        }
+        __syncthreads();
+        int4 r[SLICE_PER];
+        int level[SLICE_PER];  // of an internal cell within the slice, otherwise -1
+#pragma unroll
+        for(int k = 0; k < SLICE_PER; ++k) {
+            const int i = threadIdx.x + k * SCAN_THREADS;
+            r[k] = i < nloc ? t.rng[v0 + i] : make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for(int k = 0; k < SLICE_PER; ++k) {
+            const int i = threadIdx.x + k * SCAN_THREADS;
+            level[k] = -1;
+            if(i >= nloc) continue;
+            skip[i] = (uint16_t)min(r[k].z - v0, SLICE);
+            count[i] = (uint8_t)(r[k].y - r[k].x <= GROUP ? r[k].y - r[k].x : 255);
+            used[i] = 0;
+            if(r[k].w & 256) {
+                m[i] = msum[v0 + i];
+            } else if(r[k].z <= v1) {
+                level[k] = node_level(r[k]);
+                atomicMax(&deepest, level[k]);
+            }
+        }
+        __syncthreads();
+        for(int L = deepest; L >= 1; --L) {
+#pragma unroll
+            for(int k = 0; k < SLICE_PER; ++k) {
+                if(level[k] != L) continue;
+                const int i = threadIdx.x + k * SCAN_THREADS;
+                const int end = r[k].z - v0;
+                double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
+                int guard = 0;
+                for(int c = i + 1; c < end && guard < 8; c = skip[c], ++guard) {
+                    const double4 v = m[c];
+                    acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+                    used[c] = 1;
+                }
+                m[i] = acc;
+            }
+            __syncthreads();
+        }
+        const auto small = [&](int c) {
+            if(c < v1) return count[c - v0] <= GROUP ? (int)count[c - v0] : -1;
+            const int4 rc = t.rng[c];
+            return rc.y - rc.x <= GROUP ? rc.y - rc.x : -1;
+        };
+        const auto next = [&](int c) { return c < v1 && skip[c - v0] < SLICE ? v0 + skip[c - v0] : t.rng[c].z; };
+        int ng[SLICE_PER], at0[SLICE_PER];
+#pragma unroll
+        for(int k = 0; k < SLICE_PER; ++k) {
+            const int i = threadIdx.x + k * SCAN_THREADS;
+            ng[k] = at0[k] = 0;
+            if(i >= nloc) continue;
+            if(r[k].w & 256) continue;
+            if(level[k] >= 0) {
+                const double4 acc = m[i];
+                store_mom(t, v0 + i, acc);
+                if(!used[i]) msum[v0 + i] = acc;
+            } else {
+                const int L = node_level(r[k]), slot = atomicAdd(span_cnt + L, 1);
+                int child[8], c = v0 + i + 1;
+                const int end = min(r[k].z, total);
+#pragma unroll
+                for(int q = 0; q < 8; ++q) {
+                    child[q] = NO_CHILD;
+                    if(c >= end) continue;
+                    const int4 rc = t.rng[c];
+                    const bool spans = !(rc.w & 256) && rc.z > (c / SLICE + 1) * SLICE && rc.z > c;
+                    child[q] = spans ? -2 - c : c;
+                    c = rc.z > c ? rc.z : c + 1;
+                }
+                if(slot < span_cap) {
+                    const int64_t at = (int64_t)L * span_cap + slot;
+                    span[at] = v0 + i;
+                    span_child[2 * at] = make_int4(child[0], child[1], child[2], child[3]);
+                    span_child[2 * at + 1] = make_int4(child[4], child[5], child[6], child[7]);
+                }
+            }
+            if(r[k].y - r[k].x > GROUP) {
+                pack_groups(t.rng, v0 + i, r[k], total, runs, small, next, [&](int, int) { ++ng[k]; });
+                if(ng[k]) at0[k] = atomicAdd(&ngroups, ng[k]);
+            }
+        }
+        __syncthreads();
+        if(threadIdx.x == 0 && ngroups) group0 = atomicAdd(num_groups, ngroups);
+        __syncthreads();
+#pragma unroll
+        for(int k = 0; k < SLICE_PER; ++k) {
+            if(!ng[k]) continue;
+            int64_t g = (int64_t)group0 + at0[k];
+            pack_groups(t.rng, v0 + (int)threadIdx.x + k * SCAN_THREADS, r[k], total, runs, small, next, [&](int b, int e) {
+                if(g < group_cap) groups[g] = make_int2(b, e);
+                ++g;
+            });
+        }
+        __syncthreads();  // the slice's LDS is free
+    }
+}
+
+// Moments of the cells that span slices, in one workgroup: the children
+// within slices are fetched for all cells at once, then level after level
+// bottom-up those that span slices themselves; a barrier between levels
+// orders the children's results before their parents read them (one
+// workgroup runs on one CU, whose waves see each other's stores once past
+// the barrier).  Two chunks of cells take 84 us at
+// 2M particles, one 10 to 18 at 393k and 1M.
+__global__ void __launch_bounds__(SCAN_THREADS) spanning_kernel(TreeDev t, double4 *msum, const int *span_cnt, const int *span,
+                                                             const int4 *span_child, int span_cap)
+{
+    __shared__ int sh[SCAN_THREADS / WAVE];
+    __shared__ int off[NLEVEL];  // of the level NLEVEL - 1 - e: deepest first
+    if(*t.num_nodes <= SLICE) return;  // one slice: none spans
+    int total;
+    const int ex = block_scan((int)threadIdx.x < NLEVEL ? span_cnt[NLEVEL - 1 - threadIdx.x] : 0, sh, total);
+    if((int)threadIdx.x < NLEVEL) off[threadIdx.x] = ex;
+    __syncthreads();
+    const auto entry = [&](int k) {  // the last e with off[e] <= k
+        int lo = 0, hi = NLEVEL - 1;
+        while(lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if(off[mid] <= k) lo = mid;
+            else hi = mid - 1;
+        }
+        return lo;
+    };
+    for(int k0 = 0; k0 < total; k0 += SCAN_THREADS) {
+        const int k = k0 + threadIdx.x;
+        int e = -1, p = 0;
+        int child[8];
+        double4 v[8];
+        if(k < total) {
+            e = entry(k);
+            const int64_t at = (int64_t)(NLEVEL - 1 - e) * span_cap + k - off[e];
+            p = span[at];
+            const int4 a = span_child[2 * at], b = span_child[2 * at + 1];
+            child[0] = a.x; child[1] = a.y; child[2] = a.z; child[3] = a.w;
+            child[4] = b.x; child[5] = b.y; child[6] = b.z; child[7] = b.w;
+#pragma unroll
+            for(int q = 0; q < 8; ++q)
+                if(child[q] >= 0) v[q] = msum[child[q]];
+        }
+        const int e1 = entry(min(k0 + SCAN_THREADS, total) - 1);
+        for(int x = entry(k0); x <= e1; ++x) {
+            if(e == x) {
+                double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
+#pragma unroll
+                for(int q = 0; q < 8; ++q) {
+                    if(child[q] == NO_CHILD) continue;
+                    if(child[q] < NO_CHILD) v[q] = msum[-2 - child[q]];
+                    acc.x += v[q].x; acc.y += v[q].y; acc.z += v[q].z; acc.w += v[q].w;
+                }
+                msum[p] = acc;
+                store_mom(t, p, acc);
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -599,11 +779,14 @@ int tree_alloc(Ctx &c)
     SPHGPU_HIP(hipMalloc(&c.delta, n));
     SPHGPU_HIP(hipMalloc(&c.nn, n * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.noff, n * sizeof(int)));
+    SPHGPU_HIP(hipMalloc(&c.nbase, (grid_for(n, SCAN_THREADS) + 1) * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.t.geo, c.node_cap * sizeof(double4)));
     SPHGPU_HIP(hipMalloc(&c.t.mom, c.node_cap * sizeof(double4)));
     SPHGPU_HIP(hipMalloc(&c.t.rng, c.node_cap * sizeof(int4)));
     SPHGPU_HIP(hipMalloc(&c.t.num_nodes, sizeof(int)));
-    SPHGPU_HIP(hipMalloc(&c.lvl_nodes, c.node_cap * sizeof(int)));
+    c.span_cap = (int)grid_for(c.node_cap, SLICE);
+    SPHGPU_HIP(hipMalloc(&c.span, (size_t)NLEVEL * c.span_cap * sizeof(int)));
+    SPHGPU_HIP(hipMalloc(&c.span_child, (size_t)NLEVEL * c.span_cap * 2 * sizeof(int4)));
     SPHGPU_HIP(hipMalloc(&c.msum, c.node_cap * sizeof(double4)));
     if(c.p.gravity_is_valid) {
         SPHGPU_HIP(hipMalloc(&c.gnode, c.node_cap * sizeof(GravNode)));
@@ -616,11 +799,10 @@ int tree_alloc(Ctx &c)
         SPHGPU_HIP(hipMalloc(&c.leafhit, waves * LEAFHIT_CAP * sizeof(LeafHit)));
         SPHGPU_HIP(hipMalloc(&c.leafcnt, waves * sizeof(int)));
     }
-    if(!c.lvl) SPHGPU_HIP(hipMalloc(&c.lvl, (LVL_FILL + NLEVEL) * sizeof(int)));
+    if(!c.lvl) SPHGPU_HIP(hipMalloc(&c.lvl, LVL_SIZE * sizeof(int)));
     c.num_groups = c.lvl + LVL_GROUPS;
-    // per-level counts and offsets, the number of search groups, the sort's flag
-    if(!c.lvl_host) SPHGPU_HIP(hipHostMalloc(&c.lvl_host, LVL_FILL * sizeof(int), hipHostMallocDefault));
-    for(int k = 0; k < LVL_FILL; ++k) c.lvl_host[k] = 0;
+    if(!c.lvl_host) SPHGPU_HIP(hipHostMalloc(&c.lvl_host, LVL_HOST * sizeof(int), hipHostMallocDefault));
+    for(int k = 0; k < LVL_HOST; ++k) c.lvl_host[k] = 0;
     // buckets: the cells of the deepest level that has at most twice as many
     // cells as there are particles
     int levels = 0;
@@ -628,8 +810,10 @@ int tree_alloc(Ctx &c)
     c.bucket_bits = levels * c.D;
     c.bucket_clear = false;
     c.bucket_wait = 0;
-    SPHGPU_HIP(hipMalloc(&c.bucket_cnt, ((size_t)1 << c.bucket_bits) * sizeof(int)));
-    SPHGPU_HIP(hipMalloc(&c.bucket_off, ((size_t)1 << c.bucket_bits) * sizeof(int)));
+    const int64_t nbucket = std::max<int64_t>((int64_t)1 << c.bucket_bits, 4);  // scanned by fours
+    SPHGPU_HIP(hipMalloc(&c.bucket_cnt, nbucket * sizeof(int)));
+    SPHGPU_HIP(hipMalloc(&c.bucket_off, nbucket * sizeof(int)));
+    SPHGPU_HIP(hipMalloc(&c.bucket_base, (grid_for(nbucket, BUCKET_TILE) + 1) * sizeof(int)));
     c.group_cap = c.node_cap + n / 64 + 1;
     SPHGPU_HIP(hipMalloc(&c.groups, c.group_cap * sizeof(int2)));
     size_t bytes = 0;
@@ -637,32 +821,7 @@ int tree_alloc(Ctx &c)
     SPHGPU_HIP(rocprim::radix_sort_pairs(nullptr, bytes, c.keys, c.keys_sorted, c.idx, c.perm, (unsigned)n, 0, key_bits, c.stream));
     c.sort_tmp_bytes = bytes;
     SPHGPU_HIP(hipMalloc(&c.sort_tmp, bytes));
-    bytes = 0;
-    SPHGPU_HIP(rocprim::exclusive_scan(nullptr, bytes, c.nn, c.noff, 0, (size_t)n, rocprim::plus<int>(), c.stream));
-    size_t bucket_bytes = 0;
-    SPHGPU_HIP(rocprim::exclusive_scan(nullptr, bucket_bytes, c.bucket_cnt, c.bucket_off, 0, (size_t)1 << c.bucket_bits, rocprim::plus<int>(), c.stream));
-    bytes = std::max(bytes, bucket_bytes);
-    c.scan_tmp_bytes = bytes;
-    SPHGPU_HIP(hipMalloc(&c.scan_tmp, bytes));
     return SPHGPU_OK;
-}
-
-// The upper levels that one workgroup reduces: levels 0 .. nlev-1, each with
-// at most TOP_MAXNODES nodes (level counts from the last tree build).
-static TopLevels top_levels(const Ctx &c)
-{
-    TopLevels tl{};
-    int L = 0;
-    while(L < NLEVEL && c.lvl_host[L] == 0) ++L;  // levels start at the root's
-    tl.first = L;
-    int k = 0;
-    while(k < 16 && L + k < NLEVEL && c.lvl_host[L + k] > 0 && c.lvl_host[L + k] <= TOP_MAXNODES) {
-        tl.count[k] = c.lvl_host[L + k];
-        tl.offset[k] = c.lvl_host[NLEVEL + L + k];
-        ++k;
-    }
-    tl.nlev = k;
-    return tl;
 }
 
 // Fields that a sphgpu_integrate step writes after its tree build before
@@ -693,7 +852,7 @@ template <int D> static int tree_build_d(Ctx &c)
     c.radius_ready = false;
     const bool buckets = c.bucket_wait == 0;
     if(!buckets) --c.bucket_wait;
-    const int nbucket = 1 << c.bucket_bits, shift = G * D - c.bucket_bits;
+    const int nbucket = 1 << c.bucket_bits, nscan = std::max(nbucket, 4), shift = G * D - c.bucket_bits;
     // root geometry
     if(!c.p.periodic_is_valid) {
         const int nb = std::min(grid_for(n), 1024);
@@ -701,21 +860,20 @@ template <int D> static int tree_build_d(Ctx &c)
         hipLaunchKernelGGL(bbox_final<D>, dim3(1), dim3(WAVE), 0, c.stream, c.partial, nb, c.scal);
     }
     if(buckets && !c.bucket_clear)
-        hipLaunchKernelGGL(clear_kernel, dim3(grid_for(nbucket)), dim3(BLOCK), 0, c.stream, c.bucket_cnt, nbucket);
+        hipLaunchKernelGGL(clear_kernel, dim3(grid_for(nscan)), dim3(BLOCK), 0, c.stream, c.bucket_cnt, nscan);
     c.bucket_clear = false;
     hipLaunchKernelGGL(keys_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.s, n, c.scal, G, c.keys, c.idx,
-                       buckets ? c.bucket_cnt : nullptr, shift, c.lvl + LVL_SORT);
-    size_t bytes = 0;
+                       buckets ? c.bucket_cnt : nullptr, shift, c.lvl);
+    const BucketOff off{c.bucket_off, c.bucket_base};
     if(buckets) {
-        bytes = c.scan_tmp_bytes;
-        SPHGPU_HIP(rocprim::exclusive_scan(c.scan_tmp, bytes, c.bucket_cnt, c.bucket_off, 0, (size_t)nbucket, rocprim::plus<int>(), c.stream));
-        hipLaunchKernelGGL(bucket_scatter_kernel, dim3(grid_for(std::max(n, nbucket))), dim3(BLOCK), 0, c.stream, c.keys, c.idx, n, shift, c.bucket_off,
-                           c.bucket_cnt, nbucket, c.keys_sorted, c.perm);
+        hipLaunchKernelGGL(bucket_scan_kernel, dim3(grid_for(nscan, BUCKET_TILE)), dim3(SCAN_THREADS), 0, c.stream, (int4 *)c.bucket_cnt, nscan,
+                           (int4 *)c.bucket_off, c.bucket_base, c.lvl + LVL_TICKET);
+        hipLaunchKernelGGL(bucket_scatter_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys, c.idx, n, shift, off, c.keys_sorted, c.perm);
         c.bucket_clear = true;
         // the keys in bucket order are read, the sorted ones written
         std::swap(c.keys, c.keys_sorted);
     } else {
-        bytes = c.sort_tmp_bytes;
+        size_t bytes = c.sort_tmp_bytes;
         SPHGPU_HIP(rocprim::radix_sort_pairs(c.sort_tmp, bytes, c.keys, c.keys_sorted, c.idx, c.perm, (unsigned)n, 0, (unsigned)(G * D), c.stream));
     }
     // gather the state into key order (in sphgpu_integrate, without the
@@ -743,7 +901,7 @@ template <int D> static int tree_build_d(Ctx &c)
     }
     if(buckets) {
         r.bkeys = c.keys;
-        r.off = c.bucket_off;
+        r.off = off;
         r.shift = shift;
         r.nbucket = nbucket;
         r.keys = c.keys_sorted;
@@ -762,25 +920,20 @@ template <int D> static int tree_build_d(Ctx &c)
     }
 
     const TreeShape ts{n, G, D, c.p.tree_leaf_particle_num, c.p.tree_max_level};
-    hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn,
-                       c.lvl + LVL_SORT);
-    bytes = c.scan_tmp_bytes;
-    SPHGPU_HIP(rocprim::exclusive_scan(c.scan_tmp, bytes, c.nn, c.noff, 0, (size_t)n, rocprim::plus<int>(), c.stream));
-    hipLaunchKernelGGL(emit_nodes_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, c.delta, ts, c.nn, c.noff,
-                       c.scal, c.t, c.node_cap, c.counters, c.lvl, c.groups, c.num_groups);
-    // nodes listed by level (in c.lvl_nodes), and the search groups (they
-    // need the node ranges only), so that the level counts and the number of
-    // groups come to the host together
-    const int ngrid = grid_for(c.node_cap);
+    hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n, SCAN_THREADS)), dim3(SCAN_THREADS), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn,
+                       c.noff, c.nbase, c.lvl);
+    hipLaunchKernelGGL(emit_nodes_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, c.delta, ts, c.nn, c.noff, c.nbase,
+                       c.scal, c.s, c.t, c.msum, c.node_cap, c.counters, c.groups, c.num_groups);
     // in 1D and 2D the waves are filled from runs of small cells (2D KHI
     // step 2 % faster); in 3D whole cells stay together (the Evrard step
     // was 6 % slower with runs: less compact groups keep more candidates)
-    hipLaunchKernelGGL(level_count_groups_kernel, dim3(ngrid), dim3(BLOCK), 0, c.stream, c.t, c.lvl, c.groups, c.num_groups,
-                       c.group_cap, D < 3 ? 1 : 0);
-    hipLaunchKernelGGL(level_offsets_kernel, dim3(1), dim3(WAVE), 0, c.stream, c.lvl);
-    hipLaunchKernelGGL(level_scatter_kernel, dim3(ngrid), dim3(BLOCK), 0, c.stream, c.t, c.lvl, c.lvl_nodes);
-    SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_FILL * sizeof(int), hipMemcpyDeviceToHost, c.stream));
-    SPHGPU_HIP(hipStreamSynchronize(c.stream));
+    hipLaunchKernelGGL(slice_kernel, dim3(std::min(c.span_cap, 2 * c.num_cu)), dim3(SCAN_THREADS), 0, c.stream, c.t, c.msum, c.lvl + LVL_SPAN, c.span,
+                       c.span_child, c.span_cap, c.groups, c.num_groups, c.group_cap, D < 3 ? 1 : 0);
+    SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_HOST * sizeof(int), hipMemcpyDeviceToHost, c.stream));
+    SPHGPU_HIP(hipEventRecord(c.ev_tree, c.stream));
+    hipLaunchKernelGGL(spanning_kernel, dim3(1), dim3(SCAN_THREADS), 0, c.stream, c.t, c.msum, c.lvl + LVL_SPAN, c.span, c.span_child,
+                       c.span_cap);
+    SPHGPU_HIP(hipEventSynchronize(c.ev_tree));
     if(buckets && c.lvl_host[LVL_SORT]) {
         // a bucket was too full to be sorted: build again from the state as
         // it was, with the library's sort
@@ -790,14 +943,6 @@ template <int D> static int tree_build_d(Ctx &c)
     }
     c.ngroups = c.lvl_host[LVL_GROUPS];
     if(c.ngroups < 1 || c.ngroups > c.group_cap) return set_error(SPHGPU_E_TREE, "search groups out of range");
-    const TopLevels tl = top_levels(c);
-    for(int L = NLEVEL - 1; L >= tl.first + tl.nlev; --L) {
-        const int cnt = c.lvl_host[L];
-        if(cnt <= 0) continue;
-        hipLaunchKernelGGL(moments_level_kernel<D>, dim3(grid_for(cnt)), dim3(BLOCK), 0, c.stream, c.s, c.t,
-                           c.lvl_nodes + c.lvl_host[NLEVEL + L], cnt, c.msum);
-    }
-    if(tl.nlev > 0) hipLaunchKernelGGL(moments_top_kernel<D>, dim3(1), dim3(TOP_THREADS), 0, c.stream, c.s, c.t, c.lvl_nodes, tl, c.msum);
     SPHGPU_HIP(hipGetLastError());
     c.radius_ready = radius;
     return search_alloc(c);

@@ -1,0 +1,57 @@
+"""Nodes and moments at the edges of the tree build's tiles: node counts
+around one slice of 1,024 nodes and many, cells that span several slices,
+deep chains of single-child cells, leaves larger than a search group, and
+particle counts around the scans' tiles of 1,024 and 4,096.  Geometry and
+counts equal the oracle's pointer octree; the moments are sums of at most
+n terms in another order, so within n * 2^-52 of sum |m x| / M."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from _oracle import OracleEngine
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(n, dim, kind, rng):
+    if kind == "uniform":
+        return rng.random((n, dim))
+    if kind == "clump":  # a steep profile: deep tree, many spanning cells
+        return 0.5 + rng.normal(size=(n, dim)) * rng.random((n, 1)) ** 6
+    x = rng.random((n, dim))  # pair: two close points far from the rest
+    x[0] = 0.123456
+    x[1] = x[0] + 1e-6
+    return x
+
+
+@pytest.mark.parametrize("n,dim,kind,leaf,levels", [
+    (2, 3, "uniform", 1, 20), (30, 1, "pair", 1, 40), (64, 2, "uniform", 1, 20), (65, 2, "uniform", 1, 20), (700, 3, "uniform", 1, 20),
+    (1023, 2, "uniform", 2, 20), (1024, 3, "clump", 1, 20), (1025, 1, "uniform", 1, 50), (3000, 1, "pair", 1, 60),
+    (4096, 3, "uniform", 100, 20), (4097, 2, "clump", 16, 8), (9000, 3, "clump", 1, 6), (40000, 3, "uniform", 1, 20),
+    (1048577, 3, "uniform", 2, 20),  # more cells that span slices than one pass takes
+])
+def test_nodes_and_moments(gpu, n, dim, kind, leaf, levels):
+    from sphcode_amd import GPUEngine, ics
+    p, _ = ics.rollout(4, dim=dim)
+    p.periodic_is_valid = 0
+    p.tree_leaf_particle_num = leaf
+    p.tree_max_level = levels
+    rng = np.random.default_rng(n)
+    pos = _points(n, dim, kind, rng)
+    mass = rng.random(n) + 0.5
+    f = dict(pos=pos, vel=np.zeros((n, dim)), mass=mass, dens=np.ones(n), ene=np.ones(n), pres=np.ones(n))
+    print(f"[tree] n={n} dim={dim} {kind} leaf={leaf} levels={levels}", flush=True)
+    ref, g = OracleEngine(p), GPUEngine(p)
+    for e in (ref, g):
+        e.upload(f)
+        e.make_tree()
+    a, b = ref.tree_info(), g.tree_info()
+    assert a["num_nodes"] == b["num_nodes"]
+    assert np.array_equal(a["level"], b["level"])
+    assert np.array_equal(a["count"][1:], b["count"][1:])
+    assert np.array_equal(a["edge"], b["edge"]) and np.array_equal(a["center"], b["center"])
+    eps = n * 2.0 ** -52
+    assert np.allclose(a["mass"], b["mass"], rtol=eps, atol=0)
+    assert np.max(np.abs(a["com"][1:] - b["com"][1:])) <= 2 * eps * np.abs(pos).max()
+    g.close()
