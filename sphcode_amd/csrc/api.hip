@@ -154,15 +154,11 @@ static int alloc_buffers(Ctx &c, int64_t n)
 
 // Reads the error counters; a list overflow or node-pool exhaustion since
 // the last check becomes an error status.
-// Reads the counters (and, with the scalars, the scalars as well: they
-// share one allocation, so one copy brings both) and reports the errors
-// they record.
-static int check_flags(Ctx &c, const char *stage, bool with_scalars = false)
+// Reads the counters (`sent`: the corrector has sent them and the scalars)
+// and reports the errors they record.
+static int check_flags(Ctx &c, const char *stage, bool sent = false)
 {
-    if(with_scalars)
-        SPHGPU_HIP(hipMemcpyAsync(c.scal_host, c.scal, SCAL_SPAN + NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost,
-                                  c.stream));
-    else
+    if(!sent)
         SPHGPU_HIP(hipMemcpyAsync(c.counters_host, c.counters, NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, c.stream));
     SPHGPU_HIP(hipStreamSynchronize(c.stream));
     if(c.counters_host[C_TREE_ERR] > 0)
@@ -239,11 +235,11 @@ static int stage_pre(Ctx &c, bool walk = false)
         if((rc = search_gather(c, false))) return rc;
         kmark(c, 1);
     } else {
-        // the radii h_guess * ratio, and the search's records and boxes (set
-        // by sphgpu_integrate's tree build)
+        // the radii h_guess * ratio, the search's records and boxes and its
+        // task counters (set by sphgpu_integrate's tree build)
         if(!c.radius_ready && (rc = search_guess(c))) return rc;
+        const bool ready = c.radius_ready;
         c.radius_ready = false;
-        reset_work(c, 0);  // the search's task counters
         // the gravity walk (second stream) runs beside the search, which is
         // launched first: the walk's waves take what the search leaves free,
         // so that the longer path (search, pre-interaction, force) is not
@@ -251,7 +247,7 @@ static int stage_pre(Ctx &c, bool walk = false)
         const int bpc = search_blocks(c, walk);
         if(walk) SPHGPU_HIP(hipEventRecord(c.ev_pre, c.stream));
         kmark(c, 0);
-        if((rc = search_combined(c, true, bpc))) return rc;
+        if((rc = search_combined(c, ready, bpc))) return rc;
         if(walk && (rc = launch_gravity_walk(c))) return rc;
         walk = false;
         kmark(c, 1);
@@ -265,18 +261,18 @@ static int stage_pre(Ctx &c, bool walk = false)
         if((rc = launch_gravity_walk(c))) return rc;
     }
     kmark(c, 2);
-    if((rc = pre_compute(c))) return rc;
+    const bool speculate = combined && c.speculate && !c.record;
+    if((rc = pre_compute(c, speculate))) return rc;
     kmark(c, 3);
     c.lists_symmetric = false;
     if(combined) {
         // the combined lists hold every force pair unless some h outgrew its
         // search radius (src/pre_interaction.cpp:70 truncates the gather set)
-        if(c.speculate && !c.record) {
+        if(speculate) {
             // sphgpu_integrate: the force pass starts on the combined lists
-            // at once and stage_force checks the counters once it is queued
-            // (a truncation, which needs a new search, is rare)
-            SPHGPU_HIP(hipMemcpyAsync(c.counters_spec, c.counters, NCOUNTERS * sizeof(int64_t), hipMemcpyDeviceToHost, c.stream));
-            SPHGPU_HIP(hipEventRecord(c.ev_flags, c.stream));
+            // at once and stage_force checks the counters, which its packing
+            // sends, once it is queued (a truncation, which needs a new
+            // search, is rare)
             c.flags_pending = true;
             c.lists_symmetric = true;
             return SPHGPU_OK;
@@ -424,11 +420,13 @@ int sphgpu_create(const sphgpu_params *params, void **out)
        (e = hipHostMalloc(&c->counters_spec, NCOUNTERS * sizeof(int64_t), hipHostMallocDefault)) != hipSuccess ||
        // scalars and counters in one allocation (device and pinned host)
        (e = hipMalloc(&c->scal, SCAL_SPAN + NCOUNTER_ENTRIES * sizeof(int64_t))) != hipSuccess ||
-       (e = hipMalloc(&c->work, WORK_SLOTS * NUM_XCD * WORK_STRIDE * sizeof(int))) != hipSuccess ||
+       (e = hipMalloc(&c->work, (WORK_SLOTS * NUM_XCD + 1) * WORK_STRIDE * sizeof(int))) != hipSuccess ||
        (e = hipHostMalloc(&c->scal_host, SCAL_SPAN + NCOUNTER_ENTRIES * sizeof(int64_t), hipHostMallocDefault)) != hipSuccess) {
         delete c;
         return hip_fail(e, "sphgpu_create");
     }
+    c->ticket = c->work + WORK_SLOTS * NUM_XCD * WORK_STRIDE;
+    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(BLOCK), 0, c->stream, c->ticket, (int64_t)WORK_STRIDE, 0);
     c->counters = reinterpret_cast<int64_t *>(reinterpret_cast<char *>(c->scal) + SCAL_SPAN);
     c->counters_host = reinterpret_cast<int64_t *>(reinterpret_cast<char *>(c->scal_host) + SCAL_SPAN);
 
@@ -732,6 +730,7 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     if((rc = stage_pre(c, grav))) {
         c.speculate = false;
         c.flags_pending = false;
+        c.hvs_partials = 0;
         // later work on the main stream must not overtake the walk
         if(grav) (void)hipStreamWaitEvent(c.stream, c.ev_grav, 0);
         return rc;
@@ -743,6 +742,7 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     c.after_pack = nullptr;
     c.speculate = false;
     c.flags_pending = false;
+    c.hvs_partials = 0;
     if(rc) {
         if(grav) (void)hipStreamWaitEvent(c.stream, c.ev_grav, 0);
         return rc;
@@ -751,7 +751,7 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     if(grav) SPHGPU_HIP(hipStreamWaitEvent(c.stream, c.ev_grav, 0));
     mark(6);
     // the gravity sums are added to acc by the corrector's launch
-    if((rc = step_correct(c, grav))) return rc;
+    if((rc = step_correct(c, grav, true))) return rc;
     mark(7);
     c.kernel_marks = false;
     if((rc = check_flags(c, "integrate", true))) return rc;  // synchronises the stream
@@ -768,6 +768,21 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     return SPHGPU_OK;
 }
 
+// Tree, pre-interaction and fluid force as sphgpu_integrate does them.
+static int rollout_force(Ctx &c)
+{
+    c.reorder_light = !c.first_pre;
+    int rc = stage_tree(c);
+    c.reorder_light = false;
+    if(rc) return rc;
+    c.speculate = true;
+    if(!(rc = stage_pre(c))) rc = stage_force(c);
+    c.speculate = false;
+    c.flags_pending = false;
+    c.hvs_partials = 0;
+    return rc;
+}
+
 // One full step with a fixed dt, without timers (the rollout and its
 // recomputation use exactly this sequence).
 static int rollout_step(Ctx &c, double dt)
@@ -775,9 +790,7 @@ static int rollout_step(Ctx &c, double dt)
     int rc;
     hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(1), 0, c.stream, c.scal, (int)S_DT, dt);
     if((rc = step_predict(c))) return rc;
-    if((rc = stage_tree(c))) return rc;
-    if((rc = stage_pre(c))) return rc;
-    if((rc = stage_force(c))) return rc;
+    if((rc = rollout_force(c))) return rc;
     if((rc = gravity_compute(c))) return rc;
     return step_correct(c);
 }
@@ -796,9 +809,7 @@ static int rollout_recompute(Ctx &c, int slot)
         hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(1), 0, c.stream, c.scal, (int)S_DT, c.ro.dt);
         if((rc = step_predict(c))) return rc;
     }
-    if((rc = stage_tree(c))) return rc;
-    if((rc = stage_pre(c))) return rc;
-    return stage_force(c);
+    return rollout_force(c);
 }
 
 static int rollout_supported(const Ctx &c)

@@ -233,6 +233,30 @@ struct Xfer {
 constexpr int TIMER_SETS = 32;
 constexpr int TIMER_EVENTS = 20;
 
+// A last block added to a streaming launch: reduces block minima and sends
+// words to pinned host memory, in place of a launch and a copy between two
+// kernels (about 4 us each, and as much again until the next one starts).
+struct Report {
+    int block;              // the block that does it
+    const double *partial;  // nb block minima into *min
+    int nb;
+    double *min;
+    const int64_t *src;     // count words (src null: none) to the host
+    int64_t *dst;
+    int count;
+    __device__ __forceinline__ bool run(int b) const
+    {
+        if(!dst || b != block) return false;
+        __shared__ double sh[BLOCK / WAVE];
+        if(partial) {
+            const double m = min_partials(partial, nb, sh);
+            if(threadIdx.x == 0) *min = m;
+        }
+        for(int k = threadIdx.x; k < count; k += BLOCK) dst[k] = src[k];
+        return true;
+    }
+};
+
 struct Ctx {
     sphgpu_params p{};
     int D = 3;
@@ -243,14 +267,14 @@ struct Ctx {
     hipEvent_t ev_pre = nullptr, ev_grav = nullptr;
     hipEvent_t *ev_g = nullptr;  // the gravity stream's timing events of the current timer set
     // sphgpu_integrate's check of the combined lists, read without stalling
-    // the stream: the counters are copied after the pre-interaction (event
-    // ev_flags) and read once the force pass is queued
+    // the stream: the force pass's packing also sends the counters (event
+    // ev_flags), which are read once the force pass is queued
     hipEvent_t ev_flags = nullptr;
     bool speculate = false;      // sphgpu_integrate: assume symmetric lists, check after
     bool reorder_light = false;  // sphgpu_integrate's tree build: skip fields the step rewrites
     bool radius_ready = false;   // that build set the search radii, records and boxes
     bool stats_on = false;       // count the statistics (sphgpu_enable_stats)
-    bool flags_pending = false;  // a copy behind ev_flags awaits its check
+    bool flags_pending = false;  // the counters behind ev_flags await their check
     int64_t *counters_spec = nullptr;  // pinned host copy for that check
     // called by the force pass between its record packing and its pair
     // kernel (sphgpu_integrate starts the gravity pair pass there, so that
@@ -346,6 +370,8 @@ struct Ctx {
     // which every kernel reads), and their pinned host copies laid out alike
     double *scal = nullptr;
     double *partial = nullptr;  // block partials of reductions
+    int *ticket = nullptr;      // of reductions that end in their last block (zero between launches)
+    int hvs_partials = 0;       // block minima of h / v_sig that the force pass's packing still reduces
     int64_t *counters = nullptr;       // (char *)scal + SCAL_SPAN
     int64_t *counters_host = nullptr;  // (char *)scal_host + SCAL_SPAN
     double *scal_host = nullptr;
@@ -430,7 +456,7 @@ int search_alloc(Ctx &c);        // tile slabs for c.ngroups groups (after a tre
 int search_record(Ctx &c, int *list, int *cnt, bool force);
 // pre.hip
 int pre_initial(Ctx &c);         // initial_smoothing density
-int pre_compute(Ctx &c);         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients
+int pre_compute(Ctx &c, bool defer = false);  // defer: min h / v_sig is left to the force pass (hvs_partials)         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients
 // force.hip
 int force_compute(Ctx &c);
 // gravity.hip
@@ -460,7 +486,9 @@ int group_waves(const Ctx &c, GroupPass pass);
 int step_init_fields(Ctx &c);
 int step_timestep(Ctx &c);       // dt into scal[S_DT]
 int step_predict(Ctx &c);
-int step_correct(Ctx &c, bool add_gravity = false);  // add_gravity: acc += the gravity pass's sums first
+// add_gravity: acc += the gravity pass's sums first; report: the scalars and
+// counters also to the host
+int step_correct(Ctx &c, bool add_gravity = false, bool report = false);
 int step_energy(Ctx &c, double *out);
 int reduce_min_partials(Ctx &c, int nblocks, int slot);
 // adjoint.hip: vector-Jacobian product of one force evaluation

@@ -46,8 +46,9 @@ struct ForceArgs {
 // (rounded to the pair type), and the quotients of j's own fields.
 template <int D, int TYPE, class T>
 __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, double4 *pr, ForceRec<T> *fr,
-                                                           GradRec<T> *gr)
+                                                           GradRec<T> *gr, Report rep)
 {
+    if(rep.run(blockIdx.x)) return;
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     if(i >= n) return;
     double4 p;
@@ -394,8 +395,22 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
 template <int D, int K, int TYPE, class T> static void launch_force(Ctx &c, const ForceArgs &a, const BoxDev &box)
 {
     const int use_u = TYPE == SPHGPU_DISPH || a.use_ac;
-    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
-                       c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec);
+    Report rep{};
+    int grid = grid_for(c.n);
+    if(c.hvs_partials) {
+        // sphgpu_integrate: what the pre-interaction left to reduce, and its counters to the host
+        rep.block = grid++;
+        rep.partial = c.partial;
+        rep.nb = c.hvs_partials;
+        rep.min = c.scal + S_HVS;
+        rep.src = c.counters;
+        rep.dst = c.counters_spec;
+        rep.count = NCOUNTERS;
+        c.hvs_partials = 0;
+    }
+    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
+                       c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec, rep);
+    if(rep.dst) (void)hipEventRecord(c.ev_flags, c.stream);
     if(c.after_pack) c.after_pack_rc = c.after_pack(c);
     if(group_waves(c, GROUP_PAIRS) > 1)
         hipLaunchKernelGGL((force_kernel<D, K, TYPE, T, BLOCK / WAVE>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);

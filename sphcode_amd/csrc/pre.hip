@@ -603,7 +603,7 @@ template <class T> static void pre_t(Ctx &c, const PreArgs &a, const BoxDev &box
     }
 }
 
-int pre_compute(Ctx &c)
+int pre_compute(Ctx &c, bool defer)
 {
     PreArgs a = make_args(c);
     a.gpart = c.p.gravity_is_valid ? c.gpart : nullptr;
@@ -612,7 +612,12 @@ int pre_compute(Ctx &c)
     else pre_t<double>(c, a, box);
     SPHGPU_HIP(hipGetLastError());
     c.gpart_fresh = a.gpart != nullptr;
-    return reduce_min_partials(c, group_waves(c, GROUP_PAIRS) > 1 ? c.ngroups : group_grid(c), S_HVS);
+    const int partials = group_waves(c, GROUP_PAIRS) > 1 ? c.ngroups : group_grid(c);
+    if(defer) {
+        c.hvs_partials = partials;
+        return SPHGPU_OK;
+    }
+    return reduce_min_partials(c, partials, S_HVS);
 }
 
 }  // namespace sphgpu

@@ -637,8 +637,8 @@ static SearchArgs base_args(Ctx &c)
 // test r < max(R_i, R_j) finds every gather candidate (r < R_i) and every
 // pair with r < max(h_i, h_j) for the final h, as long as no final h exceeds
 // its search radius (the caller checks the truncation counter).  With
-// `work_ready` the caller has already cleared the task counters
-// (reset_work(c, 0)); `blocks_per_cu` sets how many blocks of four
+// `work_ready` the task counters are clear already (the tree build's last
+// launch); `blocks_per_cu` sets how many blocks of four
 // persistent waves each CU gets.
 int search_combined(Ctx &c, bool work_ready, int blocks_per_cu)
 {

@@ -31,19 +31,22 @@
 namespace sphgpu {
 
 // ------------------------------------------------------------ bounding box
-template <int D> __global__ void __launch_bounds__(BLOCK) bbox_partial(State s, int n, double *partial)
+// One block per CU; the last one to finish reduces the blocks' extents.
+constexpr int BBOX_THREADS = 1024;
+template <int D> __global__ void __launch_bounds__(BBOX_THREADS) bbox_kernel(State s, int n, double *partial, int *ticket, double *scal)
 {
+#pragma clang fp contract(off)
     double lo[D], hi[D];
 #pragma unroll
     for(int k = 0; k < D; ++k) { lo[k] = 1.7976931348623157e308; hi[k] = -1.7976931348623157e308; }
-    for(int i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK)
+    for(int i = blockIdx.x * BBOX_THREADS + threadIdx.x; i < n; i += gridDim.x * BBOX_THREADS)
 #pragma unroll
         for(int k = 0; k < D; ++k) {
             const double x = s.f[F_X + k][i];
             lo[k] = x < lo[k] ? x : lo[k];
             hi[k] = x > hi[k] ? x : hi[k];
         }
-    __shared__ double sh[2 * D][BLOCK / WAVE];
+    __shared__ double sh[2 * D][BBOX_THREADS / WAVE];
 #pragma unroll
     for(int k = 0; k < D; ++k) {
         lo[k] = wave_minv(lo[k]);
@@ -58,27 +61,22 @@ template <int D> __global__ void __launch_bounds__(BLOCK) bbox_partial(State s, 
 #pragma unroll
         for(int k = 0; k < D; ++k) {
             double a = sh[k][0], b = sh[D + k][0];
-            for(int j = 1; j < BLOCK / WAVE; ++j) {
+            for(int j = 1; j < BBOX_THREADS / WAVE; ++j) {
                 a = sh[k][j] < a ? sh[k][j] : a;
                 b = sh[D + k][j] > b ? sh[D + k][j] : b;
             }
-            partial[blockIdx.x * 2 * D + k] = a;
-            partial[blockIdx.x * 2 * D + D + k] = b;
+            put(partial + blockIdx.x * 2 * D + k, a);
+            put(partial + blockIdx.x * 2 * D + D + k, b);
         }
     }
-}
-
-// Root cube: centre (max+min)/2, edge = largest extent (src/bhtree.cpp:80-94).
-// One wave: lanes stride over the block partials, then a wave min/max
-// (exact, so the result does not depend on the order).
-template <int D> __global__ void bbox_final(const double *partial, int nblocks, double *scal)
-{
-#pragma clang fp contract(off)
-    double lo[D], hi[D];
+    if(!last_block(ticket) || threadIdx.x >= WAVE) return;
+    // Root cube: centre (max+min)/2, edge = largest extent (src/bhtree.cpp:80-94).
+    // One wave: lanes stride over the block partials, then a wave min/max
+    // (exact, so the result does not depend on the order).
     for(int k = 0; k < D; ++k) { lo[k] = 1.7976931348623157e308; hi[k] = -1.7976931348623157e308; }
-    for(int b = threadIdx.x; b < nblocks; b += WAVE)
+    for(int b = threadIdx.x; b < (int)gridDim.x; b += WAVE)
         for(int k = 0; k < D; ++k) {
-            const double a = partial[b * 2 * D + k], c = partial[b * 2 * D + D + k];
+            const double a = get(partial + b * 2 * D + k), c = get(partial + b * 2 * D + D + k);
             lo[k] = a < lo[k] ? a : lo[k];
             hi[k] = c > hi[k] ? c : hi[k];
         }
@@ -138,23 +136,13 @@ __device__ __forceinline__ int block_scan(int v, int *sh, int &total)
 
 __device__ __forceinline__ void scan_publish(int sum, int *base, int *ticket, int *sh)
 {
-    __shared__ int last;
     const int nb = gridDim.x;
-    if(threadIdx.x == 0) {
-        // The sum alone passes between the blocks, through atomics of device
-        // scope: it is out before the ticket is taken (a release would also
-        // write back all that the block's L2 holds; with it the nodes' count
-        // took 84 us instead of 34 at 2M particles).
-        __hip_atomic_store(base + blockIdx.x, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
-    }
-    __syncthreads();
-    if(!last) return;
+    if(threadIdx.x == 0) put(base + blockIdx.x, sum);
+    if(!last_block(ticket)) return;
     int carry = 0;
     for(int k0 = 0; k0 < nb; k0 += SCAN_THREADS) {
         const int k = k0 + threadIdx.x;
-        const int v = k < nb ? __hip_atomic_load(base + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        const int v = k < nb ? get(base + k) : 0;
         int total;
         const int ex = block_scan(v, sh, total);
         if(k < nb) base[k] = carry + ex;
@@ -715,8 +703,10 @@ __global__ void __launch_bounds__(SCAN_THREADS) slice_kernel(TreeDev t, double4 
 // the barrier).  Two chunks of cells take 84 us at
 // 2M particles, one 10 to 18 at 393k and 1M.
 __global__ void __launch_bounds__(SCAN_THREADS) spanning_kernel(TreeDev t, double4 *msum, const int *span_cnt, const int *span,
-                                                             const int4 *span_child, int span_cap)
+                                                             const int4 *span_child, int span_cap, int *work, int nwork)
 {
+    // the task counters of the search that follows
+    for(int k = threadIdx.x; k < nwork; k += SCAN_THREADS) work[k] = 0;
     __shared__ int sh[SCAN_THREADS / WAVE];
     __shared__ int off[NLEVEL];  // of the level NLEVEL - 1 - e: deepest first
     if(*t.num_nodes <= SLICE) return;  // one slice: none spans
@@ -855,9 +845,8 @@ template <int D> static int tree_build_d(Ctx &c)
     const int nbucket = 1 << c.bucket_bits, nscan = std::max(nbucket, 4), shift = G * D - c.bucket_bits;
     // root geometry
     if(!c.p.periodic_is_valid) {
-        const int nb = std::min(grid_for(n), 1024);
-        hipLaunchKernelGGL(bbox_partial<D>, dim3(nb), dim3(BLOCK), 0, c.stream, c.s, n, c.partial);
-        hipLaunchKernelGGL(bbox_final<D>, dim3(1), dim3(WAVE), 0, c.stream, c.partial, nb, c.scal);
+        hipLaunchKernelGGL(bbox_kernel<D>, dim3(std::min(grid_for(n, BBOX_THREADS), c.num_cu)), dim3(BBOX_THREADS), 0, c.stream, c.s, n, c.partial,
+                           c.ticket, c.scal);
     }
     if(buckets && !c.bucket_clear)
         hipLaunchKernelGGL(clear_kernel, dim3(grid_for(nscan)), dim3(BLOCK), 0, c.stream, c.bucket_cnt, nscan);
@@ -932,7 +921,7 @@ template <int D> static int tree_build_d(Ctx &c)
     SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_HOST * sizeof(int), hipMemcpyDeviceToHost, c.stream));
     SPHGPU_HIP(hipEventRecord(c.ev_tree, c.stream));
     hipLaunchKernelGGL(spanning_kernel, dim3(1), dim3(SCAN_THREADS), 0, c.stream, c.t, c.msum, c.lvl + LVL_SPAN, c.span, c.span_child,
-                       c.span_cap);
+                       c.span_cap, c.work, NUM_XCD * WORK_STRIDE);
     SPHGPU_HIP(hipEventSynchronize(c.ev_tree));
     if(buckets && c.lvl_host[LVL_SORT]) {
         // a bucket was too full to be sorted: build again from the state as
