@@ -188,9 +188,9 @@ static int stage_tree(Ctx &c)
 static int launch_gravity_walk(Ctx &c)
 {
     SPHGPU_HIP(hipStreamWaitEvent(c.gstream, c.ev_pre, 0));
-    if(c.timers_on) (void)hipEventRecord(c.ev_g[0], c.gstream);
+    if(c.kernel_marks) (void)hipEventRecord(c.ev_g[0], c.gstream);
     int rc = gravity_walk(c, c.gstream);
-    if(c.timers_on) (void)hipEventRecord(c.ev_g[1], c.gstream);
+    if(c.kernel_marks) (void)hipEventRecord(c.ev_g[1], c.gstream);
     SPHGPU_HIP(hipEventRecord(c.ev_grav, c.gstream));
     return rc;
 }
@@ -202,9 +202,9 @@ static int launch_gravity_leaves(Ctx &c)
 {
     SPHGPU_HIP(hipEventRecord(c.ev_pre, c.stream));
     SPHGPU_HIP(hipStreamWaitEvent(c.gstream, c.ev_pre, 0));
-    if(c.timers_on) (void)hipEventRecord(c.ev_g[2], c.gstream);
+    if(c.kernel_marks) (void)hipEventRecord(c.ev_g[2], c.gstream);
     int rc = gravity_leaves(c, c.gstream);
-    if(c.timers_on) (void)hipEventRecord(c.ev_g[3], c.gstream);
+    if(c.kernel_marks) (void)hipEventRecord(c.ev_g[3], c.gstream);
     SPHGPU_HIP(hipEventRecord(c.ev_grav, c.gstream));
     return rc;
 }
@@ -322,6 +322,50 @@ static int stage_force(Ctx &c)
         c.have_force = true;
     }
     return SPHGPU_OK;
+}
+
+// Tree, pre-interaction, fluid force and gravity, with no synchronisation
+// after the tree build's.  The gravity sums are left in gacc and phi (the
+// caller adds them to acc).
+//
+// Gravity runs on the second stream in two parts: the tree walk (vector-ALU
+// bound; needs the tree and positions only), started once the tree is built,
+// beside the neighbour search (which waits on dependent loads) and the
+// pre-interaction; then the recorded leaves' particle pairs (need h), beside
+// the force pass.
+static int evaluate(Ctx &c)
+{
+    // the combined pre-interaction (not the first, initial-smoothing one)
+    // rewrites h, 1/h, P, grad-h and the neighbour counts, and the force and
+    // gravity passes acc, du/dt and phi, before any kernel reads them
+    c.reorder_light = !c.first_pre;
+    int rc = stage_tree(c);
+    c.reorder_light = false;
+    if(rc) return rc;
+    const bool grav = c.p.gravity_is_valid;
+    auto mark = [&](int k) {
+        if(c.kernel_marks) (void)hipEventRecord(c.ev[k], c.stream);
+    };
+    mark(3);
+    c.speculate = true;
+    rc = stage_pre(c, grav);
+    mark(4);
+    if(!rc) {
+        // the leaf pairs start once the force pass has packed its records
+        c.after_pack = grav ? launch_gravity_leaves : nullptr;
+        rc = stage_force(c);
+        c.after_pack = nullptr;
+    }
+    c.speculate = false;
+    c.flags_pending = false;
+    c.hvs_partials = 0;
+    mark(5);
+    // later work on the main stream must not overtake the gravity pass
+    if(grav) {
+        const hipError_t e = hipStreamWaitEvent(c.stream, c.ev_grav, 0);
+        if(!rc && e != hipSuccess) return hip_fail(e, "hipStreamWaitEvent");
+    }
+    return rc;
 }
 
 }  // namespace sphgpu
@@ -641,11 +685,14 @@ int sphgpu_initialize(void *ptr)
     SPHGPU_CTX(ptr);
     SPHGPU_NEED_DATA();
     int rc;
+    c.kernel_marks = false;
     if((rc = step_init_fields(c))) return rc;
-    if((rc = sphgpu_make_tree(ptr))) return rc;
-    if((rc = sphgpu_pre_interaction(ptr))) return rc;
-    if((rc = sphgpu_fluid_force(ptr))) return rc;
-    return sphgpu_gravity_force(ptr);
+    if((rc = evaluate(c))) return rc;
+    if(c.p.gravity_is_valid && (rc = gravity_combine(c, c.stream))) return rc;
+    SPHGPU_HIP(hipMemcpyAsync(c.scal_host, c.scal, NSCALARS * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+    if((rc = check_flags(c, "initialize"))) return rc;
+    c.h_per_v_sig = c.scal_host[S_HVS];
+    return SPHGPU_OK;
 }
 
 // Adds the spans of the pending timer sets (steps that have completed) to
@@ -711,46 +758,13 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     mark(1);
     if((rc = step_predict(c))) return rc;
     mark(2);
-    // the combined pre-interaction (not the first, initial-smoothing one)
-    // rewrites h, 1/h, P, grad-h and the neighbour counts, and the force and
-    // gravity passes acc, du/dt and phi, before any kernel reads them
-    c.reorder_light = !c.first_pre;
-    rc = stage_tree(c);
-    c.reorder_light = false;
-    if(rc) return rc;
-    // Gravity runs on the second stream in two parts: the tree walk (vector-
-    // ALU bound; needs the tree and positions only), started once the tree
-    // is built, beside the neighbour search (which waits on dependent loads)
-    // and the pre-interaction; then the recorded leaves' particle pairs
-    // (need h), beside the force pass.  The gravity acceleration is added to
-    // acc once both streams are done.
-    const bool grav = c.p.gravity_is_valid;
-    mark(3);
-    c.speculate = true;
-    if((rc = stage_pre(c, grav))) {
-        c.speculate = false;
-        c.flags_pending = false;
-        c.hvs_partials = 0;
-        // later work on the main stream must not overtake the walk
-        if(grav) (void)hipStreamWaitEvent(c.stream, c.ev_grav, 0);
+    if((rc = evaluate(c))) {
+        c.kernel_marks = false;
         return rc;
     }
-    mark(4);
-    // the leaf pairs start once the force pass has packed its records
-    c.after_pack = grav ? launch_gravity_leaves : nullptr;
-    rc = stage_force(c);
-    c.after_pack = nullptr;
-    c.speculate = false;
-    c.flags_pending = false;
-    c.hvs_partials = 0;
-    if(rc) {
-        if(grav) (void)hipStreamWaitEvent(c.stream, c.ev_grav, 0);
-        return rc;
-    }
-    mark(5);
-    if(grav) SPHGPU_HIP(hipStreamWaitEvent(c.stream, c.ev_grav, 0));
     mark(6);
     // the gravity sums are added to acc by the corrector's launch
+    const bool grav = c.p.gravity_is_valid;
     if((rc = step_correct(c, grav, true))) return rc;
     mark(7);
     c.kernel_marks = false;
@@ -768,21 +782,6 @@ int sphgpu_integrate(void *ptr, double fixed_dt)
     return SPHGPU_OK;
 }
 
-// Tree, pre-interaction and fluid force as sphgpu_integrate does them.
-static int rollout_force(Ctx &c)
-{
-    c.reorder_light = !c.first_pre;
-    int rc = stage_tree(c);
-    c.reorder_light = false;
-    if(rc) return rc;
-    c.speculate = true;
-    if(!(rc = stage_pre(c))) rc = stage_force(c);
-    c.speculate = false;
-    c.flags_pending = false;
-    c.hvs_partials = 0;
-    return rc;
-}
-
 // One full step with a fixed dt, without timers (the rollout and its
 // recomputation use exactly this sequence).
 static int rollout_step(Ctx &c, double dt)
@@ -790,7 +789,7 @@ static int rollout_step(Ctx &c, double dt)
     int rc;
     hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(1), 0, c.stream, c.scal, (int)S_DT, dt);
     if((rc = step_predict(c))) return rc;
-    if((rc = rollout_force(c))) return rc;
+    if((rc = evaluate(c))) return rc;
     if((rc = gravity_compute(c))) return rc;
     return step_correct(c);
 }
@@ -809,7 +808,7 @@ static int rollout_recompute(Ctx &c, int slot)
         hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(1), 0, c.stream, c.scal, (int)S_DT, c.ro.dt);
         if((rc = step_predict(c))) return rc;
     }
-    return rollout_force(c);
+    return evaluate(c);
 }
 
 static int rollout_supported(const Ctx &c)

@@ -182,12 +182,22 @@ template <int D> __global__ void __launch_bounds__(BLOCK) energy_partial_kernel(
     }
 }
 
-__global__ void energy_final_kernel(const double *partial, int nb, double *out)
+// One partial per thread, then sums over waves and over the waves' sums (one
+// wave that added the partials one after the other took 140 us).
+constexpr int ENERGY_BLOCKS = 1024;
+__global__ void __launch_bounds__(ENERGY_BLOCKS) energy_final_kernel(const double *partial, int nb, double *out)
 {
-    if(threadIdx.x >= NE) return;
+    __shared__ double sh[NE][ENERGY_BLOCKS / WAVE];
+    const int b = threadIdx.x;
+    for(int k = 0; k < NE; ++k) {
+        const double v = wave_sum(b < nb ? partial[b * NE + k] : 0.0);
+        if(wave_lane() == 0) sh[k][b / WAVE] = v;
+    }
+    __syncthreads();
+    if(b >= NE) return;
     double t = 0.0;
-    for(int b = 0; b < nb; ++b) t += partial[b * NE + threadIdx.x];
-    out[threadIdx.x] = t;
+    for(int w = 0; w < ENERGY_BLOCKS / WAVE; ++w) t += sh[b][w];
+    out[b] = t;
 }
 
 // ------------------------------------------------------------------ host
@@ -263,10 +273,10 @@ int step_correct(Ctx &c, bool add_gravity, bool report)
 
 int step_energy(Ctx &c, double *out)
 {
-    const int nb = std::min(grid_for(c.n), 1024);
+    const int nb = std::min(grid_for(c.n), ENERGY_BLOCKS);
     SPHGPU_DISPATCH_D(c, energy_partial_kernel, nb, c.s, (int)c.n, c.partial);
-    double *dev_out = c.partial + 1024 * NE;
-    hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(WAVE), 0, c.stream, c.partial, nb, dev_out);
+    double *dev_out = c.partial + ENERGY_BLOCKS * NE;
+    hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(ENERGY_BLOCKS), 0, c.stream, c.partial, nb, dev_out);
     SPHGPU_HIP(hipGetLastError());
     double host[NE];
     SPHGPU_HIP(hipMemcpyAsync(host, dev_out, sizeof(host), hipMemcpyDeviceToHost, c.stream));
