@@ -226,6 +226,9 @@ static int stage_pre(Ctx &c, bool walk = false)
 {
     int rc;
     const bool combined = !c.first_pre;
+    const bool ready = c.radius_ready;  // by the tree build of sphgpu_integrate and its like
+    const bool packed = c.pre_packed;
+    c.radius_ready = c.pre_packed = false;
     if(c.first_pre) {
         // PreInteraction::initial_smoothing (src/pre_interaction.cpp:41-44, 171-215)
         if((rc = search_gather(c, true))) return rc;
@@ -237,9 +240,7 @@ static int stage_pre(Ctx &c, bool walk = false)
     } else {
         // the radii h_guess * ratio, the search's records and boxes and its
         // task counters (set by sphgpu_integrate's tree build)
-        if(!c.radius_ready && (rc = search_guess(c))) return rc;
-        const bool ready = c.radius_ready;
-        c.radius_ready = false;
+        if(!ready && (rc = search_guess(c))) return rc;
         // the gravity walk (second stream) runs beside the search, which is
         // launched first: the walk's waves take what the search leaves free,
         // so that the longer path (search, pre-interaction, force) is not
@@ -262,7 +263,7 @@ static int stage_pre(Ctx &c, bool walk = false)
     }
     kmark(c, 2);
     const bool speculate = combined && c.speculate && !c.record;
-    if((rc = pre_compute(c, speculate))) return rc;
+    if((rc = pre_compute(c, speculate, packed))) return rc;
     kmark(c, 3);
     c.lists_symmetric = false;
     if(combined) {

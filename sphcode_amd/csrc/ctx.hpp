@@ -137,6 +137,21 @@ template <> struct __align__(16) PreRec<double> {
 };
 static_assert(sizeof(PreRec<float>) == 48 && sizeof(PreRec<double>) == 80, "PreRec size");
 
+// Particle j's record, and its position and mass for the Newton sweeps.
+template <int D, class T> __device__ __forceinline__ PreRec<T> make_pre_rec(const State &s, int j, double4 &pm)
+{
+    PreRec<T> r{};
+#pragma unroll
+    for(int k = 0; k < 3; ++k) r.x[k] = k < D ? s.f[F_X + k][j] : 0.0;
+    pm = make_double4(r.x[0], r.x[1], r.x[2], s.f[F_MASS][j]);
+    r.m = (T)s.f[F_MASS][j];
+    r.u = (T)s.f[F_ENE][j];
+    r.c = (T)s.f[F_SOUND][j];
+#pragma unroll
+    for(int k = 0; k < D; ++k) r.v[k] = (T)s.f[F_V + k][j];
+    return r;
+}
+
 // Register budgets, as the minimum number of waves per SIMD the compiler
 // must fit (amdgpu_waves_per_eu), for kernels that wait on dependent
 // gathers and where more resident waves beat a few spilled registers
@@ -272,7 +287,8 @@ struct Ctx {
     hipEvent_t ev_flags = nullptr;
     bool speculate = false;      // sphgpu_integrate: assume symmetric lists, check after
     bool reorder_light = false;  // sphgpu_integrate's tree build: skip fields the step rewrites
-    bool radius_ready = false;   // that build set the search radii, records and boxes
+    bool radius_ready = false;   // that build set the search's radii, records and boxes
+    bool pre_packed = false;     // and the pre-interaction's records
     bool stats_on = false;       // count the statistics (sphgpu_enable_stats)
     bool flags_pending = false;  // the counters behind ev_flags await their check
     int64_t *counters_spec = nullptr;  // pinned host copy for that check
@@ -456,7 +472,9 @@ int search_alloc(Ctx &c);        // tile slabs for c.ngroups groups (after a tre
 int search_record(Ctx &c, int *list, int *cnt, bool force);
 // pre.hip
 int pre_initial(Ctx &c);         // initial_smoothing density
-int pre_compute(Ctx &c, bool defer = false);  // defer: min h / v_sig is left to the force pass (hvs_partials)         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients
+// defer: min h / v_sig is left to the force pass (hvs_partials); packed: the
+// tree build has written the records
+int pre_compute(Ctx &c, bool defer, bool packed);         // Newton h, density, pressure, grad-h, AV switches / MUSCL gradients
 // force.hip
 int force_compute(Ctx &c);
 // gravity.hip

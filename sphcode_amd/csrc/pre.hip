@@ -51,6 +51,7 @@ struct PreArgs {
     int64_t *counters;
     int stats;            // add to the statistics counters (errors are always counted)
     double *partial;      // per-block min of h / v_sig
+    bool packed;          // the tree build's reorder has written the records
     const void *prec;     // PreRec<T> per particle
     const double4 *pm;    // FP64 position and mass per particle (Newton sweeps)
     void *gpart;          // GravPart<T> per particle, written with h (gravity on)
@@ -80,16 +81,7 @@ template <int D, class T> __global__ void __launch_bounds__(BLOCK) pack_pre_kern
 {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     if(i >= n) return;
-    PreRec<T> r{};
-#pragma unroll
-    for(int k = 0; k < 3; ++k) r.x[k] = k < D ? s.f[F_X + k][i] : 0.0;
-    pm[i] = make_double4(r.x[0], r.x[1], r.x[2], s.f[F_MASS][i]);
-    r.m = (T)s.f[F_MASS][i];
-    r.u = (T)s.f[F_ENE][i];
-    r.c = (T)s.f[F_SOUND][i];
-#pragma unroll
-    for(int k = 0; k < D; ++k) r.v[k] = (T)s.f[F_V + k][i];
-    out[i] = r;
+    out[i] = make_pre_rec<D, T>(s, i, pm[i]);
 }
 
 template <int D, class T> struct CurlAcc {
@@ -576,8 +568,9 @@ int pre_initial(Ctx &c)
 
 template <int D, int K, int TYPE, class T> static void launch_pre(Ctx &c, const PreArgs &a, const BoxDev &box)
 {
-    hipLaunchKernelGGL((pack_pre_kernel<D, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n,
-                       (PreRec<T> *)c.pair_rec, c.posrec);
+    if(!a.packed)
+        hipLaunchKernelGGL((pack_pre_kernel<D, T>), dim3(grid_for(c.n)), dim3(BLOCK), 0, c.stream, c.s, (int)c.n,
+                           (PreRec<T> *)c.pair_rec, c.posrec);
     if(group_waves(c, GROUP_PAIRS) > 1)
         hipLaunchKernelGGL((pre_kernel<D, K, TYPE, T, PSW>), dim3(c.ngroups), dim3(BLOCK), 0, c.stream, c.s, box, (int)c.n, a);
     else
@@ -603,9 +596,10 @@ template <class T> static void pre_t(Ctx &c, const PreArgs &a, const BoxDev &box
     }
 }
 
-int pre_compute(Ctx &c, bool defer)
+int pre_compute(Ctx &c, bool defer, bool packed)
 {
     PreArgs a = make_args(c);
+    a.packed = packed;
     a.gpart = c.p.gravity_is_valid ? c.gpart : nullptr;
     const BoxDev box = make_box(c);
     if(c.p.precision == SPHGPU_MIXED) pre_t<float>(c, a, box);
