@@ -30,6 +30,7 @@ def _points(n, dim, kind, rng):
     (1023, 2, "uniform", 2, 20), (1024, 3, "clump", 1, 20), (1025, 1, "uniform", 1, 50), (3000, 1, "pair", 1, 60),
     (4096, 3, "uniform", 100, 20), (4097, 2, "clump", 16, 8), (9000, 3, "clump", 1, 6), (40000, 3, "uniform", 1, 20),
     (1048577, 3, "uniform", 2, 20),  # more cells that span slices than one pass takes
+    (2097153, 3, "uniform", 4, 20), (2097153, 2, "uniform", 2, 25),  # level after level
 ])
 def test_nodes_and_moments(gpu, n, dim, kind, leaf, levels):
     from sphcode_amd import GPUEngine, ics
