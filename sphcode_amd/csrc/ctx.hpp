@@ -87,8 +87,8 @@ template <> struct __align__(16) GravPart<double> {
 };
 
 // Neighbour search: bounding box of CHUNK key-consecutive particles (or of
-// 64 boxes of the level below), rounded outwards to FP32, with the largest
-// candidate radius in it.
+// 64 boxes of the level below) from the root cube's centre, rounded outwards
+// to FP32, with the largest candidate radius in it.
 constexpr int CHUNK = 32;
 struct __align__(32) ChunkBox {
     float lo[3], hi[3], r, pad;

@@ -1,8 +1,7 @@
 // FluidForce on the device, one wave per search group of at most 64
 // particles, one lane per particle, over the group's candidate tiles: the
 // tile's 64 neighbour records are staged once in LDS, and each lane then
-// takes the members of its symmetric candidate set (front | back hit
-// masks) among them, keeping the pairs with r < max(h_i, h_j), r != 0:
+// takes the members of its symmetric candidate set (its hits) among them, keeping the pairs with r < max(h_i, h_j), r != 0:
 //   SSPH  src/fluid_force.cpp:26-86, viscosity :89-106, conductivity :108-116
 //   DISPH src/disph/d_fluid_force.cpp:26-86 (pressure-energy form)
 //   GSPH  src/gsph/g_fluid_force.cpp:39-166, limiter :27-36, HLL :168-199

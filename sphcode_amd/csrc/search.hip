@@ -60,6 +60,7 @@ struct SearchArgs {
     int n;
     const double4 *srec;  // position and squared candidate radius per particle
     const double *own;    // M_SYMMETRIC: h per particle (otherwise srec's radius)
+    const double *origin; // of the boxes: the root cube's centre
     const ChunkBox *lev[3];
     int cnt[3];           // boxes per level
     const int2 *groups;
@@ -90,16 +91,23 @@ __device__ __forceinline__ double min_image1(const BoxDev &b, int k, double d)
     return r;
 }
 
-// Does box b come within reach of the group's box (centre gc, half extents
-// ge, largest radius squared hmax2)?
+// Axis k of the boxes' origin (zero where a particle has gone to infinity).
+__device__ __forceinline__ double box_origin(const double *origin, int k)
+{
+    const double o = origin[k];
+    return fabs(o) < __builtin_huge_val() ? o : 0.0;
+}
+
+// Does box b come within reach of the group's box (centre go from the boxes'
+// origin, half extents ge, largest radius squared hmax2)?
 template <int D, bool IJ>
-__device__ __forceinline__ bool box_near(const BoxDev &box, const ChunkBox &b, const double gc[D], const double ge[D], double hmax2)
+__device__ __forceinline__ bool box_near(const BoxDev &box, const ChunkBox &b, const double go[D], const double ge[D], double hmax2)
 {
     double d2 = 0.0;
 #pragma unroll
     for(int k = 0; k < D; ++k) {
         const double c = 0.5 * ((double)b.lo[k] + (double)b.hi[k]), e = 0.5 * ((double)b.hi[k] - (double)b.lo[k]);
-        const double ex = fabs(min_image1(box, k, gc[k] - c)) - (ge[k] + e);
+        const double ex = fabs(min_image1(box, k, go[k] - c)) - (ge[k] + e);
         d2 += ex > 0.0 ? ex * ex : 0.0;
     }
     double H2 = hmax2;
@@ -148,8 +156,9 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     const bool valid = lane < cnt;
     const size_t gbase = (size_t)grp * (size_t)a.wcap;
 
-    // group box: centre, half extent, largest radius squared (wave-uniform)
-    double gc[D], ge[D], hmax2;
+    // group box: centre (go: from the boxes' origin), half extent, largest
+    // radius squared (wave-uniform)
+    double gc[D], go[D], ge[D], hmax2;
     {
         const int i = gr.x + (valid ? lane : 0);
         const double4 me = a.srec[i];
@@ -159,6 +168,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
             const double lo = wave_minv(x[k]);
             const double hi = wave_maxv(x[k]);
             gc[k] = uniform_d(0.5 * (lo + hi));
+            go[k] = uniform_d(gc[k] - box_origin(a.origin, k));
             ge[k] = uniform_d(0.5 * (hi - lo) * (1.0 + 1e-12) + 1e-300);
         }
         double h2 = me.w;
@@ -223,7 +233,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     auto window = [&](int level, int base) -> uint64_t {
         const int v = base + lane;
         bool hit = false;
-        if(v < a.cnt[level]) hit = box_near<D, IJ>(box, a.lev[level][v], gc, ge, hmax2);
+        if(v < a.cnt[level]) hit = box_near<D, IJ>(box, a.lev[level][v], go, ge, hmax2);
         visited += min(WAVE, a.cnt[level] - base);
         return ballot(hit);
     };
@@ -420,8 +430,8 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 // ------------------------------------------------------------------- boxes
 // Search records (position, squared candidate radius) and the boxes of the
 // first two levels: a workgroup takes the 2,048 particles of one
-// second-level box.  rad may be null (gather search: its boxes need none;
-// the records' radius is then `own2`'s, the group's own radii).
+// second-level box.  The boxes are FP32 and count from the root cube's centre
+// (origin), so that they are as tight for a domain far from zero.
 constexpr int BOX_THREADS = 1024;
 constexpr int SUPER = CHUNK * WAVE;  // particles per second-level box
 
@@ -466,7 +476,8 @@ template <int W> __device__ __forceinline__ ChunkBox box_lanes(ChunkBox b)
 }
 
 template <int D>
-__global__ void __launch_bounds__(BOX_THREADS) chunk_boxes_kernel(State s, const double *rad, int n, double4 *srec, ChunkBox *l1, ChunkBox *l2)
+__global__ void __launch_bounds__(BOX_THREADS) chunk_boxes_kernel(State s, const double *rad, const double *origin, int n, double4 *srec,
+                                                                   ChunkBox *l1, ChunkBox *l2)
 {
     __shared__ ChunkBox sh[WAVE];
     for(int r = 0; r < SUPER / BOX_THREADS; ++r) {
@@ -484,11 +495,12 @@ __global__ void __launch_bounds__(BOX_THREADS) chunk_boxes_kernel(State s, const
             const double x[3] = {q.x, q.y, q.z};
 #pragma unroll
             for(int k = 0; k < 3; ++k) {
-                // FP32, rounded outwards (a NaN coordinate stays out of the box)
-                const float f = (float)x[k], e = fabsf(f) * 1.2e-7f + 1e-37f;
+                // FP32, rounded outwards (a NaN coordinate stays out of the
+                // box; one past FP32's range makes it boundless)
+                const float f = k < D ? (float)(x[k] - box_origin(origin, k)) : 0.0f, e = fabsf(f) * 1.2e-7f + 1e-37f;
                 if(f == f) {
-                    b.lo[k] = f - e;
-                    b.hi[k] = f + e;
+                    b.lo[k] = e < __builtin_huge_valf() ? f - e : -__builtin_huge_valf();
+                    b.hi[k] = e < __builtin_huge_valf() ? f + e : __builtin_huge_valf();
                 }
             }
             const float f = (float)h;
@@ -523,9 +535,9 @@ int search_boxes(Ctx &c, const double *rad)
     const int n = (int)c.n, n2 = grid_for(n, SUPER), n3 = grid_for(n2, WAVE);
     ChunkBox *l1 = c.boxes, *l2 = l1 + grid_for(c.cap_n, CHUNK), *l3 = l2 + grid_for(c.cap_n, SUPER);
     switch(c.D) {
-    case 1: hipLaunchKernelGGL(chunk_boxes_kernel<1>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
-    case 2: hipLaunchKernelGGL(chunk_boxes_kernel<2>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
-    default: hipLaunchKernelGGL(chunk_boxes_kernel<3>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, n, c.srec, l1, l2); break;
+    case 1: hipLaunchKernelGGL(chunk_boxes_kernel<1>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, c.scal + S_ROOT_CX, n, c.srec, l1, l2); break;
+    case 2: hipLaunchKernelGGL(chunk_boxes_kernel<2>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, c.scal + S_ROOT_CX, n, c.srec, l1, l2); break;
+    default: hipLaunchKernelGGL(chunk_boxes_kernel<3>, dim3(n2), dim3(BOX_THREADS), 0, c.stream, c.s, rad, c.scal + S_ROOT_CX, n, c.srec, l1, l2); break;
     }
     // with one third-level box the search starts at the second
     if(n3 > 1) hipLaunchKernelGGL(upper_boxes_kernel, dim3(grid_for(n3, SW)), dim3(BLOCK), 0, c.stream, l2, n2, l3);
@@ -614,6 +626,7 @@ static SearchArgs base_args(Ctx &c)
     a.n = (int)c.n;
     a.srec = c.srec;
     a.own = c.s.f[F_SML];
+    a.origin = c.scal + S_ROOT_CX;
     a.lev[0] = c.boxes;
     a.lev[1] = c.boxes + grid_for(c.cap_n, CHUNK);
     a.lev[2] = a.lev[1] + grid_for(c.cap_n, SUPER);

@@ -64,3 +64,30 @@ def test_search_sets_at_edges(gpu, n, dim, periodic, neighbours, leaf):
             for x, y in zip(ref.neighbor_sets(0), g.neighbor_sets(0)):
                 assert np.array_equal(x, y)
     g.close()
+
+
+@pytest.mark.parametrize("dim,periodic", [(1, False), (2, False), (3, False), (3, True)])
+def test_boxes_far_from_zero(gpu, dim, periodic):
+    """A domain far from zero: the FP32 boxes are as tight as near zero (the
+    same number is tested, within the root cube's rounding) and the
+    neighbour counts are the same.  Positions are multiples of 2^-26, so that
+    the shift by 2^26 is exact."""
+    from sphcode_amd import GPUEngine
+    n, shift = 9000, 2.0 ** 26
+    p, f = _state(n, dim, periodic, 16 if dim > 1 else 6, 8, seed=dim)
+    f["pos"] = np.round(f["pos"] * 2.0 ** 26) / 2.0 ** 26
+    got = []
+    for off in (0.0, shift):
+        if periodic:
+            for k in range(dim):
+                p.range_min[k], p.range_max[k] = off, off + 1.0
+        g = GPUEngine(p, stats=True)
+        g.upload(dict(f, pos=f["pos"] + off))
+        print(f"[search] dim={dim} periodic={periodic} shift={off}", flush=True)
+        g.initialize()
+        nb = g.download()["neighbor"]
+        g.integrate()
+        got.append((g.stats()["search_nodes"], nb))
+        g.close()
+    assert np.array_equal(got[0][1], got[1][1])
+    assert got[1][0] <= 1.05 * got[0][0]
