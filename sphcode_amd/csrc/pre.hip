@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             // above its h: a wave whose iterates stay below takes the later
             // sweeps over those
             const double lim = NARROW * hn;
-            lim2 = lim * lim;
+            lim2 = lim * lim * (1.0 + 1e-6);  // r < (T)h is tested on rounded values
             auto narrow_holds = [&](double h_now) -> bool { return ballot(valid && !(h_now <= lim)) == 0; };
             bool done = !valid;
             int it = 0;
