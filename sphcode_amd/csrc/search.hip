@@ -157,23 +157,31 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     const size_t gbase = (size_t)grp * (size_t)a.wcap;
 
     // group box: centre (go: from the boxes' origin), half extent, largest
-    // radius squared (wave-uniform)
+    // radius squared (wave-uniform).  A particle with a NaN coordinate is at
+    // no distance from any other: it hits nothing and stays out of the box,
+    // which would otherwise be near everything or leave out the particles
+    // whose extremes met it in the reduction.
     double gc[D], go[D], ge[D], hmax2;
+    uint64_t live;
     {
         const int i = gr.x + (valid ? lane : 0);
         const double4 me = a.srec[i];
         const double x[3] = {me.x, me.y, me.z};
+        bool in = true;
+#pragma unroll
+        for(int k = 0; k < D; ++k) in = in && x[k] == x[k];
+        live = ballot(in);
 #pragma unroll
         for(int k = 0; k < D; ++k) {
-            const double lo = wave_minv(x[k]);
-            const double hi = wave_maxv(x[k]);
+            const double lo = wave_minv(in ? x[k] : 1.7976931348623157e308);
+            const double hi = wave_maxv(in ? x[k] : -1.7976931348623157e308);
             gc[k] = uniform_d(0.5 * (lo + hi));
             go[k] = uniform_d(gc[k] - box_origin(a.origin, k));
             ge[k] = uniform_d(0.5 * (hi - lo) * (1.0 + 1e-12) + 1e-300);
         }
         double h2 = me.w;
         if constexpr(MODE == M_SYMMETRIC) h2 = a.own[i] * a.own[i];
-        hmax2 = uniform_d(wave_maxv(h2));
+        hmax2 = uniform_d(wave_maxv(in && h2 == h2 ? h2 : 0.0));
     }
 
     int nkept = 0;               // staged candidates (may pass wcap: overflow)
@@ -204,14 +212,16 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
                 // implies this)
                 const double x[3] = {c_q.x, c_q.y, c_q.z};
                 double d2b = 0.0;
+                keep = true;
 #pragma unroll
                 for(int k = 0; k < D; ++k) {
                     const double ex = fabs(min_image1(box, k, x[k] - gc[k])) - ge[k];
                     d2b += ex > 0.0 ? ex * ex : 0.0;
+                    keep = keep && x[k] == x[k];
                 }
                 double H2 = hmax2;
                 if constexpr(IJ) H2 = c_q.w > H2 ? c_q.w : H2;
-                keep = d2b <= H2 * (1.0 + 1e-9);
+                keep = keep && d2b <= H2 * (1.0 + 1e-9);
                 if constexpr(IJ) reach2 = keep && H2 > reach2 ? H2 : reach2;
             }
             const uint64_t kept = ballot(keep);
@@ -237,7 +247,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
         visited += min(WAVE, a.cnt[level] - base);
         return ballot(hit);
     };
-    for(int b3 = 0; b3 < a.cnt[2]; b3 += WAVE) {
+    for(int b3 = 0; b3 < (live ? a.cnt[2] : 0); b3 += WAVE) {
         // a level with one box is not tested
         uint64_t m3 = a.cnt[2] > 1 ? window(2, b3) : 1ull;
         while(m3) {
@@ -493,18 +503,22 @@ __global__ void __launch_bounds__(BOX_THREADS) chunk_boxes_kernel(State s, const
             q.w = h * h;
             srec[i] = q;
             const double x[3] = {q.x, q.y, q.z};
+            bool in = true;
 #pragma unroll
-            for(int k = 0; k < 3; ++k) {
-                // FP32, rounded outwards (a NaN coordinate stays out of the
-                // box; one past FP32's range makes it boundless)
-                const float f = k < D ? (float)(x[k] - box_origin(origin, k)) : 0.0f, e = fabsf(f) * 1.2e-7f + 1e-37f;
-                if(f == f) {
+            for(int k = 0; k < D; ++k) in = in && x[k] == x[k];
+            // FP32, rounded outwards (a particle with a NaN coordinate stays
+            // out of the box; a coordinate past FP32's range makes it
+            // boundless)
+            if(in) {
+#pragma unroll
+                for(int k = 0; k < 3; ++k) {
+                    const float f = k < D ? (float)(x[k] - box_origin(origin, k)) : 0.0f, e = fabsf(f) * 1.2e-7f + 1e-37f;
                     b.lo[k] = e < __builtin_huge_valf() ? f - e : -__builtin_huge_valf();
                     b.hi[k] = e < __builtin_huge_valf() ? f + e : __builtin_huge_valf();
                 }
+                const float f = (float)h;
+                b.r = f == f ? f + f * 1.2e-7f + 1e-37f : 0.0f;
             }
-            const float f = (float)h;
-            b.r = f == f ? f + f * 1.2e-7f + 1e-37f : 0.0f;
         }
         b = box_lanes<CHUNK>(b);
         if((slot & (CHUNK - 1)) == 0) sh[slot / CHUNK] = b;

@@ -42,8 +42,14 @@ template <int D> struct GroupImage {
     {
         pairs.on = b.on && (gnc & GNC_WRAP);
         move = b.on && !(gnc & GNC_WRAP);
+        // the first particle with no NaN coordinate (those that have one hit nothing)
+        bool in = true;
 #pragma unroll
-        for(int k = 0; k < D; ++k) x0[k] = uniform_d(xi[k]);
+        for(int k = 0; k < D; ++k) in = in && xi[k] == xi[k];
+        const uint64_t live = ballot(in);
+        const int first = live ? (int)__builtin_ctzll(live) : 0;
+#pragma unroll
+        for(int k = 0; k < D; ++k) x0[k] = uniform_d(__shfl(xi[k], first, WAVE));
     }
     // axis k of a staged candidate's position
     __device__ __forceinline__ double at(int k, double x) const { return move ? near_image(box, k, x0[k], x) : x; }
