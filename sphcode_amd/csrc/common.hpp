@@ -340,14 +340,16 @@ template <int D> __device__ __forceinline__ void min_image(const BoxDev &b, doub
     }
 }
 
-// Axis k of the image of x that is nearest to c: x, x - L or x + L.
-__device__ __forceinline__ double near_image(const BoxDev &b, int k, double c, double x)
+// Which image of x is nearest to c on axis k: c - x + (1, 0 or -1) L, as
+// min_image chooses it.
+__device__ __forceinline__ int near_image(const BoxDev &b, int k, double c, double x)
 {
+#pragma clang fp contract(off)
     const double d = c - x;
     const double a1 = fabs(d), a2 = fabs(d + b.len[k]), a3 = fabs(d - b.len[k]);
-    double r = x + b.len[k];
-    if(a2 <= a3 && a2 <= a1) r = x - b.len[k];
-    if(a1 <= a2 && a1 <= a3) r = x;
+    int r = -1;
+    if(a2 <= a3 && a2 <= a1) r = 1;
+    if(a1 <= a2 && a1 <= a3) r = 0;
     return r;
 }
 

@@ -94,8 +94,10 @@ struct __align__(32) ChunkBox {
     float lo[3], hi[3], r, pad;
 };
 static_assert(sizeof(ChunkBox) == 32, "ChunkBox is one 32-byte record");
-// flag in Ctx::tile_nc: the group's pairs take their own minimum images
-constexpr int GNC_WRAP = 1 << 30;
+// flags in Ctx::tile_nc, beside the count: the group's pairs take their own
+// minimum images (GNC_WRAP), or all of them that of their candidate, which is
+// a shifted one for some of them on this axis (GNC_SHIFT_AXIS << axis)
+constexpr int GNC_WRAP = 1 << 30, GNC_SHIFT_AXIS = 1 << 27, GNC_SHIFT = 7 * GNC_SHIFT_AXIS, GNC_COUNT = GNC_SHIFT_AXIS - 1;
 
 // Neighbour records of the force pass, packed once per pass so that a pair
 // reads one FP64 (x, y, z, h) record for the cut and one record of the pair
@@ -353,8 +355,8 @@ struct Ctx {
     double *leaf_rad = nullptr;
 
     // candidate tiles of the last neighbour search, per search group g
-    // (groups[g], at most 64 particles): tile_nc[g] candidates (with the flag
-    // GNC_WRAP), stored in the group's slab of tile_wcap slots starting at
+    // (groups[g], at most 64 particles): tile_nc[g] candidates (with the GNC_
+    // flags), stored in the group's slab of tile_wcap slots starting at
     // g * tile_wcap.  With T = ceil(nc / 64) tiles, staging-order candidate c
     // (key order) is lane k = c / T of tile t = c % T: tile t's 64 candidate
     // indices sit at slab + 64 t (-1 past the end), and lane l of the group
@@ -365,6 +367,7 @@ struct Ctx {
     int *tile_cand = nullptr;
     uint64_t *tile_ma = nullptr;
     uint64_t *tile_mn = nullptr;   // the pre-interaction's narrowed hits (alike)
+    int8_t *tile_img = nullptr;    // images of the candidates (GroupImage), alike
     int *tile_nc = nullptr;
     int tile_wcap = 0;             // slots per group (multiple of 64)
     int64_t tile_groups_cap = 0;   // groups the slabs are allocated for

@@ -26,6 +26,7 @@ struct ForceArgs {
     int ngroups;
     const int *cand;        // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;     // hit masks per (tile, lane): every symmetric pair
+    const int8_t *img;      // images (Ctx::tile_img)
     const int *gnc;
     int wcap;
     double gamma;
@@ -141,6 +142,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
     __shared__ double2 l_xy[SW][WAVE], l_zh[SW][WAVE];
     __shared__ ForceRec<T> l_f[SW][WAVE];
     __shared__ GradRec<T> l_g[GS ? SW : 1][GS ? WAVE : 1];
+    __shared__ int8_t l_s[FP64 ? SW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -186,8 +188,8 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         const ForceRec<T> *frec = (const ForceRec<T> *)a.frec;
         const size_t gbase = (size_t)grp * a.wcap;
         const int gnc = uniform(a.gnc[grp]);
-        const int nc = gnc & ~GNC_WRAP;
-        const GroupImage<D> img(box, gnc, xi);
+        const int nc = gnc & GNC_COUNT;
+        const GroupImage<D, T> img(box, gnc);
         const int ntile = (nc + WAVE - 1) / WAVE;
         auto stage = [&](int tt) -> uint64_t {
             const size_t o = gbase + (size_t)tt * WAVE;
@@ -195,9 +197,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) {
                 double4 q = a.posrec[jl];
-                q.x = img.at(0, q.x);
-                if constexpr(D > 1) q.y = img.at(1, q.y);
-                if constexpr(D > 2) q.z = img.at(2, q.z);
+                const int c = img.code(a.img, o + lane);
+                q.x = img.at(0, q.x, c);
+                if constexpr(D > 1) q.y = img.at(1, q.y, c);
+                if constexpr(D > 2) q.z = img.at(2, q.z, c);
+                if constexpr(FP64) l_s[w][lane] = (int8_t)c;
                 l_xy[w][lane] = make_double2(q.x, q.y);
                 l_zh[w][lane] = make_double2(q.z, q.w);
                 l_f[w][lane] = frec[jl];
@@ -214,7 +218,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             if constexpr(D > 1) xj[1] = xy.y;
             if constexpr(D > 2) xj[2] = zh.x;
             hmax = hi_d < zh.y ? zh.y : hi_d;
-            return sep2<D>(img.pairs, xi, xj, d);
+            return img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
         };
         auto pair = [&](int kc) {
             double d[D], hmax;
@@ -443,6 +447,7 @@ int force_compute(Ctx &c)
     a.ngroups = c.ngroups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
+    a.img = c.tile_img;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

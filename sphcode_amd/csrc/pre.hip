@@ -37,6 +37,7 @@ struct PreArgs {
     const int *cand;      // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;   // hit masks
     uint64_t *mn;         // narrowed masks (Ctx::tile_mn)
+    const int8_t *img;    // images (Ctx::tile_img)
     const int *gnc;
     int wcap;
     double gamma;
@@ -116,6 +117,8 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
 {
     using Kern = typename KernelOf<D, K, T>::type;
     __shared__ PosMass<T> l_r[PSW][WAVE];
+    constexpr bool FP64 = sizeof(T) == 8;
+    __shared__ int8_t l_s[FP64 ? PSW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -130,18 +133,20 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
     const int gnc = uniform(a.gnc[grp]);
-    const GroupImage<D> img(box, gnc, xi);
+    const GroupImage<D, T> img(box, gnc);
     const T h = (T)s.f[F_SML][ii];
     const Kern ker(h);
     Acc<T> rho;
     const size_t gbase = (size_t)grp * a.wcap;
-    const int ntile = ((gnc & ~GNC_WRAP) + WAVE - 1) / WAVE;
+    const int ntile = ((gnc & GNC_COUNT) + WAVE - 1) / WAVE;
     auto stage = [&](int tt) -> uint64_t {
         const size_t o = gbase + (size_t)tt * WAVE;
         const int jl = stream_ld(a.cand + o + lane);
         if(jl >= 0) {
+            const int c = img.code(a.img, o + lane);
 #pragma unroll
-            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl]);
+            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl], c);
+            if constexpr(FP64) l_s[w][lane] = (int8_t)c;
             l_r[w][lane].m = (T)s.f[F_MASS][jl];
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
@@ -150,7 +155,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         double xj[D], d[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = l_r[w][kc].x[k];
-        const T r = gather_r<T>(sep2<D>(img.pairs, xi, xj, d));
+        const T r = gather_r<T>(img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d));
         if(r < h) rho.add(l_r[w][kc].m * ker.w(ker.q_of(r)));
     };
     tile_sweep<NW>(part, ntile, stage, pair);
@@ -166,6 +171,8 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     using Kern = typename KernelOf<D, K, T>::type;
     constexpr bool NUMBER = TYPE == SPHGPU_DISPH;
     __shared__ PreRec<T> l_r[PSW][WAVE];
+    constexpr bool FP64 = sizeof(T) == 8;
+    __shared__ int8_t l_s[FP64 ? PSW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int part = w % NW;
@@ -185,7 +192,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     const int ii = valid ? i : gr.x;
     const size_t gbase = (size_t)(have ? grp : 0) * a.wcap;
     const int gnc = have ? uniform(a.gnc[grp]) : 0;
-    const int ntile = ((gnc & ~GNC_WRAP) + WAVE - 1) / WAVE;
+    const int ntile = ((gnc & GNC_COUNT) + WAVE - 1) / WAVE;
     const PreRec<T> *prec = (const PreRec<T> *)a.prec;
     double hvs = 1.7976931348623157e308;
     int64_t iters = 0, fails = 0, trunc = 0, pairs = 0;
@@ -193,7 +200,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         double xi[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
-        const GroupImage<D> img(box, gnc, xi);
+        const GroupImage<D, T> img(box, gnc);
         const double mi = s.f[F_MASS][ii];
         const double Hs = s.f[F_SML][ii];  // search radius h_guess * ratio
         const double Hs2 = Hs * Hs;
@@ -226,8 +233,10 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     const int jl = stream_ld(a.cand + o + lane);
                     if(jl >= 0) {
                         const double4 q = a.pm[jl];
-                        l_xy[lane] = make_double2(img.at(0, q.x), D > 1 ? img.at(1, q.y) : 0.0);
-                        l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z) : 0.0, q.w);
+                        const int c = img.code(a.img, o + lane);
+                        l_xy[lane] = make_double2(img.at(0, q.x, c), D > 1 ? img.at(1, q.y, c) : 0.0);
+                        l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z, c) : 0.0, q.w);
+                        if constexpr(FP64) l_s[w][lane] = (int8_t)c;
                     }
                     return done ? 0ull : stream_ld(masks + o + lane);
                 };
@@ -237,7 +246,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     xj[0] = xy.x;
                     if constexpr(D > 1) xj[1] = xy.y;
                     if constexpr(D > 2) xj[2] = zm.x;
-                    const double r2 = sep2<D>(img.pairs, xi, xj, d);
+                    const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
                     const T r = gather_r<T>(r2);
                     if(r < ht && r2 < Hs2) {
                         const T q = ker.q_of(r);
@@ -299,9 +308,11 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) {
                 PreRec<T> q = prec[jl];
+                const int c = img.code(a.img, o + lane);
 #pragma unroll
-                for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k]);
+                for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k], c);
                 l_r[w][lane] = q;
+                if constexpr(FP64) l_s[w][lane] = (int8_t)c;
             }
             return valid ? stream_ld((narrowed ? a.mn : a.ma) + o + lane) : 0ull;
         };
@@ -310,7 +321,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = pj.x[l];
-            const double r2 = sep2<D>(img.pairs, xi, xj, d);
+            const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
             const T r = gather_r<T>(r2);
             if(!(r < ht && r2 < Hs2)) return;
             ++count;
@@ -377,7 +388,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = l_r[w][kc].x[l];
-            const double r2 = sep2<D>(img.pairs, xi, xj, d);
+            const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
             return gather_r<T>(r2) < ht && r2 < Hs2;
         };
         // with all the hits, refined in 3D except for GSPH (measured slower
@@ -518,6 +529,7 @@ static PreArgs make_args(Ctx &c)
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
     a.mn = c.tile_mn;
+    a.img = c.tile_img;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

@@ -46,7 +46,7 @@
 // The combined search takes H_ij = max(R_i, R_j) with the gather radii R,
 // so that one search serves both the pre-interaction (which keeps the pairs
 // with r < R_i) and the force stage.
-#include "ctx.hpp"
+#include "tiles.hpp"
 
 #include <type_traits>
 
@@ -67,7 +67,9 @@ struct SearchArgs {
     const int *num_groups;
     int *cand;           // group slabs of candidate tiles (Ctx::tile_cand)
     uint64_t *ma;        // hit masks per (tile, lane)
-    int *gnc;            // candidates per group, with GNC_WRAP
+    int8_t *img;         // the candidates' images (Ctx::tile_img)
+    int *gnc;            // candidates per group, with the GNC_ flags
+    int exact;           // FP64 pairs
     int wcap;            // slots per group slab and per staging buffer
     int *ws_j;           // staging buffers, one per persistent wave
     int cap;             // per-particle capacity (the reference's list size)
@@ -133,6 +135,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     __shared__ int l_chunk[SW][CHUNKCAP];
     __shared__ int l_kept[NW > 1 ? SW : 1], l_hits[NW > 1 ? SW : 1][NW > 1 ? WAVE : 1];
     __shared__ double l_reach[NW > 1 ? SW : 1];
+    __shared__ int l_shift[NW > 1 ? SW : 1];
 
     const int w = uniform(threadIdx.x / WAVE);
     const int part = NW > 1 ? w : 0;  // this wave's part of the group
@@ -293,9 +296,10 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     const int T = (nc + WAVE - 1) / WAVE;
     // Periodic box: every lane's minimum image of a candidate that can be a
     // hit is the one nearest to the group's centre, if the group and its
-    // reach span less than half the box; the candidate is then moved there
-    // once.  Otherwise (the flag GNC_WRAP, also read by the pair passes)
-    // every pair takes its own minimum image.
+    // reach span less than half the box; its shift by L, 0 or -L is then
+    // settled once (and added to the pairs' differences, as a minimum image
+    // does).  Otherwise every pair takes its own minimum image.  The pair
+    // passes read which of it was so from the flags beside the count.
     bool wrap = false;
     if(box.on) {
         const double H = sqrt(uniform_d(reach));
@@ -323,6 +327,10 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
         }
     };
     int count = 0;  // hits of particle `lane`
+    int shift = 0;  // GNC_SHIFT bits: some candidate is nearest by a shifted image
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
     // V consecutive tiles from tt on, the candidates' records in p_j and p_q
     int p_j[2] = {-1, -1};
     double4 p_q[2];
@@ -330,8 +338,9 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
         constexpr bool PER = decltype(pairwise)::value;
         constexpr int V = decltype(width)::value;
         constexpr int U = PER ? 1 : 4;  // particles per pass
-        int j[V];
+        int j[V], code[V];
         double x[V][3], cw[V];
+        int moved = 0;
 #pragma unroll
         for(int v = 0; v < V; ++v) {
             j[v] = p_j[v];
@@ -340,9 +349,27 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
             x[v][2] = p_q[v].z;
             cw[v] = p_q[v].w;
             stream_st(a.cand + gbase + (size_t)(tt + v) * WAVE + lane, j[v]);
-            if(!PER && box.on && j[v] >= 0) {
+            code[v] = 0;
+            if(!PER && box.on) {
+                if(j[v] >= 0) {
 #pragma unroll
-                for(int k = 0; k < D; ++k) x[v][k] = near_image(box, k, gc[k], x[v][k]);
+                    for(int k = 0; k < D; ++k) code[v] |= (near_image(box, k, gc[k], x[v][k]) & 3) << (2 * k);
+                }
+                stream_st(a.img + gbase + (size_t)(tt + v) * WAVE + lane, (int8_t)code[v]);
+                moved |= code[v];
+            }
+        }
+        bool any = wave_any(moved != 0);
+        if(any) {
+#pragma unroll
+            for(int k = 0; k < D; ++k) shift |= wave_any((moved >> (2 * k) & 3) != 0) ? GNC_SHIFT_AXIS << k : 0;
+            if(!a.exact) {
+                // mixed precision: the pairs subtract moved coordinates (GroupImage)
+#pragma unroll
+                for(int v = 0; v < V; ++v)
+#pragma unroll
+                    for(int k = 0; k < D; ++k) x[v][k] = GroupImage<D, float>::moved(box, k, x[v][k], code[v]);
+                any = false;
             }
         }
         // the next tiles' records, while these are tested
@@ -351,42 +378,63 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
         if(V > 1 && tt + S + 1 < T) fetch_c(tt + S + 1 + lane * T, p_j[1], p_q[1]);
         // particle after particle: the lanes' compares are its hit mask
         int lo[V] = {}, hi[V] = {};
-        for(int i0 = 0; i0 < cnt; i0 += U) {
-#pragma clang fp contract(off)
-            // records past the group's last particle (srec has a spare
-            // tile of them) fill lanes that are masked off below
-            double4 q[U];
-            double o2[U];
+        auto sweep = [&](auto shifted, auto first, auto number) {
+            constexpr int V0 = decltype(first)::value, N = decltype(number)::value;
+            double s[N][D];
+            if constexpr(decltype(shifted)::value) {
 #pragma unroll
-            for(int u = 0; u < U; ++u) {
-                q[u] = srec_at(a.srec, gr.x + i0 + u);
-                o2[u] = q[u].w;
+                for(int v = 0; v < N; ++v)
+#pragma unroll
+                    for(int k = 0; k < D; ++k) s[v][k] = GroupImage<D, double>::sign(code[V0 + v], k) * box.len[k];
             }
-            if constexpr(MODE == M_SYMMETRIC) {
+            for(int i0 = 0; i0 < cnt; i0 += U) {
+#pragma clang fp contract(off)
+                // records past the group's last particle (srec has a spare
+                // tile of them) fill lanes that are masked off below
+                double4 q[U];
+                double o2[U];
 #pragma unroll
                 for(int u = 0; u < U; ++u) {
-                    const double h = a.own[gr.x + min(i0 + u, cnt - 1)];
-                    o2[u] = h * h;
+                    q[u] = srec_at(a.srec, gr.x + i0 + u);
+                    o2[u] = q[u].w;
+                }
+                if constexpr(MODE == M_SYMMETRIC) {
+#pragma unroll
+                    for(int u = 0; u < U; ++u) {
+                        const double h = a.own[gr.x + min(i0 + u, cnt - 1)];
+                        o2[u] = h * h;
+                    }
+                }
+#pragma unroll
+                for(int u = 0; u < U; ++u) {
+#pragma unroll
+                    for(int v = 0; v < N; ++v) {
+                        double d[D];
+                        d[0] = q[u].x - x[V0 + v][0];
+                        if constexpr(D > 1) d[1] = q[u].y - x[V0 + v][1];
+                        if constexpr(D > 2) d[2] = q[u].z - x[V0 + v][2];
+                        if constexpr(PER) min_image<D>(box, d);
+                        if constexpr(decltype(shifted)::value) {
+#pragma unroll
+                            for(int k = 0; k < D; ++k) d[k] = d[k] + s[v][k];
+                        }
+                        double r2 = d[0] * d[0];
+#pragma unroll
+                        for(int k = 1; k < D; ++k) r2 = r2 + d[k] * d[k];
+                        uint64_t m = ballot(r2 < o2[u]);
+                        if constexpr(IJ) m |= ballot(r2 < cw[V0 + v]);
+                        lo[V0 + v] = write_lane((int)(uint32_t)m, i0 + u, lo[V0 + v]);
+                        hi[V0 + v] = write_lane((int)(uint32_t)(m >> 32), i0 + u, hi[V0 + v]);
+                    }
                 }
             }
-#pragma unroll
-            for(int u = 0; u < U; ++u) {
-#pragma unroll
-                for(int v = 0; v < V; ++v) {
-                    double d[D];
-                    d[0] = q[u].x - x[v][0];
-                    if constexpr(D > 1) d[1] = q[u].y - x[v][1];
-                    if constexpr(D > 2) d[2] = q[u].z - x[v][2];
-                    if constexpr(PER) min_image<D>(box, d);
-                    double r2 = d[0] * d[0];
-#pragma unroll
-                    for(int k = 1; k < D; ++k) r2 = r2 + d[k] * d[k];
-                    uint64_t m = ballot(r2 < o2[u]);
-                    if constexpr(IJ) m |= ballot(r2 < cw[v]);
-                    lo[v] = write_lane((int)(uint32_t)m, i0 + u, lo[v]);
-                    hi[v] = write_lane((int)(uint32_t)(m >> 32), i0 + u, hi[v]);
-                }
-            }
+        };
+        if(!any) {
+            sweep(std::false_type{}, Zero{}, width);
+        } else {
+            // one tile after the other (the shifts take the registers of the second)
+            sweep(std::true_type{}, Zero{}, One{});
+            if constexpr(V > 1) sweep(std::true_type{}, One{}, One{});
         }
 #pragma unroll
         for(int v = 0; v < V; ++v) {
@@ -396,8 +444,6 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
             count += __popcll(mine);
         }
     };
-    using One = std::integral_constant<int, 1>;
-    using Two = std::integral_constant<int, 2>;
     if(wrap) {
         int tt = part;
         if(tt < T) fetch_c(tt + lane * T, p_j[0], p_q[0]);
@@ -411,15 +457,20 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     }
     if constexpr(NW > 1) {
         l_hits[w][lane] = count;
+        if(lane == 0) l_shift[w] = shift;
         __syncthreads();
         count = 0;
+        shift = 0;
 #pragma unroll
-        for(int k = 0; k < NW; ++k) count += l_hits[k][lane];
+        for(int k = 0; k < NW; ++k) {
+            count += l_hits[k][lane];
+            shift |= l_shift[k];
+        }
         // (the next group's first barrier comes after these reads)
         tested = part == 0 ? nkept : 0;
     }
     if(part != 0) continue;
-    if(lane == 0) a.gnc[grp] = nc | (wrap ? GNC_WRAP : 0);
+    if(lane == 0) a.gnc[grp] = nc | (wrap ? GNC_WRAP : shift);
 
     // past the reference's list capacity (its unchecked write,
     // src/bhtree.cpp:257-258) the search reports an overflow
@@ -651,6 +702,8 @@ static SearchArgs base_args(Ctx &c)
     a.num_groups = c.num_groups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
+    a.img = c.tile_img;
+    a.exact = c.p.precision == SPHGPU_FP64;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.ws_j = c.ws_j;
@@ -725,14 +778,17 @@ int search_alloc(Ctx &c)
         if(c.tile_cand) (void)hipFree(c.tile_cand);
         if(c.tile_ma) (void)hipFree(c.tile_ma);
         if(c.tile_mn) (void)hipFree(c.tile_mn);
+        if(c.tile_img) (void)hipFree(c.tile_img);
         if(c.tile_nc) (void)hipFree(c.tile_nc);
         c.tile_cand = nullptr;
         c.tile_ma = c.tile_mn = nullptr;
+        c.tile_img = nullptr;
         c.tile_nc = nullptr;
         const size_t slots = (size_t)groups * wcap;
         SPHGPU_HIP(hipMalloc(&c.tile_cand, slots * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.tile_ma, slots * sizeof(uint64_t)));
         SPHGPU_HIP(hipMalloc(&c.tile_mn, slots * sizeof(uint64_t)));
+        SPHGPU_HIP(hipMalloc(&c.tile_img, slots));
         SPHGPU_HIP(hipMalloc(&c.tile_nc, groups * sizeof(int)));
         c.tile_groups_cap = groups;
     }
@@ -758,7 +814,7 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     const int i = gr.x + lane;
     if(i >= gr.y) return;
     const size_t gbase = (size_t)grp * wcap;
-    const int nc = gnc[grp] & ~GNC_WRAP;
+    const int nc = gnc[grp] & GNC_COUNT;
     const int T = (nc + WAVE - 1) / WAVE;
     const size_t lb = list_base(i, cap);
     double xi[D];
