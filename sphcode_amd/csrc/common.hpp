@@ -437,13 +437,15 @@ template <int D, class T> struct Cubic {
     __device__ __forceinline__ T dw_coef(T q, T r) const
     {
         if(r == T(0)) return T(0);
-        return dw_coef_inv(q, div_t<T>(T(1), r));
+        return dw_coef_inv(q, r, div_t<T>(T(1), r));
     }
-    // the same given 1/r, r != 0
-    __device__ __forceinline__ T dw_coef_inv(T q, T rinv) const
+    // the same given 1/r too, r != 0 (FP64 divides: the product with a
+    // rounded 1/r is rounded twice)
+    __device__ __forceinline__ T dw_coef_inv(T q, T r, T rinv) const
     {
         const T a = fmax(T(2) - q, T(0)), b = fmax(T(1) - q, T(0));
-        return -gnorm * rinv * (T(0.75) * a * a - T(3) * b * b);
+        const T g = sizeof(T) == 8 ? -gnorm / r : -gnorm * rinv;
+        return g * (T(0.75) * a * a - T(3) * b * b);
     }
     __device__ __forceinline__ T dhw(T q) const
     {
@@ -481,7 +483,7 @@ template <int D, class T> struct WendlandC4 {
         const T t2 = t * t;
         return -gnorm * (t2 * t2 * t) * (T(1) + T(5) * q);
     }
-    __device__ __forceinline__ T dw_coef_inv(T q, T /*rinv*/) const { return dw_coef(q, T(0)); }
+    __device__ __forceinline__ T dw_coef_inv(T q, T /*r*/, T /*rinv*/) const { return dw_coef(q, T(0)); }
     __device__ __forceinline__ T dhw(T q) const
     {
         const T t = fmax(T(1) - q, T(0));

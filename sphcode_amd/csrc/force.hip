@@ -43,7 +43,8 @@ struct ForceArgs {
 };
 
 // One pass over the particles: the records the pair loop reads for j
-// (rounded to the pair type), and the quotients of j's own fields.
+// (rounded to the pair type), and the quotients of j's own fields (GSPH:
+// in mixed mode; FP64 divides by rho^2 in the pair).
 template <int D, int TYPE, class T>
 __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, double4 *pr, ForceRec<T> *fr,
                                                            GradRec<T> *gr, Report rep)
@@ -240,8 +241,10 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             for(int l = 0; l < D; ++l) rij[l] = (T)d[l];
             const ForceRec<T> fj = l_f[w][kc];
             const Kern kj(T(0), fj.hinv);  // the kernel object reads 1/h only
-            const T cwi = ki.dw_coef_inv(ki.q_of(r), rinv);
-            const T cwj = kj.dw_coef_inv(kj.q_of(r), rinv);
+            const T cwi = ki.dw_coef_inv(ki.q_of(r), r, rinv);
+            const T cwj = kj.dw_coef_inv(kj.q_of(r), r, rinv);
+            // x / r (a rounded 1/r is for FP32 and unit vectors)
+            auto over_r = [&](T x) -> T { return FP64 ? x / r : x * rinv; };
             T dwi[D], dwj[D], vj[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) {
@@ -308,7 +311,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     hll(L, R, pstar, vstar);
                 }
                 const T fi = mj * pstar * rho2_inv_i;
-                const T fjj = mj * pstar * fj.q;
+                const T fjj = FP64 ? mj * pstar / (rhoj * rhoj) : mj * pstar * fj.q;
                 T fdv = T(0);
 #pragma unroll
                 for(int l = 0; l < D; ++l) {
@@ -330,7 +333,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 if(vr < T(0)) {
                     const T alpha = T(0.5) * (alphai + fj.alpha);
                     const T bal = T(0.5) * (bali + fj.bal);
-                    const T wv = vr * rinv;
+                    const T wv = over_r(vr);
                     const T vsig = ci + cj - T(3) * wv;
                     pij = T(-0.5) * bal * alpha * vsig * wv * div_t<T>(T(2), rhoi + rhoj);
                 }
@@ -338,8 +341,8 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 if(a.use_ac) {
                     const T uj = fj.u;
                     const T pj = TYPE == SPHGPU_DISPH ? div_t<T>(uj, fj.q) : fj.q * rhoj * rhoj;
-                    const T vs = a.gravity ? fabs(vr * rinv) : sqrt_t<T>(div_t<T>(T(2) * fabs(pi_ - pj), rhoi + rhoj));
-                    ac = (T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij) * rinv;
+                    const T vs = a.gravity ? fabs(over_r(vr)) : sqrt_t<T>(div_t<T>(T(2) * fabs(pi_ - pj), rhoi + rhoj));
+                    ac = over_r((T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij));
                 }
                 const T vdwi = dotd<D, T>(vij, dwi);
                 const T vdwij = dotd<D, T>(vij, dwij);
