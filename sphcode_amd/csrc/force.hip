@@ -46,7 +46,7 @@ struct ForceArgs {
 // (rounded to the pair type), and the quotients of j's own fields (GSPH:
 // in mixed mode; FP64 divides by rho^2 in the pair).
 template <int D, int TYPE, class T>
-__global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, double4 *pr, ForceRec<T> *fr,
+__global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, int use_ac, double4 *pr, ForceRec<T> *fr,
                                                            GradRec<T> *gr, Report rep)
 {
     if(rep.run(blockIdx.x)) return;
@@ -81,6 +81,8 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
         r.p = (T)pres;
         r.q = (T)(1.0 / (rho * rho));
     }
+    // the conductivity compares pressures: P itself, and the pair divides
+    if(TYPE != SPHGPU_GSPH && use_ac) r.q = (T)pres;
     fr[i] = r;
     if constexpr(TYPE == SPHGPU_GSPH) {
         if(gr) {
@@ -337,10 +339,10 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     const T vsig = ci + cj - T(3) * wv;
                     pij = T(-0.5) * bal * alpha * vsig * wv * div_t<T>(T(2), rhoi + rhoj);
                 }
-                T ac = T(0);
+                T ac = T(0), qj = fj.q;
                 if(a.use_ac) {
-                    const T uj = fj.u;
-                    const T pj = TYPE == SPHGPU_DISPH ? div_t<T>(uj, fj.q) : fj.q * rhoj * rhoj;
+                    const T uj = fj.u, pj = fj.q;
+                    qj = TYPE == SPHGPU_DISPH ? div_t<T>(uj, pj) : div_t<T>(pj, rhoj * rhoj);
                     const T vs = a.gravity ? fabs(over_r(vr)) : sqrt_t<T>(div_t<T>(T(2) * fabs(pi_ - pj), rhoi + rhoj));
                     ac = over_r((T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij));
                 }
@@ -352,11 +354,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     const T pi_i = g2u_p_i * (mj * fj.u - gradhi);
                     const T fji = T(1) - fj.p * mu_inv_i;
                     ci_f = pi_i + T(0.5) * mj * pij;
-                    cj_f = mj * (g2u_i * fj.q * fji + T(0.5) * pij);
+                    cj_f = mj * (g2u_i * qj * fji + T(0.5) * pij);
                     de = pi_i * vdwi;
                 } else {
                     ci_f = mj * (p_rho2_i * gradhi + T(0.5) * pij);
-                    cj_f = mj * (fj.q * fj.p + T(0.5) * pij);
+                    cj_f = mj * (qj * fj.p + T(0.5) * pij);
                     de = mj * p_rho2_i * gradhi * vdwi;
                 }
 #pragma unroll
@@ -414,7 +416,7 @@ template <int D, int K, int TYPE, class T> static void launch_force(Ctx &c, cons
         rep.count = NCOUNTERS;
         c.hvs_partials = 0;
     }
-    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
+    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u, (int)a.use_ac,
                        c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec, rep);
     if(rep.dst) (void)hipEventRecord(c.ev_flags, c.stream);
     if(c.after_pack) c.after_pack_rc = c.after_pack(c);
