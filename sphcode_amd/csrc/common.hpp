@@ -402,16 +402,31 @@ template <class T> __device__ __forceinline__ T rsqrt_t(T x)
 // reciprocal (times a) and square root, each about 1 ulp, without the
 // rescaling of operands or results beyond 2^126 in size (a division in
 // frexp/ldexp form takes eight instructions, about 38 cycles a wave, against
-// 12; a rescaled square root 28 against 9).
+// 12; a rescaled square root 28 against 9).  Lanes that need it, shown by a
+// reciprocal that is zero, denormal, infinite or NaN, or by a denormal (or
+// zero or negative) radicand, take the rescaled form in a branch that others
+// pass by.
 template <class T> __device__ __forceinline__ T div_t(T a, T b)
 {
-    if constexpr(sizeof(T) == 4) return a * __builtin_amdgcn_rcpf(b);
-    else return a / b;
+    if constexpr(sizeof(T) == 4) {
+        const float r = __builtin_amdgcn_rcpf(b);
+        float q = a * r;
+        constexpr int NORMAL = 0x108;  // of v_cmp_class: normal numbers of either sign
+        if(__builtin_expect(!__builtin_amdgcn_classf(r, NORMAL), 0)) q = a / b;
+        return q;
+    } else {
+        return a / b;
+    }
 }
 template <class T> __device__ __forceinline__ T sqrt_t(T x)
 {
-    if constexpr(sizeof(T) == 4) return __builtin_amdgcn_sqrtf(x);
-    else return sqrt(x);
+    if constexpr(sizeof(T) == 4) {
+        float r = __builtin_amdgcn_sqrtf(x);
+        if(__builtin_expect(!(x >= 1.17549435e-38f), 0)) r = sqrtf(x);
+        return r;
+    } else {
+        return sqrt(x);
+    }
 }
 
 template <int D, class T> struct Cubic {

@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
         r.q = (T)(s.f[F_ENE][i] / pres);
     } else if constexpr(TYPE == SPHGPU_SSPH) {
         r.p = (T)s.f[F_GRADH][i];
-        r.q = div_t<T>((T)pres, r.rho * r.rho);
+        r.q = (T)pres / (r.rho * r.rho);
     } else {
         r.p = (T)pres;
         r.q = (T)(1.0 / (rho * rho));
@@ -233,8 +233,8 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 rinv = 1.0 / r;
             } else {
                 if(!(r2 < hmax * hmax) || r2 == 0.0) return;
-                const float r2f = fmaxf((float)r2, 1.17549435e-38f);
-                r = __builtin_amdgcn_sqrtf(r2f);
+                r = __builtin_amdgcn_sqrtf((float)r2);
+                if(__builtin_expect((float)r2 < 1.17549435e-38f, 0)) r = gather_r_f32(r2);  // denormal or zero in FP32
                 rinv = __builtin_amdgcn_rcpf(r);
             }
             ++used;
