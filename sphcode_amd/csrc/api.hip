@@ -174,6 +174,7 @@ static int check_flags(Ctx &c, const char *stage, bool sent = false)
 
 static int stage_tree(Ctx &c)
 {
+    c.tree_ready = false;
     int rc = tree_build(c);
     if(rc) return rc;
     c.tree_ready = true;
@@ -525,7 +526,12 @@ int sphgpu_set_record_sets(void *ptr, int enable)
 {
     SPHGPU_CTX(ptr);
     c.record = enable != 0;
-    if(c.uploaded && c.record && !c.rec_gather) {
+    if(c.uploaded && c.record && !c.rec_force_cnt) {
+        // (the last of the four: an earlier call may have got some of them)
+        for(int **p : {&c.rec_gather, &c.rec_gather_cnt, &c.rec_force}) {
+            if(*p) (void)hipFree(*p);
+            *p = nullptr;
+        }
         const size_t lsz = (size_t)c.cap_n * (size_t)c.cap;
         SPHGPU_HIP(hipMalloc(&c.rec_gather, lsz * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.rec_gather_cnt, c.cap_n * sizeof(int)));
@@ -545,7 +551,13 @@ int sphgpu_upload(void *ptr, const sphgpu_particles *h)
     const int D = c.D;
     if(n != c.n || !c.s.f[F_X]) {
         int rc = alloc_buffers(c, n);
-        if(rc) return rc;
+        if(rc) {
+            // the old state is gone, and the new one has no place
+            free_buffers(c);
+            c.n = 0;
+            c.uploaded = c.tree_ready = false;
+            return rc;
+        }
     }
     c.n = n;
     // every field is written: from the caller's array, or zero
@@ -574,6 +586,7 @@ int sphgpu_upload(void *ptr, const sphgpu_particles *h)
     x.dev_ints = c.s.nb;
     x.user_ints = const_cast<int32_t *>(h->neighbor);
     x.dev_id = c.s.id;
+    c.uploaded = c.tree_ready = false;  // (the fields are half of one state and half of another until it is done)
     int rc = xfer_upload(c, x, n);
     if(rc) return rc;
     c.uploaded = true;

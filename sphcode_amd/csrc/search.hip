@@ -766,7 +766,10 @@ int search_alloc(Ctx &c)
     const int64_t want = std::max<int64_t>({(int64_t)8 * c.cap, (int64_t)48 * c.p.neighbor_number, 1024});
     const int wcap = (int)std::min<int64_t>((want + WAVE - 1) / WAVE * WAVE, 1 << 22);
     const int64_t waves = (int64_t)8 * c.num_cu * SW + SW;
+    // (the capacities are zero until all of a set's buffers are there, so that
+    // a failed allocation is not taken for one later)
     if(wcap != c.tile_wcap || waves > c.ws_waves) {
+        c.ws_waves = 0;
         if(c.ws_j) (void)hipFree(c.ws_j);
         c.ws_j = nullptr;
         SPHGPU_HIP(hipMalloc(&c.ws_j, (size_t)waves * wcap * sizeof(int)));
@@ -775,6 +778,7 @@ int search_alloc(Ctx &c)
     if(wcap != c.tile_wcap || c.ngroups > c.tile_groups_cap) {
         // grow with headroom: the group count changes a little every step
         const int64_t groups = std::max<int64_t>((int64_t)c.ngroups + c.ngroups / 4 + 64, c.tile_groups_cap);
+        c.tile_groups_cap = 0;
         if(c.tile_cand) (void)hipFree(c.tile_cand);
         if(c.tile_ma) (void)hipFree(c.tile_ma);
         if(c.tile_mn) (void)hipFree(c.tile_mn);
