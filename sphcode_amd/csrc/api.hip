@@ -38,6 +38,11 @@ __global__ void fill_int_kernel(int *p, int64_t n, int v)
     if(i < n) p[i] = v;
 }
 
+void fill_int(Ctx &c, int *p, int64_t n, int v)
+{
+    hipLaunchKernelGGL(fill_int_kernel, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, p, n, v);
+}
+
 void reset_work(Ctx &c, int slot)
 {
     hipLaunchKernelGGL(fill_int_kernel, dim3(NUM_XCD * WORK_STRIDE / BLOCK), dim3(BLOCK), 0, c.stream, c.work + NUM_XCD * WORK_STRIDE * slot,
@@ -108,7 +113,7 @@ static void free_buffers(Ctx &c)
     c.tile_groups_cap = 0;
     c.ws_waves = 0;
     c.ngroups = 0;
-    fr(c.rec_gather); fr(c.rec_gather_cnt); fr(c.rec_force); fr(c.rec_force_cnt);
+    fr(c.rec_gather); fr(c.rec_gather_cnt); fr(c.rec_force); fr(c.rec_force_cnt); fr(c.rec_used);
     fr(c.partial);
     c.cap_n = 0;
 }
@@ -148,6 +153,7 @@ static int alloc_buffers(Ctx &c, int64_t n)
         SPHGPU_HIP(hipMalloc(&c.rec_gather_cnt, np * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.rec_force, lsz * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.rec_force_cnt, np * sizeof(int)));
+        SPHGPU_HIP(hipMalloc(&c.rec_used, np * sizeof(int)));
     }
     return SPHGPU_OK;
 }
@@ -525,10 +531,10 @@ int sphgpu_destroy(void *ptr)
 int sphgpu_set_record_sets(void *ptr, int enable)
 {
     SPHGPU_CTX(ptr);
-    c.record = enable != 0;
-    if(c.uploaded && c.record && !c.rec_force_cnt) {
-        // (the last of the four: an earlier call may have got some of them)
-        for(int **p : {&c.rec_gather, &c.rec_gather_cnt, &c.rec_force}) {
+    c.record = false;
+    if(c.uploaded && enable && !c.rec_used) {
+        // (the last of the five: an earlier call may have got some of them)
+        for(int **p : {&c.rec_gather, &c.rec_gather_cnt, &c.rec_force, &c.rec_force_cnt}) {
             if(*p) (void)hipFree(*p);
             *p = nullptr;
         }
@@ -537,7 +543,9 @@ int sphgpu_set_record_sets(void *ptr, int enable)
         SPHGPU_HIP(hipMalloc(&c.rec_gather_cnt, c.cap_n * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.rec_force, lsz * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.rec_force_cnt, c.cap_n * sizeof(int)));
+        SPHGPU_HIP(hipMalloc(&c.rec_used, c.cap_n * sizeof(int)));
     }
+    c.record = enable != 0;
     return SPHGPU_OK;
 }
 
@@ -1055,6 +1063,15 @@ int sphgpu_neighbor_sets(void *ptr, int kind, int32_t *counts, int32_t *lists, i
     SPHGPU_HIP(hipMemcpy(id.data(), c.s.id, n * sizeof(int), hipMemcpyDeviceToHost));
     SPHGPU_HIP(hipMemcpy(cnt.data(), kind == 0 ? c.rec_gather_cnt : c.rec_force_cnt, n * sizeof(int), hipMemcpyDeviceToHost));
     SPHGPU_HIP(hipMemcpy(lst.data(), kind == 0 ? c.rec_gather : c.rec_force, lsz * sizeof(int), hipMemcpyDeviceToHost));
+    if(kind != 0) {
+        // as many as the force pass has summed
+        std::vector<int> used(n);
+        SPHGPU_HIP(hipMemcpy(used.data(), c.rec_used, n * sizeof(int), hipMemcpyDeviceToHost));
+        for(int64_t i = 0; i < n; ++i)
+            if(std::min(used[i], c.cap) != cnt[i])
+                return set_error(SPHGPU_E_STATE, "particle " + std::to_string(id[i]) + ": the force pass summed " + std::to_string(used[i]) +
+                                                     " pairs, its set has " + std::to_string(cnt[i]));
+    }
     std::vector<std::vector<int>> sets(n);
     for(int64_t i = 0; i < n; ++i) {
         std::vector<int> &m = sets[id[i]];

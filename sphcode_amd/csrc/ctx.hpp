@@ -381,6 +381,7 @@ struct Ctx {
     // recorded sets (debug): lists in list_at addressing
     int *rec_gather = nullptr, *rec_gather_cnt = nullptr;
     int *rec_force = nullptr, *rec_force_cnt = nullptr;
+    int *rec_used = nullptr;  // pairs that the force pass has summed per particle
     bool record = false;
     bool have_gather = false, have_force = false;
 
@@ -496,6 +497,7 @@ int gravity_combine(Ctx &c, hipStream_t st);
 // Zero the NUM_XCD task counters (WORK_STRIDE ints apart) of a slot before a
 // persistent launch (slot 0: the neighbour search).
 void reset_work(Ctx &c, int slot);
+void fill_int(Ctx &c, int *p, int64_t n, int v);  // on the main stream
 constexpr int WORK_SLOTS = 1;
 // one wave per search group: grid of ceil(ngroups / 4) blocks of 4 waves,
 // block b serving groups 4 xcd_block() .. + 3

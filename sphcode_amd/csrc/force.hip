@@ -37,6 +37,7 @@ struct ForceArgs {
     const double *scal;   // S_DT
     int64_t *counters;
     int stats;            // add to the statistics counters (errors are always counted)
+    int *rec_used;          // pairs summed per particle (recorded sets), or null
     const double4 *posrec;  // x, y, z, h (FP64)
     const void *frec;       // ForceRec<T>
     const void *grec;       // GradRec<T> (GSPH second order)
@@ -388,6 +389,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         else if constexpr(D == 2) parts_sum<NW, 3>(red, part, {&acc[0].s, &acc[1].s, &dene.s});
         else parts_sum<NW, 2>(red, part, {&acc[0].s, &dene.s});
         pairs = used;
+        if(a.rec_used && valid) atomicAdd(&a.rec_used[i], used);  // (of every part)
         if(valid && part == 0) {
 #pragma unroll
             for(int k = 0; k < D; ++k) s.f[F_A + k][i] = acc[k].val();
@@ -463,6 +465,10 @@ int force_compute(Ctx &c)
     a.scal = c.scal;
     a.counters = c.counters;
     a.stats = c.stats_on ? 1 : 0;
+    if(c.record) {
+        fill_int(c, c.rec_used, c.n, 0);
+        a.rec_used = c.rec_used;
+    }
     a.posrec = c.posrec;
     a.frec = c.pair_rec;
     a.grec = c.grad_rec;

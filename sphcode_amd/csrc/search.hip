@@ -800,15 +800,16 @@ int search_alloc(Ctx &c)
     return SPHGPU_OK;
 }
 
-// The gather sets (FORCE = 0: r < R_i, sml before the pre-interaction) or the
-// force sets (r < max(h_i, h_j), r != 0, as the force pass of the precision
-// tests it: 1 FP64, 2 mixed) as lists in list_at layout, from the tiles of
-// the last search (debug): lane l of a group appends its hits in staging
-// order (candidate c = t + kT is bit k of tile t).  Entries past cap are
-// dropped (the search reports them).
-template <int D, int FORCE>
+// The gather sets (r < R_i, sml before the pre-interaction) or with FORCE the
+// force sets (r < max(h_i, h_j), r != 0, as the force pass of pair type T
+// tests it) as lists in list_at layout, from the tiles of the last search
+// (debug): lane l of a group appends its hits in staging order (candidate
+// c = t + kT is bit k of tile t).  Entries past cap are dropped (the search
+// reports them).  The force pass also records how many pairs each particle
+// summed, and sphgpu_neighbor_sets compares.
+template <int D, class T, bool FORCE>
 __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
-                                                       const int *cand, const uint64_t *ma, int wcap, int cap,
+                                                       const int *cand, const uint64_t *ma, const int8_t *images, int wcap, int cap,
                                                        int *list, int *cnt)
 {
     const int grp = xcd_block() * (BLOCK / WAVE) + (int)(threadIdx.x / WAVE);
@@ -818,8 +819,9 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     const int i = gr.x + lane;
     if(i >= gr.y) return;
     const size_t gbase = (size_t)grp * wcap;
+    const GroupImage<D, T> img(box, gnc[grp]);
     const int nc = gnc[grp] & GNC_COUNT;
-    const int T = (nc + WAVE - 1) / WAVE;
+    const int ntile = (nc + WAVE - 1) / WAVE;
     const size_t lb = list_base(i, cap);
     double xi[D];
 #pragma unroll
@@ -827,21 +829,21 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     const double h = s.f[F_SML][i], h2 = h * h;
     int wf = 0;  // entries written (at most cap)
     for(int k = 0; k < WAVE; ++k) {
-        for(int t = 0; t < T; ++t) {
-            if(t + k * T >= nc) break;
+        for(int t = 0; t < ntile; ++t) {
+            if(t + k * ntile >= nc) break;
             const size_t o = gbase + (size_t)t * WAVE;
             if(!((ma[o + lane] >> k) & 1ull)) continue;
-            const int j = cand[o + k];
+            const int j = cand[o + k], c = img.code(images, o + k);
             double xj[D], d[D];
 #pragma unroll
-            for(int q = 0; q < D; ++q) xj[q] = s.f[F_X + q][j];
-            const double r2 = sep2<D>(box, xi, xj, d);
-            if constexpr(FORCE == 0) {
+            for(int q = 0; q < D; ++q) xj[q] = img.at(q, s.f[F_X + q][j], c);
+            const double r2 = img.sep2(xi, xj, [&] { return c; }, d);
+            if constexpr(!FORCE) {
                 if(!(r2 < h2)) continue;
             } else {
                 const double hj = s.f[F_SML][j];
                 const double hmax = h < hj ? hj : h;
-                if constexpr(FORCE == 1) {
+                if constexpr(sizeof(T) == 8) {
                     const double r = sqrt(r2);
                     if(r >= hmax || r == 0.0) continue;
                 } else if(!(r2 < hmax * hmax) || r2 == 0.0) {
@@ -854,17 +856,17 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     cnt[i] = wf;
 }
 
-template <int D, int FORCE> static void launch_record_t(Ctx &c, int *list, int *cnt)
+template <int D, class T> static void launch_record_t(Ctx &c, int *list, int *cnt, bool force)
 {
-    hipLaunchKernelGGL((record_kernel<D, FORCE>), dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
-                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, list, cnt);
+    const auto kernel = force ? record_kernel<D, T, true> : record_kernel<D, T, false>;
+    hipLaunchKernelGGL(kernel, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
+                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_img, c.tile_wcap, c.cap, list, cnt);
 }
 
 template <int D> static void launch_record(Ctx &c, int *list, int *cnt, bool force)
 {
-    if(!force) launch_record_t<D, 0>(c, list, cnt);
-    else if(c.p.precision == SPHGPU_FP64) launch_record_t<D, 1>(c, list, cnt);
-    else launch_record_t<D, 2>(c, list, cnt);
+    if(c.p.precision == SPHGPU_FP64) launch_record_t<D, double>(c, list, cnt, force);
+    else launch_record_t<D, float>(c, list, cnt, force);
 }
 
 int search_record(Ctx &c, int *list, int *cnt, bool force)

@@ -121,7 +121,7 @@ int main()
         if(failed == (rc == SPHGPU_OK)) return 11;
         if(failed && sphgpu_set_record_sets(ctx, 1) != SPHGPU_OK) return 12;
         for(int *q : {c.rec_gather, c.rec_force}) need(q, (size_t)h.n * c.cap * sizeof(int), "recorded sets", k);
-        for(int *q : {c.rec_gather_cnt, c.rec_force_cnt}) need(q, h.n * sizeof(int), "recorded counts", k);
+        for(int *q : {c.rec_gather_cnt, c.rec_force_cnt, c.rec_used}) need(q, h.n * sizeof(int), "recorded counts", k);
         sphgpu_destroy(ctx);
         if(!failed) break;
     }
