@@ -499,6 +499,7 @@ int sphgpu_create(const sphgpu_params *params, void **out)
         delete c;
         return hip_fail(e, "sphgpu_create");
     }
+    xfer_attach();
     *out = c;
     return SPHGPU_OK;
 }
@@ -512,6 +513,7 @@ int sphgpu_destroy(void *ptr)
     if(c->gstream) (void)hipStreamSynchronize(c->gstream);
     adjoint_free(*c);
     xfer_free(*c);
+    xfer_detach();
     free_buffers(*c);
     if(c->scal) (void)hipFree(c->scal);  // with the counters
     if(c->work) (void)hipFree(c->work);

@@ -332,7 +332,7 @@ struct Ctx {
     int *lvl = nullptr;        // the build's counters (tree.hip's LVL_...)
     int *lvl_host = nullptr;   // the first of them (pinned host)
     hipEvent_t ev_tree = nullptr; // they are on the host
-    double4 *msum = nullptr;   // raw mass moments (sum m x, sum m)
+    double4 *msum = nullptr;   // raw mass moments (sum m x, sum m); between builds, the stage of transfers
     GravNode *gnode = nullptr; // gravity node records (gravity on)
     double *gacc = nullptr;    // gravity's acceleration, D x cap_n (gravity on)
     LeafHit *leafhit = nullptr; // split walk: LEAFHIT_CAP records per wave
@@ -397,11 +397,7 @@ struct Ctx {
     int64_t *counters_host = nullptr;  // (char *)scal_host + SCAL_SPAN
     double *scal_host = nullptr;
 
-    // staging of particle transfers: two buffers on the host (pinned) and
-    // two on the device, of xfer_half bytes each
-    void *xfer_host = nullptr, *xfer_dev = nullptr;
-    int64_t xfer_half = 0;
-    hipEvent_t ev_xfer[2] = {nullptr, nullptr};
+    hipEvent_t ev_xfer[4] = {};  // particle transfers: a slot's copy is done
 
     // host mirror of simulation scalars
     double time = 0.0, dt = 0.0, h_per_v_sig = 0.0;
@@ -460,6 +456,8 @@ BoxDev make_box(const Ctx &c);
 int xfer_upload(Ctx &c, const Xfer &x, int64_t n);    // returns when the caller's arrays are free
 int xfer_download(Ctx &c, const Xfer &x, int64_t n);
 void xfer_free(Ctx &c);
+void xfer_attach();  // an engine more; pinned memory is kept for the next transfers while there is one
+void xfer_detach();
 // tree.hip
 int tree_alloc(Ctx &c);
 int tree_build(Ctx &c);          // BHTree::make

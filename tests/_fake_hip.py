@@ -19,8 +19,9 @@ def _compile(src: pathlib.Path, out: pathlib.Path) -> pathlib.Path:
     return out
 
 
-def program(driver: str, where: pathlib.Path) -> pathlib.Path:
-    srcs = [build.SRC / s for s in build.SOURCES] + [HERE / "fake_hip.cpp", HERE / driver]
+def program(driver: str, where: pathlib.Path, without=()) -> pathlib.Path:
+    """`driver` with the library's sources, except those that it includes itself."""
+    srcs = [build.SRC / s for s in build.SOURCES if s not in without] + [HERE / "fake_hip.cpp", HERE / driver]
     with cf.ThreadPoolExecutor(8) as ex:
         objs = list(ex.map(lambda s: _compile(s, where / (s.stem + ".o")), srcs))
     exe = where / "program"
