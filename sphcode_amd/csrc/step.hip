@@ -23,6 +23,7 @@ template <int D> __global__ void __launch_bounds__(BLOCK) init_kernel(State s, i
 // (the minimum is exact, so the order does not matter); without a ticket
 // dt_final_kernel does that.
 constexpr int DT_THREADS = 1024;
+constexpr int DT_LOADS = 4;
 template <int D>
 __global__ void __launch_bounds__(DT_THREADS) dt_kernel(const double *sml, const double *ax, const double *ay, const double *az, int n, double cf,
                                                      double *partial, int *ticket, double csound, const double *h_per_v_sig, double *dt)
@@ -33,14 +34,32 @@ __global__ void __launch_bounds__(DT_THREADS) dt_kernel(const double *sml, const
     // for each particle.  A NaN or a negative q counts for nothing.
     const double sign = cf < 0.0 ? -1.0 : 1.0;
     double least = __builtin_huge_val();
-    for(int i = blockIdx.x * DT_THREADS + threadIdx.x; i < n; i += gridDim.x * DT_THREADS) {
-        double a2 = ax[i] * ax[i];
-        if constexpr(D > 1) a2 += ay[i] * ay[i];
-        if constexpr(D > 2) a2 += az[i] * az[i];
-        const double a = sqrt(a2);
-        if(a > 0.0) {
-            const double q = sml[i] / a;
-            if(q >= 0.0 && sign * q < least) least = sign * q;
+    // DT_LOADS particles at a time, all of them read before the first is used;
+    // a wave leaves out the rounds in which it has none
+    const int stride = gridDim.x * blockDim.x;
+    for(int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += DT_LOADS * stride) {
+        double x[DT_LOADS], y[DT_LOADS], z[DT_LOADS], h[DT_LOADS];
+#pragma unroll
+        for(int u = 0; u < DT_LOADS; ++u) {
+            const int j = i + u * stride;
+            if(j < n) {
+                x[u] = ax[j];
+                if constexpr(D > 1) y[u] = ay[j];
+                if constexpr(D > 2) z[u] = az[j];
+                h[u] = sml[j];
+            }
+        }
+#pragma unroll
+        for(int u = 0; u < DT_LOADS; ++u) {
+            if(i + u * stride >= n) break;
+            double a2 = x[u] * x[u];
+            if constexpr(D > 1) a2 += y[u] * y[u];
+            if constexpr(D > 2) a2 += z[u] * z[u];
+            const double a = sqrt(a2);
+            if(a > 0.0) {
+                const double q = h[u] / a;
+                if(q >= 0.0 && sign * q < least) least = sign * q;
+            }
         }
     }
     least = block_min(least, sh);
@@ -53,7 +72,7 @@ __global__ void __launch_bounds__(DT_THREADS) dt_kernel(const double *sml, const
         if(threadIdx.x == 0) put(partial + blockIdx.x, m);
         if(!ticket || !last_block(ticket)) return;
         m = 1.7976931348623157e308;
-        for(int b = threadIdx.x; b < (int)gridDim.x; b += DT_THREADS) {
+        for(int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
             const double v = get(partial + b);
             m = v < m ? v : m;
         }
@@ -75,19 +94,26 @@ __global__ void __launch_bounds__(BLOCK) dt_final_kernel(const double *partial, 
     }
 }
 
-// Up to DT_ONE particles take one block and one launch; beyond that a block
-// per CU, with a ticket (a context's own) in one launch, otherwise in two.
-// A call and its synchronisation without a ticket, one block against two
-// launches: 16.2 us against 18.2 at 2,048 particles, 17.3 and 18.2 at 4,096,
-// 19.3 and 18.6 at 8,192 (17.9 us at 4,096 with a root for each particle).
+// Up to DT_ONE particles take one block and one launch.  Beyond that a context
+// with its own ticket takes one launch of a large block per CU; without one
+// (calls on the caller's stream) a launch of small blocks and one that reduces
+// their minima.  A call and its synchronisation without a ticket, one block
+// against two launches, on arrays read before / not read since they were
+// written: 22.7 / 23.6 us and 24.8 / 24.9 at 1,000 particles, 24.6 / 26.2 and
+// 24.8 / 24.9 at 4,096, 26.9 / 28.6 and 24.8 / 25.0 at 8,192; calls one after the
+// other 11.2 us and 13.6 at 4,096.  (One block's four loads a thread went out
+// one by one before: 24.1 / 27.2 us.  Blocks of 1,024 threads for the two
+// launches: 25.6 / 27.0 us at 8,192, 33.7 / 41.2 at 2^20, where small ones take
+// 27.7 / 36.9.)
 constexpr int DT_MAX_BLOCKS = 1024;
 constexpr int DT_ONE = 4096;
 static void launch_dt(int D, int n, const double *sml, const double *const acc[3], const double *hvs, double cf, double cs,
                       double *partial, int *ticket, int num_cu, double *dt, hipStream_t st)
 {
-    const int nb = n <= DT_ONE ? 1 : std::min({grid_for(n, DT_THREADS), num_cu, DT_MAX_BLOCKS});
+    const int threads = n <= DT_ONE || ticket ? DT_THREADS : BLOCK;
+    const int nb = n <= DT_ONE ? 1 : std::min(grid_for(n, threads), ticket ? num_cu : DT_MAX_BLOCKS);
     const auto kernel = D == 1 ? dt_kernel<1> : D == 2 ? dt_kernel<2> : dt_kernel<3>;
-    hipLaunchKernelGGL(kernel, dim3(nb), dim3(DT_THREADS), 0, st, sml, acc[0], acc[1], acc[2], n, cf, partial, ticket, cs, hvs, dt);
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(threads), 0, st, sml, acc[0], acc[1], acc[2], n, cf, partial, ticket, cs, hvs, dt);
     if(nb > 1 && !ticket) hipLaunchKernelGGL(dt_final_kernel, dim3(1), dim3(BLOCK), 0, st, partial, nb, cs, hvs, dt);
 }
 
