@@ -321,6 +321,7 @@ struct Ctx {
     int bucket_bits = 0;       // leading key bits that number a bucket
     bool bucket_clear = false; // bucket_cnt is all zero
     int bucket_wait = 0;       // tree builds before the buckets are tried again
+    int tree_nodes = 0;        // of the last build (0: none yet)
     void *sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     uint8_t *delta = nullptr;

@@ -98,9 +98,10 @@ template <int D> __global__ void __launch_bounds__(BBOX_THREADS) bbox_kernel(Sta
 constexpr int NLEVEL = 72;
 
 // Layout of lvl, all cleared by the keys' kernel: the number of search
-// groups and the sort's flag (one copy takes both to the host), the scans'
-// tickets, and the number of slice-spanning cells of each level.
-constexpr int LVL_GROUPS = 0, LVL_SORT = 1, LVL_HOST = 2, LVL_TICKET = 2, LVL_SPAN = 4, LVL_SIZE = LVL_SPAN + NLEVEL;
+// groups, the sort's flag and the number of nodes (one copy takes them to the
+// host), the scans' tickets, and the number of slice-spanning cells of each
+// level.
+constexpr int LVL_GROUPS = 0, LVL_SORT = 1, LVL_NODES = 2, LVL_HOST = 3, LVL_TICKET = 3, LVL_SPAN = 5, LVL_SIZE = LVL_SPAN + NLEVEL;
 
 // ------------------------------------------------------------------- scan
 // Exclusive scans by tiles: a block scans its tile and publishes the tile's
@@ -492,7 +493,7 @@ template <int D> __device__ __forceinline__ void leaf_moments(const State &s, co
 template <int D>
 __global__ void __launch_bounds__(BLOCK) emit_nodes_kernel(const uint64_t *keys, const uint8_t *delta, TreeShape ts, const int *nn,
                                                         const int *noff, const int *base, const double *scal, State s, TreeDev t, double4 *msum,
-                                                        int64_t node_cap, int64_t *counters, int2 *groups, int *num_groups)
+                                                        int64_t node_cap, int64_t *counters, int2 *groups, int *num_groups, int *nodes_out)
 {
 #pragma clang fp contract(off)
     __shared__ int first[BLOCK + 1];  // first node of each particle
@@ -505,7 +506,7 @@ __global__ void __launch_bounds__(BLOCK) emit_nodes_kernel(const uint64_t *keys,
         first[threadIdx.x] = f;
         if((int)threadIdx.x == nb - 1) first[nb] = f + nn[b];
         if(b == 0) {
-            *t.num_nodes = total <= node_cap ? total : (int)node_cap;
+            *t.num_nodes = *nodes_out = total <= node_cap ? total : (int)node_cap;
             if(total > node_cap) atomicAdd((unsigned long long *)&counters[C_TREE_ERR], 1ull);
             t.geo[0] = make_double4(scal[S_ROOT_CX], D > 1 ? scal[S_ROOT_CY] : 0.0, D > 2 ? scal[S_ROOT_CZ] : 0.0, scal[S_ROOT_EDGE]);
             t.rng[0] = make_int4(0, ts.n, total, 1);
@@ -776,12 +777,15 @@ __global__ void __launch_bounds__(SCAN_THREADS) spanning_kernel(TreeDev t, doubl
 }
 
 // One level of them, the deepest first, by many blocks: the single workgroup
-// handles about a thousand cells in some 20 us, one batch after the other
-// (978 us at 16.8M particles), a launch for each level takes 3 us.  Taken
-// past SPAN_BATCHES particles: the tree build takes 0.96 ms instead of 1.07
-// at 3.0M particles and 4.3 instead of 5.1 at 16.8M (at 2^21 the batches
-// take 84 us, the launches 60).
-constexpr int SPAN_BATCHES = 1 << 21;
+// handles about a thousand cells in some 20 us, one batch after the other, a
+// launch for each level takes 3 us.  How many cells span slices follows the
+// nodes, so the line is drawn there, not at a number of particles (whose nodes
+// differ by a factor of ten with leafParticleNumber).  Tree build, batches
+// against launches, us: 1.90M nodes (1.5M particles, one to a leaf) 457 and 461,
+// 2.10M (1D) 398 and 391, 2.33M (4.2M particles, eight to a leaf) 918 and 914,
+// 2.40M (2.1M, one) 580 and 562, 5.8M (4.2M, one) 1,320 and 1,087; but 299k nodes
+// (4.2M particles, 32 to a leaf) 761 and 822.
+constexpr int SPAN_BATCHES = 2000000;
 __global__ void __launch_bounds__(BLOCK) spanning_level_kernel(TreeDev t, double4 *msum, const int *span_cnt, const int *span,
                                                             const int4 *span_child, int span_cap, int L, int *work, int nwork)
 {
@@ -850,6 +854,7 @@ int tree_alloc(Ctx &c)
     c.bucket_bits = levels * c.D;
     c.bucket_clear = false;
     c.bucket_wait = 0;
+    c.tree_nodes = 0;
     const int64_t nbucket = std::max<int64_t>((int64_t)1 << c.bucket_bits, 4);  // scanned by fours
     SPHGPU_HIP(hipMalloc(&c.bucket_cnt, nbucket * sizeof(int)));
     SPHGPU_HIP(hipMalloc(&c.bucket_off, nbucket * sizeof(int)));
@@ -969,7 +974,7 @@ template <int D> static int tree_build_d(Ctx &c)
     hipLaunchKernelGGL(count_nodes_kernel, dim3(grid_for(n, SCAN_THREADS)), dim3(SCAN_THREADS), 0, c.stream, c.keys_sorted, ts, c.delta, c.nn,
                        c.noff, c.nbase, c.lvl);
     hipLaunchKernelGGL(emit_nodes_kernel<D>, dim3(grid_for(n)), dim3(BLOCK), 0, c.stream, c.keys_sorted, c.delta, ts, c.nn, c.noff, c.nbase,
-                       c.scal, c.s, c.t, c.msum, c.node_cap, c.counters, c.groups, c.num_groups);
+                       c.scal, c.s, c.t, c.msum, c.node_cap, c.counters, c.groups, c.num_groups, c.lvl + LVL_NODES);
     // in 1D and 2D the waves are filled from runs of small cells (2D KHI
     // step 2 % faster); in 3D whole cells stay together (the Evrard step
     // was 6 % slower with runs: less compact groups keep more candidates)
@@ -977,7 +982,8 @@ template <int D> static int tree_build_d(Ctx &c)
                        c.span_child, c.span_cap, c.groups, c.num_groups, c.group_cap, D < 3 ? 1 : 0);
     SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_HOST * sizeof(int), hipMemcpyDeviceToHost, c.stream));
     SPHGPU_HIP(hipEventRecord(c.ev_tree, c.stream));
-    if(n > SPAN_BATCHES) {
+    // (by the last build's nodes; before the first, about as many as a lattice has)
+    if((c.tree_nodes > 0 ? c.tree_nodes : 1.3 * n / ts.leaf) > SPAN_BATCHES) {
         for(int L = std::min(G + 1, NLEVEL - 1); L >= 1; --L)
             hipLaunchKernelGGL(spanning_level_kernel, dim3(c.num_cu), dim3(BLOCK), 0, c.stream, c.t, c.msum, c.lvl + LVL_SPAN, c.span,
                                c.span_child, c.span_cap, L, c.work, NUM_XCD * WORK_STRIDE);
@@ -993,6 +999,7 @@ template <int D> static int tree_build_d(Ctx &c)
         c.bucket_wait = BUCKET_WAIT;
         return tree_build_d<D>(c);
     }
+    c.tree_nodes = c.lvl_host[LVL_NODES];
     c.ngroups = c.lvl_host[LVL_GROUPS];
     if(c.ngroups < 1 || c.ngroups > c.group_cap) return set_error(SPHGPU_E_TREE, "search groups out of range");
     SPHGPU_HIP(hipGetLastError());
