@@ -158,10 +158,9 @@ static int alloc_buffers(Ctx &c, int64_t n)
     return SPHGPU_OK;
 }
 
-// Reads the error counters; a list overflow or node-pool exhaustion since
-// the last check becomes an error status.
-// Reads the counters (`sent`: the corrector has sent them and the scalars)
-// and reports the errors they record.
+// Reads the counters (`sent`: the corrector has sent them and the scalars);
+// a list overflow or node-pool exhaustion since the last check becomes an
+// error status.
 static int check_flags(Ctx &c, const char *stage, bool sent = false)
 {
     if(!sent)
@@ -216,19 +215,19 @@ static int launch_gravity_leaves(Ctx &c)
     return rc;
 }
 
-// The pre-interaction's candidate search.  After the first call, one walk
-// finds both the gather candidates and the symmetric pairs the force stage
-// needs (search_combined); the first call keeps the reference's initial
-// smoothing and separate searches.  With `walk` the gravity walk is started
-// on the second stream just after the search's launch (mixed Evrard step
-// 4.87 -> 4.62 ms at 2^20 particles, 0.418 -> 0.398 at 20k, FP64 at 131k
-// 1.27 -> 1.20 against starting it just before).
 // Kernel-span marks of sphgpu_integrate's timers (ev[8 + k]).
 static void kmark(Ctx &c, int k)
 {
     if(c.kernel_marks) (void)hipEventRecord(c.ev[8 + k], c.stream);
 }
 
+// The pre-interaction with its candidate search.  After the first call, one
+// search finds both the gather candidates and the symmetric pairs the force
+// stage needs (search_combined); the first call keeps the reference's initial
+// smoothing and separate searches.  With `walk` the gravity walk is started
+// on the second stream just after the search's launch (mixed Evrard step
+// 4.87 -> 4.62 ms at 2^20 particles, 0.418 -> 0.398 at 20k, FP64 at 131k
+// 1.27 -> 1.20 against starting it just before).
 static int stage_pre(Ctx &c, bool walk = false)
 {
     int rc;

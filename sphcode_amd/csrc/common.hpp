@@ -70,15 +70,6 @@ __device__ __forceinline__ uint64_t wave_transpose64(uint64_t a)
     return a;
 }
 
-__device__ __forceinline__ int wave_min_int(int v)
-{
-    for(int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(v, off, WAVE);
-        v = o < v ? o : v;
-    }
-    return v;
-}
-
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 {
@@ -130,9 +121,10 @@ __device__ __forceinline__ bool last_block(int *ticket)
 
 // Persistent waves: tasks [0, ntask) are split into NUM_XCD contiguous
 // shares, and the waves of each XCD take the tasks of its share one at a
-// time from that XCD's counter (hardware deals block b to XCD b mod 8).  A wave whose share is used up moves on to the next XCD's share, so no
-// XCD idles while another still has tasks; after visiting all NUM_XCD shares
-// it gets -1.  The counters lie WORK_STRIDE ints apart: updates of one cache
+// time from that XCD's counter (hardware deals block b to XCD b mod 8).  A
+// wave whose share is used up moves on to the next XCD's share, so no XCD
+// idles while another still has tasks; after visiting all NUM_XCD shares it
+// gets -1.  The counters lie WORK_STRIDE ints apart: updates of one cache
 // line by waves of all XCDs run one after the other at about 12 ns each,
 // and with the eight counters on one line those updates alone bounded the
 // search (2D, 393,160 particles: 327 us with 2,048 waves, 687 us with
@@ -221,31 +213,6 @@ template <class T> __device__ __forceinline__ T wave_maxv(T v)
     return v;
 }
 
-// Inclusive prefix maximum over the 64 lanes of non-negative values, by
-// DPP: row shifts by 1, 2, 4, 8 within each row of 16 lanes, then lane 15's
-// value into row 1 and lane 47's into row 3, then lane 31's into rows 2 and
-// 3.  Lanes whose DPP source is outside the pattern read 0, the identity.
-__device__ __forceinline__ int wave_incl_max_nonneg(int x)
-{
-    int y;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x = y > x ? y : x;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x = y > x ? y : x;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x = y > x ? y : x;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    x = y > x ? y : x;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x = y > x ? y : x;
-    y = __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    x = y > x ? y : x;
-    return x;
-}
-
-// Lane l receives lane l-1's value; lane 0 receives 0 (DPP wave_shr:1).
-__device__ __forceinline__ int wave_shr1(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x138, 0xf, 0xf, false); }
-
 // Read of a record the kernel never writes, through the constant address
 // space: a wave-uniform address then becomes a scalar load even where the
 // kernel also stores through other pointers (which otherwise forces vector
@@ -271,11 +238,10 @@ template <class T> __device__ __forceinline__ T load_ro(const T *p)
 // hardware FP64 square root (one instruction, no refinement sequence)
 // rounded to FP32, which is the correctly rounded FP32 |r| except when the
 // FP64 result falls within its error of an FP32 rounding boundary.  The
-// search stores it and the adjoint recomputes it with this same function.
+// pre-interaction and the adjoint share it.
 __device__ __forceinline__ float gather_r_f32(double r2) { return (float)__builtin_amdgcn_sqrt(r2); }
 
 // --------------------------------------------------------------- scalar math
-template <class T> __host__ __device__ __forceinline__ T sq(T x) { return x * x; }
 template <class T> __host__ __device__ __forceinline__ T cube(T x) { return x * x * x; }
 
 // h^D (include/kernel/kernel_function.hpp:8-16)

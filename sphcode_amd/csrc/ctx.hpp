@@ -435,7 +435,6 @@ struct Ctx {
     hipEvent_t *ev = nullptr;            // the current set
     double timer_ms[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     int64_t steps = 0;
-    int64_t last_nodes = 0, last_levels = 0;
 };
 
 // Error state (per thread).

@@ -19,7 +19,8 @@
 // A variant that kept two tiles resident, so that lanes waited at a tile
 // boundary only when one ran a whole tile ahead, needed 8-15 more registers
 // and twice the LDS; it was as fast on the 3D Evrard benchmark and 7-10 %
-// slower where the pair kernels run alone (2D KHI, 3D Sedov).
+// slower where the pair kernels run alone (2D KHI, 3D Sedov), measured before
+// the Newton sweep narrowed the hits and four waves shared small groups.
 #pragma once
 
 #include "ctx.hpp"

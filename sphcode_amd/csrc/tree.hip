@@ -977,7 +977,9 @@ template <int D> static int tree_build_d(Ctx &c)
                        c.scal, c.s, c.t, c.msum, c.node_cap, c.counters, c.groups, c.num_groups, c.lvl + LVL_NODES);
     // in 1D and 2D the waves are filled from runs of small cells (2D KHI
     // step 2 % faster); in 3D whole cells stay together (the Evrard step
-    // was 6 % slower with runs: less compact groups keep more candidates)
+    // was 6 % slower with runs: less compact groups keep more candidates.
+    // Both were measured when the search walked the octree, which took about
+    // twice the box search's time, and not since)
     hipLaunchKernelGGL(slice_kernel, dim3(std::min(c.span_cap, 2 * c.num_cu)), dim3(SCAN_THREADS), 0, c.stream, c.t, c.msum, c.lvl + LVL_SPAN, c.span,
                        c.span_child, c.span_cap, c.groups, c.num_groups, c.group_cap, D < 3 ? 1 : 0);
     SPHGPU_HIP(hipMemcpyAsync(c.lvl_host, c.lvl, LVL_HOST * sizeof(int), hipMemcpyDeviceToHost, c.stream));
