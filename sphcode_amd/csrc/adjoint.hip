@@ -183,7 +183,7 @@ template <int D, int NW> struct AdjGroup {
         ntile = ((gnc & GNC_COUNT) + WAVE - 1) / WAVE;
     }
     template <class T, class R>
-    __device__ __forceinline__ uint64_t stage(const AdjArgs &a, const GroupImage<D, T> &img, int tt, double4 *l_p, R *l_r, int8_t *l_s, const R *rec) const
+    __device__ __forceinline__ uint64_t stage(const AdjArgs &a, const GroupImage<D, T> &img, int tt, double4 *l_p, R *l_r, const R *rec) const
     {
         const size_t o = gbase + (size_t)tt * WAVE;
         const int jl = stream_ld(a.cand + o + lane);
@@ -194,20 +194,19 @@ template <int D, int NW> struct AdjGroup {
             if constexpr(D > 1) q.y = img.at(1, q.y, c);
             if constexpr(D > 2) q.z = img.at(2, q.z, c);
             l_p[lane] = q;
-            if constexpr(sizeof(T) == 8) l_s[lane] = (int8_t)c;
             l_r[lane] = rec[jl];
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
     }
 };
 
-template <int D, class T> __device__ __forceinline__ double pair_sep2(const GroupImage<D, T> &img, const double xi[D], const double4 &q, const int8_t &c, double d[D])
+template <int D, class T> __device__ __forceinline__ double pair_sep2(const GroupImage<D, T> &img, const double xi[D], const double4 &q, double d[D])
 {
     double xj[D];
     xj[0] = q.x;
     if constexpr(D > 1) xj[1] = q.y;
     if constexpr(D > 2) xj[2] = q.z;
-    return img.sep2(xi, xj, [&]() -> int { return c; }, d);
+    return img.sep2(xi, xj, d);
 }
 
 // The sweep of a pass: in 3D each lane's hits are first narrowed to those
@@ -231,7 +230,6 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, A
 {
     constexpr bool FP64 = sizeof(T) == 8;
     __shared__ double4 l_p[ASW][WAVE];
-    __shared__ int8_t l_s[ASW][sizeof(T) == 8 ? WAVE : 1];  // image codes
     __shared__ AdjRec<T> l_r[ASW][WAVE];
     __shared__ PartsLds<NW> red;
     const AdjGroup<D, NW> g(a);
@@ -256,7 +254,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, A
     auto keep = [&](int kc) -> bool {
         const double4 q = l_p[w][kc];
         double dd[D];
-        const double r2 = pair_sep2<D, T>(img, xi, q, l_s[w][sizeof(T) == 8 ? kc : 0], dd);
+        const double r2 = pair_sep2<D, T>(img, xi, q, dd);
         const double hmax = hi_d < q.w ? q.w : hi_d;
         if constexpr(FP64) {
             const double r = sqrt(r2);
@@ -268,7 +266,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, A
     auto pair = [&](int kc) {
         const AdjRec<T> &j = l_r[w][kc];
         double dd[D];
-        const double r2 = pair_sep2<D, T>(img, xi, l_p[w][kc], l_s[w][sizeof(T) == 8 ? kc : 0], dd);
+        const double r2 = pair_sep2<D, T>(img, xi, l_p[w][kc], dd);
         T r;
         if constexpr(FP64) r = sqrt(r2);
         else r = sqrtf((float)r2);
@@ -321,7 +319,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, A
         Ab.add((b + sv * psii) * gi);
     };
     const AdjRec<T> *rec = (const AdjRec<T> *)a.rec;
-    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], l_s[w], rec); }, keep, pair);
+    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
 #pragma unroll
     for(int k = 0; k < D; ++k) parts_sum<NW, 2>(red, g.part, {&xb[k].s, &vb[k].s});
     parts_sum<NW, 4>(red, g.part, {&hb.s, &rhob.s, &Ab.s, &Bb.s});
@@ -358,7 +356,6 @@ template <int D, int K, class T, int NW>
 __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, AdjArgs a)
 {
     __shared__ double4 l_p[ASW][WAVE];
-    __shared__ int8_t l_s[ASW][sizeof(T) == 8 ? WAVE : 1];  // image codes
     __shared__ AdjRec<T> l_r[ASW][WAVE];
     __shared__ PartsLds<NW> red;
     const AdjGroup<D, NW> gp(a);
@@ -377,12 +374,12 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, Adj
     Acc<T> rho_a, rhop_a, rhopp_a, Dv_a, Dvh_a, Rv_a[3], Rvh_a[3];
     auto keep = [&](int kc) -> bool {
         double dd[D];
-        return pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], l_s[w][sizeof(T) == 8 ? kc : 0], dd)) < ht;
+        return pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], dd)) < ht;
     };
     auto pair = [&](int kc) {
         const AdjRec<T> &j = l_r[w][kc];
         double dd[D];
-        const double r2 = pair_sep2<D, T>(img, xi, l_p[w][kc], l_s[w][sizeof(T) == 8 ? kc : 0], dd);
+        const double r2 = pair_sep2<D, T>(img, xi, l_p[w][kc], dd);
         const T r = pair_r<T>(r2);
         const T mj = j.m;
         const KernelDerivs<T> kd = kernel_derivs_inv<D, K, T>(r, ht_inv);
@@ -410,7 +407,7 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, Adj
         }
     };
     const AdjRec<T> *rec = (const AdjRec<T> *)a.rec;
-    adj_sweep<D, NW>(gp, [&](int tt) { return gp.stage(a, img, tt, l_p[w], l_r[w], l_s[w], rec); }, keep, pair);
+    adj_sweep<D, NW>(gp, [&](int tt) { return gp.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
     parts_sum<NW, 3>(red, gp.part, {&rho_a.s, &rhop_a.s, &rhopp_a.s});
     if(a.balsara && D > 1) {
         parts_sum<NW, 4>(red, gp.part, {&Dv_a.s, &Rv_a[0].s, &Rv_a[1].s, &Rv_a[2].s});
@@ -528,7 +525,6 @@ template <int D, int K, class T, int NW>
 __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, AdjArgs a)
 {
     __shared__ double4 l_p[ASW][WAVE];
-    __shared__ int8_t l_s[ASW][sizeof(T) == 8 ? WAVE : 1];  // image codes
     __shared__ SeedRec<T> l_r[ASW][WAVE];
     __shared__ PartsLds<NW> red;
     const AdjGroup<D, NW> g(a);
@@ -547,13 +543,13 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, Adj
     Acc<T> xb[D], vb[D];
     auto keep = [&](int kc) -> bool {
         double dd[D];
-        const T r = pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], l_s[w][sizeof(T) == 8 ? kc : 0], dd));
+        const T r = pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], dd));
         return r != T(0) && (r < me.h || r < l_r[w][kc].h);
     };
     auto pair = [&](int kc) {
         const SeedRec<T> &j = l_r[w][kc];
         double dd[D];
-        const T r = pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], l_s[w][sizeof(T) == 8 ? kc : 0], dd));
+        const T r = pair_r<T>(pair_sep2<D, T>(img, xi, l_p[w][kc], dd));
         T v[D], d[D], sv = T(0);
 #pragma unroll
         for(int k = 0; k < D; ++k) {
@@ -564,7 +560,7 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, Adj
         if(r < me.h) sum_term<D, K, T>(r, d, v, sv, j.m, me.hinv, me.srho, me.srhop, me.sdv, me.srv, xb, vb);
         if(r < j.h) sum_term<D, K, T>(r, d, v, sv, me.m, j.hinv, j.srho, j.srhop, j.sdv, j.srv, xb, vb);
     };
-    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], l_s[w], rec); }, keep, pair);
+    adj_sweep<D, NW>(g, [&](int tt) { return g.stage(a, img, tt, l_p[w], l_r[w], rec); }, keep, pair);
 #pragma unroll
     for(int k = 0; k < D; ++k) parts_sum<NW, 2>(red, g.part, {&xb[k].s, &vb[k].s});
     if(!g.valid || g.part != 0) return;

@@ -286,7 +286,7 @@ template <int D> __device__ __forceinline__ double sml_guess(double m, double rh
 // of |d|, |d+L|, |d-L| in the reference's tie order.
 struct BoxDev {
     int on;
-    double lo[3], hi[3], len[3];
+    double lo[3], hi[3], len[3], inv[3];  // inv = 1 / len
 };
 
 template <int D> __device__ __forceinline__ void min_image(const BoxDev &b, double d[D])

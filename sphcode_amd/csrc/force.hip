@@ -146,7 +146,6 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
     __shared__ double2 l_xy[SW][WAVE], l_zh[SW][WAVE];
     __shared__ ForceRec<T> l_f[SW][WAVE];
     __shared__ GradRec<T> l_g[GS ? SW : 1][GS ? WAVE : 1];
-    __shared__ int8_t l_s[FP64 ? SW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -205,7 +204,6 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 q.x = img.at(0, q.x, c);
                 if constexpr(D > 1) q.y = img.at(1, q.y, c);
                 if constexpr(D > 2) q.z = img.at(2, q.z, c);
-                if constexpr(FP64) l_s[w][lane] = (int8_t)c;
                 l_xy[w][lane] = make_double2(q.x, q.y);
                 l_zh[w][lane] = make_double2(q.z, q.w);
                 l_f[w][lane] = frec[jl];
@@ -222,7 +220,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             if constexpr(D > 1) xj[1] = xy.y;
             if constexpr(D > 2) xj[2] = zh.x;
             hmax = hi_d < zh.y ? zh.y : hi_d;
-            return img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
+            return img.sep2(xi, xj, d);
         };
         auto pair = [&](int kc) {
             double d[D], hmax;

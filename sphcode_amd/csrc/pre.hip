@@ -117,8 +117,6 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
 {
     using Kern = typename KernelOf<D, K, T>::type;
     __shared__ PosMass<T> l_r[PSW][WAVE];
-    constexpr bool FP64 = sizeof(T) == 8;
-    __shared__ int8_t l_s[FP64 ? PSW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -146,7 +144,6 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
             const int c = img.code(a.img, o + lane);
 #pragma unroll
             for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl], c);
-            if constexpr(FP64) l_s[w][lane] = (int8_t)c;
             l_r[w][lane].m = (T)s.f[F_MASS][jl];
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
@@ -155,7 +152,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         double xj[D], d[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xj[k] = l_r[w][kc].x[k];
-        const T r = gather_r<T>(img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d));
+        const T r = gather_r<T>(img.sep2(xi, xj, d));
         if(r < h) rho.add(l_r[w][kc].m * ker.w(ker.q_of(r)));
     };
     tile_sweep<NW>(part, ntile, stage, pair);
@@ -171,8 +168,6 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
     using Kern = typename KernelOf<D, K, T>::type;
     constexpr bool NUMBER = TYPE == SPHGPU_DISPH;
     __shared__ PreRec<T> l_r[PSW][WAVE];
-    constexpr bool FP64 = sizeof(T) == 8;
-    __shared__ int8_t l_s[FP64 ? PSW : 1][FP64 ? WAVE : 1];  // image codes
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int part = w % NW;
@@ -236,8 +231,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                         const int c = img.code(a.img, o + lane);
                         l_xy[lane] = make_double2(img.at(0, q.x, c), D > 1 ? img.at(1, q.y, c) : 0.0);
                         l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z, c) : 0.0, q.w);
-                        if constexpr(FP64) l_s[w][lane] = (int8_t)c;
-                    }
+                                }
                     return done ? 0ull : stream_ld(masks + o + lane);
                 };
                 auto npair = [&](int kc) -> bool {
@@ -246,7 +240,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     xj[0] = xy.x;
                     if constexpr(D > 1) xj[1] = xy.y;
                     if constexpr(D > 2) xj[2] = zm.x;
-                    const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
+                    const double r2 = img.sep2(xi, xj, d);
                     const T r = gather_r<T>(r2);
                     if(r < ht && r2 < Hs2) {
                         const T q = ker.q_of(r);
@@ -312,8 +306,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
 #pragma unroll
                 for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k], c);
                 l_r[w][lane] = q;
-                if constexpr(FP64) l_s[w][lane] = (int8_t)c;
-            }
+                }
             return valid ? stream_ld((narrowed ? a.mn : a.ma) + o + lane) : 0ull;
         };
         auto fpair = [&](int kc) {
@@ -321,7 +314,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = pj.x[l];
-            const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
+            const double r2 = img.sep2(xi, xj, d);
             const T r = gather_r<T>(r2);
             if(!(r < ht && r2 < Hs2)) return;
             ++count;
@@ -388,7 +381,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             double xj[D], d[D];
 #pragma unroll
             for(int l = 0; l < D; ++l) xj[l] = l_r[w][kc].x[l];
-            const double r2 = img.sep2(xi, xj, [&]() -> int { return l_s[FP64 ? w : 0][FP64 ? kc : 0]; }, d);
+            const double r2 = img.sep2(xi, xj, d);
             return gather_r<T>(r2) < ht && r2 < Hs2;
         };
         // with all the hits, refined in 3D except for GSPH (measured slower

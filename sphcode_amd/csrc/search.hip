@@ -67,7 +67,7 @@ struct SearchArgs {
     const int *num_groups;
     int *cand;           // group slabs of candidate tiles (Ctx::tile_cand)
     uint64_t *ma;        // hit masks per (tile, lane)
-    int8_t *img;         // the candidates' images (Ctx::tile_img)
+    int8_t *img;         // the candidates' images (mixed; Ctx::tile_img)
     int *gnc;            // candidates per group, with the GNC_ flags
     int exact;           // FP64 pairs
     int wcap;            // slots per group slab and per staging buffer
@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 #pragma unroll
                     for(int k = 0; k < D; ++k) code[v] |= (near_image(box, k, gc[k], x[v][k]) & 3) << (2 * k);
                 }
-                stream_st(a.img + gbase + (size_t)(tt + v) * WAVE + lane, (int8_t)code[v]);
+                if(!a.exact) stream_st(a.img + gbase + (size_t)(tt + v) * WAVE + lane, (int8_t)code[v]);
                 moved |= code[v];
             }
         }
@@ -837,7 +837,7 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
             double xj[D], d[D];
 #pragma unroll
             for(int q = 0; q < D; ++q) xj[q] = img.at(q, s.f[F_X + q][j], c);
-            const double r2 = img.sep2(xi, xj, [&] { return c; }, d);
+            const double r2 = img.sep2(xi, xj, d);
             if constexpr(!FORCE) {
                 if(!(r2 < h2)) continue;
             } else {

@@ -235,6 +235,7 @@ BoxDev make_box(const Ctx &c)
         box.lo[k] = c.p.range_min[k];
         box.hi[k] = c.p.range_max[k];
         box.len[k] = c.p.range_max[k] - c.p.range_min[k];
+        box.inv[k] = 1.0 / box.len[k];
     }
     return box;
 }

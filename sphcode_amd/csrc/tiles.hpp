@@ -27,22 +27,22 @@
 
 namespace sphgpu {
 
-// Periodic images of a group's candidates.  Unless the group's entry in
-// Ctx::tile_nc carries GNC_WRAP, every pair's minimum image of a candidate
-// is one and the same, and the search has written which (Ctx::tile_img, a
-// signed two-bit code per axis; read if some candidate of the group has one,
-// GNC_SHIFT).  The three minimum images of a pair cost some 30 FP64 operations
-// and compares.
+// Periodic images of a group's candidates.  A group's entry in Ctx::tile_nc
+// says what they need: every pair its three images compared (GNC_WRAP: the
+// group's reach spans half the box; some 30 FP64 operations and compares), or
+// on some axes a shift by L for some candidates (GNC_SHIFT), or nothing (no
+// face of the box comes near).
 //
-// FP64 pairs take x_i - x_j + L code, which rounds as their own minimum image
-// would (L code is exact): the sets are the reference's to the last bit and
-// the sums no further from 64-bit values (a coordinate moved by L first is
-// rounded before the subtraction, and doubled that error).  Three operations
-// on each axis with such a candidate (rollout gradient of 29,791 particles
-// 7.69 -> 7.98 ms, evaluation of 110,592 1.68 -> 1.72).  Mixed pairs, whose
-// separations are rounded to FP32 next, subtract a coordinate moved by L code
-// when it was staged (rollout gradient of 262,144 particles 34.1 ms, with the
-// FP64 form 36.3).
+// With GNC_SHIFT a pair's minimum image is closer than half the box if it is a
+// hit, so that the shift is L times the rounded quotient, minus.  FP64 pairs
+// take x_i - x_j and then add it, which rounds as the reference does: the sets
+// are the reference's to the last bit and the sums no further from 64-bit
+// values (a coordinate moved by L first is rounded before the subtraction, and
+// doubled that error).  Mixed pairs, whose separations are rounded to FP32
+// next, subtract a coordinate that was moved when it was staged: the search
+// found the image (the same one for all of the group's pairs) and has written
+// it, a signed two-bit code per axis in Ctx::tile_img (rollout gradient of
+// 262,144 particles 34.1 ms, with a shift in each pair 36.3).
 template <int D, class T> struct GroupImage {
     static constexpr bool EXACT = sizeof(T) == 8;
     const BoxDev &box;
@@ -54,21 +54,23 @@ template <int D, class T> struct GroupImage {
         shift = flags & GNC_SHIFT;
     }
     static __device__ __forceinline__ double sign(int code, int k) { return (double)(code << (30 - 2 * k) >> 30); }
-    // the code of the candidate in `lane` of the tile at slot o
-    __device__ __forceinline__ int code(const int8_t *img, size_t o) const { return shift ? stream_ld(img + o) : 0; }
+    static __device__ __forceinline__ double moved(const BoxDev &box, int k, double x, int code)
+    {
+        return __builtin_fma(-sign(code, k), box.len[k], x);
+    }
+    // mixed: the code of the candidate at slot o
+    __device__ __forceinline__ int code(const int8_t *img, size_t o) const
+    {
+        return !EXACT && shift ? stream_ld(img + o) : 0;
+    }
     // axis k of a candidate's position, as it is staged
     __device__ __forceinline__ double at(int k, double x, int code) const
     {
         if constexpr(EXACT) return x;
         else return shift ? moved(box, k, x, code) : x;
     }
-    static __device__ __forceinline__ double moved(const BoxDev &box, int k, double x, int code)
-    {
-        return __builtin_fma(-sign(code, k), box.len[k], x);
-    }
-    // sep2 of a pair; code() is the candidate's
-    template <class Code>
-    __device__ __forceinline__ double sep2(const double xi[D], const double xj[D], Code &&code, double d[D]) const
+    // r_ij and its square of a pair, the position of j as it was staged
+    __device__ __forceinline__ double sep2(const double xi[D], const double xj[D], double d[D]) const
     {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -77,10 +79,9 @@ template <int D, class T> struct GroupImage {
             if(flags & GNC_WRAP) {
                 min_image<D>(box, d);
             } else {
-                const int v = code();
 #pragma unroll
                 for(int k = 0; k < D; ++k)
-                    if(flags & GNC_SHIFT_AXIS << k) d[k] = __builtin_fma(sign(v, k), box.len[k], d[k]);
+                    if(flags & GNC_SHIFT_AXIS << k) d[k] = __builtin_fma(-rint(d[k] * box.inv[k]), box.len[k], d[k]);
             }
         }
         double r2 = d[0] * d[0];
