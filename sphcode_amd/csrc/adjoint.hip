@@ -91,7 +91,6 @@ struct AdjArgs {
     int ngroups;
     const int *cand;     // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;
-    const int8_t *img;   // images (Ctx::tile_img)
     const int *gnc;
     int wcap;
     double4 *pos;        // x, y, z, h
@@ -189,10 +188,9 @@ template <int D, int NW> struct AdjGroup {
         const int jl = stream_ld(a.cand + o + lane);
         if(jl >= 0) {
             double4 q = a.pos[jl];
-            const int c = img.code(a.img, o + lane);
-            q.x = img.at(0, q.x, c);
-            if constexpr(D > 1) q.y = img.at(1, q.y, c);
-            if constexpr(D > 2) q.z = img.at(2, q.z, c);
+            q.x = img.at(0, q.x);
+            if constexpr(D > 1) q.y = img.at(1, q.y);
+            if constexpr(D > 2) q.z = img.at(2, q.z);
             l_p[lane] = q;
             l_r[lane] = rec[jl];
         }
@@ -243,7 +241,7 @@ __global__ void __launch_bounds__(BLOCK) adj_force_kernel(State s, BoxDev box, A
         vi[k] = (T)s.f[F_V + k][i];
         afi[k] = (T)W(a, W_AF + k, i);
     }
-    const GroupImage<D, T> img(box, g.gnc);
+    const GroupImage<D, T> img(box, g.gnc, xi);
     const double hi_d = s.f[F_SML][i];
     const T hi_inv = T(1) / (T)hi_d, rhoi = (T)s.f[F_DENS][i], pi_ = (T)s.f[F_PRES][i], omi = (T)s.f[F_GRADH][i];
     const T bi = (T)s.f[F_BAL][i], ci = (T)s.f[F_SOUND][i], ali = (T)s.f[F_ALPHA][i], mi = (T)s.f[F_MASS][i];
@@ -368,7 +366,7 @@ __global__ void __launch_bounds__(BLOCK) adj_pre_kernel(State s, BoxDev box, Adj
         xi[k] = s.f[F_X + k][i];
         vi[k] = (T)s.f[F_V + k][i];
     }
-    const GroupImage<D, T> img(box, gp.gnc);
+    const GroupImage<D, T> img(box, gp.gnc, xi);
     const double h = s.f[F_SML][i];
     const T ht = (T)h, ht_inv = T(1) / ht;
     Acc<T> rho_a, rhop_a, rhopp_a, Dv_a, Dvh_a, Rv_a[3], Rvh_a[3];
@@ -537,7 +535,7 @@ __global__ void __launch_bounds__(BLOCK) adj_sum_kernel(State s, BoxDev box, Adj
         xi[k] = s.f[F_X + k][i];
         vi[k] = (T)s.f[F_V + k][i];
     }
-    const GroupImage<D, T> img(box, g.gnc);
+    const GroupImage<D, T> img(box, g.gnc, xi);
     const SeedRec<T> *rec = (const SeedRec<T> *)a.seed;
     const SeedRec<T> me = rec[i];
     Acc<T> xb[D], vb[D];
@@ -635,7 +633,6 @@ int adjoint_step(Ctx &c, bool kick)
     a.ngroups = c.ngroups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
-    a.img = c.tile_img;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.pos = c.posrec;  // free after the force pass

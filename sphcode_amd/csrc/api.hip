@@ -108,7 +108,7 @@ static void free_buffers(Ctx &c)
     if(c.lvl_host) (void)hipHostFree(c.lvl_host);
     c.lvl_host = nullptr;
     fr(c.srec); fr(c.boxes); fr(c.leaf_rad);
-    fr(c.tile_cand); fr(c.tile_ma); fr(c.tile_mn); fr(c.tile_img); fr(c.tile_nc); fr(c.ws_j);
+    fr(c.tile_cand); fr(c.tile_ma); fr(c.tile_mn); fr(c.tile_nc); fr(c.ws_j);
     c.tile_wcap = 0;
     c.tile_groups_cap = 0;
     c.ws_waves = 0;

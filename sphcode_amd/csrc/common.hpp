@@ -319,6 +319,17 @@ __device__ __forceinline__ int near_image(const BoxDev &b, int k, double c, doub
     return r;
 }
 
+// Axis k of the image of x that is nearest to c: x, x - L or x + L.
+__device__ __forceinline__ double near_position(const BoxDev &b, int k, double c, double x)
+{
+    const double d = c - x;
+    const double a1 = fabs(d), a2 = fabs(d + b.len[k]), a3 = fabs(d - b.len[k]);
+    double r = x + b.len[k];
+    if(a2 <= a3 && a2 <= a1) r = x - b.len[k];
+    if(a1 <= a2 && a1 <= a3) r = x;
+    return r;
+}
+
 // r_ij = x_i - x_j with minimum image, and its squared norm summed left to
 // right without contraction (include/vector_type.hpp:194-227).
 template <int D> __device__ __forceinline__ double sep2(const BoxDev &b, const double xi[D], const double xj[D], double d[D])
@@ -364,6 +375,10 @@ template <class T> __device__ __forceinline__ T rsqrt_t(T x)
     else return rsqrt(x);
 }
 
+// a reciprocal that needs no rescaling: a normal number of either sign (the
+// classes of v_cmp_class)
+__device__ __forceinline__ bool rcp_normal(float r) { return __builtin_amdgcn_classf(r, 0x108); }
+
 // a / b and sqrt(x) of pair terms.  The FP32 forms are the hardware
 // reciprocal (times a) and square root, each about 1 ulp, without the
 // rescaling of operands or results beyond 2^126 in size (a division in
@@ -377,8 +392,7 @@ template <class T> __device__ __forceinline__ T div_t(T a, T b)
     if constexpr(sizeof(T) == 4) {
         const float r = __builtin_amdgcn_rcpf(b);
         float q = a * r;
-        constexpr int NORMAL = 0x108;  // of v_cmp_class: normal numbers of either sign
-        if(__builtin_expect(!__builtin_amdgcn_classf(r, NORMAL), 0)) q = a / b;
+        if(__builtin_expect(!rcp_normal(r), 0)) q = a / b;
         return q;
     } else {
         return a / b;

@@ -369,7 +369,6 @@ struct Ctx {
     int *tile_cand = nullptr;
     uint64_t *tile_ma = nullptr;
     uint64_t *tile_mn = nullptr;   // the pre-interaction's narrowed hits (alike)
-    int8_t *tile_img = nullptr;    // mixed: images of the candidates (GroupImage), alike
     int *tile_nc = nullptr;
     int tile_wcap = 0;             // slots per group (multiple of 64)
     int64_t tile_groups_cap = 0;   // groups the slabs are allocated for

@@ -17,6 +17,8 @@
 // gradients lie in LDS with strides that spread over all banks: alone, Evrard
 // 2^20 DISPH 725 -> 589 us (4.6e8 -> 3.9e8 vector instructions), 2^21 GSPH
 // second order 2,361 -> 1,690 us (1.53e9 -> 0.99e9).
+#include <type_traits>
+
 #include "tiles.hpp"
 
 namespace sphgpu {
@@ -26,7 +28,6 @@ struct ForceArgs {
     int ngroups;
     const int *cand;        // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;     // hit masks per (tile, lane): every symmetric pair
-    const int8_t *img;      // images (Ctx::tile_img)
     const int *gnc;
     int wcap;
     double gamma;
@@ -47,7 +48,7 @@ struct ForceArgs {
 // (rounded to the pair type), and the quotients of j's own fields (GSPH:
 // in mixed mode; FP64 divides by rho^2 in the pair).
 template <int D, int TYPE, class T>
-__global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, int use_ac, double4 *pr, ForceRec<T> *fr,
+__global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int use_u, double4 *pr, ForceRec<T> *fr,
                                                            GradRec<T> *gr, Report rep)
 {
     if(rep.run(blockIdx.x)) return;
@@ -77,13 +78,11 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
         r.q = (T)(s.f[F_ENE][i] / pres);
     } else if constexpr(TYPE == SPHGPU_SSPH) {
         r.p = (T)s.f[F_GRADH][i];
-        r.q = (T)pres / (r.rho * r.rho);
+        r.q = div_t<T>((T)pres, r.rho * r.rho);
     } else {
         r.p = (T)pres;
         r.q = (T)(1.0 / (rho * rho));
     }
-    // the conductivity compares pressures: P itself, and the pair divides
-    if(TYPE != SPHGPU_GSPH && use_ac) r.q = (T)pres;
     fr[i] = r;
     if constexpr(TYPE == SPHGPU_GSPH) {
         if(gr) {
@@ -100,31 +99,74 @@ __global__ void __launch_bounds__(BLOCK) pack_force_kernel(State s, int n, int u
     }
 }
 
-// van Leer limiter (src/gsph/g_fluid_force.cpp:27-36).
-template <class T> __device__ __forceinline__ T van_leer(T a, T b)
-{
-    const T ab = a * b;
-    return ab <= T(0) ? T(0) : div_t<T>(T(2) * ab, a + b);
-}
+template <class T> struct Star {
+    T p, v;   // pressure and velocity of the contact
+    bool ok;  // (RiemannMath)
+};
 
-// HLL with Roe-averaged wave speeds (src/gsph/g_fluid_force.cpp:168-199);
-// states are (velocity along e, density, pressure, sound speed).
-template <class T> __device__ __forceinline__ void hll(const T L[4], const T R[4], T &pstar, T &vstar)
-{
-    const T sl = sqrt_t<T>(L[1]), sr = sqrt_t<T>(R[1]);
-    const T inv = div_t<T>(T(1), sl + sr);
-    const T ut = (sl * L[0] + sr * R[0]) * inv;
-    const T ct = (sl * L[3] + sr * R[3]) * inv;
-    const T s_l = fmin(L[0] - L[3], ut - ct);
-    const T s_r = fmax(R[0] + R[3], ut + ct);
-    const T c1 = L[1] * (s_l - L[0]);
-    const T c2 = R[1] * (s_r - R[0]);
-    const T c3 = div_t<T>(T(1), c1 - c2);
-    const T c4 = L[2] - L[0] * c1;
-    const T c5 = R[2] - R[0] * c2;
-    vstar = (c5 - c4) * c3;
-    pstar = (c1 * c5 - c2 * c4) * c3;
-}
+// Quotients, roots and the limiter of a pair's Riemann problem.  In FP32 the
+// plain ones take the hardware's reciprocal and root and note in `ok` whether
+// any lay outside the range where these are right (div_t and sqrt_t); the
+// pair is then computed again with the rescaled ones: one branch a pair, and
+// ahead of it the products and sums of all terms in one block, where the
+// compiler joins them into FMAs (with a branch at each of the 14 terms it
+// cannot, and the last bits are others).
+template <class T, bool RESCALED> struct RiemannMath {
+    static constexpr bool PLAIN = sizeof(T) == 4 && !RESCALED;
+    bool ok = true;
+    __device__ __forceinline__ T div(T a, T b)
+    {
+        if constexpr(PLAIN) {
+            const float r = __builtin_amdgcn_rcpf(b);
+            ok = ok & rcp_normal(r);
+            return a * r;
+        } else {
+            return a / b;
+        }
+    }
+    __device__ __forceinline__ T root(T x)
+    {
+        if constexpr(PLAIN) {
+            ok = ok & (x >= 1.17549435e-38f);
+            return __builtin_amdgcn_sqrtf(x);
+        } else {
+            return sqrt(x);
+        }
+    }
+    // van Leer limiter (src/gsph/g_fluid_force.cpp:27-36)
+    __device__ __forceinline__ T van_leer(T a, T b)
+    {
+        const T ab = a * b;
+        if constexpr(PLAIN) {
+            const float r = __builtin_amdgcn_rcpf(a + b);
+            ok = ok & ((ab <= 0.0f) | rcp_normal(r));
+            return ab <= T(0) ? T(0) : T(2) * ab * r;
+        } else {
+            return ab <= T(0) ? T(0) : T(2) * ab / (a + b);
+        }
+    }
+    // HLL with Roe-averaged wave speeds (src/gsph/g_fluid_force.cpp:168-199);
+    // states are (velocity along e, density, pressure, sound speed)
+    __device__ __forceinline__ Star<T> hll(const T L[4], const T R[4])
+    {
+        const T sl = root(L[1]), sr = root(R[1]);
+        const T inv = div(T(1), sl + sr);
+        const T ut = (sl * L[0] + sr * R[0]) * inv;
+        const T ct = (sl * L[3] + sr * R[3]) * inv;
+        const T s_l = fmin(L[0] - L[3], ut - ct);
+        const T s_r = fmax(R[0] + R[3], ut + ct);
+        const T c1 = L[1] * (s_l - L[0]);
+        const T c2 = R[1] * (s_r - R[0]);
+        const T c3 = div(T(1), c1 - c2);
+        const T c4 = L[2] - L[0] * c1;
+        const T c5 = R[2] - R[0] * c2;
+        Star<T> st;
+        st.v = (c5 - c4) * c3;
+        st.p = (c1 * c5 - c2 * c4) * c3;
+        st.ok = ok;
+        return st;
+    }
+};
 
 template <int D, class T> __device__ __forceinline__ T dotd(const T a[D], const T b[D])
 {
@@ -146,6 +188,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
     __shared__ double2 l_xy[SW][WAVE], l_zh[SW][WAVE];
     __shared__ ForceRec<T> l_f[SW][WAVE];
     __shared__ GradRec<T> l_g[GS ? SW : 1][GS ? WAVE : 1];
+    __shared__ T l_p[GS ? 1 : SW][GS ? 1 : WAVE];  // P_j, staged with the conductivity
     __shared__ PartsLds<NW> red;
     const int w = threadIdx.x / WAVE;
     const int lane = wave_lane();
@@ -192,7 +235,7 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
         const size_t gbase = (size_t)grp * a.wcap;
         const int gnc = uniform(a.gnc[grp]);
         const int nc = gnc & GNC_COUNT;
-        const GroupImage<D, T> img(box, gnc);
+        const GroupImage<D, T> img(box, gnc, xi);
         const int ntile = (nc + WAVE - 1) / WAVE;
         auto stage = [&](int tt) -> uint64_t {
             const size_t o = gbase + (size_t)tt * WAVE;
@@ -200,15 +243,17 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) {
                 double4 q = a.posrec[jl];
-                const int c = img.code(a.img, o + lane);
-                q.x = img.at(0, q.x, c);
-                if constexpr(D > 1) q.y = img.at(1, q.y, c);
-                if constexpr(D > 2) q.z = img.at(2, q.z, c);
+                q.x = img.at(0, q.x);
+                if constexpr(D > 1) q.y = img.at(1, q.y);
+                if constexpr(D > 2) q.z = img.at(2, q.z);
                 l_xy[w][lane] = make_double2(q.x, q.y);
                 l_zh[w][lane] = make_double2(q.z, q.w);
                 l_f[w][lane] = frec[jl];
-                if constexpr(GS)
+                if constexpr(GS) {
                     if(a.second_order) l_g[GS ? w : 0][lane] = ((const GradRec<T> *)a.grec)[jl];
+                } else {
+                    if(a.use_ac) l_p[w][lane] = (T)s.f[F_PRES][jl];
+                }
             }
             return valid ? stream_ld(a.ma + o + lane) : 0ull;
         };
@@ -264,53 +309,58 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                 for(int l = 0; l < D; ++l) e[l] = rij[l] * rinv;
                 const T ve_i = dotd<D, T>(vi, e);
                 const T ve_j = dotd<D, T>(vj, e);
-                T pstar, vstar;
-                if(a.second_order) {
-                    // MUSCL reconstruction (src/gsph/g_fluid_force.cpp:98-135)
-                    T R[4], L[4];
-                    const T di = T(0.5) * (T(1) - ci * dt * rinv);
-                    const T dj = T(0.5) * (T(1) - cj * dt * rinv);
-                    const T dv = ve_i - ve_j;
-                    const GradRec<T> &grj = l_g[GS ? w : 0][GS ? kc : 0];
-                    T gvi[D], gvj[D];
+                auto riemann = [&](auto rescaled) __attribute__((always_inline)) -> Star<T> {
+                    RiemannMath<T, rescaled()> rm;
+                    if(a.second_order) {
+                        // MUSCL reconstruction (src/gsph/g_fluid_force.cpp:98-135)
+                        T R[4], L[4];
+                        const T di = T(0.5) * (T(1) - ci * dt * rinv);
+                        const T dj = T(0.5) * (T(1) - cj * dt * rinv);
+                        const T dv = ve_i - ve_j;
+                        const GradRec<T> &grj = l_g[GS ? w : 0][GS ? kc : 0];
+                        T gvi[D], gvj[D];
 #pragma unroll
-                    for(int c = 0; c < D; ++c) {
-                        T si = gri.gv[3 * c] * e[0], sj = grj.gv[3 * c] * e[0];
+                        for(int c = 0; c < D; ++c) {
+                            T si = gri.gv[3 * c] * e[0], sj = grj.gv[3 * c] * e[0];
+#pragma unroll
+                            for(int l = 1; l < D; ++l) {
+                                si += gri.gv[3 * c + l] * e[l];
+                                sj += grj.gv[3 * c + l] * e[l];
+                            }
+                            gvi[c] = si;
+                            gvj[c] = sj;
+                        }
+                        const T dve_i = dotd<D, T>(gvi, e) * r;
+                        const T dve_j = dotd<D, T>(gvj, e) * r;
+                        R[0] = ve_i - rm.van_leer(dv, dve_i) * di;
+                        L[0] = ve_j + rm.van_leer(dv, dve_j) * dj;
+                        T gdi = gri.gd[0] * e[0], gdj = grj.gd[0] * e[0];
+                        T gpi = gri.gp[0] * e[0], gpj = grj.gp[0] * e[0];
 #pragma unroll
                         for(int l = 1; l < D; ++l) {
-                            si += gri.gv[3 * c + l] * e[l];
-                            sj += grj.gv[3 * c + l] * e[l];
+                            gdi += gri.gd[l] * e[l];
+                            gdj += grj.gd[l] * e[l];
+                            gpi += gri.gp[l] * e[l];
+                            gpj += grj.gp[l] * e[l];
                         }
-                        gvi[c] = si;
-                        gvj[c] = sj;
+                        const T dd = rhoi - rhoj;
+                        R[1] = rhoi - rm.van_leer(dd, gdi * r) * di;
+                        L[1] = rhoj + rm.van_leer(dd, gdj * r) * dj;
+                        const T dp = pi_ - pj;
+                        R[2] = pi_ - rm.van_leer(dp, gpi * r) * di;
+                        L[2] = pj + rm.van_leer(dp, gpj * r) * dj;
+                        R[3] = rm.root(rm.div(gam * R[2], R[1]));
+                        L[3] = rm.root(rm.div(gam * L[2], L[1]));
+                        return rm.hll(L, R);
+                    } else {
+                        const T R[4] = {ve_i, rhoi, pi_, ci};
+                        const T L[4] = {ve_j, rhoj, pj, cj};
+                        return rm.hll(L, R);
                     }
-                    const T dve_i = dotd<D, T>(gvi, e) * r;
-                    const T dve_j = dotd<D, T>(gvj, e) * r;
-                    R[0] = ve_i - van_leer(dv, dve_i) * di;
-                    L[0] = ve_j + van_leer(dv, dve_j) * dj;
-                    T gdi = gri.gd[0] * e[0], gdj = grj.gd[0] * e[0];
-                    T gpi = gri.gp[0] * e[0], gpj = grj.gp[0] * e[0];
-#pragma unroll
-                    for(int l = 1; l < D; ++l) {
-                        gdi += gri.gd[l] * e[l];
-                        gdj += grj.gd[l] * e[l];
-                        gpi += gri.gp[l] * e[l];
-                        gpj += grj.gp[l] * e[l];
-                    }
-                    const T dd = rhoi - rhoj;
-                    R[1] = rhoi - van_leer(dd, gdi * r) * di;
-                    L[1] = rhoj + van_leer(dd, gdj * r) * dj;
-                    const T dp = pi_ - pj;
-                    R[2] = pi_ - van_leer(dp, gpi * r) * di;
-                    L[2] = pj + van_leer(dp, gpj * r) * dj;
-                    R[3] = sqrt_t<T>(div_t<T>(gam * R[2], R[1]));
-                    L[3] = sqrt_t<T>(div_t<T>(gam * L[2], L[1]));
-                    hll(L, R, pstar, vstar);
-                } else {
-                    const T R[4] = {ve_i, rhoi, pi_, ci};
-                    const T L[4] = {ve_j, rhoj, pj, cj};
-                    hll(L, R, pstar, vstar);
-                }
+                };
+                Star<T> star = riemann(std::false_type());
+                if(__builtin_expect(!star.ok, 0)) star = riemann(std::true_type());
+                const T pstar = star.p, vstar = star.v;
                 const T fi = mj * pstar * rho2_inv_i;
                 const T fjj = FP64 ? mj * pstar / (rhoj * rhoj) : mj * pstar * fj.q;
                 T fdv = T(0);
@@ -338,10 +388,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     const T vsig = ci + cj - T(3) * wv;
                     pij = T(-0.5) * bal * alpha * vsig * wv * div_t<T>(T(2), rhoi + rhoj);
                 }
-                T ac = T(0), qj = fj.q;
+                T ac = T(0);
                 if(a.use_ac) {
-                    const T uj = fj.u, pj = fj.q;
-                    qj = TYPE == SPHGPU_DISPH ? div_t<T>(uj, pj) : div_t<T>(pj, rhoj * rhoj);
+                    // pressures of their own: where they are equal, P rebuilt
+                    // from a quotient leaves the square root of its rounding
+                    const T uj = fj.u, pj = l_p[GS ? 0 : w][GS ? 0 : kc];
                     const T vs = a.gravity ? fabs(over_r(vr)) : sqrt_t<T>(div_t<T>(T(2) * fabs(pi_ - pj), rhoi + rhoj));
                     ac = over_r((T)a.alpha_ac * mj * vs * (ui - uj) * dotd<D, T>(dwij, rij));
                 }
@@ -353,11 +404,11 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
                     const T pi_i = g2u_p_i * (mj * fj.u - gradhi);
                     const T fji = T(1) - fj.p * mu_inv_i;
                     ci_f = pi_i + T(0.5) * mj * pij;
-                    cj_f = mj * (g2u_i * qj * fji + T(0.5) * pij);
+                    cj_f = mj * (g2u_i * fj.q * fji + T(0.5) * pij);
                     de = pi_i * vdwi;
                 } else {
                     ci_f = mj * (p_rho2_i * gradhi + T(0.5) * pij);
-                    cj_f = mj * (qj * fj.p + T(0.5) * pij);
+                    cj_f = mj * (fj.q * fj.p + T(0.5) * pij);
                     de = mj * p_rho2_i * gradhi * vdwi;
                 }
 #pragma unroll
@@ -416,7 +467,7 @@ template <int D, int K, int TYPE, class T> static void launch_force(Ctx &c, cons
         rep.count = NCOUNTERS;
         c.hvs_partials = 0;
     }
-    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u, (int)a.use_ac,
+    hipLaunchKernelGGL((pack_force_kernel<D, TYPE, T>), dim3(grid), dim3(BLOCK), 0, c.stream, c.s, (int)c.n, use_u,
                        c.posrec, (ForceRec<T> *)c.pair_rec, (GradRec<T> *)c.grad_rec, rep);
     if(rep.dst) (void)hipEventRecord(c.ev_flags, c.stream);
     if(c.after_pack) c.after_pack_rc = c.after_pack(c);
@@ -452,7 +503,6 @@ int force_compute(Ctx &c)
     a.ngroups = c.ngroups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
-    a.img = c.tile_img;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

@@ -37,7 +37,6 @@ struct PreArgs {
     const int *cand;      // candidate tiles (Ctx::tile_cand)
     const uint64_t *ma;   // hit masks
     uint64_t *mn;         // narrowed masks (Ctx::tile_mn)
-    const int8_t *img;    // images (Ctx::tile_img)
     const int *gnc;
     int wcap;
     double gamma;
@@ -131,7 +130,7 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
     const int gnc = uniform(a.gnc[grp]);
-    const GroupImage<D, T> img(box, gnc);
+    const GroupImage<D, T> img(box, gnc, xi);
     const T h = (T)s.f[F_SML][ii];
     const Kern ker(h);
     Acc<T> rho;
@@ -141,9 +140,8 @@ __global__ void __launch_bounds__(BLOCK) pre_initial_kernel(State s, BoxDev box,
         const size_t o = gbase + (size_t)tt * WAVE;
         const int jl = stream_ld(a.cand + o + lane);
         if(jl >= 0) {
-            const int c = img.code(a.img, o + lane);
 #pragma unroll
-            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl], c);
+            for(int k = 0; k < D; ++k) l_r[w][lane].x[k] = img.at(k, s.f[F_X + k][jl]);
             l_r[w][lane].m = (T)s.f[F_MASS][jl];
         }
         return valid ? stream_ld(a.ma + o + lane) : 0ull;
@@ -195,7 +193,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
         double xi[D];
 #pragma unroll
         for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][ii];
-        const GroupImage<D, T> img(box, gnc);
+        const GroupImage<D, T> img(box, gnc, xi);
         const double mi = s.f[F_MASS][ii];
         const double Hs = s.f[F_SML][ii];  // search radius h_guess * ratio
         const double Hs2 = Hs * Hs;
@@ -228,9 +226,8 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                     const int jl = stream_ld(a.cand + o + lane);
                     if(jl >= 0) {
                         const double4 q = a.pm[jl];
-                        const int c = img.code(a.img, o + lane);
-                        l_xy[lane] = make_double2(img.at(0, q.x, c), D > 1 ? img.at(1, q.y, c) : 0.0);
-                        l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z, c) : 0.0, q.w);
+                        l_xy[lane] = make_double2(img.at(0, q.x), D > 1 ? img.at(1, q.y) : 0.0);
+                        l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z) : 0.0, q.w);
                                 }
                     return done ? 0ull : stream_ld(masks + o + lane);
                 };
@@ -302,9 +299,8 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
             const int jl = stream_ld(a.cand + o + lane);
             if(jl >= 0) {
                 PreRec<T> q = prec[jl];
-                const int c = img.code(a.img, o + lane);
 #pragma unroll
-                for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k], c);
+                for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k]);
                 l_r[w][lane] = q;
                 }
             return valid ? stream_ld((narrowed ? a.mn : a.ma) + o + lane) : 0ull;
@@ -345,7 +341,12 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 T rv = rij[0] * vij[0];
 #pragma unroll
                 for(int l = 1; l < D; ++l) rv += rij[l] * vij[l];
-                const T vs = ci_t + pj.c - div_t<T>(T(3) * rv, r);
+                // (in FP32 by the hardware reciprocal of a normal r: the only
+                // others are below 1.2e-38)
+                T w3 = T(3) * rv;
+                if constexpr(sizeof(T) == 4) w3 *= __builtin_amdgcn_rcpf(fmaxf(r, 1.17549435e-38f));
+                else w3 /= r;
+                const T vs = ci_t + pj.c - w3;
                 vsig_max = vs > vsig_max ? vs : vsig_max;
             }
             if(need_dv) {
@@ -522,7 +523,6 @@ static PreArgs make_args(Ctx &c)
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
     a.mn = c.tile_mn;
-    a.img = c.tile_img;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
     a.gamma = c.p.gamma;

@@ -67,7 +67,6 @@ struct SearchArgs {
     const int *num_groups;
     int *cand;           // group slabs of candidate tiles (Ctx::tile_cand)
     uint64_t *ma;        // hit masks per (tile, lane)
-    int8_t *img;         // the candidates' images (mixed; Ctx::tile_img)
     int *gnc;            // candidates per group, with the GNC_ flags
     int exact;           // FP64 pairs
     int wcap;            // slots per group slab and per staging buffer
@@ -119,6 +118,9 @@ __device__ __forceinline__ bool box_near(const BoxDev &box, const ChunkBox &b, c
     }
     return d2 <= H2 * (1.0 + 1e-6);
 }
+
+// Axis k of a candidate's image code (two signed bits to an axis).
+__device__ __forceinline__ int image_sign(int code, int k) { return code << (30 - 2 * k) >> 30; }
 
 // A particle's search record through the scalar cache (i wave-uniform; the
 // records are not written by this kernel).
@@ -355,7 +357,6 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 #pragma unroll
                     for(int k = 0; k < D; ++k) code[v] |= (near_image(box, k, gc[k], x[v][k]) & 3) << (2 * k);
                 }
-                if(!a.exact) stream_st(a.img + gbase + (size_t)(tt + v) * WAVE + lane, (int8_t)code[v]);
                 moved |= code[v];
             }
         }
@@ -368,7 +369,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 #pragma unroll
                 for(int v = 0; v < V; ++v)
 #pragma unroll
-                    for(int k = 0; k < D; ++k) x[v][k] = GroupImage<D, float>::moved(box, k, x[v][k], code[v]);
+                    for(int k = 0; k < D; ++k) x[v][k] = near_position(box, k, gc[k], x[v][k]);
                 any = false;
             }
         }
@@ -385,7 +386,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
 #pragma unroll
                 for(int v = 0; v < N; ++v)
 #pragma unroll
-                    for(int k = 0; k < D; ++k) s[v][k] = GroupImage<D, double>::sign(code[V0 + v], k) * box.len[k];
+                    for(int k = 0; k < D; ++k) s[v][k] = image_sign(code[V0 + v], k) * box.len[k];
             }
             for(int i0 = 0; i0 < cnt; i0 += U) {
 #pragma clang fp contract(off)
@@ -702,7 +703,6 @@ static SearchArgs base_args(Ctx &c)
     a.num_groups = c.num_groups;
     a.cand = c.tile_cand;
     a.ma = c.tile_ma;
-    a.img = c.tile_img;
     a.exact = c.p.precision == SPHGPU_FP64;
     a.gnc = c.tile_nc;
     a.wcap = c.tile_wcap;
@@ -782,17 +782,14 @@ int search_alloc(Ctx &c)
         if(c.tile_cand) (void)hipFree(c.tile_cand);
         if(c.tile_ma) (void)hipFree(c.tile_ma);
         if(c.tile_mn) (void)hipFree(c.tile_mn);
-        if(c.tile_img) (void)hipFree(c.tile_img);
         if(c.tile_nc) (void)hipFree(c.tile_nc);
         c.tile_cand = nullptr;
         c.tile_ma = c.tile_mn = nullptr;
-        c.tile_img = nullptr;
         c.tile_nc = nullptr;
         const size_t slots = (size_t)groups * wcap;
         SPHGPU_HIP(hipMalloc(&c.tile_cand, slots * sizeof(int)));
         SPHGPU_HIP(hipMalloc(&c.tile_ma, slots * sizeof(uint64_t)));
         SPHGPU_HIP(hipMalloc(&c.tile_mn, slots * sizeof(uint64_t)));
-        SPHGPU_HIP(hipMalloc(&c.tile_img, slots));
         SPHGPU_HIP(hipMalloc(&c.tile_nc, groups * sizeof(int)));
         c.tile_groups_cap = groups;
     }
@@ -809,7 +806,7 @@ int search_alloc(Ctx &c)
 // summed, and sphgpu_neighbor_sets compares.
 template <int D, class T, bool FORCE>
 __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, const int2 *groups, int ngroups, const int *gnc,
-                                                       const int *cand, const uint64_t *ma, const int8_t *images, int wcap, int cap,
+                                                       const int *cand, const uint64_t *ma, int wcap, int cap,
                                                        int *list, int *cnt)
 {
     const int grp = xcd_block() * (BLOCK / WAVE) + (int)(threadIdx.x / WAVE);
@@ -819,13 +816,13 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
     const int i = gr.x + lane;
     if(i >= gr.y) return;
     const size_t gbase = (size_t)grp * wcap;
-    const GroupImage<D, T> img(box, gnc[grp]);
     const int nc = gnc[grp] & GNC_COUNT;
     const int ntile = (nc + WAVE - 1) / WAVE;
     const size_t lb = list_base(i, cap);
     double xi[D];
 #pragma unroll
     for(int k = 0; k < D; ++k) xi[k] = s.f[F_X + k][i];
+    const GroupImage<D, T> img(box, gnc[grp], xi);
     const double h = s.f[F_SML][i], h2 = h * h;
     int wf = 0;  // entries written (at most cap)
     for(int k = 0; k < WAVE; ++k) {
@@ -833,10 +830,10 @@ __global__ void __launch_bounds__(BLOCK) record_kernel(State s, BoxDev box, cons
             if(t + k * ntile >= nc) break;
             const size_t o = gbase + (size_t)t * WAVE;
             if(!((ma[o + lane] >> k) & 1ull)) continue;
-            const int j = cand[o + k], c = img.code(images, o + k);
+            const int j = cand[o + k];
             double xj[D], d[D];
 #pragma unroll
-            for(int q = 0; q < D; ++q) xj[q] = img.at(q, s.f[F_X + q][j], c);
+            for(int q = 0; q < D; ++q) xj[q] = img.at(q, s.f[F_X + q][j]);
             const double r2 = img.sep2(xi, xj, d);
             if constexpr(!FORCE) {
                 if(!(r2 < h2)) continue;
@@ -860,7 +857,7 @@ template <int D, class T> static void launch_record_t(Ctx &c, int *list, int *cn
 {
     const auto kernel = force ? record_kernel<D, T, true> : record_kernel<D, T, false>;
     hipLaunchKernelGGL(kernel, dim3(group_grid(c)), dim3(BLOCK), 0, c.stream, c.s, make_box(c), c.groups, c.ngroups,
-                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_img, c.tile_wcap, c.cap, list, cnt);
+                       c.tile_nc, c.tile_cand, c.tile_ma, c.tile_wcap, c.cap, list, cnt);
 }
 
 template <int D> static void launch_record(Ctx &c, int *list, int *cnt, bool force)

@@ -39,35 +39,37 @@ namespace sphgpu {
 // are the reference's to the last bit and the sums no further from 64-bit
 // values (a coordinate moved by L first is rounded before the subtraction, and
 // doubled that error).  Mixed pairs, whose separations are rounded to FP32
-// next, subtract a coordinate that was moved when it was staged: the search
-// found the image (the same one for all of the group's pairs) and has written
-// it, a signed two-bit code per axis in Ctx::tile_img (rollout gradient of
-// 262,144 particles 34.1 ms, with a shift in each pair 36.3).
+// next, subtract a coordinate that was moved when it was staged, to the image
+// nearest to any one particle of the group: it is the same one for all of its
+// pairs (rollout gradient of 262,144 particles 34.0 ms, with a shift in each
+// pair 36.3).
 template <int D, class T> struct GroupImage {
     static constexpr bool EXACT = sizeof(T) == 8;
     const BoxDev &box;
-    int flags;  // GNC_WRAP, or GNC_SHIFT's bits, or none
-    bool shift;
-    __device__ __forceinline__ GroupImage(const BoxDev &b, int gnc) : box(b)
+    int flags;     // GNC_WRAP, or GNC_SHIFT's bits, or none
+    BoxDev pairs;  // mixed: the box, on with GNC_WRAP only
+    bool move;     // mixed: some candidates are moved
+    double x0[D];  // to beside this particle, the first with no NaN coordinate (those that have one hit nothing)
+    __device__ __forceinline__ GroupImage(const BoxDev &b, int gnc, const double xi[D]) : box(b), pairs(b)
     {
         flags = b.on ? gnc & (GNC_WRAP | GNC_SHIFT) : 0;
-        shift = flags & GNC_SHIFT;
-    }
-    static __device__ __forceinline__ double sign(int code, int k) { return (double)(code << (30 - 2 * k) >> 30); }
-    static __device__ __forceinline__ double moved(const BoxDev &box, int k, double x, int code)
-    {
-        return __builtin_fma(-sign(code, k), box.len[k], x);
-    }
-    // mixed: the code of the candidate at slot o
-    __device__ __forceinline__ int code(const int8_t *img, size_t o) const
-    {
-        return !EXACT && shift ? stream_ld(img + o) : 0;
+        pairs.on = b.on && (gnc & GNC_WRAP);
+        move = b.on && (gnc & GNC_SHIFT);
+        if constexpr(!EXACT) {
+            bool in = true;
+#pragma unroll
+            for(int k = 0; k < D; ++k) in = in && xi[k] == xi[k];
+            const uint64_t live = ballot(in);
+            const int first = live ? (int)__builtin_ctzll(live) : 0;
+#pragma unroll
+            for(int k = 0; k < D; ++k) x0[k] = uniform_d(__shfl(xi[k], first, WAVE));
+        }
     }
     // axis k of a candidate's position, as it is staged
-    __device__ __forceinline__ double at(int k, double x, int code) const
+    __device__ __forceinline__ double at(int k, double x) const
     {
         if constexpr(EXACT) return x;
-        else return shift ? moved(box, k, x, code) : x;
+        else return move ? near_position(box, k, x0[k], x) : x;
     }
     // r_ij and its square of a pair, the position of j as it was staged
     __device__ __forceinline__ double sep2(const double xi[D], const double xj[D], double d[D]) const
@@ -75,7 +77,9 @@ template <int D, class T> struct GroupImage {
 #pragma clang fp contract(off)
 #pragma unroll
         for(int k = 0; k < D; ++k) d[k] = xi[k] - xj[k];
-        if(EXACT ? flags : flags & GNC_WRAP) {
+        if constexpr(!EXACT) {
+            min_image<D>(pairs, d);
+        } else if(flags) {
             if(flags & GNC_WRAP) {
                 min_image<D>(box, d);
             } else {
