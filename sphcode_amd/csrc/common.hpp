@@ -4,7 +4,8 @@
 // Distances that decide set membership (neighbour candidates, density
 // cut-off, force cut-off, cell pruning) are evaluated in the reference's
 // operation order with FP contraction disabled, so FP64 sets match the
-// reference's exactly.  Sums over pairs may be contracted.
+// reference's exactly (mixed precision moves the candidates of pairs across a
+// periodic face by L first).  Sums over pairs may be contracted.
 #pragma once
 
 #include <hip/hip_runtime.h>

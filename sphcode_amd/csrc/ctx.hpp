@@ -103,11 +103,11 @@ constexpr int GNC_WRAP = 1 << 30, GNC_SHIFT_AXIS = 1 << 27, GNC_SHIFT = 7 * GNC_
 // reads one FP64 (x, y, z, h) record for the cut and one record of the pair
 // fields (rounded to FP32 in mixed mode) instead of one load per field, and
 // divides by nothing of particle j's alone: `q` is u/P (DISPH), P/rho^2
-// (SSPH) or 1/rho^2 (GSPH), but P where conductivity compares pressures; `p`
-// is grad-h (DISPH, SSPH) or P (GSPH).  The sizes of
-// the records that lie in LDS are odd multiples of 16 bytes: lanes that read
-// different records of a tile then spread over all banks (a stride of 64
-// bytes would use a quarter of them).
+// (SSPH) or 1/rho^2 (GSPH, mixed only: FP64 pairs divide); `p` is grad-h
+// (DISPH, SSPH) or P (GSPH).  The conductivity's P_j is staged beside the
+// record.  The sizes of the records that lie in LDS are odd multiples of 16
+// bytes: lanes that read different records of a tile then spread over all
+// banks (a stride of 64 bytes would use a quarter of them).
 template <class T> struct __align__(16) ForceRec {
     T hinv, m, rho, p, c, alpha, bal, u, q;  // the kernels need 1/h only
     T v[3];

@@ -39,9 +39,11 @@
 // 3,480 -> 800 us; Evrard, 2^20 particles, leaf 32, alone 1,440 -> 780 us
 // (vector instructions 4.0e8 -> 2.5e8).
 //
-// The sets are the reference's; the reference then sorts each list by
-// distance (src/bhtree.cpp:120-124) and stops at the first r >= h, whereas
-// the pair passes here test r < h on the unsorted set -- the same set.
+// The sets are the reference's (in mixed precision but for pairs across a
+// periodic face that are closer to the cut than the rounding of a position);
+// the reference then sorts each list by distance (src/bhtree.cpp:120-124) and
+// stops at the first r >= h, whereas the pair passes here test r < h on the
+// unsorted set -- the same set.
 //
 // The combined search takes H_ij = max(R_i, R_j) with the gather radii R,
 // so that one search serves both the pre-interaction (which keeps the pairs
@@ -299,8 +301,9 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(OCC_
     // Periodic box: every lane's minimum image of a candidate that can be a
     // hit is the one nearest to the group's centre, if the group and its
     // reach span less than half the box; its shift by L, 0 or -L is then
-    // settled once (and added to the pairs' differences, as a minimum image
-    // does).  Otherwise every pair takes its own minimum image.  The pair
+    // settled once: with FP64 pairs it is added to the pairs' differences, as
+    // a minimum image does, with mixed ones the candidate is moved, as their
+    // passes do.  Otherwise every pair takes its own minimum image.  The
     // passes read which of it was so from the flags beside the count.
     bool wrap = false;
     if(box.on) {
