@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                         const double4 q = a.pm[jl];
                         l_xy[lane] = make_double2(img.at(0, q.x), D > 1 ? img.at(1, q.y) : 0.0);
                         l_zm[lane] = make_double2(D > 2 ? img.at(2, q.z) : 0.0, q.w);
-                                }
+                    }
                     return done ? 0ull : stream_ld(masks + o + lane);
                 };
                 auto npair = [&](int kc) -> bool {
@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
 #pragma unroll
                 for(int k = 0; k < D; ++k) q.x[k] = img.at(k, q.x[k]);
                 l_r[w][lane] = q;
-                }
+            }
             return valid ? stream_ld((narrowed ? a.mn : a.ma) + o + lane) : 0ull;
         };
         auto fpair = [&](int kc) {
@@ -341,11 +341,15 @@ __global__ void __launch_bounds__(BLOCK) pre_kernel(State s, BoxDev box, int n, 
                 T rv = rij[0] * vij[0];
 #pragma unroll
                 for(int l = 1; l < D; ++l) rv += rij[l] * vij[l];
-                // (in FP32 by the hardware reciprocal of a normal r: the only
-                // others are below 1.2e-38)
+                // (in FP32 by the hardware reciprocal, of a separation below
+                // its normal range after both are scaled by 2^64)
                 T w3 = T(3) * rv;
-                if constexpr(sizeof(T) == 4) w3 *= __builtin_amdgcn_rcpf(fmaxf(r, 1.17549435e-38f));
-                else w3 /= r;
+                if constexpr(sizeof(T) == 4) {
+                    const float up = r < 1.17549435e-38f ? 0x1p64f : 1.0f;
+                    w3 = w3 * up * __builtin_amdgcn_rcpf(r * up);
+                } else {
+                    w3 /= r;
+                }
                 const T vs = ci_t + pj.c - w3;
                 vsig_max = vs > vsig_max ? vs : vsig_max;
             }
