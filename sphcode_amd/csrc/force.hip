@@ -278,7 +278,15 @@ __global__ void __launch_bounds__(BLOCK) force_kernel(State s, BoxDev box, int n
             } else {
                 if(!(r2 < hmax * hmax) || r2 == 0.0) return;
                 r = __builtin_amdgcn_sqrtf((float)r2);
-                if(__builtin_expect((float)r2 < 1.17549435e-38f, 0)) r = gather_r_f32(r2);  // denormal or zero in FP32
+                if(__builtin_expect((float)r2 < 1.17549435e-38f, 0)) {
+                    // denormal or zero in FP32: direction and velocity along it
+                    // do not depend on the length, which is raised to 2^-62
+                    // (nothing against h)
+                    const int up = -62 - (ilogb(r2) >> 1);
+#pragma unroll
+                    for(int l = 0; l < D; ++l) d[l] = ldexp(d[l], up);
+                    r = gather_r_f32(ldexp(r2, 2 * up));
+                }
                 rinv = __builtin_amdgcn_rcpf(r);
             }
             ++used;
